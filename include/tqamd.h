@@ -125,7 +125,7 @@ int tq_table_quantize_host(const void *table_host, const float *r, long long n, 
  *               packed_row_stride = capacity (the chunk list of generation_test_v2.py:109-126
  *               kept as one buffer).
  *   workspace   device memory of tq_workspace_bytes(1) bytes, 64-byte aligned, or NULL: the counters from which
- *               the blocks of a large single-row job of 16-bit elements draw runs of tiles in the order in which
+ *               the blocks of a large job of 16-bit elements draw runs of tiles in the order in which
  *               they become free (compute units that run slower take fewer, and all blocks end together; the
  *               results are the same bytes).  Same contract as the workspace of tq_decompress below: zero before
  *               its first use, left zero by every launch that completes, never shared by launches that can

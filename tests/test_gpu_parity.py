@@ -269,6 +269,24 @@ def test_strided_inputs_and_outputs(pkg, oracle):
 # ---------------------------------------------------------------------------------------------
 # TurboQuantV3 orchestration
 # ---------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("rows,tokens,window,dim", [(2, 31, 1, 128), (2, 32, 1, 128), (3, 33, 7, 128), (5, 64, 64, 128), (16, 135, 64, 128),
+                                                    (128, 607, 128, 128), (7, 1000, 0, 128), (3, 4099, 128, 128), (2, 65537, 31, 128), (3, 66, 8, 64)])
+def test_rows_of_a_token_slice_give_the_bytes_of_a_dense_tensor(pkg, rows, tokens, window, dim):
+    """Rows laid end to end in the pipelined compress path (tiles that span two rows, a partial last tile, the job with and
+    without ticket counters, into a dense result and into a packed store with room left in every row): the bytes are the same."""
+    x = outlier_kv((1, rows, tokens + window, dim), seed=rows * tokens, dtype=torch.bfloat16).to(DEV)
+    comp = pkg.MSECompressor(dim, 4, seed=7, device=DEV)
+    part = x[:, :, :tokens]
+    want = comp.compress(part.contiguous())
+    got = comp.compress(part)
+    assert torch.equal(got["idx_bytes"], want["idx_bytes"]) and torch.equal(got["vec_norms"], want["vec_norms"])
+    idx = torch.zeros((1, rows, tokens + 10, dim // 2), dtype=torch.uint8, device=DEV)
+    nrm = torch.zeros((1, rows, tokens + 10), dtype=torch.float16, device=DEV)
+    comp.compress_into(part, idx[:, :, 4:4 + tokens], nrm[:, :, 4:4 + tokens])
+    assert torch.equal(idx[:, :, 4:4 + tokens], want["idx_bytes"]) and torch.equal(nrm[:, :, 4:4 + tokens], want["vec_norms"])
+    assert not idx[:, :, :4].any() and not idx[:, :, 4 + tokens:].any() and not nrm[:, :, :4].any() and not nrm[:, :, 4 + tokens:].any()
+
+
 def test_v3_residual_window_against_reference(pkg, oracle, golden):
     """K4/V2, window 16, layer 5 of 36, fp16 [2,2,40,128]: dict schema, split, packed bytes and the
     full-length fp16 outputs against the reference's."""

@@ -459,8 +459,8 @@ def compress_into(states: torch.Tensor, table: torch.Tensor, bits: int,
     check_table(table, states.shape[-1], bits)
     with _on(states.device):
         stream = _stream_handle(states.device)
-        # counters only where the kernel can use them (a large single-row job): a one-token append needs no look-up
-        ws = _workspace(states.device, stream) if rows == 1 and tokens >= 65536 else 0
+        # counters only where the kernel can use them (a large job): a one-token append needs no look-up
+        ws = _workspace(states.device, stream) if rows * tokens >= 65536 else 0
         rc = lib().tq_compress(states.data_ptr(), dtype_code(states.dtype), rows, tokens, row_stride, token_stride,
                                table.data_ptr(), states.shape[-1], bits,
                                idx_bytes.data_ptr(), vec_norms.data_ptr(), prs, ws, stream)

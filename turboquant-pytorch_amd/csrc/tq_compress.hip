@@ -105,7 +105,7 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
     if (n_tiles == 0u) return;    // an empty job of a batch: its table may be NULL, and its counters stay untouched (zero)
     const uint32_t n_full = job.n_vec / 32u;
     const bool one_row = job.tokens >= job.n_vec;
-    // Which tiles a block works on.  Single-row jobs of 16-bit elements (the pipelined path below) hand their tiles out
+    // Which tiles a block works on.  Jobs of 16-bit elements (the pipelined path below) hand their tiles out
     // as tickets of 2^tshift consecutive tiles: block b starts with ticket b; its later tickets are b + grid, b + 2 grid, ...
     // (fixed assignment) or, with a workspace, come from a counter in device memory in the order in which the blocks
     // ask, so that compute units that run slower than others (the dies of this part do not all run at one pace) take
@@ -113,7 +113,16 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
     // counter[1] = blocks of the job that are done; the last block to finish sets both back to zero, so a workspace
     // that was zero before a launch is zero after it (the contract of the decompress kernel's counters).
     // Every other job walks single tiles blockIdx.x, blockIdx.x + grid, ...
-    const bool ticket_job = ELEM == 2 && one_row && job.token_stride < (1ll << 26);
+    // Several rows (a token slice of a [B, H, S, D] tensor, a window left behind): a tile is 32 vectors of the rows laid
+    // end to end, so with at least 32 tokens a row it touches two rows at most; vectors of the second one lie `row_skip`
+    // bytes further than the tile's own stride says.  The loads take 32-bit offsets from the tile's first vector, which
+    // bounds token_stride and row_skip; rows that overlap or lie further apart take the plain loop.
+    // Bound: as for one row (memory and the power limit); the plain loop it replaces for these jobs re-divided every
+    // lane's index and waited for each tile.  4-bit bf16, all but the last 128 tokens of a row: 8 rows of 32768 tokens
+    // 27.9 -> 25.8 us, 32 such rows 105 -> 92 us, 128 rows of 8192 100 -> 91 us (a dense tensor of that size: 91 us).
+    const long long row_skip = one_row ? 0 : job.row_stride - (long long)job.tokens * job.token_stride;
+    const bool ticket_job = ELEM == 2 && job.token_stride < (1ll << 26) &&
+                            (one_row || (job.tokens >= 32u && row_skip >= 0 && row_skip < (1ll << 31)));
     // (a ticket has to outlast the pipeline's depth: the first drawn ticket is published one iteration after the start)
     uint32_t *counter = workspace && (1u << tshift) > (uint32_t)TQ_RING ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr;
     auto report_done = [&]() {      // once per block of a non-empty job, after its last draw has been answered
@@ -364,7 +373,7 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
     if (!pipelined) load_tables();
     if (pipelined) {
         if constexpr (ELEM == 2) {
-            // Single-row jobs with 16-bit elements (the KV-cache case): a software pipeline over this block's full
+            // Jobs with 16-bit elements (the KV-cache case): a software pipeline over this block's full
             // tiles t_0 .. t_{m-1}.  Tiles travel from memory straight into a ring of RING LDS slots
             // (global_load_lds_dwordx4: no registers, no LDS write instructions); iteration j
             //   waits for its own loads of t_j (issued RING-1 iterations ago) and passes the barrier: t_j is complete
@@ -435,18 +444,36 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
 #pragma unroll
             for (int i = 2; i <= P; ++i) q[i] = advance(q[i - 1]);     // (counter mode: tickets hold more than P tiles, no draw here)
             if (counter) draw();                // ticket 1: in LDS at the end of the first iteration, read per_ticket - P iterations later
+            // Row and token of a tile's first vector v, on the scalar unit: with inv_tokens = floor(2^32 / tokens) + 1 the high
+            // half of v * inv_tokens is v / tokens or one more (v < 2^31); one row: inv_tokens = 0 and the row is 0.
+            const uint32_t inv_tokens = one_row ? 0u : 0xffffffffu / job.tokens + 1u;
+            auto row_of = [&](uint32_t v) -> uint32_t {
+                const uint32_t r = (uint32_t)(((uint64_t)v * inv_tokens) >> 32);
+                return r * job.tokens > v ? r - 1u : r;
+            };
             auto issue = [&](uint32_t slot, uint32_t tl) {
                 tl = tl < n_full ? tl : n_full - 1u;
-                const uint64_t a = (uint64_t)(uintptr_t)job.states + (uint64_t)tl * (uint64_t)(32 * job.token_stride);
+                const uint32_t row = row_of(tl * 32u);
+                const uint64_t a = (uint64_t)(uintptr_t)job.states + (uint64_t)tl * (uint64_t)(32 * job.token_stride) + (uint64_t)row * (uint64_t)row_skip;
                 // (the builtin returns int: widen through uint32_t, or the low half is sign-extended into the high one)
                 const uint32_t a_hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
                 const uint32_t a_lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
                 const uint64_t base = ((uint64_t)a_hi << 32) | (uint64_t)a_lo;
+                // vectors of the tile that belong to its first row (all of them, unless a row ends inside the tile)
+                const uint32_t mine = one_row ? 32u : (row + 1u) * job.tokens - tl * 32u;
+                uint32_t off[NLOAD];
+#pragma unroll
+                for (int j = 0; j < NLOAD; ++j) off[j] = src_off[j];
+                if (mine < 32u) {       // uniform
+#pragma unroll
+                    for (int j = 0; j < NLOAD; ++j)
+                        if ((wave * NLOAD + j) * VEC_PER_LOAD + ld_vec >= mine) off[j] += (uint32_t)row_skip;
+                }
 #pragma unroll
                 for (int j = 0; j < NLOAD; ++j) {
                     const uint32_t dst = lds_wave + slot * (uint32_t)STAGE + j * 1024u;
                     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                                 :: "s"(dst), "v"(src_off[j]), "s"(base) : "memory", "m0");
+                                 :: "s"(dst), "v"(off[j]), "s"(base) : "memory", "m0");
                 }
             };
             // operand addresses inside a slot, in this wave's step order
@@ -460,8 +487,15 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
 
             // output addresses: a base per tile that is the same in every lane, plus a per-lane constant
             const uint32_t cd_lane = n * (8 * NB) + lane_slot, nd_lane = n;
+            const uint32_t slot_skip = job.packed_row_stride - job.tokens;     // packed slots between the rows (one row: not looked at)
             auto store_tile = [&](uint32_t tl, const uint32_t (&w)[NW], float nrm_of_tile) {
-                store(job.idx_bytes + (size_t)tl * (32u * (8 * NB)) + cd_lane, job.vec_norms + norm_slot((size_t)tl * 32u + nd_lane), w, nrm_of_tile);
+                if (one_row) {
+                    store(job.idx_bytes + (size_t)tl * (32u * (8 * NB)) + cd_lane, job.vec_norms + norm_slot((size_t)tl * 32u + nd_lane), w, nrm_of_tile);
+                } else {
+                    const uint32_t row = row_of(tl * 32u), v = tl * 32u + n;
+                    const uint32_t slot = v + (row + (v >= (row + 1u) * job.tokens ? 1u : 0u)) * slot_skip;
+                    store(job.idx_bytes + (size_t)slot * (8 * NB) + lane_slot, job.vec_norms + norm_slot(slot), w, nrm_of_tile);
+                }
             };
 
             auto scale_from_shares = [&](uint32_t par) {
@@ -618,7 +652,7 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
             buf = 0u;
         }
     } else if (!ticket_job && tile < n_full) {
-        // General case (several rows with their own stride, fp32 elements).  Iteration k: start the
+        // General case (fp32 elements, rows of fewer than 32 tokens or too far apart).  Iteration k: start the
         // loads of tile k+1, barrier (publishes buffer k, and everyone has finished reading buffer
         // k-1), compute and store tile k, then park tile k+1 into the other buffer.  Loads, stores
         // and the wait for the loads sit in one straight line, unpredicated: s_waitcnt vmcnt(#stores).
