@@ -375,6 +375,42 @@ int tq_attend_step(const void *queries, int q_dtype, long long rows, int group, 
                    float *q_rot, float *part_w, float *partial, int splits,
                    void *out, int out_dtype, void *stream);
 
+/*
+ * The same decode step for 16-bit elements and head dimensions 64, 96, 128 and 256 (1-bit codes: 128 only), one launch per
+ * call.  A layer is described by a record that stays the same from step to step:
+ *   k_win, v_win          window buffers: row r, slot s at element r * win_stride + s * head_dim (win_stride a multiple of 8)
+ *   k_idx .. v_norms      packed stores of packed_row_stride slots per row
+ *   table_k, table_v      codec tables (device); pi_v: the value codec's rotation, float32 [head_dim, head_dim] row-major
+ *   rows                  batch x kv heads (<= 65535); dtype: TQ_F16 or TQ_BF16, of windows, new vectors, queries and results
+ * Pointers are 16-byte aligned (packed stores: as tq_compress asks), norms 2-byte aligned.
+ *
+ * tq_decode_append: as tq_append_token (same bytes as tq_compress with rows x 1 token).
+ * tq_decode_attend: softmax(scale * q K^T) V of one query token per head ([rows, group, head_dim], group <= 16) over the first
+ *   `tokens` packed slots of every row and its window slots win_first .. win_first + n_win - 1 (n_win <= 512; not both
+ *   empty).  scratch: tq_decode_scratch_floats() float32 values (scratch_size: how many there are; TQ_ERR_CAPACITY if
+ *   too few), arrived: `rows` counters, zero before the first use and left zero by every launch that completes; neither
+ *   is shared by launches that can overlap in time.
+ * tq_decode_supported: 1 if these calls take the combination, 0 otherwise.
+ */
+typedef struct tq_decode_layer {
+    void *k_win, *v_win;
+    uint8_t *k_idx;
+    uint16_t *k_norms;
+    uint8_t *v_idx;
+    uint16_t *v_norms;
+    const void *table_k, *table_v;
+    const float *pi_v;
+    long long win_stride, packed_row_stride, rows;
+    int head_dim, dtype, bits_k, bits_v;
+} tq_decode_layer;
+
+int tq_decode_supported(int head_dim, int dtype, int bits_k, int bits_v);
+long long tq_decode_scratch_floats(long long rows, int group, int head_dim, long long tokens, long long n_win);
+int tq_decode_attend(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
+                     long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, void *out, void *stream);
+int tq_decode_append(const tq_decode_layer *layer, const void *k_new, const void *v_new, long long k_new_stride, long long v_new_stride,
+                     long long evict, long long put, long long packed_slot, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -775,3 +775,61 @@ def test_append_token_and_attend_step_through_the_c_abi(pkg, oracle):
     ref = torch.softmax(torch.einsum("rgd,rtd->rgt", q.double(), K) * scale, -1) @ V
     err = float((outs[0].double() - ref).norm() / ref.norm())
     assert err < 6e-3, err
+
+
+def _codes(idx_bytes, bits, dim):
+    """[.., G] packed bytes -> [.., dim] codes (most significant code of a byte first)."""
+    ipb = 8 // bits
+    shifts = torch.arange(ipb - 1, -1, -1, device=idx_bytes.device, dtype=torch.uint8) * bits
+    return ((idx_bytes.unsqueeze(-1) >> shifts) & ((1 << bits) - 1)).flatten(-2)[..., :dim].long()
+
+
+@pytest.mark.parametrize("dim,bits,group,dtype", [(64, (6, 4), 4, torch.float16), (64, (4, 2), 1, torch.bfloat16), (96, (4, 2), 7, torch.bfloat16),
+                                                  (96, (8, 8), 2, torch.float16), (96, (2, 3), 16, torch.bfloat16), (128, (4, 2), 4, torch.bfloat16),
+                                                  (128, (1, 1), 3, torch.float16), (128, (8, 4), 16, torch.bfloat16), (256, (4, 2), 5, torch.bfloat16),
+                                                  (256, (8, 8), 12, torch.float16), (256, (2, 4), 2, torch.bfloat16)])
+def test_one_launch_decode_step_against_float64(pkg, dim, bits, group, dtype):
+    """tq_decode_attend at the edges of its tiles: histories of 0, 1, 31 ... tokens (partial runs, one and several splits of a
+    row), windows of 1 to 512 tokens, one and many rows; float64 attention over the decoded store and the window.  The result
+    is rounded to the element type (2^-9 or 2^-12 relative, 0.29 of that in the mean square per ulp) and carries the 2^-12
+    roundings of the query term (times logits of about 10 here) and of the weights: 6e-3 and 3e-3 leave a factor of two."""
+    dec = lambda comp, idx, nrm, n: ((comp.centroids.double()[_codes(idx[:, :, :n].contiguous(), comp.bits, dim)] @ comp.Pi.double())
+                                     * nrm[:, :, :n].double().unsqueeze(-1))
+    g = torch.Generator().manual_seed(dim + group)
+    for rows, tokens, window in ((1, 0, 1), (2, 1, 16), (3, 31, 33), (1, 64, 128), (5, 513, 7), (1, 3001, 512), (40, 700, 64), (300, 90, 8)):
+        cache = pkg.V3Cache(bits[0], bits[1], residual_window=window, n_layers=40)
+        k = (torch.randn(1, rows, tokens + window, dim, generator=g) * torch.exp(0.5 * torch.randn(dim, generator=g))).to(dtype).to(DEV)
+        v = torch.randn(1, rows, tokens + window, dim, generator=g).to(dtype).to(DEV)
+        cache.append(k, v, 8)
+        for step in range(2):
+            q = torch.randn(1, rows * group, 1, dim, generator=g).to(dtype).to(DEV)
+            out = cache.attend(q, 8).double().reshape(rows, group, dim)
+            st = cache._stores[8]
+            n = st.n_compressed
+            kw, vw = (t.double() for t in st.window())
+            K = (torch.cat([dec(st.comp.key_compressor, st.k_idx, st.k_nrm, n), kw], 2) if n else kw).reshape(rows, -1, dim)
+            V = (torch.cat([dec(st.comp.val_compressor, st.v_idx, st.v_nrm, n), vw], 2) if n else vw).reshape(rows, -1, dim)
+            ref = torch.softmax(torch.matmul(q.double().reshape(rows, group, dim), K.transpose(1, 2).contiguous()) * dim ** -0.5, -1) @ V
+            err = float((out - ref).norm() / ref.norm())
+            assert err < (6e-3 if dtype == torch.bfloat16 else 3e-3), (rows, tokens, window, step, err)
+            cache.append(k[:, :, :1].contiguous(), v[:, :, :1].contiguous(), 8)
+
+
+@pytest.mark.parametrize("dim", [64, 96, 128, 256])
+@pytest.mark.parametrize("bits", [(4, 2), (8, 3), (6, 4)])
+def test_one_launch_append_stores_the_bytes_of_compress(pkg, dim, bits):
+    """tq_decode_append against MSECompressor.compress on the evicted tokens (1 to 70 rows: full and partial tiles of rows)."""
+    for rows, dtype in ((1, torch.bfloat16), (31, torch.float16), (32, torch.bfloat16), (70, torch.float16)):
+        cache = pkg.V3Cache(bits[0], bits[1], residual_window=4, n_layers=40, capacity=64)
+        k = outlier_kv((1, rows, 30, dim), seed=dim + rows, dtype=dtype).to(DEV)
+        v = outlier_kv((1, rows, 30, dim), seed=dim + rows + 1, dtype=dtype).to(DEV)
+        cache.append(k[:, :, :4], v[:, :, :4], 8)
+        for t in range(4, 30):
+            cache.append(k[:, :, t:t + 1], v[:, :, t:t + 1], 8)
+        st = cache._stores[8]
+        assert (st.n_compressed, st.n_recent) == (26, 4)
+        for comp, x, idx, nrm in ((st.comp.key_compressor, k, st.k_idx, st.k_nrm), (st.comp.val_compressor, v, st.v_idx, st.v_nrm)):
+            for t in range(26):
+                want = comp.compress(x[:, :, t:t + 1])
+                assert torch.equal(nrm[:, :, t:t + 1], want["vec_norms"]) and torch.equal(idx[:, :, t:t + 1], want["idx_bytes"]), (rows, t)
+        assert torch.equal(st.window()[0], k[:, :, 26:]) and torch.equal(st.window()[1], v[:, :, 26:])

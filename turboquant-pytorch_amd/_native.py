@@ -20,7 +20,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libtqamd.so")
-SOURCES = ("tq_host.cpp", "tq_compress.hip", "tq_decompress.hip", "tq_anydim.hip", "tq_wide.hip", "tq_attend.hip", "tq_qjl.hip")
+SOURCES = ("tq_host.cpp", "tq_compress.hip", "tq_decompress.hip", "tq_anydim.hip", "tq_wide.hip", "tq_attend.hip", "tq_qjl.hip", "tq_decode.hip")
 HEADERS = ("tq_table.h", "tq_device.h", "tq_anydim.h", "tq_wide.h", os.path.join("..", "..", "include", "tqamd.h"))
 GPU_ARCH = "gfx950"
 
@@ -150,6 +150,27 @@ class TqQjlJob(ctypes.Structure):
     ]
 
 
+class TqDecodeLayer(ctypes.Structure):
+    _fields_ = [
+        ("k_win", ctypes.c_void_p),
+        ("v_win", ctypes.c_void_p),
+        ("k_idx", ctypes.c_void_p),
+        ("k_norms", ctypes.c_void_p),
+        ("v_idx", ctypes.c_void_p),
+        ("v_norms", ctypes.c_void_p),
+        ("table_k", ctypes.c_void_p),
+        ("table_v", ctypes.c_void_p),
+        ("pi_v", ctypes.c_void_p),
+        ("win_stride", ctypes.c_longlong),
+        ("packed_row_stride", ctypes.c_longlong),
+        ("rows", ctypes.c_longlong),
+        ("head_dim", ctypes.c_int),
+        ("dtype", ctypes.c_int),
+        ("bits_k", ctypes.c_int),
+        ("bits_v", ctypes.c_int),
+    ]
+
+
 EXPORTS = (
     "tq_abi_version", "tq_status_string", "tq_device_count", "tq_bytes_per_vector",
     "tq_decision_thresholds", "tq_table_bytes", "tq_table_build", "tq_table_check", "tq_table_quantize_host",
@@ -158,6 +179,7 @@ EXPORTS = (
     "tq_qjl_compress", "tq_qjl_compress_batched", "tq_qjl_scores",
     "tq_scores", "tq_weighted_values", "tq_weighted_values_splits", "tq_attend_partials", "tq_attend_splits",
     "tq_attend_prepare", "tq_attend_merge", "tq_append_token", "tq_attend_step",
+    "tq_decode_supported", "tq_decode_scratch_floats", "tq_decode_attend", "tq_decode_append",
 )
 
 _lib = None
@@ -209,8 +231,13 @@ def lib() -> ctypes.CDLL:
     L.tq_append_token.argtypes = [vp, vp, ci, ll, ll, vp, vp, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, vp, vp, ll, ll, ll, vp]
     L.tq_attend_step.argtypes = [vp, ci, ll, ci, ctypes.c_float, vp, vp, vp, vp, ci, ll, ll, vp, vp, vp, vp, ll, ll,
                                  vp, vp, ci, ci, ci, vp, vp, vp, ci, vp, ci, vp]
+    L.tq_decode_supported.argtypes = [ci, ci, ci, ci]
+    L.tq_decode_scratch_floats.restype = ll
+    L.tq_decode_scratch_floats.argtypes = [ll, ci, ci, ll, ll]
+    L.tq_decode_attend.argtypes = [vp, vp, ci, ctypes.c_float, ll, ll, ll, vp, ll, vp, vp, vp]
+    L.tq_decode_append.argtypes = [vp, vp, vp, ll, ll, ll, ll, ll, vp]
     for name in EXPORTS:
-        if name not in ("tq_status_string", "tq_table_bytes", "tq_workspace_bytes", "tq_qjl_table_bytes"):
+        if name not in ("tq_status_string", "tq_table_bytes", "tq_workspace_bytes", "tq_qjl_table_bytes", "tq_decode_scratch_floats"):
             getattr(L, name).restype = ci
     _lib = L
     return L
@@ -290,6 +317,13 @@ def _require_gpu(t: torch.Tensor, what: str) -> None:
 
 
 ERR_ALIGN = -8      # TQ_ERR_ALIGN of include/tqamd.h
+ERR_CAPACITY = -10  # TQ_ERR_CAPACITY
+
+
+def decode_supported(head_dim: int, dtype: torch.dtype, bits_k: int, bits_v: int) -> bool:
+    """Whether the one-launch decode step (tq_decode_append, tq_decode_attend) takes this kind of layer."""
+    code = _DTYPE_CODE.get(dtype)
+    return code is not None and lib().tq_decode_supported(head_dim, code, bits_k, bits_v) == 1
 
 
 def dtype_code(dt: torch.dtype) -> int:
@@ -440,6 +474,45 @@ def step_scratch(device: torch.device, stream: int, floats: int) -> Optional[tor
     if buf is None or buf.numel() < floats:
         buf = _step_scratch[key] = torch.empty(max(floats, 1 << 16), dtype=torch.float32, device=device)
     return buf
+
+
+_arrived: Dict[Tuple[int, int], torch.Tensor] = {}
+
+
+def arrival_counters(device: torch.device, stream: int, rows: int) -> torch.Tensor:
+    """The counters through which the blocks of a row find out in tq_decode_attend which of them comes last: one zeroed
+    buffer per (device, stream), on the terms of `_workspace`.  (Never asked for while a graph is being captured.)"""
+    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
+    buf = _arrived.get(key)
+    if buf is None or buf.numel() < rows:
+        buf = _arrived[key] = torch.zeros(max(rows, 1024), dtype=torch.int32, device=device)
+    return buf
+
+
+def decode_attend(layer: TqDecodeLayer, queries: torch.Tensor, group: int, scale: float, win_first: int, n_win: int, tokens: int) -> torch.Tensor:
+    """tq_decode_attend into a new tensor of the queries' shape.  Scratch and counters are kept per stream, except while a
+    graph is being captured: then they come from the graph's own memory and the counters are cleared inside the graph."""
+    L = lib()
+    dev = queries.device
+    with _on(dev):
+        stream = _stream_handle(dev)
+        out = torch.empty_like(queries)
+        scratch = step_scratch(dev, stream, 0)
+        if scratch is None:
+            scratch = torch.empty(int(L.tq_decode_scratch_floats(layer.rows, group, layer.head_dim, tokens, n_win)), dtype=torch.float32, device=dev)
+            counters = torch.zeros(int(layer.rows), dtype=torch.int32, device=dev)
+        else:
+            counters = arrival_counters(dev, stream, layer.rows)
+        args = lambda buf: (ctypes.addressof(layer), queries.data_ptr(), group, scale, win_first, n_win, tokens, buf.data_ptr(), buf.numel(),  # noqa: E731
+                            counters.data_ptr(), out.data_ptr(), stream)
+        rc = L.tq_decode_attend(*args(scratch))
+        if rc == ERR_CAPACITY:
+            need = int(L.tq_decode_scratch_floats(layer.rows, group, layer.head_dim, tokens, n_win))
+            rc = L.tq_decode_attend(*args(step_scratch(dev, stream, need)))
+    if rc:
+        _arrived.pop((dev.index if dev.index is not None else torch.cuda.current_device(), stream), None)
+    check(rc, "tq_decode_attend")
+    return out
 
 
 def compress_into(states: torch.Tensor, table: torch.Tensor, bits: int,
@@ -678,6 +751,30 @@ def _(k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, q_rot):
     return q_rot.new_empty((q_rot.shape[0], q_rot.shape[1], max(splits, 1), q_rot.shape[2] + 2), dtype=torch.float32)
 
 
+def _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_v, k_win, v_win, scale):
+    """attend_packed through tq_decode_attend."""
+    B, Hq, _, D = q.shape
+    H, S, n_w = k_idx.shape[1], k_idx.shape[2], k_win.shape[2]
+    rows = B * H
+    win_stride = 0
+    if n_w:
+        lay_k, lay_v = row_layout(k_win), row_layout(v_win)
+        if lay_k is None or lay_v is None or lay_k != lay_v or (n_w > 1 and lay_k[3] != D) or lay_k[2] % 8 or k_win.data_ptr() % 16 or v_win.data_ptr() % 16:
+            k_win, v_win = k_win.contiguous(), v_win.contiguous()
+            lay_k = row_layout(k_win)
+        win_stride = lay_k[2] if rows > 1 else n_w * D
+    if S:
+        prs_k, prs_v = packed_row_stride(k_idx, k_norms), packed_row_stride(v_idx, v_norms)
+        if prs_k is None or prs_v is None or prs_k != prs_v:
+            k_idx, k_norms, v_idx, v_norms = k_idx.contiguous(), k_norms.contiguous(), v_idx.contiguous(), v_norms.contiguous()
+            prs_k = 0
+    layer = TqDecodeLayer(k_win.data_ptr() if n_w else None, v_win.data_ptr() if n_w else None,
+                          k_idx.data_ptr() if S else None, k_norms.data_ptr() if S else None, v_idx.data_ptr() if S else None,
+                          v_norms.data_ptr() if S else None, table_k.data_ptr(), table_v.data_ptr(), pi_v.data_ptr(), win_stride,
+                          (prs_k or S) if S else 0, rows, D, dtype_code(q.dtype), bits_k, bits_v)
+    return decode_attend(layer, q, Hq // H, scale, 0, n_w, S)
+
+
 def _attend_packed_impl(queries: torch.Tensor, k_idx: torch.Tensor, k_norms: torch.Tensor, v_idx: torch.Tensor,
                         v_norms: torch.Tensor, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int,
                         pi_k_t: torch.Tensor, pi_v: torch.Tensor, k_win: torch.Tensor, v_win: torch.Tensor,
@@ -695,6 +792,8 @@ def _attend_packed_impl(queries: torch.Tensor, k_idx: torch.Tensor, k_norms: tor
     q = queries.contiguous()
     pi_k_t, pi_v = pi_k_t.contiguous(), pi_v.contiguous()       # copies only if the caller kept a strided view
     L = lib()
+    if group <= 16 and n_w <= 512 and (k_win.dtype == v_win.dtype == q.dtype) and decode_supported(D, q.dtype, bits_k, bits_v):
+        return _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_v, k_win, v_win, scale)
     stream = _stream_handle(dev)
     q_rot = torch.empty((B, Hq, D), dtype=torch.float32, device=dev)
     part_w = torch.empty((rows, group, D + 2), dtype=torch.float32, device=dev) if n_w else None

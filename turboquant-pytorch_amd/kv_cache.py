@@ -20,6 +20,7 @@ subclass when transformers is importable.
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Dict, NamedTuple, Optional, Tuple
 
 import torch
@@ -69,6 +70,9 @@ class _LayerStore:
         self.n_recent = 0
         self.total_seq = 0
         self._consts = None
+        self._record = None
+        # decode steps of this layer take one launch each way (tq_decode_append, tq_decode_attend)
+        self.one_launch = _native.decode_supported(D, dtype, comp.key_bits, comp.value_bits)
         self.reserve(capacity)
 
     @staticmethod
@@ -100,6 +104,7 @@ class _LayerStore:
         self.k_idx, self.k_nrm, self.v_idx, self.v_nrm = new
         self.capacity = cap
         self._consts = None
+        self._record = None
 
     def consts(self) -> _StepConsts:
         """Rebuilt when the packed store moves (`reserve`)."""
@@ -114,12 +119,24 @@ class _LayerStore:
                 self.D * self.k_win.element_size())
         return c
 
+    def record(self) -> "_native.TqDecodeLayer":
+        """The layer as the one-launch decode step sees it; rebuilt when the packed store moves (`reserve`)."""
+        r = self._record
+        if r is None:
+            kc, vc = self.comp.key_compressor, self.comp.val_compressor
+            packed = [t.data_ptr() if t is not None else None for t in (self.k_idx, self.k_nrm, self.v_idx, self.v_nrm)]
+            r = self._record = _native.TqDecodeLayer(
+                self.k_win.data_ptr(), self.v_win.data_ptr(), *packed, kc.table(self.device).data_ptr(), vc.table(self.device).data_ptr(),
+                vc.pi(self.device).data_ptr(), self.win_cap * self.D, self.capacity, self.B * self.H, self.D, _native.dtype_code(self.dtype),
+                kc.bits, vc.bits)
+        return r
+
     def append_one(self, keys: torch.Tensor, values: torch.Tensor) -> bool:
         """The steady-state decode step in one library call: the window is full, its oldest token is compressed
         into the next packed slot and the new token takes the next window slot.  False (nothing done) when the
         step is not of that kind or the tensors are not laid out for it; the general path then runs."""
         rw = self.window_tokens
-        if (rw == 0 or self.D != _native.HEAD_DIM      # (the one-call step exists for the 128-wide kernels only)
+        if (rw == 0 or not (self.one_launch or self.D == _native.HEAD_DIM)
                 or self.n_recent != rw or self.w0 + rw + 1 > self.win_cap or self.n_compressed + 1 > self.capacity
                 or keys.dtype != self.dtype or values.dtype != self.dtype or keys.device != self.device
                 or values.device != self.device or torch.compiler.is_compiling()):
@@ -133,17 +150,23 @@ class _LayerStore:
             strides.append(s1 if self.H > 1 else s0)
         if rows > 1 and min(strides) < self.D:           # broadcast views: the general path copies them
             return False
-        c = self.consts()
         dev = self.device
         with _native._on(dev):
-            rc = _native.lib().tq_append_token(keys.data_ptr(), values.data_ptr(), c.dtype, strides[0], strides[1],
-                                               c.k_win, c.v_win, c.win_stride, self.w0, self.w0 + rw,
-                                               c.table_k, c.table_v, self.D, c.bits_k, c.bits_v,
-                                               c.k_idx, c.k_nrm, c.v_idx, c.v_nrm, self.capacity, self.n_compressed, rows,
-                                               _native._stream_handle(dev))
+            if self.one_launch and rows <= 65535:
+                rc = _native.lib().tq_decode_append(ctypes.addressof(self.record()), keys.data_ptr(), values.data_ptr(), strides[0], strides[1],
+                                                    self.w0, self.w0 + rw, self.n_compressed, _native._stream_handle(dev))
+            elif self.D != _native.HEAD_DIM:
+                return False
+            else:
+                c = self.consts()
+                rc = _native.lib().tq_append_token(keys.data_ptr(), values.data_ptr(), c.dtype, strides[0], strides[1],
+                                                   c.k_win, c.v_win, c.win_stride, self.w0, self.w0 + rw,
+                                                   c.table_k, c.table_v, self.D, c.bits_k, c.bits_v,
+                                                   c.k_idx, c.k_nrm, c.v_idx, c.v_nrm, self.capacity, self.n_compressed, rows,
+                                                   _native._stream_handle(dev))
         if rc == _native.ERR_ALIGN:
             return False
-        _native.check(rc, "tq_append_token")
+        _native.check(rc, "tq_decode_append" if self.one_launch else "tq_append_token")
         self.n_compressed += 1
         self.w0 += 1
         self.total_seq += 1
@@ -292,8 +315,9 @@ class V3Cache:
         scale = D ** -0.5 if scale is None else scale
         n_c, n_w = st.n_compressed, st.n_recent
         kc, vc = st.comp.key_compressor, st.comp.val_compressor
-        if D != _native.HEAD_DIM:
-            # The kernels that read packed codes directly are built for 128-wide heads.  Other head dimensions: the history
+        one_launch = st.one_launch and query_states.dtype == st.dtype and G <= 16 and n_w <= 512 and B * st.H <= 65535 and fused is not False
+        if D != _native.HEAD_DIM and not one_launch:
+            # The kernels that read packed codes directly are built for 64-, 96-, 128- and 256-wide heads.  Otherwise the history
             # is de-quantised by the codec kernels (into float32: rounding the keys to 16 bits would move logits of the size
             # this cache sees by several per cent of a softmax weight) and attended to together with the window.
             k = torch.empty((B, st.H, n_c + n_w, D), dtype=torch.float32, device=query_states.device)
@@ -357,6 +381,12 @@ class V3Cache:
             return None
         n_c, n_w = st.n_compressed, st.n_recent
         rows = B * st.H
+        if st.one_launch and query_states.dtype == st.dtype and rows <= 65535:
+            if torch.cuda.is_current_stream_capturing() or query_states.data_ptr() % 16:
+                return None
+            return _native.decode_attend(st.record(), query_states, G, scale, st.w0, n_w, n_c)
+        if D != _native.HEAD_DIM:
+            return None
         L = _native.lib()
         dev = st.device
         c = st.consts()
