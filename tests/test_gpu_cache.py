@@ -833,3 +833,39 @@ def test_one_launch_append_stores_the_bytes_of_compress(pkg, dim, bits):
                 want = comp.compress(x[:, :, t:t + 1])
                 assert torch.equal(nrm[:, :, t:t + 1], want["vec_norms"]) and torch.equal(idx[:, :, t:t + 1], want["idx_bytes"]), (rows, t)
         assert torch.equal(st.window()[0], k[:, :, 26:]) and torch.equal(st.window()[1], v[:, :, 26:])
+
+
+@pytest.mark.parametrize("dim,bits", [(64, (6, 4)), (96, (4, 2)), (256, (8, 8)), (256, (4, 4))])
+def test_decode_attention_of_other_head_dims_keeps_float32_weights(pkg, dim, bits):
+    """At 64, 96 and 256 queries and softmax weights enter the matrix products as two fp16 terms each (22 bits).  Against float64
+    over the centroids as the kernel holds them (float16) what is left is the rounding of the float16 result, 2^-11 / sqrt(12) = 1.4e-4
+    of a value on average over a binade at its lower end (2.4e-4 seen); single-term queries alone add 5e-4 at the logits here."""
+    g = torch.Generator().manual_seed(dim)
+    tokens, heads, group = 2000, 2, 4
+    cache = pkg.V3Cache(bits[0], bits[1], residual_window=32, n_layers=40)
+    k = (torch.randn(1, heads, tokens, dim, generator=g) * torch.exp(torch.randn(dim, generator=g))).half().to(DEV)
+    v = torch.randn(1, heads, tokens, dim, generator=g).half().to(DEV)
+    cache.append(k, v, 8)
+    q = (2 * torch.randn(1, heads * group, 1, dim, generator=g)).half().to(DEV)
+    out = cache.attend(q, 8).double().reshape(heads, group, dim)
+    st = cache._stores[8]
+    n = st.n_compressed
+    dec = lambda comp, idx, nrm: ((comp.centroids.half().double()[_codes(idx[:, :, :n].contiguous(), comp.bits if comp.bits < 5 else 8, dim)] @ comp.Pi.double())
+                                  * nrm[:, :, :n].double().unsqueeze(-1))
+    K = torch.cat([dec(st.comp.key_compressor, st.k_idx, st.k_nrm), st.window()[0].double()], 2).reshape(heads, -1, dim)
+    V = torch.cat([dec(st.comp.val_compressor, st.v_idx, st.v_nrm), st.window()[1].double()], 2).reshape(heads, -1, dim)
+    ref = torch.softmax(torch.matmul(q.double().reshape(heads, group, dim), K.transpose(1, 2).contiguous()) * dim ** -0.5, -1) @ V
+    err = float((out - ref).norm() / ref.norm())
+    assert err < 3.5e-4, err
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_attend_takes_queries_at_any_element_address(pkg, dim):
+    """Contiguous queries that start in the middle of a buffer, on no 16-byte boundary."""
+    cache = pkg.V3Cache(4, 2, residual_window=16, n_layers=40)
+    k, v = (outlier_kv((1, 2, 100, dim), seed=s, dtype=torch.float16).to(DEV) for s in (1, 2))
+    cache.append(k, v, 8)
+    q = torch.randn(1, 4, 1, dim, dtype=torch.float16, generator=torch.Generator().manual_seed(3)).to(DEV)
+    odd = torch.empty(4 * dim + 1, dtype=torch.float16, device=DEV)[1:].view(1, 4, 1, dim)
+    odd.copy_(q)
+    assert torch.equal(cache.attend(odd, 8), cache.attend(q, 8))

@@ -756,10 +756,12 @@ def _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_
     B, Hq, _, D = q.shape
     H, S, n_w = k_idx.shape[1], k_idx.shape[2], k_win.shape[2]
     rows = B * H
+    if q.data_ptr() % 16:
+        q = q.clone()
     win_stride = 0
     if n_w:
         lay_k, lay_v = row_layout(k_win), row_layout(v_win)
-        if lay_k is None or lay_v is None or lay_k != lay_v or (n_w > 1 and lay_k[3] != D) or lay_k[2] % 8 or k_win.data_ptr() % 16 or v_win.data_ptr() % 16:
+        if lay_k is None or lay_v is None or lay_k != lay_v or (rows > 1 and lay_k[2] < n_w * D) or (n_w > 1 and lay_k[3] != D) or lay_k[2] % 8 or k_win.data_ptr() % 16 or v_win.data_ptr() % 16:
             k_win, v_win = k_win.contiguous(), v_win.contiguous()
             lay_k = row_layout(k_win)
         win_stride = lay_k[2] if rows > 1 else n_w * D
@@ -792,7 +794,7 @@ def _attend_packed_impl(queries: torch.Tensor, k_idx: torch.Tensor, k_norms: tor
     q = queries.contiguous()
     pi_k_t, pi_v = pi_k_t.contiguous(), pi_v.contiguous()       # copies only if the caller kept a strided view
     L = lib()
-    if group <= 16 and n_w <= 512 and (k_win.dtype == v_win.dtype == q.dtype) and decode_supported(D, q.dtype, bits_k, bits_v):
+    if group <= 16 and n_w <= 512 and rows <= 65535 and (k_win.dtype == v_win.dtype == q.dtype) and decode_supported(D, q.dtype, bits_k, bits_v):
         return _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_v, k_win, v_win, scale)
     stream = _stream_handle(dev)
     q_rot = torch.empty((B, Hq, D), dtype=torch.float32, device=dev)

@@ -136,11 +136,13 @@ __device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t fir
 //     probabilities enter the value product as two (fp16) or three (bf16) terms that add up to their float32 value;
 //   * the waves' sums meet in LDS; with several splits per row the block that arrives last at the row's counter merges the
 //     records of all splits and of the window, rotates the value sums back and stores the result.
-// Queries and weights enter the packed products as one fp16 term (queries against 8-bit keys at 128: two): their 2^-12
-// roundings stay at or under what the fp16 centroids and the fp16 rotation of a de-quantised history would cost.
+// At 128 queries (against 8-bit keys: two terms) and weights enter the packed products as one fp16 term, as in tq_attend_kernel:
+// their 2^-12 roundings stay under what the fp16 centroids cost.  The other head dimensions, whose histories were attended to in
+// float32 before, take both as two terms (22 bits): the matrix cores are idle most of the time.
 template <int D, int IPBK, int IPBV>
 __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs a) {
-    constexpr bool QLO = D == 128 && IPBK == 1;          // queries as fp16 hi + lo against 8-bit keys
+    constexpr bool QLO = D != 128 || IPBK == 1;          // queries as fp16 hi + lo
+    constexpr bool PLO = D != 128;                       // weights as fp16 hi + lo
     constexpr int SETS = D == 256 ? 1 : 2;               // register sets of the loads that run one run ahead
     constexpr int PART = D + 2;
     constexpr int STEPS = D / 16, TILES = D / 32;        // query rotation: 32x32x16 matrix instructions
@@ -508,12 +510,25 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
             // ---- weights p_j |v_j| / 2^ev_ref: slice j of lane (., q4) = token 32 u + 4 q4 + j (j < 4), 32 u + 16 + 4 q4 + j - 4
             const uint32_t tok_a = 32u * u + 4u * q4, tok_b = tok_a + 16u;
             tq_half8 h;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) h[j] = (_Float16)ps[j];
             const tq_u2 vn_a = *reinterpret_cast<const tq_u2 *>(&lds_vn[wave][tok_a]);
             const tq_u2 vn_b = *reinterpret_cast<const tq_u2 *>(&lds_vn[wave][tok_b]);
             const tq_u4 nrm = {vn_a[0], vn_a[1], vn_b[0], vn_b[1]};
-            h = h * __builtin_bit_cast(tq_half8, nrm);
+            tq_u4 pl = {0u, 0u, 0u, 0u};
+            if constexpr (PLO) {
+                const tq_half8 vn8 = __builtin_bit_cast(tq_half8, nrm);
+                tq_half8 lo;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float x = ps[j] * (float)vn8[j];
+                    h[j] = (_Float16)x;
+                    lo[j] = (_Float16)(x - (float)h[j]);
+                }
+                pl = __builtin_bit_cast(tq_u4, lo);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) h[j] = (_Float16)ps[j];
+                h = h * __builtin_bit_cast(tq_half8, nrm);
+            }
             const tq_u4 pa = __builtin_bit_cast(tq_u4, h);
             auto columns = [&](auto n_tag, int c0) __attribute__((always_inline)) {
                 constexpr int N = decltype(n_tag)::value;
@@ -529,6 +544,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
                     for (int d = 0; d < 4; ++d)
                         bt[d] = __builtin_amdgcn_perm(dec[2 * d + 1][c / 2], dec[2 * d][c / 2], (c & 1) ? 0x07060302u : 0x05040100u);
                     acc[c0 + c] = mfma16_f16(pa, bt, acc[c0 + c]);
+                    if constexpr (PLO) acc[c0 + c] = mfma16_f16(pl, bt, acc[c0 + c]);
                 }
             };
             if constexpr (D == 64) columns(std::integral_constant<int, 4>{}, 0);
