@@ -197,6 +197,24 @@ int tq_decompress_batched(const tq_job *jobs_host, const tq_job *jobs_dev, int n
                           int head_dim, void *workspace, void *stream);
 
 /*
+ * Keys and values of one layer in one call.
+ * tq_compress_layer: two tq_compress calls on tensors of one layout, into dense packed buffers.
+ * tq_restore_layer: the full-length keys and values [batch, heads, tokens + n_win, head_dim] (dense) of a layer whose first `tokens`
+ *   tokens are packed (packed_row_stride as for tq_decompress) and whose last n_win (0 or more) are kept as they are, in the
+ *   output's element type: head h of sequence b of k_win / v_win starts at element b * win_batch_stride + h * win_head_stride,
+ *   its tokens follow one another.  With a window, its addresses and strides, the outputs' and the rows' lengths in bytes are
+ *   multiples of 16 (TQ_ERR_ALIGN otherwise); at most 65535 rows.
+ * The workspace is that of tq_decompress, used by the launches of the call one after the other.
+ */
+int tq_compress_layer(const void *keys, const void *values, int dtype, long long rows, long long tokens, long long row_stride, long long token_stride,
+                      const void *table_k, const void *table_v, int head_dim, int bits_k, int bits_v, uint8_t *k_idx, uint16_t *k_norms,
+                      uint8_t *v_idx, uint16_t *v_norms, void *workspace, void *stream);
+int tq_restore_layer(const uint8_t *k_idx, const uint16_t *k_norms, const uint8_t *v_idx, const uint16_t *v_norms,
+                     long long packed_row_stride, long long batch, long long heads, long long tokens, const void *table_k, const void *table_v,
+                     int head_dim, int bits_k, int bits_v, const void *k_win, const void *v_win, long long n_win, long long win_batch_stride,
+                     long long win_head_stride, void *k_out, void *v_out, int dtype, void *workspace, void *stream);
+
+/*
  * V2 key path: MSE codes of (bits - 1) bits plus one QJL sign bit per coordinate of the quantisation residual, for the
  * unbiased inner-product estimate  <q, k> ~ <q, k_mse> + ||r|| * sqrt(pi/2) / D * <S q, sign(S r)>.
  * Replaces TurboQuantCompressorV2.compress / asymmetric_attention_scores, turboquant/compressors.py:84-158 (and the

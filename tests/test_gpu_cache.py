@@ -869,3 +869,59 @@ def test_attend_takes_queries_at_any_element_address(pkg, dim):
     odd = torch.empty(4 * dim + 1, dtype=torch.float16, device=DEV)[1:].view(1, 4, 1, dim)
     odd.copy_(q)
     assert torch.equal(cache.attend(odd, 8), cache.attend(q, 8))
+
+
+def _layer_forms(dim, dtype, g):
+    """[B,H,S,D] tensors laid out in the ways a caller's may be: dense, one row, one head, token slices of a longer buffer, heads
+    and tokens exchanged, a broadcast batch; where vectors are moved element by element also an address on no 16-byte boundary."""
+    mk = lambda *shape: (torch.randn(shape, generator=g) * 2).to(dtype).to(DEV)
+    yield "dense", mk(2, 3, 70, dim)
+    yield "one row", mk(1, 1, 33, dim)
+    yield "one head", mk(3, 1, 40, dim)
+    yield "slice", mk(2, 3, 90, dim)[:, :, 5:77]
+    yield "heads last", mk(2, 50, 3, dim).transpose(1, 2)
+    if dim % 32:
+        yield "odd address", torch.empty(2 * 2 * 40 * dim + 1, dtype=dtype, device=DEV)[1:].view(2, 2, 40, dim).copy_(mk(2, 2, 40, dim))
+    yield "broadcast", mk(1, 2, 40, dim).expand(3, 2, 40, dim)
+
+
+@pytest.mark.parametrize("dim,bits", [(64, (4, 2)), (80, (4, 4)), (96, (6, 3)), (128, (4, 2)), (128, (8, 1)), (256, (3, 2))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_layer_calls_equal_the_calls_per_tensor(pkg, monkeypatch, dim, bits, dtype):
+    """compress_kv / decompress_kv through tq_compress_layer and tq_restore_layer against the same methods tensor by tensor: the same
+    bytes and values for every layout, with windows of none, one and most of the tokens."""
+    g = torch.Generator().manual_seed(dim)
+    for window in (0, 1, 32):
+        comp = pkg.TurboQuantV3(dim, key_bits=bits[0], value_bits=bits[1], residual_window=window, layer_idx=8, device=DEV)
+        for name, k in _layer_forms(dim, dtype, g):
+            v = k.flip(0).contiguous() if name in ("dense", "one row") else (k * 1 if name == "slice" else k)
+            got = comp.compress_kv(k, v)
+            got_full = comp.decompress_kv(*got)
+            with monkeypatch.context() as m:
+                m.setattr(pkg._native, "compress_layer", lambda *a: None)
+                m.setattr(pkg._native, "restore_layer", lambda *a: None)
+                want = comp.compress_kv(k, v)
+                want_full = comp.decompress_kv(*want)
+            for a, b in zip(got, want):
+                assert a["compressed"]["shape"] == b["compressed"]["shape"] and a["compressed"]["idx_pad"] == b["compressed"]["idx_pad"]
+                assert torch.equal(a["compressed"]["idx_bytes"], b["compressed"]["idx_bytes"]), (name, window)
+                assert torch.equal(a["compressed"]["vec_norms"], b["compressed"]["vec_norms"]), (name, window)
+            for a, b in zip(got_full, want_full):
+                assert a.is_contiguous() and a.dtype == b.dtype and torch.equal(a, b), (name, window)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_update_restores_the_layer_as_the_calls_per_tensor_do(pkg, monkeypatch, dim):
+    """V3Cache.update from a per-row store (packed slots between the rows) and a window that moves through its buffer."""
+    full = []
+    for fast in (True, False):
+        with monkeypatch.context() as m:
+            if not fast:
+                m.setattr(pkg._native, "restore_layer", lambda *a: None)
+            cache = pkg.V3Cache(4, 2, residual_window=8, n_layers=40)
+            x = outlier_kv((2, 3, 60, dim), seed=dim, dtype=torch.float16).to(DEV)
+            steps = [cache.update(x[:, :, :40], x[:, :, :40], 8)]
+            steps += [cache.update(x[:, :, t:t + 1], x[:, :, t:t + 1], 8) for t in range(40, 60)]
+            full.append(steps)
+    for a, b in zip(*full):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])

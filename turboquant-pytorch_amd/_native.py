@@ -180,6 +180,7 @@ EXPORTS = (
     "tq_scores", "tq_weighted_values", "tq_weighted_values_splits", "tq_attend_partials", "tq_attend_splits",
     "tq_attend_prepare", "tq_attend_merge", "tq_append_token", "tq_attend_step",
     "tq_decode_supported", "tq_decode_scratch_floats", "tq_decode_attend", "tq_decode_append",
+    "tq_compress_layer", "tq_restore_layer",
 )
 
 _lib = None
@@ -236,6 +237,8 @@ def lib() -> ctypes.CDLL:
     L.tq_decode_scratch_floats.argtypes = [ll, ci, ci, ll, ll]
     L.tq_decode_attend.argtypes = [vp, vp, ci, ctypes.c_float, ll, ll, ll, vp, ll, vp, vp, vp]
     L.tq_decode_append.argtypes = [vp, vp, vp, ll, ll, ll, ll, ll, vp]
+    L.tq_compress_layer.argtypes = [vp, vp, ci, ll, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, vp, vp, vp, vp]
+    L.tq_restore_layer.argtypes = [vp, vp, vp, vp, ll, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, ll, ll, ll, vp, vp, ci, vp, vp]
     for name in EXPORTS:
         if name not in ("tq_status_string", "tq_table_bytes", "tq_workspace_bytes", "tq_qjl_table_bytes", "tq_decode_scratch_floats"):
             getattr(L, name).restype = ci
@@ -348,7 +351,7 @@ def vector_layout(t: torch.Tensor) -> Optional[Tuple[int, int, int, int]]:
         return None
     esz = t.element_size()
     align = _vector_alignment(D, esz)
-    if (t.data_ptr() % align) or any((s * esz) % align for s in (sb, sh, ss)):
+    if (t.data_ptr() % align) or (sb * esz) % align or (sh * esz) % align or (ss * esz) % align:
         return None
     n = B * H * S
     if n == 0:
@@ -435,6 +438,7 @@ def _on(device: torch.device):
 
 
 _workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
+_COUNTED_DIMS = (64, 128)       # head dimensions whose kernels can draw their tiles from counters
 
 
 def _workspace(device: torch.device, stream: int) -> int:
@@ -515,6 +519,87 @@ def decode_attend(layer: TqDecodeLayer, queries: torch.Tensor, group: int, scale
     return out
 
 
+def compress_layer(keys: torch.Tensor, values: torch.Tensor, tokens: int, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int):
+    """The first `tokens` tokens of a layer's keys and values [B,H,S,D] compressed in one call: ((idx_bytes, vec_norms) of the keys,
+    the same of the values), or None where the two are not laid out alike, or not in a form the kernels read in place
+    (the caller then goes tensor by tensor)."""
+    shape, stride, dtype, dev = keys.shape, keys.stride(), keys.dtype, keys.device
+    if (values.shape != shape or values.stride() != stride or values.dtype != dtype or values.device != dev or dev.type != "cuda"
+            or dtype not in _DTYPE_CODE or torch.compiler.is_compiling()):
+        return None
+    B, H, _, D = shape
+    sb, sh, ss, sd = stride
+    rows = B * H
+    row_stride = sh if H > 1 else sb
+    if sd != 1 or ss < D or tokens < 1 or rows < 1 or (B > 1 and H > 1 and sb != H * sh) or (rows > 1 and row_stride < D):
+        return None
+    esz = keys.element_size()
+    align = _vector_alignment(D, esz)
+    pk, pv = keys.data_ptr(), values.data_ptr()
+    if pk % align or pv % align or (sb * esz) % align or (sh * esz) % align or (ss * esz) % align:
+        return None
+    n_rows, n_tokens = rows, tokens
+    if rows == 1:
+        row_stride = 0
+    elif row_stride == tokens * ss:
+        n_rows, n_tokens, row_stride = 1, rows * tokens, 0
+    check_table(table_k, D, bits_k)
+    check_table(table_v, D, bits_v)
+    k_idx = torch.empty((B, H, tokens, _packed_width(D, bits_k)), dtype=torch.uint8, device=dev)
+    k_nrm = torch.empty((B, H, tokens), dtype=torch.float16, device=dev)
+    v_idx = torch.empty((B, H, tokens, _packed_width(D, bits_v)), dtype=torch.uint8, device=dev)
+    v_nrm = torch.empty((B, H, tokens), dtype=torch.float16, device=dev)
+    with _on(dev):
+        stream = _stream_handle(dev)
+        ws = _workspace(dev, stream) if rows * tokens >= 65536 and D in _COUNTED_DIMS else 0
+        rc = lib().tq_compress_layer(pk, pv, _DTYPE_CODE[dtype], n_rows, n_tokens, row_stride, ss, table_k.data_ptr(), table_v.data_ptr(), D, bits_k, bits_v,
+                                     k_idx.data_ptr(), k_nrm.data_ptr(), v_idx.data_ptr(), v_nrm.data_ptr(), ws, stream)
+    if rc and ws:
+        _drop_workspace(dev, stream)
+    check(rc, "tq_compress_layer")
+    return (k_idx, k_nrm), (v_idx, v_nrm)
+
+
+def restore_layer(packed_k, packed_v, tokens: int, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int,
+                  k_win: torch.Tensor, v_win: torch.Tensor):
+    """Full-length keys and values [B,H,tokens + n_win,D] in the windows' element type, from packed pairs (idx_bytes [B,H,tokens,G],
+    vec_norms [B,H,tokens]: dense, or token slices of one per-row store) and the windows [B,H,n_win,D] behind them, in one
+    call; None where the layout is not one the call takes (the caller then goes step by step)."""
+    shape, stride, dtype, dev = k_win.shape, k_win.stride(), k_win.dtype, k_win.device
+    B, H, n_win, D = shape
+    if (v_win.shape != shape or v_win.stride() != stride or v_win.dtype != dtype or v_win.device != dev or dev.type != "cuda"
+            or dtype not in _DTYPE_CODE or tokens < 1 or B * H < 1 or B * H > 65535 or torch.compiler.is_compiling()):
+        return None
+    prs = None
+    for (idx, nrm), bits in ((packed_k, bits_k), (packed_v, bits_v)):
+        if (idx.shape != (B, H, tokens, _packed_width(D, bits)) or nrm.shape != (B, H, tokens) or idx.dtype != torch.uint8 or nrm.dtype != torch.float16
+                or idx.device != dev or nrm.device != dev):
+            return None
+        one = packed_row_stride(idx, nrm)
+        if one is None or (prs is not None and one != prs):
+            return None
+        prs = one
+    esz = k_win.element_size()
+    sb, sh, ss, sd = stride
+    pk, pv = (k_win.data_ptr(), v_win.data_ptr()) if n_win else (0, 0)
+    if n_win and (sd != 1 or (n_win > 1 and ss != D) or sb < 0 or sh < 0 or (D * esz) % 16 or (sb * esz) % 16 or (sh * esz) % 16 or pk % 16 or pv % 16):
+        return None
+    check_table(table_k, D, bits_k)
+    check_table(table_v, D, bits_v)
+    full_k = torch.empty((B, H, tokens + n_win, D), dtype=dtype, device=dev)
+    full_v = torch.empty((B, H, tokens + n_win, D), dtype=dtype, device=dev)
+    with _on(dev):
+        stream = _stream_handle(dev)
+        ws = _workspace(dev, stream) if D in _COUNTED_DIMS else 0
+        rc = lib().tq_restore_layer(packed_k[0].data_ptr(), packed_k[1].data_ptr(), packed_v[0].data_ptr(), packed_v[1].data_ptr(), prs, B, H, tokens,
+                                    table_k.data_ptr(), table_v.data_ptr(), D, bits_k, bits_v, pk, pv, n_win, sb if B > 1 else 0, sh if H > 1 else 0,
+                                    full_k.data_ptr(), full_v.data_ptr(), _DTYPE_CODE[dtype], ws, stream)
+    if rc and ws:
+        _drop_workspace(dev, stream)
+    check(rc, "tq_restore_layer")
+    return full_k, full_v
+
+
 def compress_into(states: torch.Tensor, table: torch.Tensor, bits: int,
                   idx_bytes: torch.Tensor, vec_norms: torch.Tensor) -> None:
     """Launch tq_compress on `states` ([B,H,S,128], any supported float type, last dim dense).
@@ -532,8 +617,8 @@ def compress_into(states: torch.Tensor, table: torch.Tensor, bits: int,
     check_table(table, states.shape[-1], bits)
     with _on(states.device):
         stream = _stream_handle(states.device)
-        # counters only where the kernel can use them (a large job): a one-token append needs no look-up
-        ws = _workspace(states.device, stream) if rows * tokens >= 65536 else 0
+        # counters only where the kernel can use them (a large job at 128, or at 64 in pairs): a one-token append needs no look-up
+        ws = _workspace(states.device, stream) if rows * tokens >= 65536 and states.shape[-1] in _COUNTED_DIMS else 0
         rc = lib().tq_compress(states.data_ptr(), dtype_code(states.dtype), rows, tokens, row_stride, token_stride,
                                table.data_ptr(), states.shape[-1], bits,
                                idx_bytes.data_ptr(), vec_norms.data_ptr(), prs, ws, stream)
@@ -561,7 +646,7 @@ def decompress_into(idx_bytes: torch.Tensor, vec_norms: torch.Tensor, table: tor
         stream = _stream_handle(out.device)
         rc = lib().tq_decompress(idx_bytes.data_ptr(), vec_norms.data_ptr(), prs, rows, tokens, table.data_ptr(),
                                  out.shape[-1], bits, out.data_ptr(), dtype_code(out.dtype), row_stride,
-                                 token_stride, _workspace(out.device, stream), stream)
+                                 token_stride, _workspace(out.device, stream) if out.shape[-1] in _COUNTED_DIMS else 0, stream)
     if rc:
         _drop_workspace(out.device, stream)
     check(rc, "tq_decompress")

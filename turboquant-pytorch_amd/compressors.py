@@ -211,11 +211,12 @@ class TurboQuantCompressorV2:
             term1 = torch.matmul(q, exp["k_mse"].float().transpose(-2, -1))
             ip = torch.matmul(torch.matmul(q, self._s(dev).T), exp["qjl_signs"].float().transpose(-2, -1))
             return term1 + corr * ip * compressed["residual_norm"].float().unsqueeze(-2)
-        q_rot = torch.matmul(q, self._mse.pi_transposed(dev)).contiguous()          # Pi q for every query token
         st = self._s_on.get(("t", dev))
-        if st is None:
-            st = self._s_on[("t", dev)] = (self._s(dev).T * corr).contiguous()      # sqrt(pi/2)/m S^T, made once per device
-        q_sign = torch.matmul(q, st).contiguous()
+        if st is None:      # Pi^T and sqrt(pi/2)/m S^T one behind the other, made once per device
+            st = self._s_on[("t", dev)] = torch.stack((self._mse.pi_transposed(dev), self._s(dev).T * corr)).contiguous()
+        # every query token rotated and projected, in one product: [2, B * H * S_q, D]
+        q_both = torch.matmul(q.reshape(1, -1, D), st)
+        q_rot, q_sign = q_both[0], q_both[1]
         packed = [compressed[k] if compressed[k].is_contiguous() else compressed[k].contiguous()
                   for k in ("idx_bytes", "vec_norms", "sign_bytes", "residual_norm")]
         with _native._on(dev):

@@ -97,6 +97,9 @@ class MSECompressor:
 
     def table(self, device=None) -> torch.Tensor:
         """Copy of the codec table on `device` (default: the compressor's own), uploaded on first use."""
+        t = self._tables.get(device)
+        if t is not None:
+            return t
         dev = torch.device(self.device if device is None else device)
         if dev.type == "cuda" and dev.index is None:
             dev = torch.device("cuda", torch.cuda.current_device())
@@ -254,6 +257,17 @@ class TurboQuantV3:
                 {"fp16": values, "compressed": None, "shape": (B, H, S, D), "split_at": S},
             )
         split_at = S - rw
+        kc, vc = self.key_compressor, self.val_compressor
+        packed = None
+        if values.shape == keys.shape and keys.is_cuda and kc.head_dim == vc.head_dim == D:
+            packed = _native.compress_layer(keys, values, split_at, kc.table(keys.device), vc.table(keys.device), kc.bits, vc.bits)
+        if packed is not None:
+            return tuple({
+                "compressed": {"idx_bytes": idx, "vec_norms": nrm, "shape": (B, H, split_at, D), "idx_pad": -D % (8 // comp.bits)},
+                "fp16": tensor[:, :, split_at:, :],
+                "shape": (B, H, S, D),
+                "split_at": split_at,
+            } for tensor, comp, (idx, nrm) in ((keys, kc, packed[0]), (values, vc, packed[1])))
         out = []
         for tensor, comp in ((keys, self.key_compressor), (values, self.val_compressor)):
             out.append({
@@ -270,6 +284,9 @@ class TurboQuantV3:
         """-> keys, values (B, H, S, D) in the dtype of the uncompressed window."""
         if compressed_k["compressed"] is None:
             return compressed_k["fp16"], compressed_v["fp16"]
+        full = self._restore(compressed_k, compressed_v)
+        if full is not None:
+            return full
         out = []
         for c, comp in ((compressed_k, self.key_compressor), (compressed_v, self.val_compressor)):
             B, H, S, D = c["shape"]
@@ -281,6 +298,20 @@ class TurboQuantV3:
                 full[:, :, split_at:, :].copy_(window)
             out.append(full)
         return out[0], out[1]
+
+    def _restore(self, compressed_k: dict, compressed_v: dict):
+        """Keys and values in one library call, or None where the dictionaries ask for something else than it does."""
+        shape, split_at = compressed_k["shape"], compressed_k["split_at"]
+        ck, cv, k_win, v_win = compressed_k["compressed"], compressed_v["compressed"], compressed_k["fp16"], compressed_v["fp16"]
+        B, H, S, D = shape
+        if (cv is None or compressed_v["shape"] != shape or compressed_v["split_at"] != split_at or k_win.shape != (B, H, S - split_at, D)
+                or ck["shape"] != (B, H, split_at, D) or cv["shape"] != ck["shape"] or not k_win.is_cuda):
+            return None
+        kc, vc = self.key_compressor, self.val_compressor
+        if kc.head_dim != D or vc.head_dim != D:
+            return None
+        return _native.restore_layer((ck["idx_bytes"], ck["vec_norms"]), (cv["idx_bytes"], cv["vec_norms"]), split_at, kc.table(k_win.device),
+                                     vc.table(k_win.device), kc.bits, vc.bits, k_win, v_win)
 
     def memory_bytes(self, B: int, H: int, S: int) -> dict:
         """Bytes stored including the uncompressed window (compressors_v3.py:235-265)."""

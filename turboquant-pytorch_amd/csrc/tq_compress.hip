@@ -834,6 +834,14 @@ extern "C" int tq_compress(const void *states, int dtype, long long rows, long l
     return dispatch(dtype, bits, job, nullptr, 1, (uint32_t)((n_vec + 31) / 32), workspace, false, static_cast<hipStream_t>(stream));
 }
 
+extern "C" int tq_compress_layer(const void *keys, const void *values, int dtype, long long rows, long long tokens, long long row_stride, long long token_stride,
+                                 const void *table_k, const void *table_v, int head_dim, int bits_k, int bits_v, uint8_t *k_idx, uint16_t *k_norms,
+                                 uint8_t *v_idx, uint16_t *v_norms, void *workspace, void *stream) {
+    const int rc = tq_compress(keys, dtype, rows, tokens, row_stride, token_stride, table_k, head_dim, bits_k, k_idx, k_norms, 0, workspace, stream);
+    if (rc) return rc;
+    return tq_compress(values, dtype, rows, tokens, row_stride, token_stride, table_v, head_dim, bits_v, v_idx, v_norms, 0, workspace, stream);
+}
+
 extern "C" int tq_compress_batched(const tq_job *jobs_host, const tq_job *jobs_dev, int n_jobs,
                                    int head_dim, void *workspace, void *stream) {
     if (n_jobs == 0) return TQ_OK;

@@ -493,6 +493,51 @@ extern "C" int tq_decompress(const uint8_t *idx_bytes, const uint16_t *vec_norms
     return dispatch(out_dtype, bits, job, nullptr, 1, (uint32_t)((n_vec + 31) / 32), workspace, false, static_cast<hipStream_t>(stream));
 }
 
+namespace {
+// The uncompressed window of a layer into the last tokens of its full-length tensors, keys (z = 0) and values in one launch:
+// a row of the window is one run of 16-byte pieces.  Two library copies took 2.5 us each and as much host time as a launch
+// of the codec; this one takes 2.5 us for both.
+__global__ __launch_bounds__(256) void tq_copy_window_kernel(const uint8_t *k_src, const uint8_t *v_src, uint8_t *k_dst, uint8_t *v_dst, uint32_t pieces,
+                                                             uint32_t heads, long long batch_bytes, long long head_bytes, long long dst_bytes) {
+    const uint32_t row = blockIdx.y, b = row / heads, h = row % heads;
+    const uint8_t *src = (blockIdx.z ? v_src : k_src) + (long long)b * batch_bytes + (long long)h * head_bytes;
+    uint8_t *dst = (blockIdx.z ? v_dst : k_dst) + (long long)row * dst_bytes;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < pieces; i += gridDim.x * 256u) tq_gstore16(dst + (size_t)i * 16u, tq_gload16(src + (size_t)i * 16u));
+}
+}  // namespace
+
+extern "C" int tq_restore_layer(const uint8_t *k_idx, const uint16_t *k_norms, const uint8_t *v_idx, const uint16_t *v_norms,
+                                long long packed_row_stride, long long batch, long long heads, long long tokens, const void *table_k, const void *table_v, int head_dim, int bits_k, int bits_v, const void *k_win,
+                                const void *v_win, long long n_win, long long win_batch_stride, long long win_head_stride, void *k_out, void *v_out,
+                                int dtype, void *workspace, void *stream) {
+    if (batch < 1 || heads < 1 || tokens < 1 || n_win < 0 || batch > 65535 || heads > 65535 || batch * heads > 65535 || tokens > 0x7fffffff || n_win > 0x7fffffff)
+        return TQ_ERR_SIZE;
+    if (!k_out || !v_out || (n_win && (!k_win || !v_win))) return TQ_ERR_NULL;
+    if (dtype != TQ_F32 && dtype != TQ_F16 && dtype != TQ_BF16) return TQ_ERR_DTYPE;
+    const long long rows = batch * heads, total = tokens + n_win, elem = elem_bytes(dtype);
+    const long long run = n_win * head_dim * elem, dst_row = total * head_dim * elem;
+    if (n_win) {
+        if (run > 0x7fffffffll * 16 || win_batch_stride < 0 || win_head_stride < 0) return TQ_ERR_SIZE;
+        if ((run | dst_row | (tokens * head_dim * elem) | (win_batch_stride * elem) | (win_head_stride * elem)) & 15) return TQ_ERR_ALIGN;
+        if (((uintptr_t)k_win | (uintptr_t)v_win | (uintptr_t)k_out | (uintptr_t)v_out) & 15u) return TQ_ERR_ALIGN;
+    }
+    // one row, or no window and dense packed tokens: one run of vectors on both sides
+    const bool dense = rows == 1 || (n_win == 0 && packed_row_stride == 0);
+    const long long r = dense ? 1 : rows, t = dense ? rows * tokens : tokens, rs = dense ? 0 : total * head_dim;
+    int rc = tq_decompress(k_idx, k_norms, packed_row_stride, r, t, table_k, head_dim, bits_k, k_out, dtype, rs, head_dim, workspace, stream);
+    if (rc) return rc;
+    rc = tq_decompress(v_idx, v_norms, packed_row_stride, r, t, table_v, head_dim, bits_v, v_out, dtype, rs, head_dim, workspace, stream);
+    if (rc || n_win == 0) return rc;
+    const uint32_t pieces = (uint32_t)(run / 16);
+    const uint32_t bx = (pieces + 255u) / 256u;
+    const dim3 grid(bx < 64u ? bx : 64u, (unsigned)rows, 2);
+    const long long off = tokens * head_dim * elem;
+    hipLaunchKernelGGL(tq_copy_window_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const uint8_t *>(k_win),
+                       static_cast<const uint8_t *>(v_win), static_cast<uint8_t *>(k_out) + off, static_cast<uint8_t *>(v_out) + off, pieces, (uint32_t)heads,
+                       win_batch_stride * elem, win_head_stride * elem, dst_row);
+    return (int)hipGetLastError();
+}
+
 extern "C" long long tq_workspace_bytes(int n_jobs) {
     if (n_jobs < 0 || n_jobs > TQ_MAX_JOBS) return TQ_ERR_SIZE;
     return (long long)TQ_WORKSPACE_BYTES_PER_JOB * (n_jobs > 0 ? n_jobs : 1);

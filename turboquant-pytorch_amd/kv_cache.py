@@ -278,6 +278,12 @@ class V3Cache:
         comp = st.comp
         self._push(st, key_states, value_states)
         n_c = st.n_compressed
+        if n_c and st.dtype == key_states.dtype == value_states.dtype:
+            kc, vc = comp.key_compressor, comp.val_compressor
+            full = _native.restore_layer((st.k_idx[:, :, :n_c], st.k_nrm[:, :, :n_c]), (st.v_idx[:, :, :n_c], st.v_nrm[:, :, :n_c]), n_c,
+                                         kc.table(device), vc.table(device), kc.bits, vc.bits, *st.window())
+            if full is not None:
+                return full
         total = n_c + st.n_recent
         full_k = torch.empty((B, H, total, D), dtype=key_states.dtype, device=device)
         full_v = torch.empty((B, H, total, D), dtype=value_states.dtype, device=device)
