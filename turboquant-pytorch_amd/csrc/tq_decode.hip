@@ -172,6 +172,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     __shared__ __attribute__((aligned(16))) float lds_corr[DW][16];
     __shared__ float lds_top[MAX_GROUP], lds_den[MAX_GROUP];
     __shared__ uint32_t lds_last;
+    __shared__ uint32_t lds_trips[DW];                   // runs a wave has begun
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = tq_uniform32(tid >> 6);
@@ -252,6 +253,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
         issue_values(std::integral_constant<int, 0>{}, std::false_type{}, t_first);
     }
 
+    if (tid < (uint32_t)DW) lds_trips[tid] = 0u;
     stage_lut<IPBK>(lds_lut_k, a.table_k + hk_hd->off_lut, tid);
     stage_lut<IPBV>(lds_lut_v, a.table_v + hv_hd->off_lut, tid);
 
@@ -555,8 +557,20 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     };
 
     // one trip: stage the run held in register set B, start the loads of the next run into the other set, compute
+    // The two waves of a SIMD (w and w + 4) are kept level: the one that is ahead yields.  Left alone the older of the two is
+    // served first, and the other one ends its runs without anybody to cover its waits: of a row of 16384 tokens the first
+    // waves had done their 32 runs after 69 us and waited 22 us for the others; now all take 84 us and wait one
+    // (512 rows: 213 -> 200 us).  Which wave takes which run stays fixed, so the sums do too.
+    uint32_t trips = 0u;
+    auto keep_level = [&]() __attribute__((always_inline)) {
+        ++trips;
+        volatile uint32_t *count = lds_trips;
+        if (lane == 0u) count[wave] = trips;
+        if (trips > tq_uniform32(count[wave ^ 4u])) __builtin_amdgcn_s_setprio(0); else __builtin_amdgcn_s_setprio(1);
+    };
     auto trip = [&](auto bsel, auto full_tag, uint32_t t0) __attribute__((always_inline)) {
         constexpr int B = decltype(bsel)::value;
+        keep_level();
         constexpr bool FULL = decltype(full_tag)::value;
         const uint32_t n_tok = FULL ? (uint32_t)RUN : t_end - t0;
 #pragma unroll
@@ -632,6 +646,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
             }
         }
         if (t0 < t_end) trip(std::integral_constant<int, 0>{}, std::false_type{}, t0);
+        if (lane == 0u) *(volatile uint32_t *)&lds_trips[wave] = 0xffffffffu;
+        __builtin_amdgcn_s_setprio(0);
     }
     asm volatile("" ::: "memory");
 
