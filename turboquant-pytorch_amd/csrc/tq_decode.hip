@@ -691,9 +691,10 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     }
 
     // ---- the last block of the row finishes it
-    // (one thread's fences do for the block: the barrier before them has every wave's stores in the L2, the one behind them
-    // keeps the other waves' loads back; a fence per wave wrote back and invalidated the caches eight times as often: 51 us
-    // for 8 rows x 32768 tokens)
+    // (one thread's fences do for the block: every wave waits for its own stores to reach the L2 before the barrier, which by
+    // itself waits for LDS only, and the barrier behind the fences keeps the other waves' loads back; a fence per wave wrote
+    // back and invalidated the caches eight times as often: 51 us for 8 rows x 32768 tokens)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (splits > 1u) {
         if (tid == 0u) {
