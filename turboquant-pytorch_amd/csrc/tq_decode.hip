@@ -5,9 +5,9 @@
 //                      rotated, the window is attended to and the splits are merged inside the kernel that reads the codes.
 // Few rows: a step is a chain of latencies (tables, query rotation, one or two runs per wave, merge), so launches are what
 // counts; many rows: the main loop, which is bound by the vector and LDS work of the table lookups at 60 % of the issue slots.
-// Per layer and step, six launches / these two (MI355X): 8 rows x 32768 tokens, K4/V2, 4 heads a row 48.8 -> 32.1 us;
+// Per layer and step, six launches / these two (MI355X): 8 rows x 32768 tokens, K4/V2, 4 heads a row 48.8 -> 30.0 us;
 // 512 rows x 16384 tokens 223 -> 211 us; head dimension 64, 32 rows x 6000 tokens, K6/V4 (before: de-quantised to float32 and
-// multiplied by library products) 190 -> 27 us.
+// multiplied by library products) 190 -> 25 us.
 // What they compute is what tq_compress and the prepare / partials / merge trio of tq_attend.hip compute (upstream
 // turboquant/generation_test_v2.py:96-135, score definition validate_v3.py:87); those remain for float32 elements.
 #include <atomic>
@@ -48,6 +48,20 @@ __device__ __forceinline__ tq_f4v mfma16_f16(tq_u4 a, tq_u4 b, tq_f4v c) {
 }
 __device__ __forceinline__ tq_f4v mfma16_bf16(tq_u4 a, tq_u4 b, tq_f4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tq_bf8, a), __builtin_bit_cast(tq_bf8, b), c, 0, 0, 0);
+}
+
+// Records of a row with several splits travel between blocks past the caches that are not shared (stores and loads of device
+// scope), so that nothing has to be written back or invalidated around the arrival counter: with fences there a step of
+// 8 rows x 32768 tokens took 32.0 us and now 30.0, one of 32 rows x 6000 tokens, 64 wide, 27.3 and now 24.7.  A row with one split keeps
+// its records in its own block: they stay cached (512 rows x 16384 tokens: 2 % longer otherwise).
+__device__ __forceinline__ void put_record(bool across, TQ_GLOBAL float *p, float v) {
+    if (across) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+template <bool ACROSS>
+__device__ __forceinline__ float get_record(const TQ_GLOBAL float *p) {
+    if constexpr (ACROSS) return __hip_atomic_load(const_cast<TQ_GLOBAL float *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return *p;
 }
 
 // The byte -> centroids table spread over the banks (RepLut): consecutive threads write consecutive 16-byte pieces, so the
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
         }
         constexpr float DOWN = BF ? 1.f : 1.f / 16384.f;
         TQ_GLOBAL float *rec = (TQ_GLOBAL float *)a.win_part + ((size_t)row * win_tiles + wt) * G * PART;
-        if (q4 == 0u && live) { rec[n16 * PART] = m; rec[n16 * PART + 1u] = l; }
+        if (q4 == 0u && live) { put_record(splits > 1u, rec + n16 * PART, m); put_record(splits > 1u, rec + n16 * PART + 1u, l); }
         // columns in chunks of 8 (or 4, 2): the same element of token pairs side by side, one operand per coordinate
         auto columns = [&](auto n_tag, int c0) __attribute__((always_inline)) {
             constexpr int N = decltype(n_tag)::value;
@@ -371,7 +385,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
                 for (int k = 0; k < TERMS; ++k) acc = mm(pa[k], bt, acc);
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (4u * q4 + r < G) rec[(4u * q4 + r) * PART + 2u + first + (uint32_t)c] = acc[r] * DOWN;
+                    if (4u * q4 + r < G) put_record(splits > 1u, rec + (4u * q4 + r) * PART + 2u + first + (uint32_t)c, acc[r] * DOWN);
             }
         };
         if constexpr (D == 64) columns(std::integral_constant<int, 4>{}, 0);
@@ -686,24 +700,19 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
 #pragma unroll
                 for (int w = 0; w < DW; ++w) v += __expf(mw[w] - mall) * reinterpret_cast<const float *>(lds_area[w])[g * PART + j];
             }
-            ((TQ_GLOBAL float *)dst)[h0 * PART + i] = v;
+            put_record(splits > 1u, (TQ_GLOBAL float *)dst + h0 * PART + i, v);
         }
     }
 
     // ---- the last block of the row finishes it
-    // (one thread's fences do for the block: every wave waits for its own stores to reach the L2 before the barrier, which by
-    // itself waits for LDS only, and the barrier behind the fences keeps the other waves' loads back; a fence per wave wrote
-    // back and invalidated the caches eight times as often: 51 us for 8 rows x 32768 tokens)
+    // (the records were stored at device scope: once a wave has waited for its own stores, which the barrier by itself does not
+    // do, they can be counted as there)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (splits > 1u) {
         if (tid == 0u) {
-            __threadfence();
-            const bool last = atomicAdd(a.arrived + row, 1u) == splits - 1u;
-            if (last) {
-                atomicExch(a.arrived + row, 0u);
-                __threadfence();
-            }
+            const bool last = __hip_atomic_fetch_add(a.arrived + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1u;
+            if (last) __hip_atomic_store(a.arrived + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             lds_last = last ? 1u : 0u;
         }
         __syncthreads();
@@ -722,43 +731,47 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
         }
     };
     if constexpr (ROTK == RH) load_pv(0);
-    // weights of the records: exp(reference - largest reference of the head)
-    float *wgt = reinterpret_cast<float *>(lds_lut_k);            // [head][splits + window tiles]
-    const uint32_t nrec = splits + win_tiles;
-    for (uint32_t g = wave; g < G; g += DW) {
-        float m = -3.0e38f;
-        for (uint32_t s = lane; s < nrec; s += 64u) {
-            const float x = s < splits ? part[((size_t)s * G + g) * PART] : wpart[((size_t)(s - splits) * G + g) * PART];
-            m = fmaxf(m, x);
-        }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
-        float den = 0.f;
-        for (uint32_t s = lane; s < nrec; s += 64u) {
-            const TQ_GLOBAL float *r = s < splits ? part + ((size_t)s * G + g) * PART : wpart + ((size_t)(s - splits) * G + g) * PART;
-            const float f = __expf(r[0] - m);
-            wgt[g * nrec + s] = f;
-            den = fmaf(f, r[1], den);
-        }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) den += __shfl_xor(den, d);
-        if (lane == 0u) lds_den[g] = den;
-    }
-    __syncthreads();
     float *ysum = reinterpret_cast<float *>(&lds_area[0][0]);     // [head][D]: sums in the rotated space
     float *wsum = ysum + MAX_GROUP * D;                           // [head][D]: the window's, plain
-    for (uint32_t p = tid; p < G * D; p += DTHREADS) {
-        const uint32_t g = p / D, j = p % D;
-        const float *f = wgt + g * nrec;
-        float y = 0.f, w = 0.f;
+    auto merge = [&](auto across_tag) __attribute__((always_inline)) {
+        constexpr bool ACROSS = decltype(across_tag)::value;
+        // weights of the records: exp(reference - largest reference of the head)
+        float *wgt = reinterpret_cast<float *>(lds_lut_k);            // [head][splits + window tiles]
+        const uint32_t nrec = splits + win_tiles;
+        for (uint32_t g = wave; g < G; g += DW) {
+            float m = -3.0e38f;
+            for (uint32_t s = lane; s < nrec; s += 64u) {
+                const float x = get_record<ACROSS>(s < splits ? part + ((size_t)s * G + g) * PART : wpart + ((size_t)(s - splits) * G + g) * PART);
+                m = fmaxf(m, x);
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+            float den = 0.f;
+            for (uint32_t s = lane; s < nrec; s += 64u) {
+                const TQ_GLOBAL float *r = s < splits ? part + ((size_t)s * G + g) * PART : wpart + ((size_t)(s - splits) * G + g) * PART;
+                const float f = __expf(get_record<ACROSS>(r) - m);
+                wgt[g * nrec + s] = f;
+                den = fmaf(f, get_record<ACROSS>(r + 1), den);
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) den += __shfl_xor(den, d);
+            if (lane == 0u) lds_den[g] = den;
+        }
+        __syncthreads();
+        for (uint32_t p = tid; p < G * D; p += DTHREADS) {
+            const uint32_t g = p / D, j = p % D;
+            const float *f = wgt + g * nrec;
+            float y = 0.f, w = 0.f;
 #pragma unroll 8
-        for (uint32_t s = 0; s < splits; ++s) y = fmaf(f[s], part[((size_t)s * G + g) * PART + 2u + j], y);
+            for (uint32_t s = 0; s < splits; ++s) y = fmaf(f[s], get_record<ACROSS>(part + ((size_t)s * G + g) * PART + 2u + j), y);
 #pragma unroll 4
-        for (uint32_t s = 0; s < win_tiles; ++s) w = fmaf(f[splits + s], wpart[((size_t)s * G + g) * PART + 2u + j], w);
-        ysum[p] = y;
-        wsum[p] = w;
-    }
-    __syncthreads();
+            for (uint32_t s = 0; s < win_tiles; ++s) w = fmaf(f[splits + s], get_record<ACROSS>(wpart + ((size_t)s * G + g) * PART + 2u + j), w);
+            ysum[p] = y;
+            wsum[p] = w;
+        }
+        __syncthreads();
+    };
+    if (splits > 1u) merge(std::true_type{}); else merge(std::false_type{});
     // out = (ysum @ Pi_v + wsum) / den, four heads at a time
     float *parts = reinterpret_cast<float *>(lds_lut_v);          // [part][4][D]
     for (uint32_t g0 = 0; g0 < G; g0 += 4u) {
