@@ -479,6 +479,61 @@ def test_v3cache_refuses_cpu_tensors_and_reports_state(pkg):
         pkg.V3Cache(key_bits=4, value_bits=2).attend(torch.zeros(1, 4, 1, 128), 0)
 
 
+class _Recorder:
+    """The native library with the two calls of a decode step replaced by a list of their arguments (nothing is launched)."""
+
+    def __init__(self, lib):
+        self._lib, self.calls = lib, []
+
+    def __getattr__(self, name):
+        if name in ("tq_decode_append", "tq_append_token", "tq_decode_attend", "tq_attend_step"):
+            return lambda *args: self.calls.append((name, args)) or 0
+        return getattr(self._lib, name)
+
+
+@pytest.fixture
+def recorded(pkg, monkeypatch):
+    """The cache's host logic on CPU tensors: launches of a decode step are recorded, those of the codec left out."""
+    native = pkg._native
+    rec = _Recorder(native.lib())
+    monkeypatch.setattr(native, "lib", lambda: rec)
+    monkeypatch.setattr(native, "call", lambda name, *args: rec.calls.append((name, args)))
+    monkeypatch.setattr(native, "_stream_handle", lambda device: 0)
+    monkeypatch.setattr(pkg.compressors_v3.MSECompressor, "table", lambda self, device=None: torch.from_numpy(self._table_host))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    return rec
+
+
+def _steady_cache(pkg, dim, B=2, H=8, window=4):
+    """A bf16 cache on the CPU whose window is full: the next token takes the one-call step."""
+    cache = pkg.V3Cache(4, 2, residual_window=window, n_layers=40, capacity=256)
+    x = torch.randn(B, H, window, dim).to(torch.bfloat16)
+    cache.append(x, x, 8)
+    return cache, cache._stores[8]
+
+
+@pytest.mark.parametrize("dim", [64, 96, 128, 256])
+def test_decode_step_looks_at_the_shape_of_the_values(pkg, recorded, dim):
+    """Values of another shape than the keys are not handed to the one-call step, which reads both at the store's geometry:
+    what broadcasts is broadcast by the general path, the rest is refused."""
+    cache, st = _steady_cache(pkg, dim)
+    token = lambda *shape: torch.randn(shape).to(torch.bfloat16)  # noqa: E731
+    k = token(2, 8, 1, dim)
+    cache.append(k, token(2, 8, 1, dim), 8)
+    assert [name for name, _ in recorded.calls] == ["tq_decode_append"]
+    del recorded.calls[:]
+    v = token(1, 8, 1, dim)
+    cache.append(k, v, 8)
+    assert not any(name in ("tq_decode_append", "tq_append_token") for name, _ in recorded.calls)
+    assert torch.equal(st.window()[1][:, :, -1:], v.expand(2, 8, 1, dim))
+    for shape in ((2, 8, 1, 2 * dim), (2, 8, 1, dim // 2), (2, 4, 1, dim), (2, 8, 3, dim), (4, 8, 1, dim)):
+        cache, st = _steady_cache(pkg, dim)
+        del recorded.calls[:]
+        with pytest.raises(RuntimeError):
+            cache.append(k, token(*shape), 8)
+        assert not any(name in ("tq_decode_append", "tq_append_token") for name, _ in recorded.calls), shape
+
+
 def test_tables_for_other_head_dimensions(pkg):
     """Tables for head dimensions other than 128: section sizes follow d (d/32 row tiles x d/16 steps of 1 KiB per
     operand term), the operands hold Pi in the compress tiling for both directions, and the quantiser grid may use

@@ -139,7 +139,8 @@ class _LayerStore:
         if (rw == 0 or not (self.one_launch or self.D == _native.HEAD_DIM)
                 or self.n_recent != rw or self.w0 + rw + 1 > self.win_cap or self.n_compressed + 1 > self.capacity
                 or keys.dtype != self.dtype or values.dtype != self.dtype or keys.device != self.device
-                or values.device != self.device or torch.compiler.is_compiling()):
+                or values.device != self.device or torch.compiler.is_compiling()
+                or keys.shape != (self.B, self.H, 1, self.D) or values.shape != keys.shape):    # the call reads both at the store's geometry
             return False
         rows = self.B * self.H
         strides = []
