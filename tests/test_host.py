@@ -501,6 +501,9 @@ def recorded(pkg, monkeypatch):
     monkeypatch.setattr(native, "_stream_handle", lambda device: 0)
     monkeypatch.setattr(pkg.compressors_v3.MSECompressor, "table", lambda self, device=None: torch.from_numpy(self._table_host))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    for kept in ("_workspaces", "_step_scratch", "_arrived"):       # (what the calls keep per stream)
+        monkeypatch.setattr(native, kept, {})
     return rec
 
 
@@ -532,6 +535,23 @@ def test_decode_step_looks_at_the_shape_of_the_values(pkg, recorded, dim):
         with pytest.raises(RuntimeError):
             cache.append(k, token(*shape), 8)
         assert not any(name in ("tq_decode_append", "tq_append_token") for name, _ in recorded.calls), shape
+
+
+@pytest.mark.parametrize("dim", [64, 96, 128, 256])
+def test_attend_looks_at_the_width_of_the_queries(pkg, recorded, dim):
+    """Queries of another width than the store's are refused before anything is launched: the kernel takes the width from the
+    layer's record and would read and write past them."""
+    cache, _ = _steady_cache(pkg, dim)
+    query = lambda width: torch.zeros(2, 16, 1, width, dtype=torch.bfloat16)  # noqa: E731
+    cache.attend(query(dim), 8)
+    assert [name for name, _ in recorded.calls] == ["tq_decode_attend"]
+    del recorded.calls[:]
+    for width in (32, 64, 80, 96, 128, 256):
+        for fused in (None, True, False):
+            if width != dim:
+                with pytest.raises(ValueError, match="one query token per sequence"):
+                    cache.attend(query(width), 8, fused=fused)
+    assert not recorded.calls
 
 
 def test_tables_for_other_head_dimensions(pkg):

@@ -316,7 +316,7 @@ class V3Cache:
         if st is None or st.total_seq == 0:
             raise ValueError(f"attend: nothing is cached for layer {layer_idx}")
         B, Hq, Sq, D = query_states.shape
-        if Sq != 1 or B != st.B or Hq % st.H:
+        if Sq != 1 or B != st.B or Hq % st.H or D != st.D:
             raise ValueError(f"attend needs one query token per sequence, [B={st.B}, k*{st.H}, 1, {st.D}]; got {tuple(query_states.shape)}")
         G = Hq // st.H
         scale = D ** -0.5 if scale is None else scale
