@@ -554,6 +554,40 @@ def test_attend_looks_at_the_width_of_the_queries(pkg, recorded, dim):
     assert not recorded.calls
 
 
+def test_attend_packed_looks_at_every_operand(pkg, recorded, monkeypatch):
+    """The operator's kernels take every size from the queries and the key codes: operands of another shape, element type or
+    device are refused before anything is launched."""
+    native = pkg._native
+    monkeypatch.setattr(native, "_require_gpu", lambda t, what: None)
+    comp = pkg.TurboQuantV3(64, key_bits=4, value_bits=2, layer_idx=8)
+    kc, vc = comp.key_compressor, comp.val_compressor
+    B, H, G, S, n_w, D = 2, 3, 2, 40, 8, 64
+    good = dict(queries=torch.zeros(B, H * G, 1, D, dtype=torch.bfloat16), k_idx=torch.zeros(B, H, S, 32, dtype=torch.uint8),
+                k_norms=torch.zeros(B, H, S, dtype=torch.float16), v_idx=torch.zeros(B, H, S, 16, dtype=torch.uint8),
+                v_norms=torch.zeros(B, H, S, dtype=torch.float16), table_k=kc.table(), table_v=vc.table(), bits_k=4, bits_v=2,
+                pi_k_t=kc.Pi.t(), pi_v=vc.Pi, k_win=torch.zeros(B, H, n_w, D, dtype=torch.bfloat16),
+                v_win=torch.zeros(B, H, n_w, D, dtype=torch.bfloat16), scale=0.125)
+    assert native._attend_packed_impl(**good).shape == (B, H * G, 1, D)
+    empty = {k: good[k][:, :, :0] for k in ("k_idx", "k_norms", "v_idx", "v_norms")}
+    native._attend_packed_impl(**{**good, **empty})
+    native._attend_packed_impl(**{**good, "k_win": good["k_win"][:, :, :0], "v_win": good["v_win"][:, :, :0]})
+    assert len(recorded.calls) == 3
+    del recorded.calls[:]
+    z = lambda like, *shape: torch.zeros(shape, dtype=good[like].dtype)  # noqa: E731
+    bad = [("queries", z("queries", B, H * G, 1, 96)), ("queries", z("queries", B, H * G, 2, D)), ("queries", z("queries", B, H * G + 1, 1, D)),
+           ("queries", z("queries", B + 1, H * G, 1, D)), ("k_idx", z("k_idx", B, H, S, 16)), ("k_norms", z("k_norms", B, H, S - 1)),
+           ("v_idx", z("v_idx", B, H, S - 1, 16)), ("v_idx", z("v_idx", B, H, S, 32)), ("v_norms", z("v_norms", B, 1, S)),
+           ("k_win", z("k_win", B, H, n_w, 32)), ("v_win", z("v_win", B, H, n_w - 1, D)), ("v_win", z("v_win", 1, H, n_w, D)),
+           ("pi_v", z("pi_v", 32, 32)), ("pi_k_t", z("pi_k_t", 128, 128)), ("pi_v", good["pi_v"].double()),
+           ("bits_k", 9), ("bits_v", 0),
+           ("k_norms", good["k_norms"].float()), ("v_win", good["v_win"].float()), ("v_idx", good["v_idx"].int()), ("k_win", good["k_win"].to("meta")),
+           ("v_idx", good["v_idx"].to("meta")), ("table_v", good["table_v"].to("meta"))]
+    for name, other in bad:
+        with pytest.raises(native.TqError):
+            native._attend_packed_impl(**{**good, name: other})
+        assert not recorded.calls, (name, other)
+
+
 def test_tables_for_other_head_dimensions(pkg):
     """Tables for head dimensions other than 128: section sizes follow d (d/32 row tiles x d/16 steps of 1 KiB per
     operand term), the operands hold Pi in the compress tiling for both directions, and the quantiser grid may use

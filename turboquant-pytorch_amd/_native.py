@@ -862,13 +862,38 @@ def _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_
     return decode_attend(layer, q, Hq // H, scale, 0, n_w, S)
 
 
+def _check_attend_packed(queries, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_k_t, pi_v, k_win, v_win):
+    """The kernels take every size from the queries and the key codes; what does not fit them would be read out of range."""
+    B, Hq, Sq, D = queries.shape
+    H, S, n_w = k_idx.shape[1], k_idx.shape[2], k_win.shape[2]
+    fits = (Sq == 1 and H > 0 and Hq % H == 0 and 1 <= bits_k <= 8 and 1 <= bits_v <= 8
+            and pi_k_t.shape == pi_v.shape == (D, D) and pi_k_t.dtype == pi_v.dtype == torch.float32)
+    used = [table_k, table_v, pi_k_t, pi_v]
+    if S:
+        fits = (fits and k_idx.shape == (B, H, S, _packed_width(D, bits_k)) and v_idx.shape == (B, H, S, _packed_width(D, bits_v))
+                and k_norms.shape == v_norms.shape == (B, H, S) and k_idx.dtype == v_idx.dtype == torch.uint8
+                and k_norms.dtype == v_norms.dtype == torch.float16)
+        used += [k_idx, k_norms, v_idx, v_norms]
+    if n_w:
+        fits = fits and k_win.shape == v_win.shape == (B, H, n_w, D) and k_win.dtype == v_win.dtype
+        used += [k_win, v_win]
+    if not fits:
+        raise TqError(f"attend_packed: operands do not fit queries {tuple(queries.shape)}, key codes {tuple(k_idx.shape)} and a window of {n_w}")
+    if any(t.device != queries.device for t in used):
+        raise TqError(f"attend_packed: every operand must live on {queries.device}, as the queries do")
+    check_table(table_k, D, bits_k)
+    check_table(table_v, D, bits_v)
+
+
 def _attend_packed_impl(queries: torch.Tensor, k_idx: torch.Tensor, k_norms: torch.Tensor, v_idx: torch.Tensor,
                         v_norms: torch.Tensor, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int,
                         pi_k_t: torch.Tensor, pi_v: torch.Tensor, k_win: torch.Tensor, v_win: torch.Tensor,
                         scale: float) -> torch.Tensor:
     """Decode-step attention of queries [B,Hq,1,D] over a packed history ([B,H,S,..] store slices, S may be 0)
-    plus uncompressed window tokens [B,H,n_w,D] (n_w may be 0, not both): three launches."""
+    plus uncompressed window tokens [B,H,n_w,D] (n_w may be 0, not both): one launch where tq_decode_attend takes the
+    combination, otherwise three."""
     _require_gpu(queries, "queries")
+    _check_attend_packed(queries, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_k_t, pi_v, k_win, v_win)
     B, Hq, _, D = queries.shape
     H = k_idx.shape[1]
     S = k_idx.shape[2]
