@@ -4,8 +4,10 @@ Codebook and rotation against tables written by the reference, the quantiser tab
 brute force, byte accounting and layer-bit selection against the reference's outputs, error
 behaviour of the C entry points, and that the library exports what include/tqamd.h declares.
 """
+import copy
 import ctypes
 import os
+import pickle
 import re
 import shutil
 import subprocess
@@ -586,6 +588,28 @@ def test_attend_packed_looks_at_every_operand(pkg, recorded, monkeypatch):
         with pytest.raises(native.TqError):
             native._attend_packed_impl(**{**good, name: other})
         assert not recorded.calls, (name, other)
+
+
+@pytest.mark.parametrize("dim,dtype", [(64, torch.bfloat16), (128, torch.float16), (128, torch.float32)])
+def test_a_cache_can_be_copied_after_a_decode_step(pkg, recorded, dim, dtype):
+    """deepcopy and pickle of a cache (a prompt's cache kept for several continuations) whose layers hold the addresses of their
+    buffers for the decode step: the copy holds its own."""
+    cache = pkg.V3Cache(4, 2, residual_window=4, n_layers=40, capacity=256)
+    x = torch.randn(2, 8, 5, dim).to(dtype)
+    cache.append(x[:, :, :4], x[:, :, :4], 8)
+    for _ in range(2):
+        cache.append(x[:, :, 4:], x[:, :, 4:], 8)
+        cache.attend(x[:, :, 4:], 8)
+    st = cache._stores[8]
+    where = lambda s: (s.record().k_win, s.record().v_idx, s.record().table_k) if s.one_launch else (s.consts().k_win, s.consts().v_idx, s.consts().pi_v)  # noqa: E731
+    before = where(st)
+    for copied in (copy.deepcopy(cache), pickle.loads(pickle.dumps(cache))):
+        other = copied._stores[8]
+        assert where(st) == before
+        assert where(other)[0] == other.k_win.data_ptr() and where(other)[1] == other.v_idx.data_ptr()
+        assert all(a != b for a, b in zip(where(other)[:2], before))
+        assert (other.n_compressed, other.n_recent, other.w0) == (st.n_compressed, st.n_recent, st.w0)
+        assert torch.equal(other.k_win.view(torch.uint8), st.k_win.view(torch.uint8))       # (bits: the recorded step has written nothing)
 
 
 def test_tables_for_other_head_dimensions(pkg):

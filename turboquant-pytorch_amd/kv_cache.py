@@ -75,6 +75,10 @@ class _LayerStore:
         self.one_launch = _native.decode_supported(D, dtype, comp.key_bits, comp.value_bits)
         self.reserve(capacity)
 
+    def __getstate__(self):
+        """A copy (deepcopy, pickle) has buffers of its own: the addresses kept for the decode step stay behind."""
+        return {**self.__dict__, "_consts": None, "_record": None}
+
     @staticmethod
     def _width(D: int, bits: int) -> int:
         ipb = 8 // bits
