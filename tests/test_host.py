@@ -11,6 +11,7 @@ import pickle
 import re
 import shutil
 import subprocess
+import weakref
 
 import numpy as np
 import pytest
@@ -485,11 +486,11 @@ class _Recorder:
     """The native library with the two calls of a decode step replaced by a list of their arguments (nothing is launched)."""
 
     def __init__(self, lib):
-        self._lib, self.calls = lib, []
+        self._lib, self.calls, self.answer = lib, [], lambda name, args: 0
 
     def __getattr__(self, name):
         if name in ("tq_decode_append", "tq_append_token", "tq_decode_attend", "tq_attend_step"):
-            return lambda *args: self.calls.append((name, args)) or 0
+            return lambda *args: self.calls.append((name, args)) or self.answer(name, args)
         return getattr(self._lib, name)
 
 
@@ -610,6 +611,33 @@ def test_a_cache_can_be_copied_after_a_decode_step(pkg, recorded, dim, dtype):
         assert all(a != b for a, b in zip(where(other)[:2], before))
         assert (other.n_compressed, other.n_recent, other.w0) == (st.n_compressed, st.n_recent, st.w0)
         assert torch.equal(other.k_win.view(torch.uint8), st.k_win.view(torch.uint8))       # (bits: the recorded step has written nothing)
+
+
+def test_scratch_of_a_large_decode_step_is_given_back(pkg, recorded, monkeypatch):
+    """What a stream keeps for its decode steps is bounded: a step that needs more takes it for the call, and holds it until
+    the launch has been made."""
+    native = pkg._native
+    handed = []
+    kept = native.step_scratch
+
+    def watched(*args):
+        buf = kept(*args)
+        handed.append(weakref.ref(buf))
+        return buf
+
+    monkeypatch.setattr(native, "step_scratch", watched)
+
+    def answer(name, args):
+        assert handed[-1]() is not None and args[7] == handed[-1]().data_ptr()
+        need = recorded._lib.tq_decode_scratch_floats(rows, 16, 128, args[6], args[5])
+        return 0 if args[8] >= need else native.ERR_CAPACITY
+
+    recorded.answer = answer
+    for rows, n_win in ((8, 128), (4096, 512), (8, 512), (300, 512)):
+        layer = native.TqDecodeLayer(rows=rows, head_dim=128)
+        native.decode_attend(layer, torch.zeros(rows, 16, 128, dtype=torch.float16), 16, 1.0, 0, n_win, 100)
+        assert sum(t.numel() for t in native._step_scratch.values()) <= native.SCRATCH_KEPT
+    assert max(args[8] for _, args in recorded.calls) > native.SCRATCH_KEPT
 
 
 def test_tables_for_other_head_dimensions(pkg):

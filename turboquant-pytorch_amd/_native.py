@@ -463,12 +463,15 @@ def _drop_workspace(device: torch.device, stream: int) -> None:
 
 
 _step_scratch: Dict[Tuple[int, int], torch.Tensor] = {}
+SCRATCH_KEPT = 1 << 24          # float32 values a stream keeps at most: 64 MiB
 
 
 def step_scratch(device: torch.device, stream: int, floats: int) -> Optional[torch.Tensor]:
-    """float32 scratch of a decode step (rotated queries, window record, split records), one buffer per
+    """float32 scratch of a decode step (rotated queries, window records, split records), one buffer per
     (device, stream), grown on demand: the steps of all layers on a stream run one after the other.  One entry per
-    stream that ever ran a decode step, kept for the life of the process (a few hundred KiB each).
+    stream that ever ran a decode step, kept for the life of the process: a few hundred KiB for a handful of sequences, 5 MiB for
+    512 rows of 4 heads with a window of 128 tokens (a record per 32 window tokens and head), SCRATCH_KEPT at most.  What needs
+    more gets a tensor of its own, which the caller holds until its launches have been queued on `stream`.
     None while a graph is being captured: the caller then takes the general path, whose scratch comes from the
     graph's own memory pool."""
     if torch.cuda.is_current_stream_capturing():
@@ -476,7 +479,9 @@ def step_scratch(device: torch.device, stream: int, floats: int) -> Optional[tor
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     buf = _step_scratch.get(key)
     if buf is None or buf.numel() < floats:
-        buf = _step_scratch[key] = torch.empty(max(floats, 1 << 16), dtype=torch.float32, device=device)
+        buf = torch.empty(max(floats, 1 << 16), dtype=torch.float32, device=device)
+        if floats <= SCRATCH_KEPT:
+            _step_scratch[key] = buf
     return buf
 
 
@@ -511,8 +516,8 @@ def decode_attend(layer: TqDecodeLayer, queries: torch.Tensor, group: int, scale
                             counters.data_ptr(), out.data_ptr(), stream)
         rc = L.tq_decode_attend(*args(scratch))
         if rc == ERR_CAPACITY:
-            need = int(L.tq_decode_scratch_floats(layer.rows, group, layer.head_dim, tokens, n_win))
-            rc = L.tq_decode_attend(*args(step_scratch(dev, stream, need)))
+            scratch = step_scratch(dev, stream, int(L.tq_decode_scratch_floats(layer.rows, group, layer.head_dim, tokens, n_win)))
+            rc = L.tq_decode_attend(*args(scratch))
     if rc:
         _arrived.pop((dev.index if dev.index is not None else torch.cuda.current_device(), stream), None)
     check(rc, "tq_decode_attend")
