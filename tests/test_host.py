@@ -483,13 +483,13 @@ def test_v3cache_refuses_cpu_tensors_and_reports_state(pkg):
 
 
 class _Recorder:
-    """The native library with the two calls of a decode step replaced by a list of their arguments (nothing is launched)."""
+    """The native library with the calls of a decode step and of the V2 scores replaced by a list of their arguments (nothing is launched)."""
 
     def __init__(self, lib):
         self._lib, self.calls, self.answer = lib, [], lambda name, args: 0
 
     def __getattr__(self, name):
-        if name in ("tq_decode_append", "tq_append_token", "tq_decode_attend", "tq_attend_step"):
+        if name in ("tq_decode_append", "tq_append_token", "tq_decode_attend", "tq_attend_step", "tq_qjl_scores"):
             return lambda *args: self.calls.append((name, args)) or self.answer(name, args)
         return getattr(self._lib, name)
 
@@ -589,6 +589,21 @@ def test_attend_packed_looks_at_every_operand(pkg, recorded, monkeypatch):
         with pytest.raises(native.TqError):
             native._attend_packed_impl(**{**good, name: other})
         assert not recorded.calls, (name, other)
+
+
+def test_v2_scores_look_at_the_shape_of_the_queries(pkg, recorded, monkeypatch):
+    """The scores kernel reads a rotated and a projected query per row of the keys: queries of another width, batch or head
+    count are refused before anything is launched."""
+    monkeypatch.setattr(pkg._native, "_require_gpu", lambda t, what: None)
+    comp = pkg.TurboQuantCompressorV2(128, 3, seed=42)
+    packed = comp.empty_packed(2, 4, 50, "cpu")
+    assert comp.asymmetric_attention_scores(torch.zeros(2, 4, 3, 128), packed).shape == (2, 4, 3, 50)
+    assert [name for name, _ in recorded.calls] == ["tq_qjl_scores"]
+    del recorded.calls[:]
+    for shape in ((2, 4, 2, 64), (2, 4, 3, 256), (2, 4, 1, 384), (1, 4, 3, 128), (2, 2, 3, 128), (2, 1, 3, 128), (4, 4, 3, 128)):
+        with pytest.raises(ValueError, match="do not fit keys"):
+            comp.asymmetric_attention_scores(torch.zeros(shape), packed)
+        assert not recorded.calls, shape
 
 
 @pytest.mark.parametrize("dim,dtype", [(64, torch.bfloat16), (128, torch.float16), (128, torch.float32)])

@@ -211,6 +211,8 @@ class TurboQuantCompressorV2:
             term1 = torch.matmul(q, exp["k_mse"].float().transpose(-2, -1))
             ip = torch.matmul(torch.matmul(q, self._s(dev).T), exp["qjl_signs"].float().transpose(-2, -1))
             return term1 + corr * ip * compressed["residual_norm"].float().unsqueeze(-2)
+        if q.shape[-1] != D or q.numel() != B * H * S_q * D:       # the kernel reads one query per row of the keys, the reshape below would take any width
+            raise ValueError(f"queries {tuple(q.shape)} do not fit keys {(B, H, S_k, D)}: [{B}, {H}, S_q, {D}] expected")
         st = self._s_on.get(("t", dev))
         if st is None:      # Pi^T and sqrt(pi/2)/m S^T one behind the other, made once per device
             st = self._s_on[("t", dev)] = torch.stack((self._mse.pi_transposed(dev), self._s(dev).T * corr)).contiguous()
