@@ -628,6 +628,22 @@ def test_a_cache_can_be_copied_after_a_decode_step(pkg, recorded, dim, dtype):
         assert torch.equal(other.k_win.view(torch.uint8), st.k_win.view(torch.uint8))       # (bits: the recorded step has written nothing)
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+def test_a_cache_pickled_before_the_one_launch_step(pkg, recorded, dim):
+    """The layers of such a cache have neither a record nor a route, and at 128 the addresses of the process that wrote them."""
+    cache, st = _steady_cache(pkg, dim)
+    k = torch.randn(2, 8, 1, dim).to(torch.bfloat16)
+    state = {**st.__dict__, "_consts": "addresses"}
+    del state["one_launch"], state["_record"]
+    old = type(st).__new__(type(st))
+    old.__setstate__(state)
+    cache._stores[8] = old
+    assert old._consts is None
+    cache.append(k, k, 8)
+    cache.attend(k, 8)
+    assert [name for name, _ in recorded.calls] == ["tq_decode_append", "tq_decode_attend"]
+
+
 def test_scratch_of_a_large_decode_step_is_given_back(pkg, recorded, monkeypatch):
     """What a stream keeps for its decode steps is bounded: a step that needs more takes it for the call, and holds it until
     the launch has been made."""

@@ -79,6 +79,12 @@ class _LayerStore:
         """A copy (deepcopy, pickle) has buffers of its own: the addresses kept for the decode step stay behind."""
         return {**self.__dict__, "_consts": None, "_record": None}
 
+    def __setstate__(self, state):
+        """Also of a cache pickled before there was a one-launch step, which may hold addresses of the process that wrote it."""
+        self.__dict__.update(state)
+        self._consts = self._record = None
+        self.one_launch = _native.decode_supported(self.D, self.dtype, self.comp.key_bits, self.comp.value_bits)
+
     @staticmethod
     def _width(D: int, bits: int) -> int:
         ipb = 8 // bits
