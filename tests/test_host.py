@@ -606,6 +606,15 @@ def test_v2_scores_look_at_the_shape_of_the_queries(pkg, recorded, monkeypatch):
         assert not recorded.calls, shape
 
 
+def test_v2_compressor_pickled_with_its_projection_alone(pkg, recorded, monkeypatch):
+    """A compressor that has computed scores keeps the matrix for them; one pickled when that was S^T alone gets its own."""
+    monkeypatch.setattr(pkg._native, "_require_gpu", lambda t, what: None)
+    comp = pkg.TurboQuantCompressorV2(128, 3, seed=42)
+    comp._s_on[("t", torch.device("cpu"))] = comp.S.T.contiguous()
+    other = pickle.loads(pickle.dumps(comp))
+    assert other.asymmetric_attention_scores(torch.zeros(1, 2, 1, 128), other.empty_packed(1, 2, 10, "cpu")).shape == (1, 2, 1, 10)
+
+
 @pytest.mark.parametrize("dim,dtype", [(64, torch.bfloat16), (128, torch.float16), (128, torch.float32)])
 def test_a_cache_can_be_copied_after_a_decode_step(pkg, recorded, dim, dtype):
     """deepcopy and pickle of a cache (a prompt's cache kept for several continuations) whose layers hold the addresses of their

@@ -213,9 +213,9 @@ class TurboQuantCompressorV2:
             return term1 + corr * ip * compressed["residual_norm"].float().unsqueeze(-2)
         if q.shape[-1] != D or q.numel() != B * H * S_q * D:       # the kernel reads one query per row of the keys, the reshape below would take any width
             raise ValueError(f"queries {tuple(q.shape)} do not fit keys {(B, H, S_k, D)}: [{B}, {H}, S_q, {D}] expected")
-        st = self._s_on.get(("t", dev))
+        st = self._s_on.get(("both", dev))
         if st is None:      # Pi^T and sqrt(pi/2)/m S^T one behind the other, made once per device
-            st = self._s_on[("t", dev)] = torch.stack((self._mse.pi_transposed(dev), self._s(dev).T * corr)).contiguous()
+            st = self._s_on[("both", dev)] = torch.stack((self._mse.pi_transposed(dev), self._s(dev).T * corr)).contiguous()
         # every query token rotated and projected, in one product: [2, B * H * S_q, D]
         q_both = torch.matmul(q.reshape(1, -1, D), st)
         q_rot, q_sign = q_both[0], q_both[1]
