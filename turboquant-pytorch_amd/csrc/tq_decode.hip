@@ -155,7 +155,8 @@ __device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t fir
 // float32 before, take both as two terms (22 bits): the matrix cores are idle most of the time.
 template <int D, int IPBK, int IPBV>
 __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs a) {
-    constexpr bool QLO = D != 128 || IPBK == 1;          // queries as fp16 hi + lo
+    constexpr int QT = D != 128 || IPBK == 1 ? 2 : 1;    // fp16 terms of a rotated query
+    constexpr int QREG = D == 256 && (IPBK == 1 || IPBV == 1) ? 1 : QT;      // terms held in registers, the others in LDS (see below)
     constexpr bool PLO = D != 128;                       // weights as fp16 hi + lo
     constexpr int SETS = D == 256 ? 1 : 2;               // register sets of the loads that run one run ahead
     constexpr int PART = D + 2;
@@ -183,6 +184,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     __shared__ __attribute__((aligned(16))) uint8_t lds_area[DW][AREA];
     __shared__ __attribute__((aligned(16))) float lds_kn[DW][RUN];
     __shared__ __attribute__((aligned(16))) uint16_t lds_vn[DW][RUN];     // value norms / 2^ev_ref as fp16
+    __shared__ __attribute__((aligned(16))) tq_u4 lds_q[QT > QREG ? (QT - QREG) * SK : 1][TQ_WAVE];
     __shared__ __attribute__((aligned(16))) float lds_corr[DW][16];
     __shared__ float lds_top[MAX_GROUP], lds_den[MAX_GROUP];
     __shared__ uint32_t lds_last;
@@ -401,9 +403,10 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     }
     __syncthreads();
 
-    // ---- B operand of the score product: fp16 of q * 2^(10 - e), e = binary exponent of the head's largest magnitude
-    tq_u4 qb[SK];
-    tq_u4 ql[QLO ? SK : 1];
+    // ---- B operand of the score product: fp16 of q * 2^(10 - e), e = binary exponent of the head's largest magnitude.  At 256 with
+    // 8-bit codes on either side registers run out (28 spilled with 8-bit keys and values): the low term, the same in every wave, lies
+    // in LDS and serves both blocks of a step (128 rows x 8000 tokens, K8/V8: 211 -> 156 us).
+    tq_u4 qb[QREG][SK];
     float c1;                // score in base-2 units = t * c1, t = accumulator * key norm
     float rowscale;          // natural score = t * rowscale
     {
@@ -427,15 +430,21 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
         c1 = rowscale * 1.44269504088896341f;
 #pragma unroll
         for (int s = 0; s < SK; ++s) {
-            tq_half8 h, l;
+            tq_half8 term[QT];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float y = live ? x[8 * s + i] * up : 0.f;
-                h[i] = (_Float16)y;
-                l[i] = (_Float16)(y - (float)h[i]);
+                float y = live ? x[8 * s + i] * up : 0.f;
+#pragma unroll
+                for (int k = 0; k < QT; ++k) {
+                    term[k][i] = (_Float16)y;
+                    y -= (float)term[k][i];
+                }
             }
-            qb[s] = __builtin_bit_cast(tq_u4, h);
-            if constexpr (QLO) ql[s] = __builtin_bit_cast(tq_u4, l);
+#pragma unroll
+            for (int k = 0; k < QREG; ++k) qb[k][s] = __builtin_bit_cast(tq_u4, term[k]);
+#pragma unroll
+            for (int k = QREG; k < QT; ++k)         // the same in every wave
+                if (wave == 0u) lds_q[(k - QREG) * SK + s][lane] = __builtin_bit_cast(tq_u4, term[k]);
         }
     }
     __syncthreads();         // (the queries' LDS is the waves' staging area from here on)
@@ -461,16 +470,30 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
         tq_f4v sc[SUB][2];   // register r of block b = token 32 u + 16 b + 4 q4 + r
 #pragma unroll
         for (int u = 0; u < SUB; ++u) {
+            sc[u][0] = sc[u][1] = tq_f4v{0.f, 0.f, 0.f, 0.f};
+            if (!FULL && 32u * u >= n_tok) continue;       // uniform
+            auto step = [&](int b, int s, const tq_u4 (&q)[QT]) __attribute__((always_inline)) {
+                const tq_u4 kd = decode_rep<IPBK, NWK>(kraw[u][b], s, lut_k);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                sc[u][b] = tq_f4v{0.f, 0.f, 0.f, 0.f};
-                if (!FULL && 32u * u >= n_tok) continue;   // uniform
+                for (int k = 0; k < QT; ++k) sc[u][b] = mfma16_f16(kd, q[k], sc[u][b]);
+            };
+            auto terms = [&](int s, tq_u4 (&q)[QT]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int k = 0; k < QT; ++k) q[k] = k < QREG ? qb[k < QREG ? k : 0][s] : lds_q[(k - QREG) * SK + s][lane];
+            };
+            tq_u4 q[QT];
+            if constexpr (QREG == QT) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int s = 0; s < SK; ++s) { terms(s, q); step(b, s, q); }
+            } else {         // a term from LDS serves both blocks
 #pragma unroll
                 for (int s = 0; s < SK; ++s) {
-                    const tq_u4 kd = decode_rep<IPBK, NWK>(kraw[u][b], s, lut_k);
-                    sc[u][b] = mfma16_f16(kd, qb[s], sc[u][b]);
-                    if constexpr (QLO) sc[u][b] = mfma16_f16(kd, ql[s], sc[u][b]);
-                    if (D == 256 && s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                    terms(s, q);
+                    step(0, s, q);
+                    step(1, s, q);
+                    if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);
                 }
             }
         }
