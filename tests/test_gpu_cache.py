@@ -859,6 +859,46 @@ def test_decode_attention_of_other_head_dims_keeps_float32_weights(pkg, dim, bit
     assert err < 3.5e-4, err
 
 
+def _exact_attention(st, q, scale):
+    """float64 attention over a layer's store and window, the centroids rounded to float16 as the kernels hold them."""
+    B, Hq, _, D = q.shape
+    n = st.n_compressed
+    dec = lambda comp, idx, nrm: ((comp.centroids.half().double()[_codes(idx[:, :, :n].contiguous(), comp.bits if comp.bits < 5 else 8, D)] @ comp.Pi.double())  # noqa: E731
+                                  * nrm[:, :, :n].double().unsqueeze(-1))
+    K = torch.cat([dec(st.comp.key_compressor, st.k_idx, st.k_nrm), st.window()[0].double()], 2)
+    V = torch.cat([dec(st.comp.val_compressor, st.v_idx, st.v_nrm), st.window()[1].double()], 2)
+    s = torch.matmul(q.double().reshape(B, st.H, Hq // st.H, D), K.transpose(-2, -1).contiguous()) * scale
+    return torch.matmul(torch.softmax(s, -1), V).reshape(q.shape)
+
+
+def _one_heavy_token(pkg, dim, bits, at, orders, norm):
+    """A cache of 30 tokens (one wave takes them all) and a window of 32, one head, in which the token `at` has a zero value and 2^orders[g] times the weight
+    of every other token for query head g; the others of its part (history or window) share one value of this norm."""
+    g = torch.Generator().manual_seed(dim)
+    k, v = torch.zeros(1, 1, 62, dim), torch.zeros(1, 1, 62, dim)
+    u, val = torch.randn(2, dim, generator=g)
+    lo, hi = (0, 30) if at < 30 else (30, 62)
+    v[:, :, lo:hi] = val * (norm / val.norm())
+    v[:, :, at] = 0
+    k[:, :, at] = 40 * u / u.norm()
+    q = torch.stack([u / u.norm() * (o * np.log(2.0) / 40 * dim ** 0.5) for o in orders])
+    cache = pkg.V3Cache(bits[0], bits[1], residual_window=32, n_layers=40)
+    cache.append(k.half().to(DEV), v.half().to(DEV), 8)
+    return cache, q.half().reshape(1, len(orders), 1, dim).to(DEV)
+
+
+@pytest.mark.parametrize("dim,bits", [(64, (6, 4)), (96, (6, 2)), (256, (8, 8)), (256, (6, 4))])
+def test_decode_attention_keeps_the_bits_of_small_weights(pkg, dim, bits):
+    """One packed token takes nearly all the weight, the others 2^-21 to 2^-22.5 of it each (as float32: 24 bits).  A weight's terms lie on a
+    grid of 2^-34 of the largest one, which is 2^-11.5 of the smallest here; the result is rounded to float16, 2^-11 / sqrt(3) in the
+    mean square at most: 4.5e-4 in all.  Terms on a grid of 2^-30 gave 4.6e-4 to 6.5e-4."""
+    cache, q = _one_heavy_token(pkg, dim, bits, 7, [21 + 1.5 * i / 15 for i in range(16)], 3e4)
+    out = cache.attend(q, 8).double()
+    ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
+    err = float((out - ref).norm() / ref.norm())
+    assert err < 4.5e-4, err
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_attend_takes_queries_at_any_element_address(pkg, dim):
     """Contiguous queries that start in the middle of a buffer, on no 16-byte boundary."""

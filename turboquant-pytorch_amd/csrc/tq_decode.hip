@@ -151,13 +151,18 @@ __device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t fir
 //   * the waves' sums meet in LDS; with several splits per row the block that arrives last at the row's counter merges the
 //     records of all splits and of the window, rotates the value sums back and stores the result.
 // At 128 queries (against 8-bit keys: two terms) and weights enter the packed products as one fp16 term, as in tq_attend_kernel:
-// their 2^-12 roundings stay under what the fp16 centroids cost.  The other head dimensions, whose histories were attended to in
-// float32 before, take both as two terms (22 bits): the matrix cores are idle most of the time.
+// their 2^-12 roundings stay under what the fp16 centroids cost.  The other head dimensions are as exact as float32 arithmetic:
+//   * queries enter as two fp16 terms, Pi of fp16 caches as well (22 bits each).  Logits that come about by cancellation, where the
+//     roundings show, are off by 0.5 to 0.8 of what the same products in float32 are off by (rotation and score, 64 to 256 wide).
+//   * weights enter as three fp16 terms of p * 2^P_SHIFT * (value norm / 2^ev_ref) <= 2^15: 24 bits or more down to 2^-10 of the
+//     reference weight times the largest value norm's binade, a grid of 2^-34 of that below (the smaller SLACK_LOG2, the finer).
+//     Two terms on a grid of 2^-30 lost up to 2^-8 of weights around 2^-22 of the reference, a short history behind one token
+//     that takes nearly everything.  The third one costs 4 to 5 % where rows are many (96 wide, 512 rows x 8000 tokens: 102 -> 107 us).
 template <int D, int IPBK, int IPBV>
 __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs a) {
     constexpr int QT = D != 128 || IPBK == 1 ? 2 : 1;    // fp16 terms of a rotated query
     constexpr int QREG = D == 256 && (IPBK == 1 || IPBV == 1) ? 1 : QT;      // terms held in registers, the others in LDS (see below)
-    constexpr bool PLO = D != 128;                       // weights as fp16 hi + lo
+    constexpr int PT = D != 128 ? 3 : 1;                 // fp16 terms of a weight
     constexpr int SETS = D == 256 ? 1 : 2;               // register sets of the loads that run one run ahead
     constexpr int PART = D + 2;
     constexpr int STEPS = D / 16, TILES = D / 32;        // query rotation: 32x32x16 matrix instructions
@@ -170,7 +175,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     constexpr int SUB = RUN / 32;
     constexpr int VPB = GBV % 16 ? 8 : 16;               // value codes are staged in pieces of this size
     constexpr int VBYTES = RUN * GBV, VPIECES = VBYTES / VPB, NVP = (VPIECES + 63) / 64;
-    constexpr int SLACK_LOG2 = 8;
+    constexpr int SLACK_LOG2 = PT == 1 ? 8 : 4;          // (several terms: the smaller it is, the finer the grid of small weights)
     constexpr int P_SHIFT = 14 - SLACK_LOG2;             // p * 2^P_SHIFT * (value norm / 2^ev_ref < 2) <= 2^15 fits fp16
     constexpr int HR = D == 256 ? 8 : MAX_GROUP;         // heads per round of the merge through LDS
     constexpr int AREA = VBYTES > HR * PART * 4 ? VBYTES : HR * PART * 4;    // per wave: staged value codes, later its sums
@@ -183,7 +188,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     __shared__ __attribute__((aligned(16))) uint8_t lds_lut_v[32768];
     __shared__ __attribute__((aligned(16))) uint8_t lds_area[DW][AREA];
     __shared__ __attribute__((aligned(16))) float lds_kn[DW][RUN];
-    __shared__ __attribute__((aligned(16))) uint16_t lds_vn[DW][RUN];     // value norms / 2^ev_ref as fp16
+    __shared__ __attribute__((aligned(16))) std::conditional_t<PT == 1, uint16_t, float> lds_vn[DW][RUN];     // value norms / 2^ev_ref (uint16_t: as fp16)
     __shared__ __attribute__((aligned(16))) tq_u4 lds_q[QT > QREG ? (QT - QREG) * SK : 1][TQ_WAVE];
     __shared__ __attribute__((aligned(16))) float lds_corr[DW][16];
     __shared__ float lds_top[MAX_GROUP], lds_den[MAX_GROUP];
@@ -548,27 +553,29 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
             l_run += lsum;
             // ---- weights p_j |v_j| / 2^ev_ref: slice j of lane (., q4) = token 32 u + 4 q4 + j (j < 4), 32 u + 16 + 4 q4 + j - 4
             const uint32_t tok_a = 32u * u + 4u * q4, tok_b = tok_a + 16u;
-            tq_half8 h;
-            const tq_u2 vn_a = *reinterpret_cast<const tq_u2 *>(&lds_vn[wave][tok_a]);
-            const tq_u2 vn_b = *reinterpret_cast<const tq_u2 *>(&lds_vn[wave][tok_b]);
-            const tq_u4 nrm = {vn_a[0], vn_a[1], vn_b[0], vn_b[1]};
-            tq_u4 pl = {0u, 0u, 0u, 0u};
-            if constexpr (PLO) {
-                const tq_half8 vn8 = __builtin_bit_cast(tq_half8, nrm);
-                tq_half8 lo;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float x = ps[j] * (float)vn8[j];
-                    h[j] = (_Float16)x;
-                    lo[j] = (_Float16)(x - (float)h[j]);
-                }
-                pl = __builtin_bit_cast(tq_u4, lo);
-            } else {
+            tq_u4 pa[PT];
+            if constexpr (PT == 1) {
+                const tq_u2 vn_a = *reinterpret_cast<const tq_u2 *>(&lds_vn[wave][tok_a]);
+                const tq_u2 vn_b = *reinterpret_cast<const tq_u2 *>(&lds_vn[wave][tok_b]);
+                const tq_u4 nrm = {vn_a[0], vn_a[1], vn_b[0], vn_b[1]};
+                tq_half8 h;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) h[j] = (_Float16)ps[j];
                 h = h * __builtin_bit_cast(tq_half8, nrm);
+                pa[0] = __builtin_bit_cast(tq_u4, h);
+            } else {
+                const float4 va = *reinterpret_cast<const float4 *>(&lds_vn[wave][tok_a]), vb = *reinterpret_cast<const float4 *>(&lds_vn[wave][tok_b]);
+                float x[8] = {ps[0] * va.x, ps[1] * va.y, ps[2] * va.z, ps[3] * va.w, ps[4] * vb.x, ps[5] * vb.y, ps[6] * vb.z, ps[7] * vb.w};
+#pragma unroll
+                for (int k = 0; k < PT; ++k)
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const auto two = __builtin_amdgcn_cvt_pkrtz(x[2 * d], x[2 * d + 1]);
+                        pa[k][d] = __builtin_bit_cast(uint32_t, two);
+                        x[2 * d] -= (float)two[0];
+                        x[2 * d + 1] -= (float)two[1];
+                    }
             }
-            const tq_u4 pa = __builtin_bit_cast(tq_u4, h);
             auto columns = [&](auto n_tag, int c0) __attribute__((always_inline)) {
                 constexpr int N = decltype(n_tag)::value;
                 uint32_t dec[8][N / 2];      // per token: N coordinates of the lane as fp16
@@ -582,8 +589,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
 #pragma unroll
                     for (int d = 0; d < 4; ++d)
                         bt[d] = __builtin_amdgcn_perm(dec[2 * d + 1][c / 2], dec[2 * d][c / 2], (c & 1) ? 0x07060302u : 0x05040100u);
-                    acc[c0 + c] = mfma16_f16(pa, bt, acc[c0 + c]);
-                    if constexpr (PLO) acc[c0 + c] = mfma16_f16(pl, bt, acc[c0 + c]);
+#pragma unroll
+                    for (int k = 0; k < PT; ++k) acc[c0 + c] = mfma16_f16(pa[k], bt, acc[c0 + c]);
                 }
             };
             if constexpr (D == 64) columns(std::integral_constant<int, 4>{}, 0);
@@ -638,8 +645,11 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
                 ev_ref = ev;
             }
             const _Float16 vh = __builtin_bit_cast(_Float16, vn_buf[B]);
-            const _Float16 vs = (_Float16)ldexpf((float)vh, -ev_ref);
-            if (RUN == 64 || lane < (uint32_t)RUN) lds_vn[wave][lane] = __builtin_bit_cast(uint16_t, vs);
+            const float vs = ldexpf((float)vh, -ev_ref);
+            if (RUN == 64 || lane < (uint32_t)RUN) {
+                if constexpr (PT == 1) lds_vn[wave][lane] = __builtin_bit_cast(uint16_t, (_Float16)vs);
+                else lds_vn[wave][lane] = vs;
+            }
         }
         const uint32_t t_next = t0 + RUN * DW;
         constexpr auto nsel = std::integral_constant<int, SETS == 2 ? 1 - B : 0>{};
