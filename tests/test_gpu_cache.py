@@ -899,6 +899,17 @@ def test_decode_attention_keeps_the_bits_of_small_weights(pkg, dim, bits):
     assert err < 4.5e-4, err
 
 
+@pytest.mark.parametrize("dim", [64, 96, 128, 256])
+def test_window_attention_keeps_the_bits_of_small_weights(pkg, dim):
+    """The same inside the window of a float16 cache, 2^-28 to 2^-31: nothing but the rounding of the result is left (5 % for single
+    elements that round the other way).  Probabilities as two float16 terms are off by twice to three times that."""
+    cache, q = _one_heavy_token(pkg, dim, (6, 4), 40, [28 + 3 * i / 15 for i in range(16)], 5e4)
+    out = cache.attend(q, 8).double()
+    ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
+    rounding = float((ref.half().double() - ref).norm())
+    assert float((out - ref).norm()) < 1.05 * rounding
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_attend_takes_queries_at_any_element_address(pkg, dim):
     """Contiguous queries that start in the middle of a buffer, on no 16-byte boundary."""

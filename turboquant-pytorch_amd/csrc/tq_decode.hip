@@ -50,6 +50,19 @@ __device__ __forceinline__ tq_f4v mfma16_bf16(tq_u4 a, tq_u4 b, tq_f4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tq_bf8, a), __builtin_bit_cast(tq_bf8, b), c, 0, 0, 0);
 }
 
+// Exact split of eight fp16 values into two bf16 terms each: a truncation keeps eight of the eleven bits, the rest fits the second.
+__device__ __forceinline__ void split_f16x8(tq_u4 v, tq_u4 &hi, tq_u4 &lo) {
+    const tq_half8 h = __builtin_bit_cast(tq_half8, v);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const uint32_t x0 = __float_as_uint((float)h[2 * d]), x1 = __float_as_uint((float)h[2 * d + 1]);
+        const uint32_t r0 = __float_as_uint(__uint_as_float(x0) - __uint_as_float(x0 & 0xffff0000u));
+        const uint32_t r1 = __float_as_uint(__uint_as_float(x1) - __uint_as_float(x1 & 0xffff0000u));
+        hi[d] = __builtin_amdgcn_perm(x1, x0, 0x07060302u);
+        lo[d] = __builtin_amdgcn_perm(r1, r0, 0x07060302u);
+    }
+}
+
 // Records of a row with several splits travel between blocks past the caches that are not shared (stores and loads of device
 // scope), so that nothing has to be written back or invalidated around the arrival counter: with fences there a step of
 // 8 rows x 32768 tokens took 32.0 us and now 30.0, one of 32 rows x 6000 tokens, 64 wide, 27.3 and now 24.7.  A row with one split keeps
@@ -147,7 +160,8 @@ __device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t fir
 // of the value product, whose B operand is built in the lanes from the staged codes.  Around it, in the same launch:
 //   * waves 0 .. D/32 - 1 rotate the row's queries on the matrix cores (operands of the key codec's table, every term of Pi:
 //     fp32-grade), while the other waves attend to the window, 32 tokens each: raw 16-bit keys and queries multiply exactly,
-//     probabilities enter the value product as two (fp16) or three (bf16) terms that add up to their float32 value;
+//     probabilities enter the value product as three bf16 terms that add up to their float32 value, fp16 values as two that add up to
+//     theirs (two fp16 terms of a probability lie on a grid of 2^-38 of the largest one: at 2^-30 of it eight bits were left);
 //   * the waves' sums meet in LDS; with several splits per row the block that arrives last at the row's counter merges the
 //     records of all splits and of the window, rotates the value sums back and stores the result.
 // At 128 queries (against 8-bit keys: two terms) and weights enter the packed products as one fp16 term, as in tq_attend_kernel:
@@ -351,22 +365,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
         }
         l += __shfl_xor(l, 16);
         l += __shfl_xor(l, 32);
-        constexpr int TERMS = BF ? 3 : 2;
-        tq_u4 pa[TERMS];
-        if constexpr (BF) {
-            split_f32x8(p, pa[0], pa[1], pa[2]);
-        } else {
-            tq_half8 h, lo;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float x = p[j] * 16384.f;
-                h[j] = (_Float16)x;
-                lo[j] = (_Float16)(x - (float)h[j]);
-            }
-            pa[0] = __builtin_bit_cast(tq_u4, h);
-            pa[1] = __builtin_bit_cast(tq_u4, lo);
-        }
-        constexpr float DOWN = BF ? 1.f : 1.f / 16384.f;
+        tq_u4 pa[3];
+        split_f32x8(p, pa[0], pa[1], pa[2]);
         TQ_GLOBAL float *rec = (TQ_GLOBAL float *)a.win_part + ((size_t)row * win_tiles + wt) * G * PART;
         if (q4 == 0u && live) { put_record(splits > 1u, rec + n16 * PART, m); put_record(splits > 1u, rec + n16 * PART + 1u, l); }
         // columns in chunks of 8 (or 4, 2): the same element of token pairs side by side, one operand per coordinate
@@ -388,11 +388,16 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
                 for (int d = 0; d < 4; ++d)
                     bt[d] = __builtin_amdgcn_perm(v[2 * d + 1][c / 2], v[2 * d][c / 2], (c & 1) ? 0x07060302u : 0x05040100u);
                 tq_f4v acc = tq_f4v{0.f, 0.f, 0.f, 0.f};
+                tq_u4 hi = bt, lo;
+                if constexpr (!BF) split_f16x8(bt, hi, lo);
 #pragma unroll
-                for (int k = 0; k < TERMS; ++k) acc = mm(pa[k], bt, acc);
+                for (int k = 0; k < 3; ++k) {
+                    acc = mfma16_bf16(pa[k], hi, acc);
+                    if constexpr (!BF) acc = mfma16_bf16(pa[k], lo, acc);
+                }
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (4u * q4 + r < G) put_record(splits > 1u, rec + (4u * q4 + r) * PART + 2u + first + (uint32_t)c, acc[r] * DOWN);
+                    if (4u * q4 + r < G) put_record(splits > 1u, rec + (4u * q4 + r) * PART + 2u + first + (uint32_t)c, acc[r]);
             }
         };
         if constexpr (D == 64) columns(std::integral_constant<int, 4>{}, 0);
