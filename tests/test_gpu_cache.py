@@ -910,6 +910,30 @@ def test_window_attention_keeps_the_bits_of_small_weights(pkg, dim):
     assert float((out - ref).norm()) < 1.05 * rounding
 
 
+@pytest.mark.parametrize("dim", [64, 96, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_infinite_window_values_stay_in_their_coordinate(pkg, dim, dtype):
+    """Infinities and a NaN among the values of the window come out in their own coordinate as attention in float32 gives them, for tokens of
+    every part of a tile, the last token of a partial tile (which is read again for the rest of it) and the token of weight one."""
+    g = torch.Generator().manual_seed(dim)
+    for window in (1, 45):
+        k = torch.randn(1, 2, 50 + window, dim, generator=g).to(dtype)
+        v = torch.randn(1, 2, 50 + window, dim, generator=g).to(dtype)
+        q = torch.randn(1, 8, 1, dim, generator=g).to(dtype)
+        k[:, :, -1] = q[:, ::4, 0] * 4                 # (the largest probability is exactly one)
+        v[:, :, -1, 1], v[:, :, -1, dim - 2] = float("inf"), -float("inf")
+        if window > 1:
+            v[:, :, 50, 3], v[:, :, 50 + 20, 5], v[:, :, 50 + 31, 6], v[:, :, 50 + 33, 9] = float("inf"), -float("inf"), float("nan"), float("inf")
+            v[:, :, 50 + 2, 10], v[:, :, 50 + 3, 10] = float("inf"), -float("inf")
+        cache = pkg.V3Cache(4, 2, residual_window=window, n_layers=40)
+        cache.append(k.to(DEV), v.to(DEV), 8)
+        out = cache.attend(q.to(DEV), 8).double()
+        ref = _exact_attention(cache._stores[8], q.to(DEV), dim ** -0.5)
+        fin = ref.isfinite()
+        assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out[ref.isinf()], ref[ref.isinf()])
+        assert float((out[fin] - ref[fin]).norm() / ref[fin].norm()) < (6e-3 if dtype == torch.bfloat16 else 3e-3)
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_attend_takes_queries_at_any_element_address(pkg, dim):
     """Contiguous queries that start in the middle of a buffer, on no 16-byte boundary."""

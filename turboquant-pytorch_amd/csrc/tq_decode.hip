@@ -381,13 +381,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
                 else if constexpr (N == 4) { const tq_u2 x = tq_gload8(src); v[j][0] = x[0]; v[j][1] = x[1]; }
                 else v[j][0] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src);
             }
-#pragma unroll
-            for (int c = 0; c < N; ++c) {
-                tq_u4 bt;
-#pragma unroll
-                for (int d = 0; d < 4; ++d)
-                    bt[d] = __builtin_amdgcn_perm(v[2 * d + 1][c / 2], v[2 * d][c / 2], (c & 1) ? 0x07060302u : 0x05040100u);
-                tq_f4v acc = tq_f4v{0.f, 0.f, 0.f, 0.f};
+            float odd = 0.f;         // NaN once a sum is not finite
+            auto column = [&](uint32_t c, tq_u4 bt, tq_f4v acc) __attribute__((always_inline)) {
                 tq_u4 hi = bt, lo;
                 if constexpr (!BF) split_f16x8(bt, hi, lo);
 #pragma unroll
@@ -396,8 +391,42 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
                     if constexpr (!BF) acc = mfma16_bf16(pa[k], lo, acc);
                 }
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (4u * q4 + r < G) put_record(splits > 1u, rec + (4u * q4 + r) * PART + 2u + first + (uint32_t)c, acc[r]);
+                for (int r = 0; r < 4; ++r) {
+                    odd = fmaf(acc[r], 0.f, odd);
+                    if (4u * q4 + r < G) put_record(splits > 1u, rec + (4u * q4 + r) * PART + 2u + first + c, acc[r]);
+                }
+            };
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                tq_u4 bt;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    bt[d] = __builtin_amdgcn_perm(v[2 * d + 1][c / 2], v[2 * d][c / 2], (c & 1) ? 0x07060302u : 0x05040100u);
+                column((uint32_t)c, bt, tq_f4v{0.f, 0.f, 0.f, 0.f});
+            }
+            if (__any(odd != odd)) {
+                // An infinite (or NaN) value met a lower term of its probability that is zero, or the zero weight of a token read
+                // again.  Once more: such values as bf16 against the leading terms, tokens past the end left out.
+#pragma unroll 1
+                for (uint32_t c = 0; c < (uint32_t)N; ++c) {
+                    tq_u4 bt, wild;
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        uint32_t pair = 0u;
+#pragma unroll
+                        for (int k = 0; k < 2; ++k) {
+                            const uint32_t t = 16u * (d / 2) + 4u * q4 + 2u * (d % 2) + k;
+                            if (t < left) pair |= (uint32_t)tq_gload2(reinterpret_cast<const uint16_t *>(vw + (size_t)t * (2 * D)) + first + c) << (16 * k);
+                        }
+                        constexpr uint32_t EXPO = BF ? 0x7f807f80u : 0x7c007c00u, ONE = BF ? 0x00800080u : 0x04000400u;
+                        const uint32_t mask = ((((pair & EXPO) + ONE) >> 15) & 0x00010001u) * 0xffffu;     // exponent all ones
+                        wild[d] = pair & mask;
+                        if constexpr (!BF)
+                            wild[d] = (wild[d] & 0x80008000u) | (mask & 0x7f807f80u) | ((((wild[d] & 0x03ff03ffu) + 0x03ff03ffu) >> 4) & 0x00400040u);
+                        bt[d] = pair & ~mask;
+                    }
+                    column(c, bt, mfma16_bf16(pa[0], wild, tq_f4v{0.f, 0.f, 0.f, 0.f}));
+                }
             }
         };
         if constexpr (D == 64) columns(std::integral_constant<int, 4>{}, 0);
