@@ -934,6 +934,38 @@ def test_infinite_window_values_stay_in_their_coordinate(pkg, dim, dtype):
         assert float((out[fin] - ref[fin]).norm() / ref[fin].norm()) < (6e-3 if dtype == torch.bfloat16 else 3e-3)
 
 
+@pytest.mark.parametrize("dim,bits", [(64, 4), (64, 8), (96, 4), (128, 8), (256, 4), (256, 8)])
+def test_logits_that_cancel_are_as_exact_as_float32(pkg, dim, bits):
+    """Queries almost orthogonal to a packed key, scaled up until the roundings of rotation and score show in the result: it is no
+    further from float64 than rotation and score in float32 are (queries and, in float16 caches, Pi enter as two float16 terms)."""
+    g = torch.Generator().manual_seed(dim + bits)
+    heads, group = 32, 8
+    cache = pkg.V3Cache(bits, 4, residual_window=1, n_layers=40)
+    k = torch.zeros(1, heads, 3, dim)
+    k[:, :, 0] = torch.randn(1, heads, dim, generator=g)
+    v = torch.randn(1, heads, 3, dim, generator=g)
+    v[:, :, 2] = 0
+    cache.append(k.half().to(DEV), v.half().to(DEV), 8)
+    st = cache._stores[8]
+    kc = st.comp.key_compressor
+    codes = kc.centroids.half().double()[_codes(st.k_idx[0, :, :1].contiguous(), bits, dim)][:, 0]       # the keys' directions, rotated
+    unit = codes @ kc.Pi.double()
+    q = torch.randn(heads, 2048, dim, generator=g).double().to(DEV)
+    q = (q - (q @ unit.unsqueeze(-1)) * unit.unsqueeze(1) / (unit * unit).sum(-1)[:, None, None]).half()
+    nearest = (q.double() @ unit.unsqueeze(-1)).squeeze(-1).abs().argsort(dim=1)[:, :group]
+    q = torch.gather(q, 1, nearest.unsqueeze(-1).expand(-1, -1, dim)).reshape(1, heads * group, 1, dim).contiguous()
+    scale = 2.0 ** 17 / (float(st.k_nrm[0, :, 0].float().mean()) * dim ** 0.5)
+    ref = _exact_attention(st, q, scale)
+    err = float((cache.attend(q, 8, scale=scale).double() - ref).norm())
+    rot = torch.matmul(q.float().reshape(heads, group, dim), kc.Pi.t().contiguous()) * scale
+    first = (torch.matmul(rot, codes.float().unsqueeze(-1)) * st.k_nrm[0, :, :1].float().unsqueeze(-1)).double()
+    vc = st.comp.val_compressor
+    vals = (vc.centroids.half().double()[_codes(st.v_idx[0, :, :2].contiguous(), 4, dim)] @ vc.Pi.double()) * st.v_nrm[0, :, :2, None].double()
+    probs = torch.softmax(torch.cat([first, torch.zeros_like(first), torch.zeros_like(first)], -1), -1)
+    f32 = torch.matmul(probs[..., :2], vals).reshape(q.shape)
+    assert err <= float((f32 - ref).norm()), (err, float((f32 - ref).norm()))
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_attend_takes_queries_at_any_element_address(pkg, dim):
     """Contiguous queries that start in the middle of a buffer, on no 16-byte boundary."""

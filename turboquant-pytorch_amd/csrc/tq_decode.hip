@@ -158,8 +158,8 @@ __device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t fir
 // tokens of the split, loaded one run ahead; scores transposed (A = decoded keys, B = rotated queries, heads padded to 16
 // columns), softmax in base 2 against a lazily moved per-head reference, probabilities times value norms as the A operand
 // of the value product, whose B operand is built in the lanes from the staged codes.  Around it, in the same launch:
-//   * waves 0 .. D/32 - 1 rotate the row's queries on the matrix cores (operands of the key codec's table, every term of Pi:
-//     fp32-grade), while the other waves attend to the window, 32 tokens each: raw 16-bit keys and queries multiply exactly,
+//   * waves 0 .. D/32 - 1 rotate the row's queries on the matrix cores (operands of the key codec's table; Pi as three bf16 terms that
+//     add up to its float32 value, or for fp16 queries as two fp16 terms, 22 bits), while the other waves attend to the window, 32 tokens each: raw 16-bit keys and queries multiply exactly,
 //     probabilities enter the value product as three bf16 terms that add up to their float32 value, fp16 values as two that add up to
 //     theirs (two fp16 terms of a probability lie on a grid of 2^-38 of the largest one: at 2^-30 of it eight bits were left);
 //   * the waves' sums meet in LDS; with several splits per row the block that arrives last at the row's counter merges the
