@@ -1,6 +1,8 @@
 """GPU tests of the append-in-place packed store (packed_row_stride of the C ABI) and of the
 streaming cache built on it, against the dense kernels, the CPU oracle and the bookkeeping of
 the reference's generation-time cache (generation_test_v2.py:80-165)."""
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -837,7 +839,7 @@ def test_one_launch_append_stores_the_bytes_of_compress(pkg, dim, bits):
 
 @pytest.mark.parametrize("dim,bits", [(64, (6, 4)), (96, (4, 2)), (256, (8, 8)), (256, (4, 4))])
 def test_decode_attention_of_other_head_dims_keeps_float32_weights(pkg, dim, bits):
-    """At 64, 96 and 256 queries and softmax weights enter the matrix products as two fp16 terms each (22 bits).  Against float64
+    """At 64, 96 and 256 queries enter the matrix products as two fp16 terms (22 bits) and softmax weights as three.  Against float64
     over the centroids as the kernel holds them (float16) what is left is the rounding of the float16 result, 2^-11 / sqrt(12) = 1.4e-4
     of a value on average over a binade at its lower end (2.4e-4 seen); single-term queries alone add 5e-4 at the logits here."""
     g = torch.Generator().manual_seed(dim)
@@ -976,6 +978,60 @@ def test_attend_takes_queries_at_any_element_address(pkg, dim):
     odd = torch.empty(4 * dim + 1, dtype=torch.float16, device=DEV)[1:].view(1, 4, 1, dim)
     odd.copy_(q)
     assert torch.equal(cache.attend(odd, 8), cache.attend(q, 8))
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_attend_replayed_from_a_graph(pkg, dim):
+    """A captured decode step brings its own scratch and clears its arrival counters itself: replays between eager steps of another
+    shape on the same stream give the bytes of the eager call (several splits a row: the last block of a row finishes it)."""
+    cache, other = (pkg.V3Cache(4, 2, residual_window=16, n_layers=40) for _ in range(2))
+    k, v = (outlier_kv((1, 2, 5000, dim), seed=s, dtype=torch.bfloat16).to(DEV) for s in (1, 2))
+    cache.append(k, v, 8)
+    other.append(k[:, :, :700].expand(3, 2, 700, dim), v[:, :, :700].expand(3, 2, 700, dim), 8)
+    qs = torch.randn(6, 1, 8, 1, dim, generator=torch.Generator().manual_seed(dim)).to(torch.bfloat16).to(DEV)
+    q3 = qs[:1, 0].expand(3, 8, 1, dim).contiguous()
+    want = [cache.attend(q, 8) for q in qs]
+    want_other = other.attend(q3, 8)
+    q = qs[0].clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        cache.attend(q, 8)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = cache.attend(q, 8)
+    for i, expected in enumerate(want):
+        q.copy_(qs[i])
+        assert torch.equal(other.attend(q3, 8), want_other)
+        graph.replay()
+        assert torch.equal(out, expected), i
+        torch.cuda.synchronize()
+        assert torch.equal(cache.attend(qs[i], 8), expected), i
+
+
+def test_decode_steps_on_two_streams(pkg):
+    """Steps of two caches queued on two streams without waiting for each other: scratch and counters are each stream's own."""
+    caches, q = [], torch.randn(1, 8, 1, 128, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(DEV)
+    for tokens in (6000, 9000):
+        cache = pkg.V3Cache(4, 2, residual_window=16, n_layers=40, capacity=tokens + 64)
+        k, v = (outlier_kv((1, 2, tokens, 128), seed=tokens + s, dtype=torch.bfloat16).to(DEV) for s in (1, 2))
+        cache.append(k, v, 8)
+        caches.append((cache, k, v))
+    runs = []
+    for streams in ((torch.cuda.current_stream(),) * 2, (torch.cuda.Stream(), torch.cuda.Stream())):
+        torch.cuda.synchronize()
+        outs, copies = ([], []), [copy.deepcopy(c) for c, _, _ in caches]
+        torch.cuda.synchronize()
+        for step in range(20):
+            for i, (_, k, v) in enumerate(caches):
+                with torch.cuda.stream(streams[i]):
+                    copies[i].append(k[:, :, step:step + 1], v[:, :, step:step + 1], 8)
+                    outs[i].append(copies[i].attend(q, 8))
+        torch.cuda.synchronize()
+        runs.append(outs)
+    for i in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(runs[0][i], runs[1][i]))
 
 
 def _layer_forms(dim, dtype, g):

@@ -272,8 +272,8 @@ def test_strided_inputs_and_outputs(pkg, oracle):
 @pytest.mark.parametrize("rows,tokens,window,dim", [(2, 31, 1, 128), (2, 32, 1, 128), (3, 33, 7, 128), (5, 64, 64, 128), (16, 135, 64, 128),
                                                     (128, 607, 128, 128), (7, 1000, 0, 128), (3, 4099, 128, 128), (2, 65537, 31, 128), (3, 66, 8, 64)])
 def test_rows_of_a_token_slice_give_the_bytes_of_a_dense_tensor(pkg, rows, tokens, window, dim):
-    """Rows laid end to end in the pipelined compress path (tiles that span two rows, a partial last tile, the job with and
-    without ticket counters, into a dense result and into a packed store with room left in every row): the bytes are the same."""
+    """Rows laid end to end in the pipelined compress path (tiles that span two rows, a partial last tile, into a dense result and into
+    a packed store with room left in every row): the bytes are the same.  (Jobs too small for ticket counters; see below.)"""
     x = outlier_kv((1, rows, tokens + window, dim), seed=rows * tokens, dtype=torch.bfloat16).to(DEV)
     comp = pkg.MSECompressor(dim, 4, seed=7, device=DEV)
     part = x[:, :, :tokens]
@@ -285,6 +285,36 @@ def test_rows_of_a_token_slice_give_the_bytes_of_a_dense_tensor(pkg, rows, token
     comp.compress_into(part, idx[:, :, 4:4 + tokens], nrm[:, :, 4:4 + tokens])
     assert torch.equal(idx[:, :, 4:4 + tokens], want["idx_bytes"]) and torch.equal(nrm[:, :, 4:4 + tokens], want["vec_norms"])
     assert not idx[:, :, :4].any() and not idx[:, :, 4 + tokens:].any() and not nrm[:, :, :4].any() and not nrm[:, :, 4 + tokens:].any()
+
+
+@pytest.mark.parametrize("dim,rows,tokens", [(128, 33, 32641), (64, 33, 65282)])
+def test_rows_of_a_token_slice_drawn_from_ticket_counters(pkg, dim, rows, tokens):
+    """The same in jobs large enough for their tiles to be drawn from counters (runs of 8 tiles, four or more a block): one job, and small
+    jobs that share a launch of many.  The bytes are those without a workspace, and the counters are zero afterwards."""
+    native = pkg._native
+    comp = pkg.MSECompressor(dim, 4, seed=7, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    x = torch.randn(1, rows, tokens + 32, dim, generator=g, device=DEV).to(torch.bfloat16)
+    ws = torch.zeros(int(native.lib().tq_workspace_bytes(1)), dtype=torch.uint8, device=DEV)
+    got = []
+    for workspace in (None, ws.data_ptr()):
+        idx = torch.zeros(1, rows, tokens, dim // 2, dtype=torch.uint8, device=DEV)
+        nrm = torch.zeros(1, rows, tokens, dtype=torch.float16, device=DEV)
+        native.check(native.lib().tq_compress(x.data_ptr(), native.dtype_code(x.dtype), rows, tokens, x.stride(1), dim, comp.table().data_ptr(), dim, 4,
+                                              idx.data_ptr(), nrm.data_ptr(), 0, workspace, torch.cuda.current_stream().cuda_stream), "tq_compress")
+        got.append((idx, nrm))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and not bool(ws.any())
+    jobs, many = [], 40
+    for i in range(many):
+        n = 11000 + 2 * i                    # (64: pairs)
+        jobs.append({"states": x[:, i % 30:i % 30 + 3, 2:2 + n], "idx_bytes": torch.zeros(1, 3, n, dim // 2, dtype=torch.uint8, device=DEV),
+                     "vec_norms": torch.zeros(1, 3, n, dtype=torch.float16, device=DEV), "table": comp.table(), "bits": 4})
+    jl = native.JobList(jobs, DEV)
+    jl.compress()
+    for job in jobs:
+        want = comp.compress(job["states"].contiguous())
+        assert torch.equal(job["idx_bytes"], want["idx_bytes"]) and torch.equal(job["vec_norms"], want["vec_norms"])
+    assert int(jl.workspace.sum()) == 0
 
 
 def test_v3_residual_window_against_reference(pkg, oracle, golden):
