@@ -8,7 +8,6 @@
 // and the value side is rotated back once per query head.  These kernels replace the pair
 // "de-quantise the whole history (generation_test_v2.py:131-135), then let the model multiply by
 // it" (score definition: validate_v3.py:87) for single-token decode steps.
-#include <atomic>
 
 #include "tq_device.h"
 
@@ -1237,23 +1236,6 @@ __global__ __launch_bounds__(512) void tq_attend_merge_kernel(MergeArgs a) {
     }
 }
 
-int device_cus(int &cus) {
-    static std::atomic<int> cache[64];   // per device; threads that race here store the same value
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return (int)e;
-    if (dev < 0 || dev >= 64) return TQ_ERR_NO_DEVICE;
-    int c = cache[dev].load(std::memory_order_relaxed);
-    if (c == 0) {
-        e = hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e != hipSuccess) return (int)e;
-        c = c > 0 ? c : 1;
-        cache[dev].store(c, std::memory_order_relaxed);
-    }
-    cus = c;
-    return 0;
-}
-
 int check_packed(const uint8_t *idx_bytes, const uint16_t *vec_norms, long long packed_row_stride, long long rows,
                  long long tokens, const void *table, int head_dim, int bits) {
     if (bits < 1 || bits > 8) return TQ_ERR_BITS;
@@ -1280,7 +1262,7 @@ extern "C" int tq_scores(const uint8_t *idx_bytes, const uint16_t *vec_norms, lo
     if (scores_stride < tokens) return TQ_ERR_SIZE;
     if (((uintptr_t)q_rot & 3u) || ((uintptr_t)scores & 3u)) return TQ_ERR_ALIGN;
     int cus = 0;
-    rc = device_cus(cus);
+    rc = tq_device_cus(cus);
     if (rc) return rc;
     ScoreArgs a;
     a.idx_bytes = idx_bytes;
@@ -1320,7 +1302,7 @@ extern "C" int tq_qjl_scores(const uint8_t *idx_bytes, const uint16_t *vec_norms
         ((uintptr_t)scores & 3u))
         return TQ_ERR_ALIGN;
     int cus = 0;
-    rc = device_cus(cus);
+    rc = tq_device_cus(cus);
     if (rc) return rc;
     QjlScoreArgs a;
     a.idx_bytes = idx_bytes;
@@ -1355,7 +1337,7 @@ extern "C" int tq_qjl_scores(const uint8_t *idx_bytes, const uint16_t *vec_norms
 extern "C" int tq_weighted_values_splits(long long rows, long long tokens) {
     if (rows <= 0 || tokens <= 0) return 1;
     int cus = 0;
-    if (device_cus(cus)) cus = 256;
+    if (tq_device_cus(cus)) cus = 256;
     long long splits = ((long long)cus * 8 + rows - 1) / rows;       // ~8 four-wave blocks per compute unit
     const long long most = (tokens + 128 * WV_WAVES - 1) / (128 * WV_WAVES);
     if (splits > most) splits = most;
@@ -1423,7 +1405,7 @@ int launch_attend(int ipbv, dim3 grid, dim3 block, hipStream_t s, const AttendAr
 extern "C" int tq_attend_splits(long long rows, long long tokens) {
     if (rows <= 0 || tokens <= 0) return 1;
     int cus = 0;
-    if (device_cus(cus)) cus = 256;
+    if (tq_device_cus(cus)) cus = 256;
     // One eight-wave block is resident per compute unit.  Few rows: as many splits as fill the chip once (a
     // second generation of blocks would stage its tables again: 17 instead of 23 us for 8 rows x 32K tokens).
     // Many rows: two generations, which balances blocks of unequal speed better than one.
@@ -1509,7 +1491,7 @@ extern "C" int tq_attend_merge(const float *partial, int splits, const float *pa
     a.group = (uint32_t)group; a.splits = (uint32_t)splits; a.out_dtype = out_dtype;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     int cus = 0;
-    if (device_cus(cus)) cus = 256;
+    if (tq_device_cus(cus)) cus = 256;
     const dim3 block(512);
     if (group == 1 || rows * 2 <= cus) {                     // few rows: one block per (row, head)
         hipLaunchKernelGGL(tq_attend_merge_kernel<1>, dim3((unsigned)(rows * group)), block, 0, st, a);

@@ -10,7 +10,6 @@
 // multiplied by library products) 190 -> 25 us.
 // What they compute is what tq_compress and the prepare / partials / merge trio of tq_attend.hip compute (upstream
 // turboquant/generation_test_v2.py:96-135, score definition validate_v3.py:87); those remain for float32 elements.
-#include <atomic>
 #include <type_traits>
 
 #include "tq_device.h"
@@ -67,6 +66,9 @@ __device__ __forceinline__ void split_f16x8(tq_u4 v, tq_u4 &hi, tq_u4 &lo) {
 // scope), so that nothing has to be written back or invalidated around the arrival counter: with fences there a step of
 // 8 rows x 32768 tokens took 32.0 us and now 30.0, one of 32 rows x 6000 tokens, 64 wide, 27.3 and now 24.7.  A row with one split keeps
 // its records in its own block: they stay cached (512 rows x 16384 tokens: 2 % longer otherwise).
+// No release and acquire of the language stand behind this order, all accesses are relaxed: it rests on the hardware, where a
+// store of device scope counts in vmcnt until every compute unit sees it, and on both sides going through put_record and
+// get_record.  Plain accesses to a record of a row with several splits would be a race.
 __device__ __forceinline__ void put_record(bool across, TQ_GLOBAL float *p, float v) {
     if (across) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else *p = v;
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     __shared__ __attribute__((aligned(16))) std::conditional_t<PT == 1, uint16_t, float> lds_vn[DW][RUN];     // value norms / 2^ev_ref (uint16_t: as fp16)
     __shared__ __attribute__((aligned(16))) tq_u4 lds_q[QT > QREG ? (QT - QREG) * SK : 1][TQ_WAVE];
     __shared__ __attribute__((aligned(16))) float lds_corr[DW][16];
-    __shared__ float lds_top[MAX_GROUP], lds_den[MAX_GROUP];
+    __shared__ float lds_den[MAX_GROUP];
     __shared__ uint32_t lds_last;
     __shared__ uint32_t lds_trips[DW];                   // runs a wave has begun
 
@@ -772,8 +774,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     }
 
     // ---- the last block of the row finishes it
-    // (the records were stored at device scope: once a wave has waited for its own stores, which the barrier by itself does not
-    // do, they can be counted as there)
+    // (the records were stored at device scope: once every wave has waited for its own stores, which the barrier by itself does not
+    // do, thread 0 may count the block as done, see put_record)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (splits > 1u) {
@@ -1034,23 +1036,6 @@ __global__ __launch_bounds__(D / 32 * TQ_WAVE) void tq_decode_append_kernel(Appe
 }
 
 // ---- host side --------------------------------------------------------------------------------------------------------
-int device_cus(int &cus) {
-    static std::atomic<int> cache[64];   // per device; threads that race here store the same value
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return (int)e;
-    if (dev < 0 || dev >= 64) return TQ_ERR_NO_DEVICE;
-    int c = cache[dev].load(std::memory_order_relaxed);
-    if (c == 0) {
-        e = hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e != hipSuccess) return (int)e;
-        c = c > 0 ? c : 1;
-        cache[dev].store(c, std::memory_order_relaxed);
-    }
-    cus = c;
-    return 0;
-}
-
 bool decode_supported(int head_dim, int bits_k, int bits_v) {
     if (bits_k < 1 || bits_k > 8 || bits_v < 1 || bits_v > 8) return false;
     if (head_dim == 128) return true;
@@ -1093,7 +1078,7 @@ void launch_append(dim3 grid, hipStream_t s, const AppendArgs &a) {
 int decode_splits(long long rows, long long tokens) {
     if (rows <= 0 || tokens <= 0) return 1;
     int cus = 0;
-    if (device_cus(cus)) cus = 256;
+    if (tq_device_cus(cus)) cus = 256;
     // One block is resident per compute unit.  A launch takes as many rounds of blocks as rows * splits fill the chip, each as
     // long as a block's tokens (in trips of its eight waves) plus about what 1000 tokens take for tables, query rotation and
     // result, and what 600 more take where the splits of a row have to be merged.

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/tqamd.h"
 #include "tq_table.h"
 
@@ -330,6 +332,24 @@ __device__ __forceinline__ tq_u4 decode_rep(const uint32_t (&raw)[NW], int s, co
         out = *reinterpret_cast<const tq_u4 *>(lut + (b << 7));
     }
     return out;
+}
+
+// Compute units of the current device.
+static inline int tq_device_cus(int &cus) {
+    static std::atomic<int> cache[64];   // per device; threads that race here store the same value
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return (int)e;
+    if (dev < 0 || dev >= 64) return TQ_ERR_NO_DEVICE;
+    int c = cache[dev].load(std::memory_order_relaxed);
+    if (c == 0) {
+        e = hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e != hipSuccess) return (int)e;
+        c = c > 0 ? c : 1;
+        cache[dev].store(c, std::memory_order_relaxed);
+    }
+    cus = c;
+    return 0;
 }
 
 // 64-wide vectors can go through the 128-wide kernels two at a time when the two vectors of every pair are neighbours in

@@ -177,7 +177,7 @@ class _LayerStore:
                                                    _native._stream_handle(dev))
         if rc == _native.ERR_ALIGN:
             return False
-        _native.check(rc, "tq_decode_append" if self.one_launch else "tq_append_token")
+        _native.check(rc, "tq_decode_append" if self.one_launch and rows <= 65535 else "tq_append_token")
         self.n_compressed += 1
         self.w0 += 1
         self.total_seq += 1
