@@ -4,12 +4,15 @@
 //   tq_decode_attend   softmax(scale q K^T) V over the packed history and the uncompressed window, one launch: the queries are
 //                      rotated, the window is attended to and the splits are merged inside the kernel that reads the codes.
 // Few rows: a step is a chain of latencies (tables, query rotation, one or two runs per wave, merge), so launches are what
-// counts; many rows: the main loop, which is bound by the vector and LDS work of the table lookups at 60 % of the issue slots.
-// Per layer and step, six launches / these two (MI355X): 8 rows x 32768 tokens, K4/V2, 4 heads a row 48.8 -> 30.0 us;
-// 512 rows x 16384 tokens 223 -> 211 us; head dimension 64, 32 rows x 6000 tokens, K6/V4 (before: de-quantised to float32 and
-// multiplied by library products) 190 -> 25 us.
+// counts; many rows: the main loop, which is bound by the vector and LDS work of the table lookups (counted on this kernel at
+// 512 rows x 16384 tokens: vector instructions take 60 % of the issue slots, the LDS is busy 44 % of the time).
+// Per layer and whole step, six launches / these two (MI355X): 8 rows x 32768 tokens, K4/V2, 4 heads a row 48.9 -> 30.1 us;
+// 512 rows x 16384 tokens 226 -> 212 us, of which attention 200-204; head dimension 64, 32 rows x 6000 tokens, K6/V4 (before:
+// de-quantised to float32 and multiplied by library products) 190 -> 25 us.  Attention alone at 256, 32 rows x 6000 tokens, before /
+// this: K4/V2 307 -> 43 us, K8/V8 344 -> 58 us.
 // What they compute is what tq_compress and the prepare / partials / merge trio of tq_attend.hip compute (upstream
-// turboquant/generation_test_v2.py:96-135, score definition validate_v3.py:87); those remain for float32 elements.
+// turboquant/generation_test_v2.py:96-135, score definition validate_v3.py:87); at 128 those remain for float32 caches, queries of
+// another type than the cache's and more than 65535 rows.  A value whose norm is infinite in float16 makes its row's results NaN, as there.
 #include <type_traits>
 
 #include "tq_device.h"
@@ -640,7 +643,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(DecodeArgs 
     // The two waves of a SIMD (w and w + 4) are kept level: the one that is ahead yields.  Left alone the older of the two is
     // served first, and the other one ends its runs without anybody to cover its waits: of a row of 16384 tokens the first
     // waves had done their 32 runs after 69 us and waited 22 us for the others; now all take 84 us and wait one
-    // (512 rows: 213 -> 200 us).  Which wave takes which run stays fixed, so the sums do too.
+    // (512 rows, the launch, median over eight layers in turn: 208 -> 200-204 us).  Which wave takes which run stays fixed, so the sums do too.
     uint32_t trips = 0u;
     auto keep_level = [&]() __attribute__((always_inline)) {
         ++trips;

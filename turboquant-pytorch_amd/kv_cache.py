@@ -334,7 +334,8 @@ class V3Cache:
         kc, vc = st.comp.key_compressor, st.comp.val_compressor
         one_launch = st.one_launch and query_states.dtype == st.dtype and G <= 16 and n_w <= 512 and B * st.H <= 65535 and fused is not False
         if D != _native.HEAD_DIM and not one_launch:
-            # The kernels that read packed codes directly are built for 64-, 96-, 128- and 256-wide heads.  Otherwise the history
+            # The kernels that read packed codes directly are built for 128-wide heads, and at 64, 96 and 256 for 16-bit caches of up
+            # to 65535 rows, windows of 512 tokens and 16 query heads a kv head.  Otherwise the history
             # is de-quantised by the codec kernels (into float32: rounding the keys to 16 bits would move logits of the size
             # this cache sees by several per cent of a softmax weight) and attended to together with the window.
             k = torch.empty((B, st.H, n_c + n_w, D), dtype=torch.float32, device=query_states.device)
@@ -357,8 +358,8 @@ class V3Cache:
                 return out
         kw, vw = st.window()
         if fused and n_w <= 512:
-            # three launches: rotate the queries + window statistics, one pass over the packed history,
-            # log-sum-exp merge + rotation back + cast
+            # one launch where tq_decode_attend takes the layer; otherwise three: rotate the queries + window statistics, one
+            # pass over the packed history, log-sum-exp merge + rotation back + cast
             if n_c:
                 packed = (st.k_idx[:, :, :n_c], st.k_nrm[:, :, :n_c], st.v_idx[:, :, :n_c], st.v_nrm[:, :, :n_c])
             else:                                   # nothing has left the window yet: an empty history
