@@ -817,6 +817,24 @@ def test_one_launch_decode_step_against_float64(pkg, dim, bits, group, dtype):
             cache.append(k[:, :, :1].contiguous(), v[:, :, :1].contiguous(), 8)
 
 
+@pytest.mark.parametrize("dim,bits", [(64, (4, 4)), (64, (8, 2)), (96, (4, 2)), (96, (8, 8)), (128, (4, 2)), (128, (2, 1)), (128, (8, 8)), (256, (4, 2)), (256, (8, 4))])
+def test_decode_attention_with_heads_side_by_side(pkg, dim, bits):
+    """Up to 4 and up to 8 query heads of a row share the columns of the matrix products with 4 and 2 blocks of 16 tokens: every group
+    size around those bounds, histories that end inside each block of a run, against float64 over the store as the kernel holds it.
+    float16 results round to 2^-11 / sqrt(12) of a value (1.4e-4, twice that at the lower end of a binade); at 128 the 2^-12 roundings of
+    query and weight come on top (times logits of about 3 here): 3.5e-4 and 1.5e-3."""
+    g = torch.Generator().manual_seed(dim + bits[0])
+    for rows, tokens in ((2, 15), (1, 17), (3, 47), (1, 63), (2, 65), (1, 545), (1, 4099)):
+        cache = pkg.V3Cache(bits[0], bits[1], residual_window=3, n_layers=40)
+        k, v = (torch.randn(1, rows, tokens + 3, dim, generator=g).half().to(DEV) for _ in range(2))
+        cache.append(k, v, 8)
+        for group in (1, 2, 4, 5, 8, 9, 16):
+            q = torch.randn(1, rows * group, 1, dim, generator=g).half().to(DEV)
+            ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
+            err = float((cache.attend(q, 8).double().reshape(ref.shape) - ref).norm() / ref.norm())
+            assert err < (1.5e-3 if dim == 128 else 3.5e-4), (rows, tokens, group, err)
+
+
 @pytest.mark.parametrize("dim", [64, 96, 128, 256])
 @pytest.mark.parametrize("bits", [(4, 2), (8, 3), (6, 4)])
 def test_one_launch_append_stores_the_bytes_of_compress(pkg, dim, bits):
