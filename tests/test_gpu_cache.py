@@ -835,6 +835,22 @@ def test_decode_attention_with_heads_side_by_side(pkg, dim, bits):
             assert err < (1.5e-3 if dim == 128 else 3.5e-4), (rows, tokens, group, err)
 
 
+@pytest.mark.parametrize("dim,tokens,window", [(64, 34000, 260), (96, 17000, 40), (128, 70000, 128), (256, 20000, 5)])
+def test_decode_attention_merges_many_splits(pkg, dim, tokens, window):
+    """One row over many blocks: more records than a lane has under way at a time (32) and than a wave has lanes, several windows' tiles
+    among them, against float64 over the store as the kernel holds it.  Bounds as in test_decode_attention_with_heads_side_by_side; the many
+    tokens of about equal weight leave results of 0.01, where float16 still rounds to 2^-11 of a value."""
+    g = torch.Generator().manual_seed(dim)
+    cache = pkg.V3Cache(4, 2, residual_window=window, n_layers=40)
+    k, v = (torch.randn(1, 1, tokens + window, dim, generator=g).half().to(DEV) for _ in range(2))
+    cache.append(k, v, 8)
+    for group in (1, 8, 16):
+        q = 2 * torch.randn(1, group, 1, dim, generator=g).half().to(DEV)
+        ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
+        err = float((cache.attend(q, 8).double() - ref).norm() / ref.norm())
+        assert err < (1.5e-3 if dim == 128 else 3.5e-4), (group, err)
+
+
 @pytest.mark.parametrize("dim", [64, 96, 128, 256])
 @pytest.mark.parametrize("bits", [(4, 2), (8, 3), (6, 4)])
 def test_one_launch_append_stores_the_bytes_of_compress(pkg, dim, bits):

@@ -563,8 +563,8 @@ __global__ __launch_bounds__(AT_WAVES *TQ_WAVE, AT_WAVES / 4) void tq_attend_ker
     const TqTableHeader *hv_hd = reinterpret_cast<const TqTableHeader *>(a.table_v);
     RepLut<IPBK>::stage(lds_lut_k, a.table_k + hk_hd->off_lut, tid, AT_WAVES * TQ_WAVE);
     RepLut<IPBV>::stage(lds_lut_v, a.table_v + hv_hd->off_lut, tid, AT_WAVES * TQ_WAVE);
-    const uint32_t lut_k = tq_lds_offset(lds_lut_k) + RepLut<IPBK>::lane_offset(lane);
-    const uint32_t lut_v = tq_lds_offset(lds_lut_v) + RepLut<IPBV>::lane_offset(lane);
+    const uint8_t *lut_k = lds_lut_k + RepLut<IPBK>::lane_offset(lane);
+    const uint8_t *lut_v = lds_lut_v + RepLut<IPBV>::lane_offset(lane);
 
     const uint32_t G = a.group;
     const bool live = n16 < G;

@@ -26,7 +26,7 @@ constexpr int MAX_GROUP = 16;
 constexpr int WIN_TILE = 32;
 constexpr int MAX_WINDOW = 512;
 constexpr int MAX_SPLITS = 256;     // (the merge keeps a weight per record and head in 32 KiB of LDS)
-static_assert(MAX_GROUP * (MAX_SPLITS + MAX_WINDOW / WIN_TILE) * 4 <= 32768, "weights of the records");
+static_assert(MAX_GROUP * (MAX_SPLITS + MAX_WINDOW / WIN_TILE) * 4 <= 32768, "weights of the records");    // (both multiples of a batch)
 
 }  // namespace
 

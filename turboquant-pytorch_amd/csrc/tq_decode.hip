@@ -192,15 +192,16 @@ int decode_splits(long long rows, long long tokens) {
     int cus = 0;
     if (tq_device_cus(cus)) cus = 256;
     // One block is resident per compute unit.  A launch takes as many rounds of blocks as rows * splits fill the chip, each as
-    // long as a block's tokens (in trips of its eight waves) plus about what 1000 tokens take for tables, query rotation and
-    // result, and what 600 more take where the splits of a row have to be merged.
-    long long most = (tokens + 64 * DW - 1) / (64 * DW);
+    // long as a block's tokens plus about what 2000 tokens take for tables, query rotation and result, and 400 more where the splits
+    // of a row have to be merged; every record to merge counts like 12 tokens.  Blocks of less than 192 tokens gain nothing.
+    // (Best of a sweep / what this rule takes, us a launch, K4/V2: 8 x 32768 tokens 18.3 / 18.4 with 32 splits, 20.0 with 16 and 25.3 with 48;
+    // 2 x 8738 12.4 / 12.6; 8 x 1024 12.0 / 12.4, 14.9 in one split; 160 x 6000 34.6 / 34.6 in one split, 40.4 with 3; 128 x 4182 23.2 with 2.)
+    long long most = (tokens + 191) / 192;
     if (most > MAX_SPLITS) most = MAX_SPLITS;
     long long best = 1, best_cost = 0;
     for (long long s = 1; s <= most; ++s) {
         const long long rounds = (rows * s + cus - 1) / cus;
-        const long long trips = ((tokens + s - 1) / s + 64 * DW - 1) / (64 * DW);
-        const long long cost = rounds * (trips * 64 * DW + 1000 + (s > 1 ? 600 : 0));
+        const long long cost = rounds * ((tokens + s - 1) / s + 2000 + (s > 1 ? 400 : 0)) + 12 * s;
         if (s == 1 || cost < best_cost) { best = s; best_cost = cost; }
         if (rounds > 16 && s > 1) break;
     }
@@ -271,9 +272,14 @@ extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *querie
     a.tokens = (uint32_t)tokens;
     a.packed_row_stride = (uint32_t)layer->packed_row_stride;
     a.group = (uint32_t)group;
-    a.chunk = (uint32_t)(((tokens + splits - 1) / splits + 63) / 64 * 64);
+    a.chunk = (uint32_t)(((tokens + splits - 1) / splits + 15) / 16 * 16);
     a.n_win = (uint32_t)n_win;
     a.bf16 = layer->dtype == TQ_BF16 ? 1u : 0u;
+    if (!tokens) {       // no history: the loads that every wave starts with find the tables instead, and nothing is done with them
+        a.k_idx = a.table_k; a.v_idx = a.table_v;
+        a.k_norms = reinterpret_cast<const uint16_t *>(a.table_k); a.v_norms = reinterpret_cast<const uint16_t *>(a.table_v);
+        a.packed_row_stride = 0;
+    }
     const dim3 grid((unsigned)splits, (unsigned)rows, 1);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const int ik = 8 / layer->bits_k, iv = 8 / layer->bits_v;

@@ -35,16 +35,26 @@ __device__ __forceinline__ void split_f16x8(tq_u4 v, tq_u4 &hi, tq_u4 &lo) {
 // its records in its own block: they stay cached (512 rows x 16384 tokens: 2 % longer otherwise).
 // No release and acquire of the language stand behind this order, all accesses are relaxed: it rests on the hardware, where a
 // store of device scope counts in vmcnt until every compute unit sees it, and on both sides going through put_record and
-// get_record.  Plain accesses to a record of a row with several splits would be a race.
+// Records.  Plain accesses to a record of a row with several splits would be a race.
 __device__ __forceinline__ void put_record(bool across, TQ_GLOBAL float *p, float v) {
     if (across) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else *p = v;
 }
+// Two neighbours in one access (the pair need not be one value to the other side, only each half of it).
 template <bool ACROSS>
-__device__ __forceinline__ float get_record(const TQ_GLOBAL float *p) {
-    if constexpr (ACROSS) return __hip_atomic_load(const_cast<TQ_GLOBAL float *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else return *p;
+__device__ __forceinline__ void put_record2(TQ_GLOBAL float *p, float a, float b) {
+    const tq_u2 v = {__float_as_uint(a), __float_as_uint(b)};
+    if constexpr (ACROSS) __hip_atomic_store(reinterpret_cast<TQ_GLOBAL uint64_t *>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *reinterpret_cast<TQ_GLOBAL tq_u2 *>(p) = v;
 }
+// Records of a row, from the first float of the first one, as a buffer: four (or two) neighbours in one access of device scope (the
+// cache-policy bits of a load can be given to the buffer form only), and what lies past the last record reads as zero.
+struct Records {
+    __amdgpu_buffer_rsrc_t rsrc;
+    __device__ __forceinline__ Records(const float *p, uint32_t floats) : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, floats * 4u, 0x00020000)) {}
+    template <bool ACROSS> __device__ __forceinline__ tq_u4 load4(uint32_t at) const { return __builtin_amdgcn_raw_buffer_load_b128(rsrc, at * 4u, 0, ACROSS ? 16 : 0); }
+    template <bool ACROSS> __device__ __forceinline__ tq_u2 load2(uint32_t at) const { return __builtin_amdgcn_raw_buffer_load_b64(rsrc, at * 4u, 0, ACROSS ? 16 : 0); }
+};
 
 // Lanes L apart exchanged between two registers (L = 32: upper half of a with lower half of b; 16: the odd quarters of a with the
 // even ones of b) and added: a summed over both where b's half (quarter) does not lie, b where it does.
@@ -58,32 +68,106 @@ __device__ __forceinline__ float fold(float a, float b) {
 // Tokens a wave takes per trip: 32 where registers are short.
 constexpr int decode_run(int d, int ipbk, int ipbv) { return d == 256 || (d > 64 && (ipbk == 1 || ipbv == 1)) ? 32 : 64; }
 
-// The byte -> centroids table spread over the banks (RepLut): consecutive threads write consecutive 16-byte pieces, so the
-// writes are free of conflicts; the eight threads of a table row read the same entry.
+// Over the lanes of a wave: within rows of 16 by rotation, then rows, then halves (no trip through the LDS as __shfl_xor takes).
+template <typename Op>
+__device__ __forceinline__ float reduce_rows(float x, Op op) {       // over the four lanes 16 apart
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return op(__uint_as_float(h[0]), __uint_as_float(h[1]));
+}
+template <typename Op>
+__device__ __forceinline__ float reduce_wave(float x, Op op) {
+    x = op(x, __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x128, 0xf, 0xf, true)));
+    x = op(x, __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x124, 0xf, 0xf, true)));
+    x = op(x, __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x122, 0xf, 0xf, true)));
+    x = op(x, __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x121, 0xf, 0xf, true)));
+    return reduce_rows(x, op);
+}
+struct OpMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
+struct OpAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
+
+// The byte -> centroids tables of keys and values, spread over the banks (RepLut), side by side: 256 rows of 256 bytes, the
+// keys' entry in the first half of a row and the values' in the second.  The address of a lane's slot of an entry is then the byte,
+// moved up by eight bits, with the lane's offset below it: one v_perm_b32, where 128-byte rows took two or three instructions (and
+// v_dot4_u32_u8, one as well, is followed by idle cycles before its result can be used as an address).
+// Consecutive threads write consecutive 16-byte pieces, so the writes are free of conflicts; the eight threads of a table
+// row read the same entry.
+template <int B, typename T>
+__device__ __forceinline__ T lut_entry(const uint8_t *lut, uint32_t raw, uint32_t slot) {      // entry <byte B of raw>
+    return *reinterpret_cast<const T *>(lut + __builtin_amdgcn_perm(raw, slot, 0x0c0c0000u | ((4u + B) << 8)));
+}
 template <int IPB>
-__device__ __forceinline__ void stage_lut(uint8_t *lds, const uint8_t *src, uint32_t tid) {
-    constexpr int ES = 2 * IPB;
-    constexpr int TRIPS = 256 * 8 / DTHREADS;
+struct Lut {
+    static constexpr int ES = 2 * IPB;
+    static constexpr int TRIPS = 256 * 8 / DTHREADS;
     tq_u4 v[TRIPS];
+    __device__ __forceinline__ void load(const uint8_t *src, uint32_t tid) {
 #pragma unroll
-    for (int k = 0; k < TRIPS; ++k) {
-        const TQ_GLOBAL uint8_t *g = (const TQ_GLOBAL uint8_t *)src + ((k * DTHREADS + tid) >> 3) * ES;
-        if constexpr (ES == 2) {
-            const uint32_t x = *reinterpret_cast<const TQ_GLOBAL uint16_t *>(g);
-            v[k] = tq_u4{x, x, x, x};
-        } else if constexpr (ES == 4) {
-            const uint32_t x = *reinterpret_cast<const TQ_GLOBAL uint32_t *>(g);
-            v[k] = tq_u4{x, x, x, x};
-        } else if constexpr (ES == 8) {
-            const tq_u2 x = *reinterpret_cast<const TQ_GLOBAL tq_u2 *>(g);
-            v[k] = tq_u4{x[0], x[1], x[0], x[1]};
-        } else {
-            v[k] = *reinterpret_cast<const TQ_GLOBAL tq_u4 *>(g);
+        for (int k = 0; k < TRIPS; ++k) {
+            const TQ_GLOBAL uint8_t *g = (const TQ_GLOBAL uint8_t *)src + ((k * DTHREADS + tid) >> 3) * ES;
+            if constexpr (ES == 2) v[k][0] = *reinterpret_cast<const TQ_GLOBAL uint16_t *>(g);
+            else if constexpr (ES == 4) v[k][0] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>(g);
+            else if constexpr (ES == 8) { const tq_u2 x = *reinterpret_cast<const TQ_GLOBAL tq_u2 *>(g); v[k][0] = x[0]; v[k][1] = x[1]; }
+            else v[k] = *reinterpret_cast<const TQ_GLOBAL tq_u4 *>(g);
         }
     }
+    __device__ __forceinline__ void store(uint8_t *lds, uint32_t tid) {
 #pragma unroll
-    for (int k = 0; k < TRIPS; ++k) *reinterpret_cast<tq_u4 *>(lds + (k * DTHREADS + tid) * 16u) = v[k];
-}
+        for (int k = 0; k < TRIPS; ++k) {
+            const tq_u4 x = ES <= 4 ? tq_u4{v[k][0], v[k][0], v[k][0], v[k][0]} : ES == 8 ? tq_u4{v[k][0], v[k][1], v[k][0], v[k][1]} : v[k];
+            const uint32_t piece = k * DTHREADS + tid;
+            *reinterpret_cast<tq_u4 *>(lds + (piece >> 3) * 256u + (piece & 7u) * 16u) = x;
+        }
+    }
+};
+
+// Rotated queries of a row, q_rot[g][j] = scale * sum_i Pi[j][i] q[g][i]: a wave's 32 coordinates on the matrix cores, from the operands
+// of the key codec's table (Pi as three bf16 terms that add up to its float32 value, or for fp16 queries as two fp16 terms, 22 bits).
+// Loads and products apart, so that other loads can be under way between them.
+template <int D, bool BF>
+struct Rotation {
+    static constexpr int STEPS = D / 16, CH = STEPS < 8 ? STEPS : 8, TERMS = BF ? 3 : 2;     // CH: steps whose operands are in flight together
+    tq_u4 q[CH], p[TERMS][CH];
+    const uint8_t *qsrc, *asrc;
+    __device__ __forceinline__ void fetch(int s0) {
+#pragma unroll
+        for (int s = 0; s < CH; ++s) {
+            q[s] = tq_gload16(qsrc + (s0 + s) * 32);
+#pragma unroll
+            for (int t = 0; t < TERMS; ++t) p[t][s] = tq_gload16(asrc + (size_t)t * TQ_OPERAND_BYTES_FOR(D) + (size_t)(s0 + s) * 1024u);
+        }
+    }
+    // queries: the row's, [group][D]
+    __device__ __forceinline__ void load(const uint8_t *queries, uint32_t group, const uint8_t *table_k, uint32_t tile, uint32_t lane) {
+        const uint32_t n = lane & 31u, hk = lane >> 5;
+        qsrc = queries + ((size_t)(n < group ? n : 0u) * D + 8u * hk) * 2u;
+        asrc = table_k + (BF ? TQ_OFF_A_BF16(D) : TQ_OFF_A_F16) + ((size_t)tile * STEPS * 64u + lane) * 16u;
+        fetch(0);
+    }
+    // qrot: [MAX_GROUP] rows of `stride` floats
+    __device__ __forceinline__ void finish(float *qrot, uint32_t stride, float scale, uint32_t tile, uint32_t lane) {
+        static_assert(STEPS % CH == 0, "whole chunks");
+        const uint32_t n = lane & 31u, hk = lane >> 5;
+        tq_f16v acc = tq_zero16();
+#pragma unroll 1
+        for (int s0 = 0;;) {
+#pragma unroll
+            for (int s = 0; s < CH; ++s)
+#pragma unroll
+                for (int t = 0; t < TERMS; ++t) acc = BF ? mfma_bf16(p[t][s], q[s], acc) : mfma_f16(p[t][s], q[s], acc);
+            s0 += CH;
+            if (s0 >= STEPS) break;
+            fetch(s0);
+        }
+        const float f = BF ? scale : scale * (1.0f / (float)(1 << TQ_F16_PI_SHIFT));
+        if (n < (uint32_t)MAX_GROUP) {
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+                *reinterpret_cast<float4 *>(qrot + n * stride + 32u * tile + 16u * hk + r) = make_float4(acc[r] * f, acc[r + 1] * f, acc[r + 2] * f, acc[r + 3] * f);
+        }
+    }
+};
 
 // Coordinates of a lane on the value side, D / 16 of them: contiguous for multiples of 64; four of the first 64 and two of
 // the last 32 for 96, so that a group of them never starts inside a packed byte that another lane shares more than once.
@@ -96,32 +180,32 @@ __device__ __forceinline__ uint32_t value_coord(uint32_t n16, int c) {
 // N consecutive coordinates (8, 4 or 2) of a staged value vector -> fp16 pairs; `codes` points at the vector's packed bytes,
 // first = index of the first coordinate.
 template <int IPB, int N>
-__device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t first, uint32_t lut, uint32_t (&out)[N / 2]) {
+__device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t first, const uint8_t *lut, uint32_t slot, uint32_t (&out)[N / 2]) {
     if constexpr (IPB == 8) {
         static_assert(N == 8, "whole bytes");
-        const tq_u4 v = tq_rep_entry<0, tq_u4>(codes[first / 8u], lut);
+        const tq_u4 v = lut_entry<0, tq_u4>(lut, codes[first / 8u], slot);
         out[0] = v[0]; out[1] = v[1]; out[2] = v[2]; out[3] = v[3];
     } else if constexpr (IPB == 4) {
         if constexpr (N == 8) {
             const uint32_t two = *reinterpret_cast<const uint16_t *>(codes + first / 4u);
-            const tq_u2 a = tq_rep_entry<0, tq_u2>(two, lut), b = tq_rep_entry<1, tq_u2>(two, lut);
+            const tq_u2 a = lut_entry<0, tq_u2>(lut, two, slot), b = lut_entry<1, tq_u2>(lut, two, slot);
             out[0] = a[0]; out[1] = a[1]; out[2] = b[0]; out[3] = b[1];
         } else if constexpr (N == 4) {
-            const tq_u2 a = tq_rep_entry<0, tq_u2>(codes[first / 4u], lut);
+            const tq_u2 a = lut_entry<0, tq_u2>(lut, codes[first / 4u], slot);
             out[0] = a[0]; out[1] = a[1];
         } else {        // half a byte
-            out[0] = tq_rep_entry<0, uint32_t>(codes[first / 4u], lut + 2u * (first & 3u));
+            out[0] = lut_entry<0, uint32_t>(lut, codes[first / 4u], slot + 2u * (first & 3u));
         }
     } else if constexpr (IPB == 2) {
         uint32_t raw;
         if constexpr (N == 8) raw = *reinterpret_cast<const uint32_t *>(codes + first / 2u);
         else if constexpr (N == 4) raw = *reinterpret_cast<const uint16_t *>(codes + first / 2u);
         else raw = codes[first / 2u];
-        out[0] = tq_rep_entry<0, uint32_t>(raw, lut);
-        if constexpr (N >= 4) out[1] = tq_rep_entry<1, uint32_t>(raw, lut);
+        out[0] = lut_entry<0, uint32_t>(lut, raw, slot);
+        if constexpr (N >= 4) out[1] = lut_entry<1, uint32_t>(lut, raw, slot);
         if constexpr (N == 8) {
-            out[2] = tq_rep_entry<2, uint32_t>(raw, lut);
-            out[3] = tq_rep_entry<3, uint32_t>(raw, lut);
+            out[2] = lut_entry<2, uint32_t>(lut, raw, slot);
+            out[3] = lut_entry<3, uint32_t>(lut, raw, slot);
         }
     } else {
         uint32_t raw[2] = {0u, 0u};
@@ -130,26 +214,208 @@ __device__ __forceinline__ void decode_values(const uint8_t *codes, uint32_t fir
         else raw[0] = *reinterpret_cast<const uint16_t *>(codes + first);
 #pragma unroll
         for (int i = 0; i < N / 2; i += 2) {
-            out[i] = (uint32_t)tq_rep_entry<0, uint16_t>(raw[i / 2], lut) | ((uint32_t)tq_rep_entry<1, uint16_t>(raw[i / 2], lut) << 16);
-            if constexpr (N > 2) out[i + 1] = (uint32_t)tq_rep_entry<2, uint16_t>(raw[i / 2], lut) | ((uint32_t)tq_rep_entry<3, uint16_t>(raw[i / 2], lut) << 16);
+            out[i] = (uint32_t)lut_entry<0, uint16_t>(lut, raw[i / 2], slot) | ((uint32_t)lut_entry<1, uint16_t>(lut, raw[i / 2], slot) << 16);
+            if constexpr (N > 2) out[i + 1] = (uint32_t)lut_entry<2, uint16_t>(lut, raw[i / 2], slot) | ((uint32_t)lut_entry<3, uint16_t>(lut, raw[i / 2], slot) << 16);
         }
     }
 }
 
+// The eight coordinates of step s among a lane's key bytes -> fp16 operand.
+template <int IPB, int NW>
+__device__ __forceinline__ tq_u4 decode_keys(const uint32_t (&raw)[NW], int s, const uint8_t *lut, uint32_t slot) {
+    tq_u4 out;
+    if constexpr (IPB == 1) {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            const uint32_t r = raw[2 * s + d];
+            out[2 * d] = (uint32_t)lut_entry<0, uint16_t>(lut, r, slot) | ((uint32_t)lut_entry<1, uint16_t>(lut, r, slot) << 16);
+            out[2 * d + 1] = (uint32_t)lut_entry<2, uint16_t>(lut, r, slot) | ((uint32_t)lut_entry<3, uint16_t>(lut, r, slot) << 16);
+        }
+    } else if constexpr (IPB == 2) {
+        out[0] = lut_entry<0, uint32_t>(lut, raw[s], slot);
+        out[1] = lut_entry<1, uint32_t>(lut, raw[s], slot);
+        out[2] = lut_entry<2, uint32_t>(lut, raw[s], slot);
+        out[3] = lut_entry<3, uint32_t>(lut, raw[s], slot);
+    } else if constexpr (IPB == 4) {
+        const uint32_t r = raw[s / 2];
+        const tq_u2 v0 = s % 2 ? lut_entry<2, tq_u2>(lut, r, slot) : lut_entry<0, tq_u2>(lut, r, slot);
+        const tq_u2 v1 = s % 2 ? lut_entry<3, tq_u2>(lut, r, slot) : lut_entry<1, tq_u2>(lut, r, slot);
+        out = tq_u4{v0[0], v0[1], v1[0], v1[1]};
+    } else {
+        const uint32_t r = raw[s / 4];
+        out = s % 4 == 0 ? lut_entry<0, tq_u4>(lut, r, slot) : s % 4 == 1 ? lut_entry<1, tq_u4>(lut, r, slot) : s % 4 == 2 ? lut_entry<2, tq_u4>(lut, r, slot) : lut_entry<3, tq_u4>(lut, r, slot);
+    }
+    return out;
+}
+
+// 32 tokens of a row's uncompressed window: raw 16-bit keys and queries multiply exactly; probabilities enter the value product as three
+// bf16 terms that add up to their float32 value, fp16 values as two that add up to theirs (two fp16 terms of a probability lie on a
+// grid of 2^-38 of the largest one: at 2^-30 of it eight bits were left).  Record: [head][largest score, sum, D sums].  The values are
+// loaded with the keys: their latency is the same, and a step of few rows waits for both.
+template <int D, bool BF>
+struct WindowTile {
+    static constexpr int SK = D / 32, NC = D / 16;
+    static constexpr int VW = D == 256 ? 0 : NC / 2;         // words of a token's columns held from the start (256: registers are short)
+    tq_u4 q[SK], k[SK][2];
+    uint32_t v[8][VW ? VW : 1];
+    const uint8_t *kw, *vw;
+    uint32_t left;
+
+    static __device__ __forceinline__ uint32_t token(int j, uint32_t q4) { return 16u * (j / 4) + 4u * q4 + (uint32_t)(j % 4); }
+    template <int N> __device__ __forceinline__ void load_columns(uint32_t (&dst)[8][N / 2], uint32_t lane, int c0) const {
+        const uint32_t first = value_coord<D>(lane & 15u, c0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {      // past the end the last token is read again and not used
+            const uint8_t *src = vw + (size_t)min(token(j, lane >> 4), left - 1u) * (2 * D) + 2u * first;
+            if constexpr (N == 8) { const tq_u4 x = tq_gload16(src); dst[j][0] = x[0]; dst[j][1] = x[1]; dst[j][2] = x[2]; dst[j][3] = x[3]; }
+            else if constexpr (N == 4) { const tq_u2 x = tq_gload8(src); dst[j][0] = x[0]; dst[j][1] = x[1]; }
+            else dst[j][0] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src);
+        }
+    }
+    __device__ __forceinline__ void load(const TqDecodeArgs &a, uint32_t row, uint32_t wt, uint32_t lane) {
+        const uint32_t n16 = lane & 15u, q4 = lane >> 4, t0 = wt * WIN_TILE;
+        left = min((uint32_t)WIN_TILE, a.n_win - t0);
+        kw = a.k_win + ((size_t)row * a.win_stride + (size_t)t0 * D) * 2u;
+        vw = a.v_win + ((size_t)row * a.win_stride + (size_t)t0 * D) * 2u;
+        const uint8_t *qs = a.queries + (((size_t)row * a.group + (n16 < a.group ? n16 : 0u)) * D + 8u * q4) * 2u;
+#pragma unroll
+        for (int s = 0; s < SK; ++s) {
+            q[s] = tq_gload16(qs + 64 * s);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) k[s][b] = tq_gload16(kw + (size_t)min(16u * b + n16, left - 1u) * (2 * D) + 64 * s + 16u * q4);
+        }
+        if constexpr (D == 64 || D == 128) load_columns<NC>(v, lane, 0);
+        else if constexpr (D == 96) {
+            uint32_t two[8][2], one[8][1];
+            load_columns<4>(two, lane, 0);
+            load_columns<2>(one, lane, 4);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) { v[j][0] = two[j][0]; v[j][1] = two[j][1]; v[j][VW - 1] = one[j][0]; }
+        }
+    }
+    __device__ __forceinline__ void finish(const TqDecodeArgs &a, TQ_GLOBAL float *rec, bool across, uint32_t lane) {
+        constexpr int PART = D + 2;
+        const uint32_t n16 = lane & 15u, q4 = lane >> 4, G = a.group;
+        auto mm = [](tq_u4 x, tq_u4 y, tq_f4v c) { return BF ? mfma16_bf16(x, y, c) : mfma16_f16(x, y, c); };
+        tq_f4v sc[2] = {tq_f4v{0.f, 0.f, 0.f, 0.f}, tq_f4v{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < SK; ++s)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) sc[b] = mm(k[s][b], q[s], sc[b]);
+        float t[8], m = -3.0e38f, l = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            t[j] = sc[j / 4][j % 4] * a.scale;       // token(j) of the tile, head n16
+            if (token(j, q4) >= left) t[j] = -3.0e38f;
+            m = fmaxf(m, t[j]);
+        }
+        m = reduce_rows(m, OpMax());
+        float p[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            p[j] = token(j, q4) < left ? __expf(t[j] - m) : 0.f;
+            l += p[j];
+        }
+        l = reduce_rows(l, OpAdd());
+        tq_u4 pa[3];
+        split_f32x8(p, pa[0], pa[1], pa[2]);
+        if (q4 == 0u && n16 < G) { put_record(across, rec + n16 * PART, m); put_record(across, rec + n16 * PART + 1u, l); }
+        // columns in chunks of 8 (or 4, 2): the same element of token pairs side by side, one operand per coordinate
+        auto columns = [&](auto n_tag, int c0, const auto &w, int w0) __attribute__((always_inline)) {
+            constexpr int N = decltype(n_tag)::value;
+            const uint32_t first = value_coord<D>(n16, c0);
+            float odd = 0.f;         // NaN once a sum is not finite
+            auto column = [&](tq_u4 bt, tq_f4v acc) __attribute__((always_inline)) {
+                tq_u4 hi = bt, lo;
+                if constexpr (!BF) split_f16x8(bt, hi, lo);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    acc = mfma16_bf16(pa[i], hi, acc);
+                    if constexpr (!BF) acc = mfma16_bf16(pa[i], lo, acc);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) odd = fmaf(acc[r], 0.f, odd);
+                return acc;
+            };
+            tq_f4v sum[N];
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                tq_u4 bt;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    bt[d] = __builtin_amdgcn_perm(w[2 * d + 1][w0 + c / 2], w[2 * d][w0 + c / 2], (c & 1) ? 0x07060302u : 0x05040100u);
+                sum[c] = column(bt, tq_f4v{0.f, 0.f, 0.f, 0.f});
+            }
+            auto store = [&](auto across_tag) __attribute__((always_inline)) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (4u * q4 + r < G) {
+#pragma unroll
+                        for (int c = 0; c < N; c += 2) put_record2<decltype(across_tag)::value>(rec + (4u * q4 + r) * PART + 2u + first + c, sum[c][r], sum[c + 1][r]);
+                    }
+                }
+            };
+            if (across) store(std::true_type{}); else store(std::false_type{});
+            if (__any(odd != odd)) {
+                // An infinite (or NaN) value met a lower term of its probability that is zero, or the zero weight of a token read
+                // again.  Once more: such values as bf16 against the leading terms, tokens past the end left out.
+#pragma unroll 1
+                for (uint32_t c = 0; c < (uint32_t)N; ++c) {
+                    tq_u4 bt, wild;
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        uint32_t pair = 0u;
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            const uint32_t tt = 16u * (d / 2) + 4u * q4 + 2u * (d % 2) + i;
+                            if (tt < left) pair |= (uint32_t)tq_gload2(reinterpret_cast<const uint16_t *>(vw + (size_t)tt * (2 * D)) + first + c) << (16 * i);
+                        }
+                        constexpr uint32_t EXPO = BF ? 0x7f807f80u : 0x7c007c00u, ONE = BF ? 0x00800080u : 0x04000400u;
+                        const uint32_t mask = ((((pair & EXPO) + ONE) >> 15) & 0x00010001u) * 0xffffu;     // exponent all ones
+                        wild[d] = pair & mask;
+                        if constexpr (!BF)
+                            wild[d] = (wild[d] & 0x80008000u) | (mask & 0x7f807f80u) | ((((wild[d] & 0x03ff03ffu) + 0x03ff03ffu) >> 4) & 0x00400040u);
+                        bt[d] = pair & ~mask;
+                    }
+                    const tq_f4v again = column(bt, mfma16_bf16(pa[0], wild, tq_f4v{0.f, 0.f, 0.f, 0.f}));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (4u * q4 + r < G) put_record(across, rec + (4u * q4 + r) * PART + 2u + first + c, again[r]);
+                }
+            }
+        };
+        if constexpr (D == 64) columns(std::integral_constant<int, 4>{}, 0, v, 0);
+        else if constexpr (D == 96) { columns(std::integral_constant<int, 4>{}, 0, v, 0); columns(std::integral_constant<int, 2>{}, 4, v, 2); }
+        else if constexpr (D == 128) columns(std::integral_constant<int, 8>{}, 0, v, 0);
+        else {
+#pragma unroll 1
+            for (int c0 = 0; c0 < NC; c0 += 8) {
+                uint32_t w[8][4];
+                load_columns<8>(w, lane, c0);
+                columns(std::integral_constant<int, 8>{}, c0, w, 0);
+            }
+        }
+    }
+};
+
 // Block (split, row), eight waves.  The main loop is the one of tq_attend_kernel (tq_attend.hip): a wave takes runs of 32 or 64
-// tokens of the split, loaded one run ahead; scores transposed (A = decoded keys, B = rotated queries, heads padded to 16
+// tokens of the split, loaded one run ahead; scores transposed (A = decoded keys, B = rotated queries, heads in the 16
 // columns), softmax in base 2 against a lazily moved per-head reference, probabilities times value norms as the A operand
 // of the value product, whose B operand is built in the lanes from the staged codes.  Around it, in the same launch:
-//   * waves 0 .. D/32 - 1 rotate the row's queries on the matrix cores (operands of the key codec's table; Pi as three bf16 terms that
-//     add up to its float32 value, or for fp16 queries as two fp16 terms, 22 bits), while the other waves attend to the window, 32 tokens each: raw 16-bit keys and queries multiply exactly,
-//     probabilities enter the value product as three bf16 terms that add up to their float32 value, fp16 values as two that add up to
-//     theirs (two fp16 terms of a probability lie on a grid of 2^-38 of the largest one: at 2^-30 of it eight bits were left);
+//   * waves 0 .. D/32 - 1 rotate the row's queries on the matrix cores (Rotation), the other waves attend to the window, 32 tokens
+//     each (WindowTile);
 //   * the waves' sums meet in LDS; with several splits per row the block that arrives last at the row's counter merges the
 //     records of all splits and of the window, rotates the value sums back and stores the result.
+// With few rows that is a chain of latencies, and what keeps it short (8 rows x 32768 tokens, K4/V2, 4 heads, 22 splits; clock stamps
+// of a launch before / after): all loads of the start issued at once in the order of their use, tables found without their header, queries
+// rotated by 4.2 / 2.5 us; the window's values loaded with its keys and its sums stored without a branch for each, 7.0 / 4.5; the block's
+// tokens dealt out evenly; records merged with one trip to memory and a code of a few hundred bytes (code that runs once is fetched from
+// the L2 as it goes: 1 us for 2.4 KiB of it), rows of Pi_v under way before the block knows that it needs them, last arrival to result 5.5 / 3.4.
+// Whole step of 32 layers 948 -> 778 us; 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
 // The matrix products have 16 columns and a row of the cache seldom 16 query heads.  C blocks of 16 tokens share them (C = 4 for up to 4
 // heads, 2 for up to 8): every block's scores are computed for the heads repeated C times, a lane keeps those of its own column's
 // block, and the weights of the other blocks are zeros in its column of the value product.  The softmax of a token then costs 1 / C
-// of what it did; columns of one head are added at the end.  With table addresses as one instruction (tq_rep_entry): 512 rows x 16384
+// of what it did; columns of one head are added at the end.  With table addresses as one instruction: 512 rows x 16384
 // tokens, K4/V2, 4 heads 202 -> 194 us; 64 wide, K6/V4, 512 rows x 32768 tokens, 4 heads 387 -> 357 us; 8 heads even (107 us at 256 rows).  Runs of
 // 32 tokens have no room for C = 4.
 // At 128 queries (against 8-bit keys: two terms) and weights enter the packed products as one fp16 term, as in tq_attend_kernel:
@@ -165,9 +431,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     constexpr int QT = D != 128 || IPBK == 1 ? 2 : 1;    // fp16 terms of a rotated query
     constexpr int QREG = D == 256 && (IPBK == 1 || IPBV == 1) ? 1 : QT;      // terms held in registers, the others in LDS (see below)
     constexpr int PT = D != 128 ? 3 : 1;                 // fp16 terms of a weight
-    constexpr int SETS = D == 256 ? 1 : 2;               // register sets of the loads that run one run ahead
     constexpr int PART = D + 2;
-    constexpr int STEPS = D / 16, TILES = D / 32;        // query rotation: 32x32x16 matrix instructions
+    constexpr int TILES = D / 32;                        // waves that rotate queries
     constexpr int SK = D / 32;                           // score product: steps of 32 coordinates, 8 per lane
     constexpr int NC = D / 16;                           // value coordinates per lane
     constexpr int KB = D / 4 / IPBK;                     // key bytes per lane and token (D / 4 coordinates)
@@ -183,19 +448,20 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     constexpr int VBYTES = RUN * GBV, VPIECES = VBYTES / VPB, NVP = (VPIECES + 63) / 64;
     constexpr int SLACK_LOG2 = PT == 1 ? 8 : 4;          // (several terms: the smaller it is, the finer the grid of small weights)
     constexpr int P_SHIFT = 14 - SLACK_LOG2;             // p * 2^P_SHIFT * (value norm / 2^ev_ref < 2) <= 2^15 fits fp16
-    constexpr int HR = D == 256 ? 8 : MAX_GROUP;         // heads per round of the merge through LDS
+    constexpr int HR = D == 256 && C == 1 ? 8 : HEADS;   // heads per round of the merge through LDS
     constexpr int AREA = VBYTES > HR * PART * 4 ? VBYTES : HR * PART * 4;    // per wave: staged value codes, later its sums
     constexpr int QROW = D + 4;                          // rotated queries in LDS, floats per head
     constexpr int ROTP = DTHREADS / (D / 4) >= 16 ? 16 : DTHREADS / (D / 4);     // parts of the contraction when rotating back
     constexpr int ROTK = D / ROTP;                       // rows of Pi_v per part
-    static_assert(DW * AREA >= MAX_GROUP * QROW * 4 && DW * AREA >= 2 * MAX_GROUP * D * 4 && ROTP * 4 * D * 4 <= 32768, "LDS areas too small");
+    constexpr int RG = C == 4 ? 4 : 8;                   // heads rotated back at a time
+    static_assert(DW * AREA >= 2 * MAX_GROUP * D * 4 && ROTP * RG * D * 4 <= 65536, "LDS areas too small");
 
-    __shared__ __attribute__((aligned(16))) uint8_t lds_lut_k[32768];
-    __shared__ __attribute__((aligned(16))) uint8_t lds_lut_v[32768];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds_lut[65536];      // (the strictest alignment: lies at address 0, where no base has to be added)
     __shared__ __attribute__((aligned(16))) uint8_t lds_area[DW][AREA];
     __shared__ __attribute__((aligned(16))) float lds_kn[DW][RUN];
     __shared__ __attribute__((aligned(16))) std::conditional_t<PT == 1, uint16_t, float> lds_vn[DW][RUN];     // value norms / 2^ev_ref (uint16_t: as fp16)
     __shared__ __attribute__((aligned(16))) tq_u4 lds_q[QT > QREG ? (QT - QREG) * SK : 1][TQ_WAVE];
+    __shared__ __attribute__((aligned(16))) float lds_qrot[MAX_GROUP][QROW];
     __shared__ __attribute__((aligned(16))) float lds_corr[DW][16];
     __shared__ float lds_den[MAX_GROUP];
     __shared__ uint32_t lds_last;
@@ -205,8 +471,6 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     const uint32_t wave = tq_uniform32(tid >> 6);
     const uint32_t row = blockIdx.y, split = blockIdx.x, splits = gridDim.x;
     const uint32_t n16 = lane & 15u, q4 = lane >> 4;
-    const TqTableHeader *hk_hd = reinterpret_cast<const TqTableHeader *>(a.table_k);
-    const TqTableHeader *hv_hd = reinterpret_cast<const TqTableHeader *>(a.table_v);
     const uint32_t G = a.group;
     const uint32_t head = n16 % HEADS, cls = n16 / HEADS;
     const bool live = head < G;
@@ -215,225 +479,115 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     const uint32_t t_end = min(a.tokens, t_begin + a.chunk);
     const size_t slot0 = (size_t)row * a.packed_row_stride;
     uint8_t *vcodes = lds_area[wave];
+    // Runs of a wave: in every whole round of the block one of RUN tokens; what is left of the block's tokens is dealt out evenly, in
+    // blocks of 16 tokens, so that no wave works on a whole run alone at the end.
+    const uint32_t rounds = (t_end - t_begin) / (RUN * DW);
+    const uint32_t rest0 = t_begin + rounds * (RUN * DW);
+    const uint32_t share = (t_end - rest0 + 16u * DW - 1u) / (16u * DW) * 16u;
+    const uint32_t tail0 = min(t_end, rest0 + wave * share), n_tail = min(t_end, tail0 + share) - tail0;
+    auto run_start = [&](uint32_t i) { return i < rounds ? t_begin + (i * DW + wave) * RUN : tail0; };
+    auto run_tokens = [&](uint32_t i) { return i < rounds ? (uint32_t)RUN : i == rounds ? n_tail : 0u; };
 
-    // Loads of a run, issued one run ahead into the other of two register sets.  At 256, where registers are short, there is
-    // one set: values and norms are loaded again as soon as the run has been staged, keys when its scores are done.
-    uint32_t kraw_buf[SETS][SUB][2][NWK];
-    tq_u4 vpiece_buf[SETS][NVP];
-    uint16_t kn_buf[SETS], vn_buf[SETS];
-    auto issue_keys = [&](auto bsel, auto full_tag, uint32_t t0) __attribute__((always_inline)) {
-        constexpr int B = decltype(bsel)::value;
-        constexpr bool FULL = decltype(full_tag)::value;     // the run has all its tokens: no address is clamped
-        auto &kraw_next = kraw_buf[B];
-        const uint32_t n_tok = FULL ? (uint32_t)RUN : min((uint32_t)RUN, t_end - t0);
+    // Loads of a run, issued one run ahead: values and norms again as soon as the run has been staged, keys when its scores are done.
+    // (A second register set, with keys issued a little earlier, made two copies of the loop: no faster with many rows, and with few every
+    // copy is fetched for the first time, 512 rows x 16384 tokens 171 against 171 us, 128 rows x 4182 tokens 24.6 against 25.1.)
+    uint32_t kraw[SUB][2][NWK];
+    tq_u4 vpiece[NVP];
+    uint16_t kn_raw, vn_raw;
+    // n_tok >= 1: what lies past the last token is read as that token.  One form for whole and partial runs: with a branch between two
+    // the registers are merged behind it, and that waits for the loads just issued.
+    auto issue_keys = [&](uint32_t t0, uint32_t n_tok) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < SUB; ++u)
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 const uint32_t tl = 32u * u + 16u * b + n16;
-                const uint8_t *src = a.k_idx + (slot0 + t0 + ((FULL || tl < n_tok) ? tl : 0u)) * (4 * KB) + q4 * KB;
+                const uint8_t *src = a.k_idx + (slot0 + t0) * (4 * KB) + min(tl, n_tok - 1u) * (4 * KB) + q4 * KB;
                 if constexpr (KB % 16 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 16; ++p) {
                         const tq_u4 v = tq_gload16(src + 16 * p);
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) kraw_next[u][b][4 * p + i] = v[i];
+                        for (int i = 0; i < 4; ++i) kraw[u][b][4 * p + i] = v[i];
                     }
                 } else if constexpr (KB % 8 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 8; ++p) {
                         const tq_u2 v = tq_gload8(src + 8 * p);
-                        kraw_next[u][b][2 * p] = v[0]; kraw_next[u][b][2 * p + 1] = v[1];
+                        kraw[u][b][2 * p] = v[0]; kraw[u][b][2 * p + 1] = v[1];
                     }
                 } else if constexpr (KB % 4 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 4; ++p)
-                        kraw_next[u][b][p] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src + 4 * p);
+                        kraw[u][b][p] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src + 4 * p);
                 } else {
                     static_assert(KB % 2 == 0, "key bytes of a lane");
                     uint32_t h[KB / 2];
 #pragma unroll
                     for (int p = 0; p < KB / 2; ++p) h[p] = tq_gload2(reinterpret_cast<const uint16_t *>(src) + p);
 #pragma unroll
-                    for (int p = 0; p < NWK; ++p) kraw_next[u][b][p] = h[2 * p] | (2 * p + 1 < KB / 2 ? h[2 * p + 1 < KB / 2 ? 2 * p + 1 : 0] << 16 : 0u);
+                    for (int p = 0; p < NWK; ++p) kraw[u][b][p] = h[2 * p] | (2 * p + 1 < KB / 2 ? h[2 * p + 1 < KB / 2 ? 2 * p + 1 : 0] << 16 : 0u);
                 }
             }
     };
-    auto issue_values = [&](auto bsel, auto full_tag, uint32_t t0) __attribute__((always_inline)) {
-        constexpr int B = decltype(bsel)::value;
-        constexpr bool FULL = decltype(full_tag)::value;
-        auto &vpiece_next = vpiece_buf[B];
-        const uint32_t n_tok = FULL ? (uint32_t)RUN : min((uint32_t)RUN, t_end - t0);
+    auto issue_values = [&](uint32_t t0, uint32_t n_tok) __attribute__((always_inline)) {
         const uint8_t *vsrc = a.v_idx + (slot0 + t0) * GBV;
 #pragma unroll
         for (int p = 0; p < NVP; ++p) {
-            const uint32_t piece = p * 64u + lane;
-            const bool ok = piece < VPIECES && (FULL || piece * VPB < n_tok * GBV);
-            if constexpr (VPB == 16) vpiece_next[p] = tq_gload16(vsrc + (ok ? piece : 0u) * 16u);
-            else { const tq_u2 v = tq_gload8(vsrc + (ok ? piece : 0u) * 8u); vpiece_next[p][0] = v[0]; vpiece_next[p][1] = v[1]; }
+            const uint32_t piece = min(p * 64u + lane, min((uint32_t)VPIECES, n_tok * (GBV / VPB)) - 1u);
+            if constexpr (VPB == 16) vpiece[p] = tq_gload16(vsrc + piece * 16u);
+            else { const tq_u2 v = tq_gload8(vsrc + piece * 8u); vpiece[p][0] = v[0]; vpiece[p][1] = v[1]; }
         }
-        kn_buf[B] = lane < n_tok ? tq_gload2(a.k_norms + slot0 + t0 + lane) : (uint16_t)0;
-        vn_buf[B] = lane < n_tok ? tq_gload2(a.v_norms + slot0 + t0 + lane) : (uint16_t)0;   // tokens past the end weigh nothing
+        const uint32_t own = min(lane, n_tok - 1u);       // (lanes past the end: see trip)
+        kn_raw = tq_gload2(a.k_norms + slot0 + t0 + own);
+        vn_raw = tq_gload2(a.v_norms + slot0 + t0 + own);
     };
-    const uint32_t t_first = t_begin + RUN * wave;
-    if (t_first < t_end) {
-        issue_keys(std::integral_constant<int, 0>{}, std::false_type{}, t_first);
-        issue_values(std::integral_constant<int, 0>{}, std::false_type{}, t_first);
-    }
 
+    // ---- start: loads in the order in which their data is used, nothing waits for what it does not need.  Tables, then the operands of
+    // the query rotation (the first waves) or a tile of the window (from the last wave down), then the first run; a wave that has no run
+    // reads the row's first token (of a row without history, what the host put there instead).
+    const uint32_t win_tiles = (a.n_win + WIN_TILE - 1u) / WIN_TILE;     // tile w goes to the block of split w % splits
+    uint32_t wt = DW - 1u - wave;
+    TQ_GLOBAL float *wrec = (TQ_GLOBAL float *)a.win_part + (size_t)row * win_tiles * G * PART;
     if (tid < (uint32_t)DW) lds_trips[tid] = 0u;
-    stage_lut<IPBK>(lds_lut_k, a.table_k + hk_hd->off_lut, tid);
-    stage_lut<IPBV>(lds_lut_v, a.table_v + hv_hd->off_lut, tid);
-
-    // ---- rotated queries: q_rot[g][j] = scale * sum_i Pi[j][i] q[g][i], wave w the coordinates 32 w .. 32 w + 31
-    float *qrot = reinterpret_cast<float *>(&lds_area[0][0]);
-    if (wave < (uint32_t)TILES) {
-        const uint32_t n = lane & 31u, hk = lane >> 5;
-        const uint8_t *qsrc = a.queries + (((size_t)row * G + (n < G ? n : 0u)) * D + 8u * hk) * 2u;
-        const uint8_t *asrc = a.table_k + (a.bf16 ? hk_hd->off_a_bf16 : hk_hd->off_a_f16) + ((size_t)wave * STEPS * 64u + lane) * 16u;
-        tq_f16v acc = tq_zero16();
-        auto rotate = [&](auto bf_tag) __attribute__((always_inline)) {
-            constexpr bool BF = decltype(bf_tag)::value;
-            constexpr int TERMS = BF ? 3 : 2, CH = 4;        // steps whose operands are in flight together
-#pragma unroll 1
-            for (int s0 = 0; s0 < STEPS; s0 += 2 * CH) {
-                tq_u4 q[2 * CH], p[TERMS][2 * CH];
-#pragma unroll
-                for (int s = 0; s < 2 * CH; ++s) {
-                    if (s0 + s < STEPS) {
-                        q[s] = tq_gload16(qsrc + (s0 + s) * 32);
-#pragma unroll
-                        for (int t = 0; t < TERMS; ++t) p[t][s] = tq_gload16(asrc + (size_t)t * TQ_OPERAND_BYTES_FOR(D) + (size_t)(s0 + s) * 1024u);
-                    }
-                }
-#pragma unroll
-                for (int s = 0; s < 2 * CH; ++s) {
-                    if (s0 + s < STEPS) {
-#pragma unroll
-                        for (int t = 0; t < TERMS; ++t) acc = BF ? mfma_bf16(p[t][s], q[s], acc) : mfma_f16(p[t][s], q[s], acc);
-                    }
-                }
-            }
-        };
-        if (a.bf16) rotate(std::true_type{}); else rotate(std::false_type{});
-        const float f = a.bf16 ? a.scale : a.scale * (1.0f / (float)(1 << TQ_F16_PI_SHIFT));
-        if (n < (uint32_t)MAX_GROUP) {
-#pragma unroll
-            for (int r = 0; r < 16; r += 4)
-                *reinterpret_cast<float4 *>(qrot + n * QROW + 32u * wave + 16u * hk + r) = make_float4(acc[r] * f, acc[r + 1] * f, acc[r + 2] * f, acc[r + 3] * f);
-        }
-    }
-
-    // ---- the window: tile w of 32 tokens goes to the block of split w % splits, there to the waves from the last one down
-    const uint32_t win_tiles = (a.n_win + WIN_TILE - 1u) / WIN_TILE;
-    auto window_tile = [&](auto bf_tag, uint32_t wt) __attribute__((always_inline)) {
+    Lut<IPBK> table_k;
+    Lut<IPBV> table_v;
+    table_k.load(a.table_k + TQ_OFF_LUT(D), tid);
+    table_v.load(a.table_v + TQ_OFF_LUT(D), tid);
+    __builtin_amdgcn_sched_barrier(0);
+    auto first_run = [&]() __attribute__((always_inline)) {
+        const uint32_t n0 = run_tokens(0u), t0 = n0 ? run_start(0u) : 0u;
+        __builtin_amdgcn_sched_barrier(0);
+        issue_keys(t0, max(n0, 1u));
+        issue_values(t0, max(n0, 1u));
+        __builtin_amdgcn_sched_barrier(0);
+        table_k.store(lds_lut, tid);
+        table_v.store(lds_lut + 128, tid);
+    };
+    auto start = [&](auto bf_tag) __attribute__((always_inline)) {
         constexpr bool BF = decltype(bf_tag)::value;
-        auto mm = [](tq_u4 x, tq_u4 y, tq_f4v c) { return BF ? mfma16_bf16(x, y, c) : mfma16_f16(x, y, c); };
-        const uint32_t t0 = wt * WIN_TILE, left = min((uint32_t)WIN_TILE, a.n_win - t0);
-        const uint8_t *kw = a.k_win + ((size_t)row * a.win_stride + (size_t)t0 * D) * 2u;
-        const uint8_t *vw = a.v_win + ((size_t)row * a.win_stride + (size_t)t0 * D) * 2u;
-        const bool one = n16 < G;        // (a column per head here)
-        const uint8_t *qs = a.queries + (((size_t)row * G + (one ? n16 : 0u)) * D + 8u * q4) * 2u;
-        tq_f4v sc[2] = {tq_f4v{0.f, 0.f, 0.f, 0.f}, tq_f4v{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-        for (int s = 0; s < SK; ++s) {
-            const tq_u4 q = tq_gload16(qs + 64 * s);
-#pragma unroll
-            for (int b = 0; b < 2; ++b)      // past the end the last token is read again and not used
-                sc[b] = mm(tq_gload16(kw + (size_t)min(16u * b + n16, left - 1u) * (2 * D) + 64 * s + 16u * q4), q, sc[b]);
+        if (wave < (uint32_t)TILES) {
+            Rotation<D, BF> r;
+            r.load(a.queries + (size_t)row * G * D * 2u, G, a.table_k, wave, lane);
+            first_run();
+            r.finish(&lds_qrot[0][0], QROW, a.scale, wave, lane);
+        } else if (split + wt * splits < win_tiles) {
+            WindowTile<D, BF> w;
+            w.load(a, row, split + wt * splits, lane);
+            first_run();
+            w.finish(a, wrec + (size_t)(split + wt * splits) * G * PART, splits > 1u, lane);
+            wt += DW;
+        } else {
+            first_run();
         }
-        float t[8], m = -3.0e38f, l = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            t[j] = sc[j / 4][j % 4] * a.scale;       // token 16 (j / 4) + 4 q4 + j % 4 of the tile, head n16
-            if (16u * (j / 4) + 4u * q4 + (j % 4) >= left) t[j] = -3.0e38f;
-            m = fmaxf(m, t[j]);
-        }
-        m = fmaxf(m, __shfl_xor(m, 16));
-        m = fmaxf(m, __shfl_xor(m, 32));
-        float p[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            p[j] = 16u * (j / 4) + 4u * q4 + (j % 4) < left ? __expf(t[j] - m) : 0.f;
-            l += p[j];
-        }
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
-        tq_u4 pa[3];
-        split_f32x8(p, pa[0], pa[1], pa[2]);
-        TQ_GLOBAL float *rec = (TQ_GLOBAL float *)a.win_part + ((size_t)row * win_tiles + wt) * G * PART;
-        if (q4 == 0u && one) { put_record(splits > 1u, rec + n16 * PART, m); put_record(splits > 1u, rec + n16 * PART + 1u, l); }
-        // columns in chunks of 8 (or 4, 2): the same element of token pairs side by side, one operand per coordinate
-        auto columns = [&](auto n_tag, int c0) __attribute__((always_inline)) {
-            constexpr int N = decltype(n_tag)::value;
-            uint32_t v[8][N / 2];
-            const uint32_t first = value_coord<D>(n16, c0);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint8_t *src = vw + (size_t)min(16u * (j / 4) + 4u * q4 + (j % 4), left - 1u) * (2 * D) + 2u * first;
-                if constexpr (N == 8) { const tq_u4 x = tq_gload16(src); v[j][0] = x[0]; v[j][1] = x[1]; v[j][2] = x[2]; v[j][3] = x[3]; }
-                else if constexpr (N == 4) { const tq_u2 x = tq_gload8(src); v[j][0] = x[0]; v[j][1] = x[1]; }
-                else v[j][0] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src);
-            }
-            float odd = 0.f;         // NaN once a sum is not finite
-            auto column = [&](uint32_t c, tq_u4 bt, tq_f4v acc) __attribute__((always_inline)) {
-                tq_u4 hi = bt, lo;
-                if constexpr (!BF) split_f16x8(bt, hi, lo);
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    acc = mfma16_bf16(pa[k], hi, acc);
-                    if constexpr (!BF) acc = mfma16_bf16(pa[k], lo, acc);
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    odd = fmaf(acc[r], 0.f, odd);
-                    if (4u * q4 + r < G) put_record(splits > 1u, rec + (4u * q4 + r) * PART + 2u + first + c, acc[r]);
-                }
-            };
-#pragma unroll
-            for (int c = 0; c < N; ++c) {
-                tq_u4 bt;
-#pragma unroll
-                for (int d = 0; d < 4; ++d)
-                    bt[d] = __builtin_amdgcn_perm(v[2 * d + 1][c / 2], v[2 * d][c / 2], (c & 1) ? 0x07060302u : 0x05040100u);
-                column((uint32_t)c, bt, tq_f4v{0.f, 0.f, 0.f, 0.f});
-            }
-            if (__any(odd != odd)) {
-                // An infinite (or NaN) value met a lower term of its probability that is zero, or the zero weight of a token read
-                // again.  Once more: such values as bf16 against the leading terms, tokens past the end left out.
 #pragma unroll 1
-                for (uint32_t c = 0; c < (uint32_t)N; ++c) {
-                    tq_u4 bt, wild;
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        uint32_t pair = 0u;
-#pragma unroll
-                        for (int k = 0; k < 2; ++k) {
-                            const uint32_t t = 16u * (d / 2) + 4u * q4 + 2u * (d % 2) + k;
-                            if (t < left) pair |= (uint32_t)tq_gload2(reinterpret_cast<const uint16_t *>(vw + (size_t)t * (2 * D)) + first + c) << (16 * k);
-                        }
-                        constexpr uint32_t EXPO = BF ? 0x7f807f80u : 0x7c007c00u, ONE = BF ? 0x00800080u : 0x04000400u;
-                        const uint32_t mask = ((((pair & EXPO) + ONE) >> 15) & 0x00010001u) * 0xffffu;     // exponent all ones
-                        wild[d] = pair & mask;
-                        if constexpr (!BF)
-                            wild[d] = (wild[d] & 0x80008000u) | (mask & 0x7f807f80u) | ((((wild[d] & 0x03ff03ffu) + 0x03ff03ffu) >> 4) & 0x00400040u);
-                        bt[d] = pair & ~mask;
-                    }
-                    column(c, bt, mfma16_bf16(pa[0], wild, tq_f4v{0.f, 0.f, 0.f, 0.f}));
-                }
-            }
-        };
-        if constexpr (D == 64) columns(std::integral_constant<int, 4>{}, 0);
-        else if constexpr (D == 96) { columns(std::integral_constant<int, 4>{}, 0); columns(std::integral_constant<int, 2>{}, 4); }
-        else {
-#pragma unroll 1
-            for (int c0 = 0; c0 < NC; c0 += 8) columns(std::integral_constant<int, 8>{}, c0);
+        for (; split + wt * splits < win_tiles; wt += DW) {
+            WindowTile<D, BF> w;
+            w.load(a, row, split + wt * splits, lane);
+            w.finish(a, wrec + (size_t)(split + wt * splits) * G * PART, splits > 1u, lane);
         }
     };
-    for (uint32_t k = DW - 1u - wave; split + k * splits < win_tiles; k += DW) {
-        if (a.bf16) window_tile(std::true_type{}, split + k * splits);
-        else window_tile(std::false_type{}, split + k * splits);
-    }
+    if (a.bf16) start(std::true_type{}); else start(std::false_type{});
     __syncthreads();
 
     // ---- B operand of the score product: fp16 of q * 2^(10 - e), e = binary exponent of the head's largest magnitude.  At 256 with
@@ -443,7 +597,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     float c1;                // score in base-2 units = t * c1, t = accumulator * key norm
     float rowscale;          // natural score = t * rowscale
     {
-        const float *q = qrot + head * QROW + (D / 4) * q4;
+        const float *q = &lds_qrot[head][(D / 4) * q4];
         float x[D / 4];
 #pragma unroll
         for (int i = 0; i < D / 4; i += 4) {
@@ -453,8 +607,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         float big = 0.f;
 #pragma unroll
         for (int i = 0; i < D / 4; ++i) big = fmaxf(big, fabsf(x[i]));
-        big = fmaxf(big, __shfl_xor(big, 16));
-        big = fmaxf(big, __shfl_xor(big, 32));
+        big = reduce_rows(big, OpMax());
         int e = 0;
         if (big > 0.f && big < __builtin_inff()) (void)frexpf(big, &e);
         e = e < -100 ? -100 : e;
@@ -480,10 +633,9 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 if (wave == 0u) lds_q[(k - QREG) * SK + s][lane] = __builtin_bit_cast(tq_u4, term[k]);
         }
     }
-    __syncthreads();         // (the queries' LDS is the waves' staging area from here on)
+    if constexpr (QT > QREG) __syncthreads();
 
-    const uint32_t lut_k = tq_lds_offset(lds_lut_k) + RepLut<IPBK>::lane_offset(lane);
-    const uint32_t lut_v = tq_lds_offset(lds_lut_v) + RepLut<IPBV>::lane_offset(lane);
+    const uint32_t slot_k = RepLut<IPBK>::lane_offset(lane), slot_v = 128u + RepLut<IPBV>::lane_offset(lane);
     tq_f4v acc[NC];          // weighted value sums: register r = column 4 q4 + r of the scores (head and block of tokens), c = coordinate value_coord(n16, c)
 #pragma unroll
     for (int c = 0; c < NC; ++c) acc[c] = tq_f4v{0.f, 0.f, 0.f, 0.f};
@@ -496,17 +648,15 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
 
     // one run of staged tokens; FULL: all of them exist.  The score products of all its tiles come first, so that a later
     // tile's matrix work runs under an earlier one's softmax.
-    auto run = [&](auto bsel, auto full_tag, uint32_t n_tok, uint32_t t_next) __attribute__((always_inline)) {
-        constexpr int B = decltype(bsel)::value;
+    auto run = [&](auto full_tag, uint32_t n_tok, uint32_t t_next, uint32_t n_next) __attribute__((always_inline)) {
         constexpr bool FULL = decltype(full_tag)::value;
-        const auto &kraw = kraw_buf[B];
         tq_f4v sc[SUB][2];   // register r of block b = token 32 u + 16 b + 4 q4 + r
 #pragma unroll
         for (int u = 0; u < SUB; ++u) {
             sc[u][0] = sc[u][1] = tq_f4v{0.f, 0.f, 0.f, 0.f};
             if (!FULL && 32u * u >= n_tok) continue;       // uniform
             auto step = [&](int b, int s, const tq_u4 (&q)[QT]) __attribute__((always_inline)) {
-                const tq_u4 kd = decode_rep<IPBK, NWK>(kraw[u][b], s, lut_k);
+                const tq_u4 kd = decode_keys<IPBK, NWK>(kraw[u][b], s, lds_lut, slot_k);
 #pragma unroll
                 for (int k = 0; k < QT; ++k) sc[u][b] = mfma16_f16(kd, q[k], sc[u][b]);
             };
@@ -530,10 +680,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 }
             }
         }
-        if constexpr (SETS == 1 && FULL) {
-            if (t_next + RUN <= t_end) issue_keys(bsel, std::true_type{}, t_next);
-            else if (t_next < t_end) issue_keys(bsel, std::false_type{}, t_next);
-        }
+        if constexpr (FULL) issue_keys(t_next, n_next);
 #pragma unroll
         for (int u = 0; u < RUN / UNIT; ++u) {
             if (!FULL && (uint32_t)(UNIT * u) >= n_tok) break;  // uniform
@@ -633,7 +780,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                     const uint32_t first = value_coord<D>(n16, c0);
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        decode_values<IPBV, N>(vcodes + ((j < 4 ? tok_a : tok_b) + (uint32_t)(j % 4)) * GBV, first, lut_v, dec[j]);
+                        decode_values<IPBV, N>(vcodes + ((j < 4 ? tok_a : tok_b) + (uint32_t)(j % 4)) * GBV, first, lds_lut, slot_v, dec[j]);
 #pragma unroll
                     for (int c = 0; c < N; ++c) {
                         tq_u4 bt;
@@ -652,7 +799,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         }
     };
 
-    // one trip: stage the run held in register set B, start the loads of the next run into the other set, compute
+    // one trip: stage the run that has been loaded, start the loads of the next one, compute
     // The two waves of a SIMD (w and w + 4) are kept level: the one that is ahead yields.  Left alone the older of the two is
     // served first, and the other one ends its runs without anybody to cover its waits: of a row of 16384 tokens the first
     // waves had done their 32 runs after 69 us and waited 22 us for the others; now all take 84 us and wait one
@@ -660,28 +807,28 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     uint32_t trips = 0u;
     auto keep_level = [&]() __attribute__((always_inline)) {
         ++trips;
-        volatile uint32_t *count = lds_trips;
+        volatile __attribute__((address_space(3))) uint32_t *count = (__attribute__((address_space(3))) uint32_t *)lds_trips;
         if (lane == 0u) count[wave] = trips;
         if (trips > tq_uniform32(count[wave ^ 4u])) __builtin_amdgcn_s_setprio(0); else __builtin_amdgcn_s_setprio(1);
     };
-    auto trip = [&](auto bsel, auto full_tag, uint32_t t0) __attribute__((always_inline)) {
-        constexpr int B = decltype(bsel)::value;
+    auto trip = [&](auto full_tag, uint32_t i) __attribute__((always_inline)) {
         keep_level();
         constexpr bool FULL = decltype(full_tag)::value;
-        const uint32_t n_tok = FULL ? (uint32_t)RUN : t_end - t0;
+        const uint32_t n_tok = FULL ? (uint32_t)RUN : run_tokens(i);
 #pragma unroll
         for (int p = 0; p < NVP; ++p) {
             const uint32_t piece = p * 64u + lane;
             if (VPIECES % 64 == 0 || piece < VPIECES) {
-                if constexpr (VPB == 16) *reinterpret_cast<tq_u4 *>(vcodes + piece * 16u) = vpiece_buf[B][p];
-                else *reinterpret_cast<tq_u2 *>(vcodes + piece * 8u) = tq_u2{vpiece_buf[B][p][0], vpiece_buf[B][p][1]};
+                if constexpr (VPB == 16) *reinterpret_cast<tq_u4 *>(vcodes + piece * 16u) = vpiece[p];
+                else *reinterpret_cast<tq_u2 *>(vcodes + piece * 8u) = tq_u2{vpiece[p][0], vpiece[p][1]};
             }
         }
         {
-            const _Float16 kh = __builtin_bit_cast(_Float16, kn_buf[B]);
+            const _Float16 kh = __builtin_bit_cast(_Float16, kn_raw);
             if (RUN == 64 || lane < (uint32_t)RUN) lds_kn[wave][lane] = (float)kh;     // one token per lane
             // does a value norm of this run exceed the reference exponent?  (a vote; a handful of times per wave)
-            uint32_t e = ((uint32_t)vn_buf[B] >> 10) & 31u;
+            const uint16_t vn = (FULL && RUN == 64) || lane < n_tok ? vn_raw : (uint16_t)0;   // tokens past the end weigh nothing
+            uint32_t e = ((uint32_t)vn >> 10) & 31u;
             if (__any((int)max(e, 1u) - 15 > ev_ref)) {
                 // largest exponent field of the run: row-wise running maximum, then the four row ends
                 e = max(e, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e, 0x111, 0xf, 0xf, true));
@@ -696,56 +843,29 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 for (int c = 0; c < NC; ++c) acc[c] *= f;
                 ev_ref = ev;
             }
-            const _Float16 vh = __builtin_bit_cast(_Float16, vn_buf[B]);
+            const _Float16 vh = __builtin_bit_cast(_Float16, vn);
             const float vs = ldexpf((float)vh, -ev_ref);
             if (RUN == 64 || lane < (uint32_t)RUN) {
                 if constexpr (PT == 1) lds_vn[wave][lane] = __builtin_bit_cast(uint16_t, (_Float16)vs);
                 else lds_vn[wave][lane] = vs;
             }
         }
-        const uint32_t t_next = t0 + RUN * DW;
-        constexpr auto nsel = std::integral_constant<int, SETS == 2 ? 1 - B : 0>{};
-        if constexpr (FULL) {
-            if (t_next + RUN <= t_end) {
-                if constexpr (SETS == 2) issue_keys(nsel, std::true_type{}, t_next);
-                issue_values(nsel, std::true_type{}, t_next);
-            } else if (t_next < t_end) {
-                if constexpr (SETS == 2) issue_keys(nsel, std::false_type{}, t_next);
-                issue_values(nsel, std::false_type{}, t_next);
-            }
-        }
+        // (behind the last run the row's first token is read again)
+        const uint32_t n_more = run_tokens(i + 1u), t_next = n_more ? run_start(i + 1u) : 0u, n_next = max(n_more, 1u);
+        if constexpr (FULL) issue_values(t_next, n_next);
         asm volatile("" ::: "memory");    // staged with one access width, read back with others (LDS serves a wave in order)
         __builtin_amdgcn_wave_barrier();
-        run(bsel, full_tag, n_tok, t_next);
+        run(full_tag, n_tok, t_next, n_next);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_wave_barrier();
-        return t_next;
     };
     {
         // whole runs in the loop, the partial one (a wave has one at most) behind it: with both kinds in one loop body the
         // accumulators are copied where they meet and registers spill
-        uint32_t t0 = t_first;
-        while (t0 + RUN <= t_end) {
-            t0 = trip(std::integral_constant<int, 0>{}, std::true_type{}, t0);
-            if constexpr (SETS == 2) {
-                if (t0 + RUN > t_end) {       // what has been loaded last moves to the set the partial run is taken from
-#pragma unroll
-                    for (int u = 0; u < SUB; ++u)
-#pragma unroll
-                        for (int b = 0; b < 2; ++b)
-#pragma unroll
-                            for (int i = 0; i < NWK; ++i) kraw_buf[0][u][b][i] = kraw_buf[SETS - 1][u][b][i];
-#pragma unroll
-                    for (int p = 0; p < NVP; ++p) vpiece_buf[0][p] = vpiece_buf[SETS - 1][p];
-                    kn_buf[0] = kn_buf[SETS - 1];
-                    vn_buf[0] = vn_buf[SETS - 1];
-                    break;
-                }
-                t0 = trip(std::integral_constant<int, SETS - 1>{}, std::true_type{}, t0);
-            }
-        }
-        if (t0 < t_end) trip(std::integral_constant<int, 0>{}, std::false_type{}, t0);
-        if (lane == 0u) *(volatile uint32_t *)&lds_trips[wave] = 0xffffffffu;
+        uint32_t i = 0u;
+        while (run_tokens(i) == (uint32_t)RUN) trip(std::true_type{}, i++);
+        if (run_tokens(i)) trip(std::false_type{}, i);
+        if (lane == 0u) *(volatile __attribute__((address_space(3))) uint32_t *)&lds_trips[wave] = 0xffffffffu;
         __builtin_amdgcn_s_setprio(0);
     }
     asm volatile("" ::: "memory");
@@ -796,22 +916,30 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
             }
         }
         __syncthreads();
-        const uint32_t total = min((uint32_t)HR, G - h0) * PART;
-        for (uint32_t i = tid; i < total; i += DTHREADS) {
-            const uint32_t g = i / PART, j = i % PART;
-            float mw[DW], mall = -3.0e38f;
+        for (uint32_t i = 2u * tid; i < min((uint32_t)HR, G - h0) * D; i += 2u * DTHREADS) {
+            const uint32_t g = i / D, j = i % D;
+            const float *rec = reinterpret_cast<const float *>(lds_area[0]) + g * PART;      // wave w: AREA bytes further
+            float f[DW], mall = -3.0e38f, v0 = 0.f, v1 = 0.f;
 #pragma unroll
             for (int w = 0; w < DW; ++w) {
-                mw[w] = reinterpret_cast<const float *>(lds_area[w])[g * PART];
-                mall = fmaxf(mall, mw[w]);
+                f[w] = rec[w * (AREA / 4)];
+                mall = fmaxf(mall, f[w]);
             }
-            float v = mall;
-            if (j != 0u) {
-                v = 0.f;
 #pragma unroll
-                for (int w = 0; w < DW; ++w) v += __expf(mw[w] - mall) * reinterpret_cast<const float *>(lds_area[w])[g * PART + j];
+            for (int w = 0; w < DW; ++w) {
+                f[w] = __expf(f[w] - mall);
+                const float2 two = *reinterpret_cast<const float2 *>(rec + w * (AREA / 4) + 2u + j);
+                v0 += f[w] * two.x;
+                v1 += f[w] * two.y;
             }
-            put_record(splits > 1u, (TQ_GLOBAL float *)dst + h0 * PART + i, v);
+            TQ_GLOBAL float *out = (TQ_GLOBAL float *)dst + (h0 + g) * PART;
+            if (splits > 1u) put_record2<true>(out + 2u + j, v0, v1); else put_record2<false>(out + 2u + j, v0, v1);
+            if (j == 0u) {
+                float l = 0.f;
+#pragma unroll
+                for (int w = 0; w < DW; ++w) l += f[w] * rec[w * (AREA / 4) + 1];
+                if (splits > 1u) put_record2<true>(out, mall, l); else put_record2<false>(out, mall, l);
+            }
         }
     }
 
@@ -820,6 +948,16 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     // do, thread 0 may count the block as done, see put_record)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    // rows of Pi_v for the rotation back: thread (four columns, part) takes ROTK of them.  Loaded while the counter is asked whether
+    // they are needed (all blocks but one of a row load them for nothing: 4 D^2 bytes from the L2); wave 0, which asks, afterwards.
+    const uint32_t rc = (tid % (D / 4)) * 4u, rp = tid / (D / 4);
+    tq_u4 pv[ROTK];
+    auto load_pv = [&]() __attribute__((always_inline)) {
+        const uint8_t *src = reinterpret_cast<const uint8_t *>(a.pi_v + (size_t)(min(rp, (uint32_t)ROTP - 1u) * ROTK) * D + rc);
+#pragma unroll
+        for (int k = 0; k < ROTK; ++k) pv[k] = tq_gload16(src + k * (D * 4));
+    };
+    if (wave) load_pv();
     if (splits > 1u) {
         if (tid == 0u) {
             const bool last = __hip_atomic_fetch_add(a.arrived + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1u;
@@ -829,93 +967,112 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         __syncthreads();
         if (!lds_last) return;
     }
-    const TQ_GLOBAL float *part = (const TQ_GLOBAL float *)a.partial + (size_t)row * splits * G * PART;
-    const TQ_GLOBAL float *wpart = (const TQ_GLOBAL float *)a.win_part + (size_t)row * win_tiles * G * PART;
-    // rows of Pi_v for the rotation back: thread (four columns, part) takes ROTK of them
-    const uint32_t rc = (tid % (D / 4)) * 4u, rp = tid / (D / 4);
-    constexpr int RH = ROTK > 8 ? 8 : ROTK;           // held at a time
-    tq_u4 pv[RH];
-    auto load_pv = [&](int k0) {
-        if (rp < (uint32_t)ROTP) {
-#pragma unroll
-            for (int k = 0; k < RH; ++k) pv[k] = tq_gload16(reinterpret_cast<const uint8_t *>(a.pi_v + (size_t)(rp * ROTK + k0 + k) * D + rc));
-        }
-    };
-    if constexpr (ROTK == RH) load_pv(0);
+    if (!wave) load_pv();
     float *ysum = reinterpret_cast<float *>(&lds_area[0][0]);     // [head][D]: sums in the rotated space
     float *wsum = ysum + MAX_GROUP * D;                           // [head][D]: the window's, plain
+    // One trip to memory where few records meet: references and sums of exp of a head's records (a lane each) and the sums (four columns
+    // a lane, every fourth record; the quarters of a wave are added in registers) are under way together.  Little code: it runs once
+    // and is fetched for the first time (33 loads a lane, written out: 2.0 us from the first to the last of them, now 0.4).
     auto merge = [&](auto across_tag) __attribute__((always_inline)) {
         constexpr bool ACROSS = decltype(across_tag)::value;
+        constexpr int YB = 8;                                         // records a lane has under way
+        const uint32_t step = G * PART, nrec = splits + win_tiles;    // (a row's records lie within 4.5 MiB)
+        const Records part(a.partial + (size_t)row * splits * step, splits * step), wpart(a.win_part + (size_t)row * win_tiles * step, win_tiles * step);
         // weights of the records: exp(reference - largest reference of the head)
-        float *wgt = reinterpret_cast<float *>(lds_lut_k);            // [head][splits + window tiles]
-        const uint32_t nrec = splits + win_tiles;
-        for (uint32_t g = wave; g < G; g += DW) {
-            float m = -3.0e38f;
-            for (uint32_t s = lane; s < nrec; s += 64u) {
-                const float x = get_record<ACROSS>(s < splits ? part + ((size_t)s * G + g) * PART : wpart + ((size_t)(s - splits) * G + g) * PART);
-                m = fmaxf(m, x);
-            }
+        float *wgt = reinterpret_cast<float *>(lds_lut);              // [head][splits, then window tiles: each up to a multiple of 4, zeros behind]
+        const uint32_t wfirst = (splits + 3u) / 4u * 4u, wrow = wfirst + (win_tiles + 3u) / 4u * 4u;
+        auto place = [&](uint32_t s) { return s < splits ? s : wfirst + s - splits; };
+        auto head_of = [&](uint32_t s, uint32_t g) { return s < splits ? part.load2<ACROSS>(s * step + g * PART) : wpart.load2<ACROSS>((s - splits) * step + g * PART); };
+        tq_u2 ml = {0u, 0u};
+        tq_u4 y[YB], w;
+        if (wave < G && lane < nrec) ml = head_of(lane, wave);
+        auto fetch = [&](uint32_t off, uint32_t s0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+            for (int s = 0; s < YB; ++s) y[s] = part.load4<ACROSS>((s0 + 4u * s + q4) * step + off);
+        };
+        const uint32_t col = (wave * 16u + n16) * 4u;                 // + DTHREADS: further heads
+        fetch(col / D * PART + 2u + col % D, 0u);
+        w = wpart.load4<ACROSS>(q4 * step + col / D * PART + 2u + col % D);
+        for (uint32_t g = wave; g < G; g += DW) {
+            if (g != wave && lane < nrec) ml = head_of(lane, g);
+            float m = lane < nrec ? __uint_as_float(ml[0]) : -3.0e38f;
+            for (uint32_t s = lane + 64u; s < nrec; s += 64u) m = fmaxf(m, __uint_as_float(head_of(s, g)[0]));
+            m = reduce_wave(m, OpMax());
+            for (uint32_t s = lane; s < wrow; s += 64u) wgt[g * wrow + s] = 0.f;      // (the LDS serves a wave in order)
+            asm volatile("" ::: "memory");
             float den = 0.f;
             for (uint32_t s = lane; s < nrec; s += 64u) {
-                const TQ_GLOBAL float *r = s < splits ? part + ((size_t)s * G + g) * PART : wpart + ((size_t)(s - splits) * G + g) * PART;
-                const float f = __expf(get_record<ACROSS>(r) - m);
-                wgt[g * nrec + s] = f;
-                den = fmaf(f, get_record<ACROSS>(r + 1), den);
+                const tq_u2 r = s == lane ? ml : head_of(s, g);
+                const float f = __expf(__uint_as_float(r[0]) - m);
+                wgt[g * wrow + place(s)] = f;
+                den = fmaf(f, __uint_as_float(r[1]), den);
             }
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) den += __shfl_xor(den, d);
+            den = reduce_wave(den, OpAdd());
             if (lane == 0u) lds_den[g] = den;
         }
         __syncthreads();
-        for (uint32_t p = tid; p < G * D; p += DTHREADS) {
-            const uint32_t g = p / D, j = p % D;
-            const float *f = wgt + g * nrec;
-            float y = 0.f, w = 0.f;
-#pragma unroll 8
-            for (uint32_t s = 0; s < splits; ++s) y = fmaf(f[s], get_record<ACROSS>(part + ((size_t)s * G + g) * PART + 2u + j), y);
-#pragma unroll 4
-            for (uint32_t s = 0; s < win_tiles; ++s) w = fmaf(f[splits + s], get_record<ACROSS>(wpart + ((size_t)s * G + g) * PART + 2u + j), w);
-            ysum[p] = y;
-            wsum[p] = w;
+        for (uint32_t p = col; p < G * D; p += DTHREADS) {
+            const uint32_t g = p / D, off = g * PART + 2u + p % D;
+            const float *f = wgt + g * wrow + q4;
+            float ys[4] = {0.f, 0.f, 0.f, 0.f}, ws[4] = {0.f, 0.f, 0.f, 0.f};
+            for (uint32_t s0 = 0; s0 < splits; s0 += 4 * YB) {
+                if (p != col || s0) fetch(off, s0);
+#pragma unroll
+                for (int s = 0; s < YB; ++s) {
+                    if (s0 + 4u * s >= splits) break;     // (uniform)
+                    const float fs = f[s0 + 4 * s];       // (zero for what lies past the last record)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) ys[c] = fmaf(fs, __uint_as_float(y[s][c]), ys[c]);
+                }
+            }
+            for (uint32_t s0 = 0; s0 < win_tiles; s0 += 4u) {
+                if (p != col || s0) w = wpart.load4<ACROSS>((s0 + q4) * step + off);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) ws[c] = fmaf(f[wfirst + s0], __uint_as_float(w[c]), ws[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                ys[c] = reduce_rows(ys[c], OpAdd());
+                ws[c] = reduce_rows(ws[c], OpAdd());
+            }
+            if (q4 == 0u) {
+                *reinterpret_cast<float4 *>(ysum + p) = make_float4(ys[0], ys[1], ys[2], ys[3]);
+                *reinterpret_cast<float4 *>(wsum + p) = make_float4(ws[0], ws[1], ws[2], ws[3]);
+            }
         }
         __syncthreads();
     };
     if (splits > 1u) merge(std::true_type{}); else merge(std::false_type{});
-    // out = (ysum @ Pi_v + wsum) / den, four heads at a time
-    float *parts = reinterpret_cast<float *>(lds_lut_v);          // [part][4][D]
-    for (uint32_t g0 = 0; g0 < G; g0 += 4u) {
-        float x[4][4];
+    // out = (ysum @ Pi_v + wsum) / den, RG heads at a time
+    float *parts = reinterpret_cast<float *>(lds_lut);            // [part][RG][D]
+    for (uint32_t g0 = 0; g0 < G; g0 += RG) {
+        float x[RG][4];
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+        for (int g = 0; g < RG; ++g)
 #pragma unroll
             for (int c = 0; c < 4; ++c) x[g][c] = 0.f;
-#pragma unroll 1
-        for (int k0 = 0; k0 < ROTK; k0 += RH) {
-            if constexpr (ROTK != RH) load_pv(k0);
-            if (rp < (uint32_t)ROTP) {
+        if (rp < (uint32_t)ROTP) {
 #pragma unroll
-                for (int k = 0; k < RH; ++k)
+            for (int k = 0; k < ROTK; k += 2)
 #pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const float y = ysum[(g0 + g) * D + rp * ROTK + k0 + k];     // (heads past the last one: whatever lies there, not stored)
+                for (int g = 0; g < RG; ++g) {
+                    // (heads past the last one: whatever lies there, not stored)
+                    const float2 y = *reinterpret_cast<const float2 *>(ysum + (g0 + g) * D + rp * ROTK + k);
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) x[g][c] = fmaf(y, __uint_as_float(pv[k][c]), x[g][c]);
-                    }
-            }
+                    for (int c = 0; c < 4; ++c) x[g][c] = fmaf(y.y, __uint_as_float(pv[k + 1][c]), fmaf(y.x, __uint_as_float(pv[k][c]), x[g][c]));
+                }
         }
         if (g0) __syncthreads();
         if (rp < (uint32_t)ROTP) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) *reinterpret_cast<float4 *>(parts + (rp * 4u + g) * D + rc) = make_float4(x[g][0], x[g][1], x[g][2], x[g][3]);
+            for (int g = 0; g < RG; ++g) *reinterpret_cast<float4 *>(parts + (rp * RG + g) * D + rc) = make_float4(x[g][0], x[g][1], x[g][2], x[g][3]);
         }
         __syncthreads();
-        for (uint32_t p = tid; p < min(4u, G - g0) * D; p += DTHREADS) {
+        for (uint32_t p = tid; p < min((uint32_t)RG, G - g0) * D; p += DTHREADS) {
             const uint32_t g = p / D, j = p % D;
             float v = 0.f;
 #pragma unroll
-            for (int q = 0; q < ROTP; ++q) v += parts[((uint32_t)q * 4u + g) * D + j];
+            for (int q = 0; q < ROTP; ++q) v += parts[((uint32_t)q * RG + g) * D + j];
             v = (v + wsum[(g0 + g) * D + j]) / lds_den[g0 + g];
             TQ_GLOBAL uint16_t *o = (TQ_GLOBAL uint16_t *)a.out + ((size_t)row * G + g0 + g) * D + j;
             if (a.bf16) { const __bf16 h = (__bf16)v; *o = __builtin_bit_cast(uint16_t, h); }

@@ -303,40 +303,33 @@ struct RepLut {
     }
 };
 
-// Address of entry <byte B of raw> of a replicated table, `lut` = the lane's slot of entry 0: raw.byte[B] * 128 + lut as one
-// instruction (a dot product of four bytes with three zero weights) where extracting, shifting and adding take two or three.
-// A lookup is one LDS read of 2 to 4 clocks a compute unit, so those instructions were what the attention loop issued most.
-typedef const __attribute__((address_space(3))) uint8_t *tq_lds_ptr;
-static __device__ __forceinline__ uint32_t tq_lds_offset(const uint8_t *p) { return (uint32_t)(uintptr_t)(tq_lds_ptr)p; }
-template <int B, typename T>
-static __device__ __forceinline__ T tq_rep_entry(uint32_t raw, uint32_t lut) {
-    return *(const __attribute__((address_space(3))) T *)(uintptr_t)__builtin_amdgcn_udot4(raw, 0x80u << (8 * B), lut, false);
-}
-
-// decode_step against a replicated table; `lut` = the lane's slot of entry 0 (tq_lds_offset)
+// decode_step against a replicated table; `lut` already points at the lane's slot of entry 0
 template <int IPB, int NW>
-__device__ __forceinline__ tq_u4 decode_rep(const uint32_t (&raw)[NW], int s, uint32_t lut) {
+__device__ __forceinline__ tq_u4 decode_rep(const uint32_t (&raw)[NW], int s, const uint8_t *lut) {
     tq_u4 out;
     if constexpr (IPB == 1) {
 #pragma unroll
-        for (int d = 0; d < 2; ++d) {
-            const uint32_t r = raw[2 * s + d];
-            out[2 * d] = (uint32_t)tq_rep_entry<0, uint16_t>(r, lut) | ((uint32_t)tq_rep_entry<1, uint16_t>(r, lut) << 16);
-            out[2 * d + 1] = (uint32_t)tq_rep_entry<2, uint16_t>(r, lut) | ((uint32_t)tq_rep_entry<3, uint16_t>(r, lut) << 16);
+        for (int d = 0; d < 4; ++d) {
+            const uint32_t b0 = (raw[2 * s + (2 * d) / 4] >> (8 * ((2 * d) % 4))) & 0xffu;
+            const uint32_t b1 = (raw[2 * s + (2 * d + 1) / 4] >> (8 * ((2 * d + 1) % 4))) & 0xffu;
+            const uint32_t lo = *reinterpret_cast<const uint16_t *>(lut + (b0 << 7));
+            const uint32_t hi = *reinterpret_cast<const uint16_t *>(lut + (b1 << 7));
+            out[d] = lo | (hi << 16);
         }
     } else if constexpr (IPB == 2) {
-        out[0] = tq_rep_entry<0, uint32_t>(raw[s], lut);
-        out[1] = tq_rep_entry<1, uint32_t>(raw[s], lut);
-        out[2] = tq_rep_entry<2, uint32_t>(raw[s], lut);
-        out[3] = tq_rep_entry<3, uint32_t>(raw[s], lut);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) out[d] = *reinterpret_cast<const uint32_t *>(lut + (((raw[s] >> (8 * d)) & 0xffu) << 7));
     } else if constexpr (IPB == 4) {
-        const uint32_t r = raw[s / 2];
-        const tq_u2 v0 = s % 2 ? tq_rep_entry<2, tq_u2>(r, lut) : tq_rep_entry<0, tq_u2>(r, lut);
-        const tq_u2 v1 = s % 2 ? tq_rep_entry<3, tq_u2>(r, lut) : tq_rep_entry<1, tq_u2>(r, lut);
-        out = tq_u4{v0[0], v0[1], v1[0], v1[1]};
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const uint32_t b = (raw[s / 2] >> (16 * (s % 2) + 8 * q)) & 0xffu;
+            const tq_u2 v = *reinterpret_cast<const tq_u2 *>(lut + (b << 7));
+            out[2 * q] = v[0];
+            out[2 * q + 1] = v[1];
+        }
     } else {
-        const uint32_t r = raw[s / 4];
-        out = s % 4 == 0 ? tq_rep_entry<0, tq_u4>(r, lut) : s % 4 == 1 ? tq_rep_entry<1, tq_u4>(r, lut) : s % 4 == 2 ? tq_rep_entry<2, tq_u4>(r, lut) : tq_rep_entry<3, tq_u4>(r, lut);
+        const uint32_t b = (raw[s / 4] >> (8 * (s % 4))) & 0xffu;
+        out = *reinterpret_cast<const tq_u4 *>(lut + (b << 7));
     }
     return out;
 }

@@ -103,15 +103,14 @@ bool supported_head_dim(int d) { return d >= TQ_ANYDIM_MIN && d <= TQ_ANYDIM_MAX
 
 Layout layout_for(int head_dim, int bits) {
     const uint32_t levels = 1u << bits, ipb = 8u / (uint32_t)bits;
-    const uint32_t operand = (uint32_t)TQ_OPERAND_BYTES_FOR(head_dim);
     Layout L{};
-    uint32_t off = sizeof(TqTableHeader);
-    L.off_a_f16 = off;      off += 2 * operand;
-    L.off_a_bf16 = off;     off += 3 * operand;
-    L.off_at_f16 = off;     off += 2 * operand;
-    L.off_grid = off;       off += round_up(TQ_GRID_LDS_BYTES, 256);
+    L.off_a_f16 = TQ_OFF_A_F16;
+    L.off_a_bf16 = TQ_OFF_A_BF16(head_dim);
+    L.off_at_f16 = TQ_OFF_AT_F16(head_dim);
+    L.off_grid = TQ_OFF_GRID(head_dim);
     L.lut_entry_bytes = 2 * ipb;
-    L.off_lut = off;        off += round_up(256 * L.lut_entry_bytes, 256);
+    L.off_lut = TQ_OFF_LUT(head_dim);
+    uint32_t off = L.off_lut + round_up(256 * L.lut_entry_bytes, 256);
     L.off_centroids = off;  off += round_up(levels * 4, 256);
     L.off_thresholds = off; off += round_up(levels * 4, 256);
     if (head_dim == TQ_HEAD_DIM / 2) {

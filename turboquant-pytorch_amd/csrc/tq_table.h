@@ -65,6 +65,14 @@
 #define TQ_GRID_COPY_STRIDE(bits) (TQ_GRID_LDS_BYTES / TQ_GRID_COPIES(bits))
 #define TQ_GRID_MAX_CELLS(bits) (TQ_GRID_COPY_STRIDE(bits) / 8)
 
+// Sections every table of a head dimension has at the same place whatever its width (the header holds them too): a kernel whose
+// launch is a chain of a few loads takes them from here and saves the load of the header in front.
+#define TQ_OFF_A_F16 256u
+#define TQ_OFF_A_BF16(d) (TQ_OFF_A_F16 + 2u * TQ_OPERAND_BYTES_FOR(d))
+#define TQ_OFF_AT_F16(d) (TQ_OFF_A_BF16(d) + 3u * TQ_OPERAND_BYTES_FOR(d))
+#define TQ_OFF_GRID(d) (TQ_OFF_AT_F16(d) + 2u * TQ_OPERAND_BYTES_FOR(d))
+#define TQ_OFF_LUT(d) (TQ_OFF_GRID(d) + TQ_GRID_LDS_BYTES)
+
 struct TqGridCell {
     float threshold;
     uint32_t base;
@@ -101,7 +109,8 @@ struct TqTableHeader {
     uint32_t padded_dim;      // TQ_PADDED_DIM(head_dim): the dimension of the operand sets
     uint32_t reserved[41];
 };
-static_assert(sizeof(TqTableHeader) == 256, "header is one 256-byte block");
+static_assert(sizeof(TqTableHeader) == TQ_OFF_A_F16, "header is one 256-byte block");
+static_assert(TQ_GRID_LDS_BYTES % 256 == 0 && TQ_OPERAND_BYTES_FOR(8) % 256 == 0, "sections start on 256-byte boundaries");
 
 // --- table of the V2 key path (MSE codes + 1-bit QJL signs of the residual) ---------------------------------------
 // Operand tiles in the compress tiling above (tile = wave, out = 32w + 16h + r, input = 16s + 8hk + i), as fp16 terms
