@@ -282,6 +282,14 @@ int tq_qjl_compress_batched(const tq_qjl_job *jobs_host, const tq_qjl_job *jobs_
 int tq_qjl_scores(const uint8_t *idx_bytes, const uint16_t *vec_norms, const uint8_t *sign_bytes, const uint16_t *residual_norm,
                   long long rows, long long tokens, const void *table_dev, int head_dim, int mse_bits,
                   const float *q_rot, const float *q_sign, long long n_queries, float *scores, void *stream);
+/*
+ * The same scores for up to 8 query tokens per row from the raw queries [rows, n_queries, head_dim] (`dtype`, contiguous), which are rotated
+ * and projected in the launch: `both_dev` holds Pi^T and sqrt(pi/2) / head_dim * S^T one behind the other (float32, 16-byte aligned).
+ * head_dim 128, rows <= 65535.
+ */
+int tq_qjl_query_scores(const uint8_t *idx_bytes, const uint16_t *vec_norms, const uint8_t *sign_bytes, const uint16_t *residual_norm,
+                        long long rows, long long tokens, const void *table_dev, const float *both_dev, int head_dim, int mse_bits,
+                        const void *queries, int dtype, long long n_queries, float *scores, void *stream);
 
 /*
  * tq_decompress_batched for callers that cannot allocate device memory and have no workspace to pass: code

@@ -209,3 +209,24 @@ def test_v2_keys_at_other_head_dimensions(pkg, oracle, D, bits, dtype):
     keep = same.reshape(4, 1, n_tok).repeat(9, axis=1)
     err = (np.abs(got.reshape(4, 9, n_tok) - want) / scale)[keep]
     assert err.max() < 1e-3
+
+
+@pytest.mark.parametrize("bits,dtype", [(2, torch.bfloat16), (3, torch.float16), (4, torch.float32), (7, torch.bfloat16)])
+def test_v2_scores_of_few_queries_equal_those_of_many(pkg, bits, dtype):
+    """Up to 8 query tokens a row are rotated and projected inside the scores launch, more of them by library products in front of another
+    kernel.  Both products are float32 (2^-23 of |q| each, some 12 roundings of a dot product: 1.4e-6 |q| |k|); where that moves the
+    projected query across a rounding of its single fp16 term, 2^-11 of a coordinate of the correction moves with it: 128 such
+    coordinates of a correction of up to 0.6 |q| |k|, at random, 2^-11 * 0.6 / sqrt(128) = 2.6e-5 |q| |k| if all of them did."""
+    comp = pkg.TurboQuantCompressorV2(128, bits, seed=5, device=DEV)
+    g = torch.Generator().manual_seed(bits)
+    for rows, tokens in ((1, 1), (3, 63), (2, 65), (1, 513), (2, 1100), (300, 40)):
+        x = outlier_kv((1, rows, tokens, 128), seed=tokens, dtype=torch.bfloat16).to(DEV)
+        packed = comp.compress(x)
+        q = torch.randn(1, rows, 9, 128, generator=g).to(dtype).to(DEV)
+        many = comp.asymmetric_attention_scores(q, packed)
+        scale = q.double().norm(dim=-1)[..., None] * x.double().norm(dim=-1)[:, :, None, :]
+        for n in (1, 3, 8):
+            few = comp.asymmetric_attention_scores(q[:, :, :n], packed)
+            assert few.shape == (1, rows, n, tokens)
+            err = float(((few.double() - many[:, :, :n].double()).abs() / scale[:, :, :n]).max())
+            assert err < 3e-5, (rows, tokens, n, err)

@@ -20,14 +20,15 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libtqamd.so")
-SOURCES = ("tq_host.cpp", "tq_compress.hip", "tq_decompress.hip", "tq_anydim.hip", "tq_wide.hip", "tq_attend.hip", "tq_qjl.hip",
+SOURCES = ("tq_host.cpp", "tq_compress.hip", "tq_decompress.hip", "tq_anydim.hip", "tq_wide.hip", "tq_attend.hip", "tq_qjl.hip", "tq_qjl_scores.hip",
            "tq_decode.hip", "tq_decode_d64.hip", "tq_decode_d96.hip", "tq_decode_d128_narrow.hip", "tq_decode_d128_wide.hip", "tq_decode_d256.hip")
-HEADERS = ("tq_table.h", "tq_device.h", "tq_anydim.h", "tq_wide.h", "tq_decode.h", "tq_decode_kernel.h", os.path.join("..", "..", "include", "tqamd.h"))
+HEADERS = ("tq_table.h", "tq_device.h", "tq_anydim.h", "tq_wide.h", "tq_lut.h", "tq_decode.h", "tq_decode_kernel.h", os.path.join("..", "..", "include", "tqamd.h"))
 GPU_ARCH = "gfx950"
 
 TQ_F32, TQ_F16, TQ_BF16 = 0, 1, 2
 _DTYPE_CODE = {torch.float32: TQ_F32, torch.float16: TQ_F16, torch.bfloat16: TQ_BF16}
 HEAD_DIM = 128
+MAX_QUERY_SCORES = 8    # query tokens a row that tq_qjl_query_scores takes
 
 
 class TqError(RuntimeError):
@@ -177,7 +178,7 @@ EXPORTS = (
     "tq_decision_thresholds", "tq_table_bytes", "tq_table_build", "tq_table_check", "tq_table_quantize_host",
     "tq_compress", "tq_decompress", "tq_compress_batched", "tq_decompress_batched", "tq_workspace_bytes",
     "tq_decompress_batched_noalloc", "tq_qjl_table_bytes", "tq_qjl_table_build", "tq_qjl_signs",
-    "tq_qjl_compress", "tq_qjl_compress_batched", "tq_qjl_scores",
+    "tq_qjl_compress", "tq_qjl_compress_batched", "tq_qjl_scores", "tq_qjl_query_scores",
     "tq_scores", "tq_weighted_values", "tq_weighted_values_splits", "tq_attend_partials", "tq_attend_splits",
     "tq_attend_prepare", "tq_attend_merge", "tq_append_token", "tq_attend_step",
     "tq_decode_supported", "tq_decode_scratch_floats", "tq_decode_attend", "tq_decode_append",
@@ -230,6 +231,7 @@ def lib() -> ctypes.CDLL:
     L.tq_qjl_compress.argtypes = [vp, ci, ll, ll, vp, vp, ci, ci, vp, vp, vp, vp, vp]
     L.tq_qjl_compress_batched.argtypes = [vp, vp, ci, ci, vp]
     L.tq_qjl_scores.argtypes = [vp, vp, vp, vp, ll, ll, vp, ci, ci, vp, vp, ll, vp, vp]
+    L.tq_qjl_query_scores.argtypes = [vp, vp, vp, vp, ll, ll, vp, vp, ci, ci, vp, ci, ll, vp, vp]
     L.tq_append_token.argtypes = [vp, vp, ci, ll, ll, vp, vp, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, vp, vp, ll, ll, ll, vp]
     L.tq_attend_step.argtypes = [vp, ci, ll, ci, ctypes.c_float, vp, vp, vp, vp, ci, ll, ll, vp, vp, vp, vp, ll, ll,
                                  vp, vp, ci, ci, ci, vp, vp, vp, ci, vp, ci, vp]

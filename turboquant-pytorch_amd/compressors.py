@@ -204,23 +204,32 @@ class TurboQuantCompressorV2:
         if out.numel() == 0:
             return out
         _native._require_gpu(queries, "queries")
-        q = queries.float()
-        dev = q.device
+        dev = queries.device
         if D != _native.HEAD_DIM:       # other head dimensions: the reconstruction from the MSE kernels, the rest as tensor operations
+            q = queries.float()
             exp = self.reference_format(compressed)
             term1 = torch.matmul(q, exp["k_mse"].float().transpose(-2, -1))
             ip = torch.matmul(torch.matmul(q, self._s(dev).T), exp["qjl_signs"].float().transpose(-2, -1))
             return term1 + corr * ip * compressed["residual_norm"].float().unsqueeze(-2)
-        if q.shape[-1] != D or q.numel() != B * H * S_q * D:       # the kernel reads one query per row of the keys, the reshape below would take any width
-            raise ValueError(f"queries {tuple(q.shape)} do not fit keys {(B, H, S_k, D)}: [{B}, {H}, S_q, {D}] expected")
+        if queries.shape[-1] != D or queries.numel() != B * H * S_q * D:       # the kernels read one query per row of the keys, the reshape below would take any width
+            raise ValueError(f"queries {tuple(queries.shape)} do not fit keys {(B, H, S_k, D)}: [{B}, {H}, S_q, {D}] expected")
         st = self._s_on.get(("both", dev))
         if st is None:      # Pi^T and sqrt(pi/2)/m S^T one behind the other, made once per device
             st = self._s_on[("both", dev)] = torch.stack((self._mse.pi_transposed(dev), self._s(dev).T * corr)).contiguous()
+        packed = [compressed[k] if compressed[k].is_contiguous() else compressed[k].contiguous()
+                  for k in ("idx_bytes", "vec_norms", "sign_bytes", "residual_norm")]
+        if S_q <= _native.MAX_QUERY_SCORES and queries.dtype in _native._DTYPE_CODE and B * H <= 65535:
+            q = queries.contiguous()
+            with _native._on(dev):
+                rc = _native.lib().tq_qjl_query_scores(packed[0].data_ptr(), packed[1].data_ptr(), packed[2].data_ptr(), packed[3].data_ptr(),
+                                                       B * H, S_k, self._mse.table(dev).data_ptr(), st.data_ptr(), D, self.mse_bits,
+                                                       q.data_ptr(), _native._DTYPE_CODE[q.dtype], S_q, out.data_ptr(), _native._stream_handle(dev))
+            _native.check(rc, "tq_qjl_query_scores")
+            return out
+        q = queries.float()
         # every query token rotated and projected, in one product: [2, B * H * S_q, D]
         q_both = torch.matmul(q.reshape(1, -1, D), st)
         q_rot, q_sign = q_both[0], q_both[1]
-        packed = [compressed[k] if compressed[k].is_contiguous() else compressed[k].contiguous()
-                  for k in ("idx_bytes", "vec_norms", "sign_bytes", "residual_norm")]
         with _native._on(dev):
             rc = _native.lib().tq_qjl_scores(packed[0].data_ptr(), packed[1].data_ptr(), packed[2].data_ptr(), packed[3].data_ptr(),
                                              B * H, S_k, self._mse.table(dev).data_ptr(), D, self.mse_bits,
