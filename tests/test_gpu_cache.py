@@ -1107,6 +1107,23 @@ def test_layer_calls_equal_the_calls_per_tensor(pkg, monkeypatch, dim, bits, dty
                 assert a.is_contiguous() and a.dtype == b.dtype and torch.equal(a, b), (name, window)
 
 
+@pytest.mark.parametrize("dim,dtype", [(128, torch.bfloat16), (64, torch.float16), (80, torch.bfloat16), (256, torch.float16)])
+def test_large_layers_equal_the_calls_per_tensor(pkg, dim, dtype):
+    """Layers large enough for blocks to draw their tiles from counters (64 and 128: keys and values have a pair of counters each in one
+    record of the workspace), with keys and values of different widths, twice in a row: the counters are zero again behind a call."""
+    g = torch.Generator().manual_seed(dim)
+    tokens = 26003 if dim == 128 else 52007 if dim == 64 else 9001
+    k, v = (torch.randn(1, 16, tokens, dim, generator=g).to(dtype).to(DEV) for _ in range(2))
+    comp = pkg.TurboQuantV3(dim, key_bits=6, value_bits=2, residual_window=77, layer_idx=8, device=DEV)
+    want = [c.compress(x[:, :, :-77].contiguous()) for c, x in ((comp.key_compressor, k), (comp.val_compressor, v))]
+    full = [torch.cat([c.decompress(w).to(dtype), x[:, :, -77:]], 2) for c, w, x in zip((comp.key_compressor, comp.val_compressor), want, (k, v))]
+    for _ in range(2):
+        packed = comp.compress_kv(k, v)
+        for got, w in zip(packed, want):
+            assert torch.equal(got["compressed"]["idx_bytes"], w["idx_bytes"]) and torch.equal(got["compressed"]["vec_norms"], w["vec_norms"])
+        assert all(torch.equal(a, b) for a, b in zip(comp.decompress_kv(*packed), full))
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_update_restores_the_layer_as_the_calls_per_tensor_do(pkg, monkeypatch, dim):
     """V3Cache.update from a per-row store (packed slots between the rows) and a window that moves through its buffer."""

@@ -461,23 +461,21 @@ __global__ __launch_bounds__(MAX_WAVES *TQ_WAVE, 2) void tq_anydim_decompress_ke
 // against 640 bytes puts this width on the matrix side of the roofline: the kernel is bound by the matrix rate the part
 // sustains, not by memory.
 template <int DTYPE, int BITS>
-__global__ __launch_bounds__(512, 1) void tq_d256_compress_kernel(TqDevJob job0, const tq_job *jobs) {
+__device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock blk, uint8_t *lds) {
     static_assert(DTYPE == TQ_F16 || DTYPE == TQ_BF16, "16-bit inputs");
     constexpr int D = 256, STEPS = D / 16, PIECES = D * 2 / 16;     // 32 pieces of 16 bytes per vector
     constexpr int IPB = 8 / BITS, NB = 16 / IPB, NW = NB < 4 ? 1 : NB / 4;
     constexpr int TILE_BYTES = 32 * D * 2;
 
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint8_t *lds_grid = lds;                                                        // single copy, bases unshifted
     uint8_t (*lds_stage)[TILE_BYTES] = reinterpret_cast<uint8_t (*)[TILE_BYTES]>(lds + TQ_GRID_LDS_BYTES);
     float (*lds_ss)[32] = reinterpret_cast<float (*)[32]>(lds + TQ_GRID_LDS_BYTES + 2 * TILE_BYTES);     // [3][32]
 
-    const TqDevJob job = tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2));
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = tq_uniform32(tid >> 6);
     const uint32_t n = lane & 31u, hk = lane >> 5;
     const uint32_t n_tiles = (job.n_vec + 31u) / 32u;
-    if (blockIdx.x >= n_tiles) return;        // also: an empty job of a batch, whose table may be NULL
+    if (blk.x >= n_tiles) return;        // also: an empty job of a batch, whose table may be NULL
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
 
     // loads of a tile: piece i = l * 512 + tid of the tile's 1024 is piece i % 32 of vector i / 32, so that the 32 pieces
@@ -492,7 +490,7 @@ __global__ __launch_bounds__(512, 1) void tq_d256_compress_kernel(TqDevJob job0,
             pre[l] = tq_gload16(job.states + tq_vec_offset(job, v) + ld_piece * 16u);
         }
     };
-    issue_loads(blockIdx.x);
+    issue_loads(blk.x);
 
     tq_u4 areg[2][STEPS];
     {
@@ -558,7 +556,7 @@ __global__ __launch_bounds__(512, 1) void tq_d256_compress_kernel(TqDevJob job0,
             if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (SEARCH) {
-            const uint32_t v = (blockIdx.x + (j - 1u) * gridDim.x) * 32u + n;
+            const uint32_t v = (blk.x + (j - 1u) * blk.grid) * 32u + n;
             if (v < job.n_vec) {
                 const uint32_t slot = tq_packed_slot(job, v);
                 uint8_t *dst = job.idx_bytes + (size_t)slot * g_bytes + (2u * wave + hk) * NB;
@@ -574,11 +572,11 @@ __global__ __launch_bounds__(512, 1) void tq_d256_compress_kernel(TqDevJob job0,
         }
     };
 
-    const uint32_t m = (n_tiles - blockIdx.x + gridDim.x - 1u) / gridDim.x;     // this block's tiles
+    const uint32_t m = (n_tiles - blk.x + blk.grid - 1u) / blk.grid;     // this block's tiles
     // one trip: the tile after this one sets out while this one is rotated, and is parked behind the trip's work
     auto trip = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
         const bool more = j + 1u < m;
-        if (more) issue_loads(blockIdx.x + (j + 1u) * gridDim.x);
+        if (more) issue_loads(blk.x + (j + 1u) * blk.grid);
         __syncthreads();        // tile j and its sums are parked, and nobody reads buffer (j + 1) & 1 any more
         iteration(rot_tag, search_tag, j, acc_new, acc_old);
         if (more) park((j + 1u) & 1u, (j + 1u) % 3u);
@@ -601,13 +599,35 @@ __global__ __launch_bounds__(512, 1) void tq_d256_compress_kernel(TqDevJob job0,
     else trip(F{}, T{}, m, acc_a, acc_b);
 }
 
+template <int DTYPE, int BITS>
+__global__ __launch_bounds__(512, 1) void tq_d256_compress_kernel(TqDevJob job0, const tq_job *jobs) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    d256_compress_job<DTYPE, BITS>(tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2)), TqBlock{blockIdx.x, gridDim.x}, lds);
+}
+
+// keys and values of a layer
+template <int DTYPE>
+__global__ __launch_bounds__(512, 1) void tq_d256_compress_layer_kernel(TqLayer l) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t which = tq_layer_job(l);
+    const TqDevJob job = tq_uniform_job(which ? l.job[1] : l.job[0]);
+    const TqBlock blk = tq_layer_block(l, which);
+    switch (which ? l.bits[1] : l.bits[0]) {
+        case 1: d256_compress_job<DTYPE, 1>(job, blk, lds); break;
+        case 2: d256_compress_job<DTYPE, 2>(job, blk, lds); break;
+        case 3: d256_compress_job<DTYPE, 3>(job, blk, lds); break;
+        case 4: d256_compress_job<DTYPE, 4>(job, blk, lds); break;
+        default: d256_compress_job<DTYPE, 8>(job, blk, lds); break;
+    }
+}
+
 // decompress: a block is four waves that share tiles of 32 vectors; wave w keeps the rows [64w, 64w+64) of Pi^T as A
 // operands for all 16 steps (the leading fp16 term: 128 registers).  The packed bytes of a tile are fetched one tile
 // ahead (every thread the bytes of 32 codes), turned into fp16 centroids through the byte -> centroids table and parked
 // in a double-buffered swizzled LDS tile that all four waves read as B operands; the scaled, rounded results go through
 // a second LDS tile so that the stores are 512 contiguous bytes per vector.
 template <int DTYPE, int IPB>
-__global__ __launch_bounds__(256, 2) void tq_d256_decompress_kernel(TqDevJob job0, const tq_job *jobs) {
+__device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock blk, uint8_t *lds) {
     static_assert(DTYPE == TQ_F16 || DTYPE == TQ_BF16, "16-bit outputs");
     constexpr int D = 256, STEPS = D / 16;
     constexpr int TILE_BYTES = 32 * D * 2;
@@ -615,19 +635,17 @@ __global__ __launch_bounds__(256, 2) void tq_d256_decompress_kernel(TqDevJob job
     constexpr int RAW = 32 / IPB;                  // packed bytes of a thread's 32 codes: 4, 8, 16, 32
     constexpr int RW = RAW / 4;                    // as dwords
 
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint8_t *lds_lut = lds;
     uint8_t (*lds_y)[TILE_BYTES] = reinterpret_cast<uint8_t (*)[TILE_BYTES]>(lds + 4096);
     uint8_t *lds_out = lds + 4096 + 2 * TILE_BYTES;
     float (*lds_norm)[32] = reinterpret_cast<float (*)[32]>(lds + 4096 + 3 * TILE_BYTES);       // [2][32]
 
-    const TqDevJob job = tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2));
     uint8_t *out_base = const_cast<uint8_t *>(job.states);
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = tq_uniform32(tid >> 6);
     const uint32_t n = lane & 31u, hk = lane >> 5;
     const uint32_t n_tiles = (job.n_vec + 31u) / 32u;
-    if (blockIdx.x >= n_tiles) return;
+    if (blk.x >= n_tiles) return;
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
     const uint32_t g_bytes = D / IPB;
 
@@ -652,7 +670,7 @@ __global__ __launch_bounds__(256, 2) void tq_d256_decompress_kernel(TqDevJob job
         }
         if (chunk == 0u) norm_bits = tq_gload2(job.vec_norms + slot);
     };
-    issue_loads(blockIdx.x);
+    issue_loads(blk.x);
 
     tq_u4 areg[2][STEPS];       // row tiles 2w, 2w + 1
     {
@@ -700,11 +718,11 @@ __global__ __launch_bounds__(256, 2) void tq_d256_decompress_kernel(TqDevJob job
     const uint32_t op_base = n * (D * 2) + (((hk << 3) ^ (n & 31u)) << 4);
     auto op_step = [](int s) { return (uint32_t)((((2 * (s & 1)) << 3) | (s >> 1)) << 4); };
 
-    const uint32_t m = (n_tiles - blockIdx.x + gridDim.x - 1u) / gridDim.x;
+    const uint32_t m = (n_tiles - blk.x + blk.grid - 1u) / blk.grid;
     decode(0u);
     for (uint32_t j = 0; j < m; ++j) {
-        const uint32_t tl = blockIdx.x + j * gridDim.x;
-        if (j + 1u < m) issue_loads(tl + gridDim.x);
+        const uint32_t tl = blk.x + j * blk.grid;
+        if (j + 1u < m) issue_loads(tl + blk.grid);
         __syncthreads();        // tile j is decoded; the output tile of the last iteration has been read
         const uint8_t *ys = lds_y[j & 1u];
         tq_f16v acc[2] = {tq_zero16(), tq_zero16()};
@@ -745,6 +763,29 @@ __global__ __launch_bounds__(256, 2) void tq_d256_decompress_kernel(TqDevJob job
         }
         if (j + 1u < m) decode((j + 1u) & 1u);
     }
+}
+
+template <int DTYPE, int IPB>
+__global__ __launch_bounds__(256, 2) void tq_d256_decompress_kernel(TqDevJob job0, const tq_job *jobs) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    d256_decompress_job<DTYPE, IPB>(tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2)), TqBlock{blockIdx.x, gridDim.x}, lds);
+}
+
+// keys and values of a layer and its window
+template <int DTYPE>
+__global__ __launch_bounds__(256, 2) void tq_d256_restore_layer_kernel(TqLayer l, TqWindowCopy window) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t which = tq_layer_job(l);
+    const TqDevJob job = tq_uniform_job(which ? l.job[1] : l.job[0]);
+    const TqBlock blk = tq_layer_block(l, which);
+    tq_with_window(window, [&]() __attribute__((always_inline)) {
+        switch (8 / (which ? l.bits[1] : l.bits[0])) {
+            case 8: d256_decompress_job<DTYPE, 8>(job, blk, lds); break;
+            case 4: d256_decompress_job<DTYPE, 4>(job, blk, lds); break;
+            case 2: d256_decompress_job<DTYPE, 2>(job, blk, lds); break;
+            default: d256_decompress_job<DTYPE, 1>(job, blk, lds); break;
+        }
+    });
 }
 
 // ---- host side --------------------------------------------------------------------------
@@ -797,24 +838,52 @@ int launch(K kernel, uint32_t (&raised)[MAX_DEVICES], L lds_for, uint32_t nt_max
     return (int)hipGetLastError();
 }
 
-// Launch of one of the 256-wide kernels: `threads` per block, `resident` blocks per compute unit, `lds` bytes of dynamic LDS.
-template <typename K>
-int launch_d256(K kernel, bool (&raised)[MAX_DEVICES], uint32_t lds, uint32_t threads, int resident, const TqDevJob &job,
-                const tq_job *jobs_dev, int n_jobs, uint32_t max_vec, hipStream_t stream) {
+// 256-wide kernels: threads per block, blocks per compute unit, bytes of dynamic LDS
+struct D256Compress { static constexpr uint32_t THREADS = 512, RESIDENT = 1, LDS = TQ_GRID_LDS_BYTES + 2u * 32u * 256u * 2u + 3u * 32u * 4u; };
+struct D256Decompress { static constexpr uint32_t THREADS = 256, RESIDENT = 2, LDS = 4096u + 3u * 32u * 256u * 2u + 2u * 32u * 4u; };
+
+// Blocks the current device holds at once; raises the kernel's LDS limit, once per device (`raised` is the kernel's own).
+template <typename S, typename K>
+int d256_slots(K kernel, bool (&raised)[MAX_DEVICES], int &slots) {
     int dev = 0, cus = 0;
     const int rc = device_cus(dev, cus);
     if (rc) return rc;
-    {
-        std::lock_guard<std::mutex> lock(host_state_mutex);
-        if (!raised[dev]) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return (int)e;
-            raised[dev] = true;
-        }
+    std::lock_guard<std::mutex> lock(host_state_mutex);
+    if (!raised[dev]) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::LDS);
+        if (e != hipSuccess) return (int)e;
+        raised[dev] = true;
     }
-    const uint32_t tiles = (max_vec + 31u) / 32u;
-    const uint32_t bx = tq_blocks_per_job(tiles, cus * resident, n_jobs);
-    hipLaunchKernelGGL(kernel, dim3(bx, (unsigned)n_jobs, 1), dim3(threads, 1, 1), lds, stream, job, jobs_dev);
+    slots = cus * (int)S::RESIDENT;
+    return 0;
+}
+template <typename S, typename K>
+int launch_d256(K kernel, bool (&raised)[MAX_DEVICES], const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_vec, hipStream_t stream) {
+    int slots = 0;
+    const int rc = d256_slots<S>(kernel, raised, slots);
+    if (rc) return rc;
+    const uint32_t bx = tq_blocks_per_job((max_vec + 31u) / 32u, slots, n_jobs);
+    hipLaunchKernelGGL(kernel, dim3(bx, (unsigned)n_jobs, 1), dim3(S::THREADS, 1, 1), S::LDS, stream, job, jobs_dev);
+    return (int)hipGetLastError();
+}
+template <int DTYPE>
+int launch_d256_compress_layer(TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+    static bool raised[MAX_DEVICES] = {};
+    int slots = 0;
+    const int rc = d256_slots<D256Compress>(&tq_d256_compress_layer_kernel<DTYPE>, raised, slots);
+    if (rc) return rc;
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)slots, cost_k, cost_v);
+    hipLaunchKernelGGL((tq_d256_compress_layer_kernel<DTYPE>), dim3(blocks), dim3(D256Compress::THREADS), D256Compress::LDS, stream, l);
+    return (int)hipGetLastError();
+}
+template <int DTYPE>
+int launch_d256_restore_layer(TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+    static bool raised[MAX_DEVICES] = {};
+    int slots = 0;
+    const int rc = d256_slots<D256Decompress>(&tq_d256_restore_layer_kernel<DTYPE>, raised, slots);
+    if (rc) return rc;
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)slots, cost_k, cost_v);
+    hipLaunchKernelGGL((tq_d256_restore_layer_kernel<DTYPE>), dim3(blocks), dim3(D256Decompress::THREADS), D256Decompress::LDS, stream, l, w);
     return (int)hipGetLastError();
 }
 
@@ -823,8 +892,7 @@ int launch_compress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uin
     if constexpr (DTYPE != TQ_F32) {
         if (d == 256u) {
             static bool raised256[MAX_DEVICES] = {};
-            constexpr uint32_t lds = TQ_GRID_LDS_BYTES + 2u * 32u * 256u * 2u + 3u * 32u * 4u;
-            return launch_d256(&tq_d256_compress_kernel<DTYPE, BITS>, raised256, lds, 512u, 1, job, jobs_dev, n_jobs, max_vec, s);
+            return launch_d256<D256Compress>(&tq_d256_compress_kernel<DTYPE, BITS>, raised256, job, jobs_dev, n_jobs, max_vec, s);
         }
     }
     const uint32_t dp = TQ_PADDED_DIM(d);
@@ -855,8 +923,7 @@ int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, u
     if constexpr (DTYPE != TQ_F32) {
         if (d == 256u) {
             static bool raised256[MAX_DEVICES] = {};
-            constexpr uint32_t lds = 4096u + 3u * 32u * 256u * 2u + 2u * 32u * 4u;
-            return launch_d256(&tq_d256_decompress_kernel<DTYPE, IPB>, raised256, lds, 256u, 2, job, jobs_dev, n_jobs, max_vec, s);
+            return launch_d256<D256Decompress>(&tq_d256_decompress_kernel<DTYPE, IPB>, raised256, job, jobs_dev, n_jobs, max_vec, s);
         }
     }
     const uint32_t dp = TQ_PADDED_DIM(d);
@@ -911,4 +978,20 @@ int tq_anydim_decompress(int dtype, int bits, int head_dim, const TqDevJob &sing
         case TQ_BF16: return decompress_bits<TQ_BF16>(bits, single, jobs_dev, n_jobs, max_vec, d, stream);
         default: return TQ_ERR_DTYPE;
     }
+}
+
+bool tq_anydim_layer_supported(int head_dim, int dtype) {
+    return tq_wide_supported(head_dim, dtype) || (head_dim == 256 && (dtype == TQ_F16 || dtype == TQ_BF16));
+}
+
+int tq_anydim_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+    if (!tq_anydim_layer_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
+    if (head_dim != 256) return tq_wide_compress_layer(dtype, head_dim, l, n_vec, cost_k, cost_v, stream);
+    return dtype == TQ_F16 ? launch_d256_compress_layer<TQ_F16>(l, n_vec, cost_k, cost_v, stream) : launch_d256_compress_layer<TQ_BF16>(l, n_vec, cost_k, cost_v, stream);
+}
+
+int tq_anydim_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+    if (!tq_anydim_layer_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
+    if (head_dim != 256) return tq_wide_restore_layer(dtype, head_dim, l, w, n_vec, cost_k, cost_v, stream);
+    return dtype == TQ_F16 ? launch_d256_restore_layer<TQ_F16>(l, w, n_vec, cost_k, cost_v, stream) : launch_d256_restore_layer<TQ_BF16>(l, w, n_vec, cost_k, cost_v, stream);
 }

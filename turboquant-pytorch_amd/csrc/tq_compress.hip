@@ -72,9 +72,30 @@ __device__ __forceinline__ bool run_tail(F &step) {
     }
 }
 
+// LDS of a block, the same arrays for every width (several bodies in one kernel share them).  Arrays of their own and not one structure:
+// the compiler then knows that the tiles, the grid and the sums do not overlap, and orders their accesses freely (one structure: the
+// pipelined loop waits more, compress launches of the 32-layer cache + 2 %).
+template <int DTYPE>
+struct CompressLds {
+    static constexpr int ELEM = InTraits<DTYPE>::ELEM;
+    static constexpr int RING = ELEM == 2 ? TQ_RING : 2;     // staged tiles
+    using Grid = uint8_t[TQ_GRID_LDS_BYTES];
+    using Stage = uint8_t[RING][32 * TQ_HEAD_DIM * ELEM];
+    using Part = float[2][32][4];      // sum of squares of the tile's vectors, one share per wave (pipelined path)
+    using Ss = float[2][32];           // the same, whole (16-bit inputs)
+    using Ssh = float[2][32][2];       // the same per half of a row (rows that are pairs of 64-wide vectors)
+    using Tk = uint32_t[4];            // ticket k of the block sits in slot k % 4 (counter mode only)
+    static __device__ __forceinline__ Grid &grid() { __shared__ __attribute__((aligned(16))) Grid a; return a; }
+    static __device__ __forceinline__ Stage &stage() { __shared__ __attribute__((aligned(1024))) Stage a; return a; }
+    static __device__ __forceinline__ Part &part() { __shared__ __attribute__((aligned(16))) Part a; return a; }
+    static __device__ __forceinline__ Ss &ss() { __shared__ Ss a; return a; }
+    static __device__ __forceinline__ Ssh &ssh() { __shared__ Ssh a; return a; }
+    static __device__ __forceinline__ Tk &tk() { __shared__ Tk a; return a; }
+};
+
+// One block's share of a job; `workspace`: the job's two counters, or NULL.
 template <int DTYPE, int BITS>
-__global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace,
-                                                                                          uint32_t tshift, uint32_t paired) {
+__device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, uint32_t *workspace, uint32_t tshift, uint32_t paired) {
     using T = InTraits<DTYPE>;
     using P = Pack<BITS>;
     constexpr int ELEM = T::ELEM;
@@ -85,18 +106,17 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
     constexpr int VEC_PER_LOAD = 64 / PIECES;          // vectors covered by one load instruction
     constexpr int NB = P::NB, NW = P::NW;
 
-    // grid copies first, so that their LDS addresses are small compile-time immediates
-    constexpr int RING = ELEM == 2 ? TQ_RING : 2;     // staged tiles
-    __shared__ __attribute__((aligned(16))) uint8_t lds_grid[TQ_GRID_LDS_BYTES];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds_stage[RING][STAGE];
-    __shared__ float lds_ss[2][32];   // sum of squares of the tile's vectors (16-bit inputs)
-    __shared__ float lds_ssh[2][32][2];   // the same per half of a row (rows that are pairs of 64-wide vectors)
-    __shared__ __attribute__((aligned(16))) float lds_part[2][32][4];   // the same, one share per wave (pipelined path)
+    constexpr int RING = CompressLds<DTYPE>::RING;
+    auto &lds_grid = CompressLds<DTYPE>::grid();
+    auto &lds_stage = CompressLds<DTYPE>::stage();
+    auto &lds_ss = CompressLds<DTYPE>::ss();
+    auto &lds_ssh = CompressLds<DTYPE>::ssh();
+    auto &lds_part = CompressLds<DTYPE>::part();
+    auto &tk = CompressLds<DTYPE>::tk();
 
     // paired: the job's vectors are 64 wide and the kernel works on pairs of them as 128-wide rows (diag(Pi, Pi) from the
     // table's pair sections).  Everything is as for 128-wide vectors except the norm: one per half of a row; the
     // coordinates of wave w belong to half w / 2.
-    const TqDevJob job = tq_uniform_job(tq_pair_job(tq_load_job(job0, jobs, blockIdx.y, ELEM), paired != 0u));
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
@@ -112,7 +132,7 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
     // fewer tiles and all blocks of a job end together.  counter[0] = tiles handed out beyond every block's first ticket,
     // counter[1] = blocks of the job that are done; the last block to finish sets both back to zero, so a workspace
     // that was zero before a launch is zero after it (the contract of the decompress kernel's counters).
-    // Every other job walks single tiles blockIdx.x, blockIdx.x + grid, ...
+    // Every other job walks single tiles blk.x, blk.x + grid, ...
     // Several rows (a token slice of a [B, H, S, D] tensor, a window left behind): a tile is 32 vectors of the rows laid
     // end to end, so with at least 32 tokens a row it touches two rows at most; vectors of the second one lie `row_skip`
     // bytes further than the tile's own stride says.  The loads take 32-bit offsets from the tile's first vector, which
@@ -124,21 +144,21 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
     const bool ticket_job = ELEM == 2 && job.token_stride < (1ll << 26) &&
                             (one_row || (job.tokens >= 32u && row_skip >= 0 && row_skip < (1ll << 31)));
     // (a ticket has to outlast the pipeline's depth: the first drawn ticket is published one iteration after the start)
-    uint32_t *counter = workspace && (1u << tshift) > (uint32_t)TQ_RING ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr;
+    uint32_t *counter = workspace && (1u << tshift) > (uint32_t)TQ_RING ? workspace : nullptr;
     auto report_done = [&]() {      // once per block of a non-empty job, after its last draw has been answered
         if (counter && tid == 0) {
-            if (atomicAdd(counter + 1, 1u) == gridDim.x - 1u) {
+            if (atomicAdd(counter + 1, 1u) == blk.grid - 1u) {
                 atomicExch(counter, 0u);
                 atomicExch(counter + 1, 0u);
             }
         }
     };
-    uint32_t tile = ticket_job ? blockIdx.x << tshift : blockIdx.x;
+    uint32_t tile = ticket_job ? blk.x << tshift : blk.x;
     if (tile >= n_tiles) {        // whole block idle (uniform)
         report_done();
         return;
     }
-    const uint32_t tile_stride = gridDim.x;
+    const uint32_t tile_stride = blk.grid;
 
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
 
@@ -404,9 +424,8 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
             // ---- the block's sequence of tiles.  q[i] = the tile of iteration j - 1 + i while iteration j runs: q[0] is
             // searched and stored, q[1] rotated, q[P] loaded.  All of it lives in scalar registers.  A value >= n_full
             // marks the end (the sequence of a block only grows); loads past the end re-read the job's last full tile.
-            __shared__ uint32_t tk[4];          // ticket k of the block sits in slot k % 4 (counter mode only)
             const uint32_t per_ticket = 1u << tshift;
-            const uint32_t drawn_origin = gridDim.x << tshift;
+            const uint32_t drawn_origin = blk.grid << tshift;
             uint32_t q[P + 1];
             uint32_t left = per_ticket - 1u;    // tiles of the head's ticket beyond the head
             uint32_t kt = 0;                    // tickets the head has entered beyond the first
@@ -437,7 +456,7 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
                     draw();
                     return base;
                 }
-                return (blockIdx.x + kt * gridDim.x) << tshift;
+                return (blk.x + kt * blk.grid) << tshift;
             };
             q[0] = 0xffffffffu;
             q[1] = tile;
@@ -685,6 +704,30 @@ __global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compr
     report_done();
 }
 
+template <int DTYPE, int BITS>
+__global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace,
+                                                                                          uint32_t tshift, uint32_t paired) {
+    const TqDevJob job = tq_uniform_job(tq_pair_job(tq_load_job(job0, jobs, blockIdx.y, InTraits<DTYPE>::ELEM), paired != 0u));
+    compress_job<DTYPE, BITS>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr,
+                              tshift, paired);
+}
+
+// keys and values of a layer; their counters share one job's record of the workspace
+template <int DTYPE>
+__global__ __launch_bounds__(CTHREADS, InTraits<DTYPE>::MIN_WAVES) void tq_compress_layer_kernel(TqLayer l, uint32_t *workspace, uint32_t tshift, uint32_t paired) {
+    const uint32_t which = tq_layer_job(l);
+    const TqDevJob job = tq_uniform_job(tq_pair_job(which ? l.job[1] : l.job[0], paired != 0u));
+    const TqBlock blk = tq_layer_block(l, which);
+    uint32_t *counters = workspace ? workspace + which * (TQ_WORKSPACE_BYTES_PER_JOB / 8) : nullptr;
+    switch (which ? l.bits[1] : l.bits[0]) {
+        case 1: compress_job<DTYPE, 1>(job, blk, counters, tshift, paired); break;
+        case 2: compress_job<DTYPE, 2>(job, blk, counters, tshift, paired); break;
+        case 3: compress_job<DTYPE, 3>(job, blk, counters, tshift, paired); break;
+        case 4: compress_job<DTYPE, 4>(job, blk, counters, tshift, paired); break;
+        default: compress_job<DTYPE, 8>(job, blk, counters, tshift, paired); break;
+    }
+}
+
 // ---- host side --------------------------------------------------------------------------
 
 constexpr int MAX_DEVICES = 64;
@@ -720,25 +763,30 @@ int query_device(DeviceInfo &info) {
 #define TQ_COMPRESS_TICKET_SHIFT 3
 #endif
 
+// Blocks of a kernel that are resident per compute unit (registers and LDS decide): a grid is that many per unit, each walking its share
+// of the tiles.  Asked once per device; `resident_on` is the kernel's own.
+template <typename K>
+int resident_blocks(K kernel, const DeviceInfo &info, int (&resident_on)[MAX_DEVICES], int &resident) {
+    std::lock_guard<std::mutex> lock(host_state_mutex);
+    if (resident_on[info.dev] == 0) {
+        int nb = 0;
+        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, CTHREADS, 0);
+        if (e != hipSuccess) return (int)e;
+        resident_on[info.dev] = nb > 0 ? nb : 1;
+    }
+    resident = resident_on[info.dev];
+    return 0;
+}
+
 template <int DTYPE, int BITS>
 int launch_compress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *workspace, bool paired, hipStream_t stream) {
     DeviceInfo info;
     int rc = query_device(info);
     if (rc) return rc;
-    // blocks resident per compute unit for this instantiation (registers and LDS decide): the grid
-    // is that many blocks per unit, each walking its share of the tiles.  Asked once per device.
+    static int resident_on[MAX_DEVICES] = {};
     int resident;
-    {
-        static int resident_on[MAX_DEVICES] = {};
-        std::lock_guard<std::mutex> lock(host_state_mutex);
-        if (resident_on[info.dev] == 0) {
-            int nb = 0;
-            hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, tq_compress_kernel<DTYPE, BITS>, CTHREADS, 0);
-            if (e != hipSuccess) return (int)e;
-            resident_on[info.dev] = nb > 0 ? nb : 1;
-        }
-        resident = resident_on[info.dev];
-    }
+    rc = resident_blocks(tq_compress_kernel<DTYPE, BITS>, info, resident_on, resident);
+    if (rc) return rc;
     // Tickets from a counter pay off once every block has several to draw; below that (and without a workspace) the
     // blocks walk single tiles b, b + grid, ..., which splits a small job most evenly.
     uint32_t bx = tq_blocks_per_job(max_tiles, info.cus * resident, n_jobs);
@@ -755,6 +803,30 @@ int launch_compress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uin
     }
     dim3 grid(bx, (unsigned)n_jobs, 1), block(CTHREADS, 1, 1);
     hipLaunchKernelGGL((tq_compress_kernel<DTYPE, BITS>), grid, block, 0, stream, job, jobs_dev, counters, tshift, paired ? 1u : 0u);
+    return (int)hipGetLastError();
+}
+
+template <int DTYPE>
+int launch_layer(TqLayer &l, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, void *workspace, bool paired, hipStream_t stream) {
+    DeviceInfo info;
+    int rc = query_device(info);
+    if (rc) return rc;
+    static int resident_on[MAX_DEVICES] = {};
+    int resident;
+    rc = resident_blocks(tq_compress_layer_kernel<DTYPE>, info, resident_on, resident);
+    if (rc) return rc;
+    const uint32_t slots = (uint32_t)(info.cus * resident);
+    uint32_t blocks = tq_layer_blocks(l, tiles, slots, cost_k, cost_v), tshift = 0;
+    uint32_t *counters = nullptr;
+    if (workspace && InTraits<DTYPE>::ELEM == 2 && TQ_COMPRESS_TICKET_SHIFT > 0) {       // as in launch_compress
+        const uint32_t tickets = (tiles + (1u << TQ_COMPRESS_TICKET_SHIFT) - 1u) >> TQ_COMPRESS_TICKET_SHIFT;
+        if (2u * tickets >= 4u * slots) {
+            blocks = tq_layer_blocks(l, tickets, slots, cost_k, cost_v);
+            tshift = TQ_COMPRESS_TICKET_SHIFT;
+            counters = static_cast<uint32_t *>(workspace);
+        }
+    }
+    hipLaunchKernelGGL((tq_compress_layer_kernel<DTYPE>), dim3(blocks), dim3(CTHREADS), 0, stream, l, counters, tshift, paired ? 1u : 0u);
     return (int)hipGetLastError();
 }
 
@@ -837,7 +909,39 @@ extern "C" int tq_compress(const void *states, int dtype, long long rows, long l
 extern "C" int tq_compress_layer(const void *keys, const void *values, int dtype, long long rows, long long tokens, long long row_stride, long long token_stride,
                                  const void *table_k, const void *table_v, int head_dim, int bits_k, int bits_v, uint8_t *k_idx, uint16_t *k_norms,
                                  uint8_t *v_idx, uint16_t *v_norms, void *workspace, void *stream) {
-    const int rc = tq_compress(keys, dtype, rows, tokens, row_stride, token_stride, table_k, head_dim, bits_k, k_idx, k_norms, 0, workspace, stream);
+    long long n_vec = 0;
+    int rc = check_job(keys, dtype, rows, tokens, row_stride, token_stride, table_k, head_dim, bits_k, k_idx, k_norms, 0, &n_vec);
+    if (!rc) rc = check_job(values, dtype, rows, tokens, row_stride, token_stride, table_v, head_dim, bits_v, v_idx, v_norms, 0, &n_vec);
+    if (rc) return rc;
+    if ((uintptr_t)workspace & 63u) return TQ_ERR_ALIGN;
+    if (n_vec == 0) return TQ_OK;
+    const bool paired = tq_pairable(rows, tokens, token_stride, 0, head_dim, k_idx) && tq_pairable(rows, tokens, token_stride, 0, head_dim, v_idx);
+    if (head_dim == TQ_HEAD_DIM || paired || tq_anydim_layer_supported(head_dim, dtype)) {
+        const int eb = elem_bytes(dtype);
+        TqLayer l{};
+        for (int i = 0; i < 2; ++i) {
+            TqDevJob &job = l.job[i];
+            job.states = static_cast<const uint8_t *>(i ? values : keys);
+            job.idx_bytes = i ? v_idx : k_idx;
+            job.vec_norms = i ? v_norms : k_norms;
+            job.table = static_cast<const uint8_t *>(i ? table_v : table_k);
+            job.n_vec = (uint32_t)n_vec;
+            job.tokens = job.packed_row_stride = (uint32_t)tokens;
+            job.row_stride = row_stride * eb;
+            job.token_stride = token_stride * eb;
+            l.bits[i] = i ? bits_v : bits_k;
+        }
+        const uint32_t cost_k = (uint32_t)tq_vector_bytes(head_dim, eb, bits_k), cost_v = (uint32_t)tq_vector_bytes(head_dim, eb, bits_v);
+        const hipStream_t s = static_cast<hipStream_t>(stream);
+        if (head_dim != TQ_HEAD_DIM && !paired) return tq_anydim_compress_layer(dtype, head_dim, l, (uint32_t)n_vec, cost_k, cost_v, s);
+        const uint32_t tiles = (uint32_t)(((paired ? n_vec / 2 : n_vec) + 31) / 32);
+        switch (dtype) {
+            case TQ_F32: return launch_layer<TQ_F32>(l, tiles, cost_k, cost_v, workspace, paired, s);
+            case TQ_F16: return launch_layer<TQ_F16>(l, tiles, cost_k, cost_v, workspace, paired, s);
+            default: return launch_layer<TQ_BF16>(l, tiles, cost_k, cost_v, workspace, paired, s);
+        }
+    }
+    rc = tq_compress(keys, dtype, rows, tokens, row_stride, token_stride, table_k, head_dim, bits_k, k_idx, k_norms, 0, workspace, stream);
     if (rc) return rc;
     return tq_compress(values, dtype, rows, tokens, row_stride, token_stride, table_v, head_dim, bits_v, v_idx, v_norms, 0, workspace, stream);
 }

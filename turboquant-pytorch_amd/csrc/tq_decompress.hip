@@ -60,8 +60,9 @@ __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
     return (float)__builtin_bit_cast(_Float16, h);
 }
 
+// One block's share of a job; `counter`: the job's two counters, or NULL; lds: decompress_lds_bytes.
 template <int DTYPE, int IPB>
-__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace, uint32_t paired) {
+__device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk, uint32_t *counter, uint32_t paired, uint8_t *lds, uint32_t (&tk)[3]) {
     using T = OutTraits<DTYPE>;
     constexpr int ELEM = T::ELEM;
     constexpr int VEC_BYTES = TQ_HEAD_DIM * ELEM;   // 256 or 512
@@ -72,11 +73,8 @@ __global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompres
     constexpr int NB = 64 / IPB;                    // packed bytes per lane
     constexpr int NW = NB / 4;                      // dwords per lane: 2, 4, 8, 16
 
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-
     // paired: the job's vectors are 64 wide; two neighbours are one 128-wide row here (diag(Pi, Pi)^T from the table's pair
     // section).  Lane half hk decodes and produces the second vector of the pair; only its norm is its own.
-    const TqDevJob job = tq_pair_job(tq_load_job(job0, jobs, blockIdx.y, ELEM), paired != 0u);
     uint8_t *out_base = const_cast<uint8_t *>(job.states);
 
     const uint32_t tid = threadIdx.x;
@@ -92,10 +90,9 @@ __global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompres
 
     // tickets: counter[0] = tiles handed out beyond every block's first ticket, counter[1] = blocks of this job that are done.
     // The first ticket of a block is fixed (block b: tiles b * WAVES ...), so its loads can start before anything else.
-    __shared__ uint32_t tk[3];         // ticket k of the block sits in slot k % 3
-    uint32_t *counter = workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr;
-    const uint32_t first = blockIdx.x * T::WAVES;
-    const uint32_t drawn_origin = gridDim.x * T::WAVES;
+    // (ticket k of the block sits in tk[k % 3])
+    const uint32_t first = blk.x * T::WAVES;
+    const uint32_t drawn_origin = blk.grid * T::WAVES;
     uint32_t fixed_next = first + drawn_origin;
     // thread 0 only.  The ticket is computed from the atomic's result on the spot, which makes the drawing wave wait for
     // its own outstanding loads and stores once per ticket.  Measured against a form that leaves the result untouched
@@ -333,11 +330,38 @@ __global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompres
     // launch.  All accesses to the counters are device-scope atomics, which are performed in one place;
     // no fence is needed, and a release fence here would write back the L2's share of the output first.
     if (counter && tid == 0) {
-        if (atomicAdd(counter + 1, 1u) == gridDim.x - 1u) {
+        if (atomicAdd(counter + 1, 1u) == blk.grid - 1u) {
             atomicExch(counter, 0u);
             atomicExch(counter + 1, 0u);
         }
     }
+}
+
+template <int DTYPE, int IPB>
+__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace, uint32_t paired) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ uint32_t tk[3];
+    const TqDevJob job = tq_pair_job(tq_load_job(job0, jobs, blockIdx.y, OutTraits<DTYPE>::ELEM), paired != 0u);
+    decompress_job<DTYPE, IPB>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr, paired, lds, tk);
+}
+
+// keys and values of a layer and its window; the two jobs' counters share one job's record of the workspace
+template <int DTYPE>
+__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t *workspace, uint32_t paired) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ uint32_t tk[3];
+    const uint32_t which = tq_layer_job(l);
+    const TqDevJob job = tq_pair_job(which ? l.job[1] : l.job[0], paired != 0u);
+    const TqBlock blk = tq_layer_block(l, which);
+    uint32_t *counter = workspace ? workspace + which * (TQ_WORKSPACE_BYTES_PER_JOB / 8) : nullptr;
+    tq_with_window(window, [&]() __attribute__((always_inline)) {
+        switch (8 / (which ? l.bits[1] : l.bits[0])) {
+            case 8: decompress_job<DTYPE, 8>(job, blk, counter, paired, lds, tk); break;
+            case 4: decompress_job<DTYPE, 4>(job, blk, counter, paired, lds, tk); break;
+            case 2: decompress_job<DTYPE, 2>(job, blk, counter, paired, lds, tk); break;
+            default: decompress_job<DTYPE, 1>(job, blk, counter, paired, lds, tk); break;
+        }
+    });
 }
 
 // Sets n 32-bit words to zero.  A kernel rather than hipMemsetAsync, so that a caller may record the launch
@@ -389,6 +413,21 @@ int static_counters(uint32_t **out) {
     return 0;
 }
 
+// Raises a kernel's LDS limit, once per device (`configured` is the kernel's own).
+int allow_lds(const void *kernel, size_t lds, bool (&configured)[MAX_DEVICES]) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return (int)e;
+    if (dev < 0 || dev >= MAX_DEVICES) return TQ_ERR_NO_DEVICE;
+    std::lock_guard<std::mutex> lock(host_state_mutex);
+    if (!configured[dev]) {
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+        configured[dev] = true;
+    }
+    return 0;
+}
+
 template <int DTYPE, int IPB>
 int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *workspace, bool paired,
                       hipStream_t stream) {
@@ -397,26 +436,32 @@ int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, u
     int rc = device_cus(cus);
     if (rc) return rc;
     constexpr size_t lds = decompress_lds_bytes<DTYPE>();
-    {   // the kernel's LDS limit is raised once per device (one flag table per instantiation)
-        static bool configured[MAX_DEVICES] = {};
-        int dev = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e != hipSuccess) return (int)e;
-        if (dev < 0 || dev >= MAX_DEVICES) return TQ_ERR_NO_DEVICE;
-        std::lock_guard<std::mutex> lock(host_state_mutex);
-        if (!configured[dev]) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(&tq_decompress_kernel<DTYPE, IPB>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return (int)e;
-            configured[dev] = true;
-        }
-    }
+    static bool configured[MAX_DEVICES] = {};
+    rc = allow_lds(reinterpret_cast<const void *>(&tq_decompress_kernel<DTYPE, IPB>), lds, configured);
+    if (rc) return rc;
     const uint32_t want = (max_tiles + T::WAVES - 1) / T::WAVES;
     const uint32_t bx = tq_blocks_per_job(want, cus, n_jobs);
     dim3 grid(bx, (unsigned)n_jobs, 1), block(T::WAVES * TQ_WAVE, 1, 1);
     // tickets pay off once every block has several to draw; below that the fixed assignment starts sooner
     uint32_t *counters = want >= 4u * bx ? static_cast<uint32_t *>(workspace) : nullptr;
     hipLaunchKernelGGL((tq_decompress_kernel<DTYPE, IPB>), grid, block, lds, stream, job, jobs_dev, counters, paired ? 1u : 0u);
+    return (int)hipGetLastError();
+}
+
+template <int DTYPE>
+int launch_layer(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, void *workspace, bool paired, hipStream_t stream) {
+    using T = OutTraits<DTYPE>;
+    int cus = 0;
+    int rc = device_cus(cus);
+    if (rc) return rc;
+    constexpr size_t lds = decompress_lds_bytes<DTYPE>();
+    static bool configured[MAX_DEVICES] = {};
+    rc = allow_lds(reinterpret_cast<const void *>(&tq_restore_layer_kernel<DTYPE>), lds, configured);
+    if (rc) return rc;
+    const uint32_t want = (tiles + T::WAVES - 1) / T::WAVES;
+    const uint32_t blocks = tq_layer_blocks(l, want, (uint32_t)cus, cost_k, cost_v);
+    uint32_t *counters = 2u * want >= 4u * blocks ? static_cast<uint32_t *>(workspace) : nullptr;      // as in launch_decompress
+    hipLaunchKernelGGL((tq_restore_layer_kernel<DTYPE>), dim3(blocks), dim3(T::WAVES * TQ_WAVE), lds, stream, l, window, counters, paired ? 1u : 0u);
     return (int)hipGetLastError();
 }
 
@@ -496,7 +541,7 @@ extern "C" int tq_decompress(const uint8_t *idx_bytes, const uint16_t *vec_norms
 namespace {
 // The uncompressed window of a layer into the last tokens of its full-length tensors, keys (z = 0) and values in one launch:
 // a row of the window is one run of 16-byte pieces.  Two library copies took 2.5 us each and as much host time as a launch
-// of the codec; this one takes 2.5 us for both.
+// of the codec; this one takes 2.5 us for both.  (For layers that tq_restore_layer_kernel and its kind do not take.)
 __global__ __launch_bounds__(256) void tq_copy_window_kernel(const uint8_t *k_src, const uint8_t *v_src, uint8_t *k_dst, uint8_t *v_dst, uint32_t pieces,
                                                              uint32_t heads, long long batch_bytes, long long head_bytes, long long dst_bytes) {
     const uint32_t row = blockIdx.y, b = row / heads, h = row % heads;
@@ -524,14 +569,58 @@ extern "C" int tq_restore_layer(const uint8_t *k_idx, const uint16_t *k_norms, c
     // one row, or no window and dense packed tokens: one run of vectors on both sides
     const bool dense = rows == 1 || (n_win == 0 && packed_row_stride == 0);
     const long long r = dense ? 1 : rows, t = dense ? rows * tokens : tokens, rs = dense ? 0 : total * head_dim;
-    int rc = tq_decompress(k_idx, k_norms, packed_row_stride, r, t, table_k, head_dim, bits_k, k_out, dtype, rs, head_dim, workspace, stream);
+    long long n_vec = 0;
+    int rc = check_job(k_out, dtype, r, t, rs, head_dim, table_k, head_dim, bits_k, k_idx, k_norms, packed_row_stride, &n_vec);
+    if (!rc) rc = check_job(v_out, dtype, r, t, rs, head_dim, table_v, head_dim, bits_v, v_idx, v_norms, packed_row_stride, &n_vec);
+    if (rc) return rc;
+    if ((uintptr_t)workspace & 63u) return TQ_ERR_ALIGN;
+    const bool paired = tq_pairable(r, t, head_dim, packed_row_stride, head_dim, k_idx) && tq_pairable(r, t, head_dim, packed_row_stride, head_dim, v_idx);
+    const long long off = tokens * head_dim * elem;
+    if ((head_dim == TQ_HEAD_DIM || paired || tq_anydim_layer_supported(head_dim, dtype)) && 2 * rows * (run / 16) < 0xffffffffll) {
+        TqLayer l{};
+        for (int i = 0; i < 2; ++i) {
+            TqDevJob &job = l.job[i];
+            job.states = static_cast<const uint8_t *>(i ? v_out : k_out);
+            job.idx_bytes = const_cast<uint8_t *>(i ? v_idx : k_idx);
+            job.vec_norms = const_cast<uint16_t *>(i ? v_norms : k_norms);
+            job.table = static_cast<const uint8_t *>(i ? table_v : table_k);
+            job.n_vec = (uint32_t)n_vec;
+            job.tokens = (uint32_t)t;
+            job.packed_row_stride = (uint32_t)(packed_row_stride ? packed_row_stride : t);
+            job.row_stride = rs * elem;
+            job.token_stride = head_dim * elem;
+            l.bits[i] = i ? bits_v : bits_k;
+        }
+        TqWindowCopy w{};
+        if (n_win) {
+            w.src[0] = static_cast<const uint8_t *>(k_win);
+            w.src[1] = static_cast<const uint8_t *>(v_win);
+            w.dst[0] = static_cast<uint8_t *>(k_out) + off;
+            w.dst[1] = static_cast<uint8_t *>(v_out) + off;
+            w.pieces = (uint32_t)(run / 16);
+            w.heads = (uint32_t)heads;
+            w.total = (uint32_t)(2 * rows * (run / 16));
+            w.batch_bytes = win_batch_stride * elem;
+            w.head_bytes = win_head_stride * elem;
+            w.dst_bytes = dst_row;
+        }
+        const uint32_t cost_k = (uint32_t)tq_vector_bytes(head_dim, (int)elem, bits_k), cost_v = (uint32_t)tq_vector_bytes(head_dim, (int)elem, bits_v);
+        const hipStream_t s = static_cast<hipStream_t>(stream);
+        if (head_dim != TQ_HEAD_DIM && !paired) return tq_anydim_restore_layer(dtype, head_dim, l, w, (uint32_t)n_vec, cost_k, cost_v, s);
+        const uint32_t tiles = (uint32_t)(((paired ? n_vec / 2 : n_vec) + 31) / 32);
+        switch (dtype) {
+            case TQ_F32: return launch_layer<TQ_F32>(l, w, tiles, cost_k, cost_v, workspace, paired, s);
+            case TQ_F16: return launch_layer<TQ_F16>(l, w, tiles, cost_k, cost_v, workspace, paired, s);
+            default: return launch_layer<TQ_BF16>(l, w, tiles, cost_k, cost_v, workspace, paired, s);
+        }
+    }
+    rc = tq_decompress(k_idx, k_norms, packed_row_stride, r, t, table_k, head_dim, bits_k, k_out, dtype, rs, head_dim, workspace, stream);
     if (rc) return rc;
     rc = tq_decompress(v_idx, v_norms, packed_row_stride, r, t, table_v, head_dim, bits_v, v_out, dtype, rs, head_dim, workspace, stream);
     if (rc || n_win == 0) return rc;
     const uint32_t pieces = (uint32_t)(run / 16);
     const uint32_t bx = (pieces + 255u) / 256u;
     const dim3 grid(bx < 64u ? bx : 64u, (unsigned)rows, 2);
-    const long long off = tokens * head_dim * elem;
     hipLaunchKernelGGL(tq_copy_window_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const uint8_t *>(k_win),
                        static_cast<const uint8_t *>(v_win), static_cast<uint8_t *>(k_out) + off, static_cast<uint8_t *>(v_out) + off, pieces, (uint32_t)heads,
                        win_batch_stride * elem, win_head_stride * elem, dst_row);

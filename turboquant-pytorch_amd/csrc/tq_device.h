@@ -48,6 +48,72 @@ __device__ __forceinline__ TqDevJob tq_load_job(const TqDevJob &single, const tq
     return job;
 }
 
+// A block's place among the blocks of its job, and their number.
+struct TqBlock {
+    uint32_t x, grid;
+};
+
+// Keys and values of a layer in one launch (plain calls of tq_compress_layer and tq_restore_layer): blocks [0, split) work on the
+// keys, the others on the values, each with the body of its own code width; blocks are dealt out by the bytes a vector costs.
+// A launch of its own for each paid for start and drain twice, with half the chip idle at the seam.  us a layer, compress + restore, two
+// launches each way and one for the window / one and one: 8 x 32640 tokens, bf16, K4/V2 95 / 81; 16 x 3968, fp16, K6/V4 44.5 / 35.5; 8 x 16256, 256 wide
+// 140 / 132; 32 x 5873, 80 wide 76 / 63.
+struct TqLayer {
+    TqDevJob job[2];
+    uint32_t split;
+    int bits[2];
+};
+__device__ __forceinline__ uint32_t tq_layer_job(const TqLayer &l) { return blockIdx.x >= l.split ? 1u : 0u; }
+__device__ __forceinline__ TqBlock tq_layer_block(const TqLayer &l, uint32_t which) {
+    return which ? TqBlock{blockIdx.x - l.split, gridDim.x - l.split} : TqBlock{blockIdx.x, l.split};
+}
+// Blocks of such a launch: as many as are resident at once (`slots`), at most `want` for either job, one each at least; sets l.split.
+static inline uint32_t tq_layer_blocks(TqLayer &l, uint32_t want, uint32_t slots, uint32_t cost_k, uint32_t cost_v) {
+    uint32_t total = want < slots / 2u ? 2u * want : slots;
+    if (total < 2u) total = 2u;
+    uint32_t k = (uint32_t)((unsigned long long)total * cost_k / (cost_k + cost_v));
+    if (k < 1u) k = 1u;
+    if (k > total - 1u) k = total - 1u;
+    uint32_t v = total - k;
+    if (k > want) k = want;
+    if (v > want) v = want;
+    l.split = k;
+    return k + v;
+}
+
+// The uncompressed window of a layer into the last tokens of its full-length tensors, by the blocks that de-quantise the tokens before
+// it: a row of the window is one run of 16-byte pieces, `pieces` a row, total = 2 * rows * pieces (keys first; 0: no window).  The first
+// piece of a thread is loaded before the block's own work and stored behind it, so that nothing waits for it.
+struct TqWindowCopy {
+    const uint8_t *src[2];
+    uint8_t *dst[2];
+    uint32_t pieces, heads, total;
+    long long batch_bytes, head_bytes, dst_bytes;
+};
+struct TqWindowPiece {
+    const uint8_t *src;
+    uint8_t *dst;
+    __device__ __forceinline__ TqWindowPiece(const TqWindowCopy &w, uint32_t i) {
+        const uint32_t half = w.total / 2u, which = i >= half ? 1u : 0u, j = i - which * half;
+        const uint32_t row = j / w.pieces, p = j - row * w.pieces, b = row / w.heads, h = row - b * w.heads;
+        src = (which ? w.src[1] : w.src[0]) + (long long)b * w.batch_bytes + (long long)h * w.head_bytes + (size_t)p * 16u;
+        dst = (which ? w.dst[1] : w.dst[0]) + (long long)row * w.dst_bytes + (size_t)p * 16u;
+    }
+};
+template <typename F>
+__device__ __forceinline__ void tq_with_window(const TqWindowCopy &w, F work) {
+    const uint32_t threads = gridDim.x * blockDim.x, first = blockIdx.x * blockDim.x + threadIdx.x;
+    tq_u4 v = {0u, 0u, 0u, 0u};
+    if (first < w.total) v = *reinterpret_cast<const TQ_GLOBAL tq_u4 *>((const TQ_GLOBAL uint8_t *)TqWindowPiece(w, first).src);
+    work();
+    if (first < w.total) *reinterpret_cast<TQ_GLOBAL tq_u4 *>((TQ_GLOBAL uint8_t *)TqWindowPiece(w, first).dst) = v;
+    for (uint32_t i = first; i < w.total && w.total - i > threads;) {      // (no overflow: total may be close to 2^32)
+        i += threads;
+        const TqWindowPiece p(w, i);
+        *reinterpret_cast<TQ_GLOBAL tq_u4 *>((TQ_GLOBAL uint8_t *)p.dst) = *reinterpret_cast<const TQ_GLOBAL tq_u4 *>((const TQ_GLOBAL uint8_t *)p.src);
+    }
+}
+
 // Two 64-wide vectors that lie next to each other are one 128-wide row to the 128-wide kernels (rotated by diag(Pi, Pi)):
 // the job seen that way.  The host has checked that every row holds an even number of tokens, 64 elements apart.
 __device__ __forceinline__ TqDevJob tq_pair_job(TqDevJob j, bool paired) {
@@ -371,6 +437,11 @@ static inline uintptr_t tq_packed_alignment(int head_dim, int bits) {
     const uintptr_t g = (uintptr_t)((head_dim + (8 / bits) - 1) / (8 / bits));
     const uintptr_t low = g & (~g + 1);
     return low < 16 ? low : 16;
+}
+
+// Bytes that compressing or de-quantising a vector moves.
+static inline long long tq_vector_bytes(int head_dim, int elem_bytes, int bits) {
+    return (long long)head_dim * elem_bytes + (head_dim + (8 / bits) - 1) / (8 / bits) + 2;
 }
 
 // Alignment of the vectors themselves (pointer and strides, in bytes): 16, except for head dimensions that are not a

@@ -9,3 +9,6 @@ int tq_wide_compress(int dtype, int bits, int head_dim, const TqDevJob &single, 
                      uint32_t max_vec, hipStream_t stream);
 int tq_wide_decompress(int dtype, int bits, int head_dim, const TqDevJob &single, const tq_job *jobs_dev, int n_jobs,
                        uint32_t max_vec, hipStream_t stream);
+// keys and values of a layer in one launch (TqLayer: everything but `split` filled in)
+int tq_wide_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream);
+int tq_wide_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream);

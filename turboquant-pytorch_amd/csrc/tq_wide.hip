@@ -44,24 +44,22 @@ __device__ __forceinline__ uint32_t rotated_piece(uint32_t p, uint32_t v) {
 }
 
 template <int DTYPE, int BITS, int D, bool RAGGED>
-__global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD) void tq_wide_compress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t dl) {
+__device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
     static_assert(DTYPE == TQ_F16 || DTYPE == TQ_BF16, "16-bit inputs");
     using W = Wide<D>;
     constexpr int STEPS = W::STEPS, PIECES = W::PIECES, ROW = W::ROW, THREADS = W::THREADS;
     constexpr int IPB = 8 / BITS, NB = 16 / IPB, NW = NB < 4 ? 1 : NB / 4;
     constexpr int CPS = (16 + STEPS - 1) / STEPS;      // coordinates searched per step of the contraction
 
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint8_t *lds_grid = lds;                                                        // single copy, bases unshifted
     uint8_t (*lds_stage)[W::TILE_BYTES] = reinterpret_cast<uint8_t (*)[W::TILE_BYTES]>(lds + TQ_GRID_LDS_BYTES);
     float (*lds_part)[32][PIECES] = reinterpret_cast<float (*)[32][PIECES]>(lds + TQ_GRID_LDS_BYTES + 2 * W::TILE_BYTES);   // [3]
 
-    const TqDevJob job = tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2));
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = tq_uniform32(tid >> 6);
     const uint32_t n = lane & 31u, hk = lane >> 5;
     const uint32_t n_tiles = (job.n_vec + 31u) / 32u;
-    if (blockIdx.x >= n_tiles) return;        // also: an empty job of a batch, whose table may be NULL
+    if (blk.x >= n_tiles) return;        // also: an empty job of a batch, whose table may be NULL
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
 
     // loads of a tile: piece i = l * THREADS + tid of the tile's 32 * PIECES is piece i % PIECES of vector i / PIECES;
@@ -96,7 +94,7 @@ __global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD)
             }
         }
     };
-    issue_loads(blockIdx.x);
+    issue_loads(blk.x);
 
     tq_u4 areg[2][STEPS];
     {
@@ -173,7 +171,7 @@ __global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD)
             if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);      // keep the steps in this order (register pressure)
         }
         if constexpr (SEARCH) {
-            const uint32_t v = (blockIdx.x + (j - 1u) * gridDim.x) * 32u + n;
+            const uint32_t v = (blk.x + (j - 1u) * blk.grid) * 32u + n;
             if (v < job.n_vec) {
                 const uint32_t slot = tq_packed_slot(job, v);
                 uint8_t *dst = job.idx_bytes + (size_t)slot * g_bytes + (2u * wave + hk) * NB;
@@ -196,11 +194,11 @@ __global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD)
         }
     };
 
-    const uint32_t m = (n_tiles - blockIdx.x + gridDim.x - 1u) / gridDim.x;     // this block's tiles
+    const uint32_t m = (n_tiles - blk.x + blk.grid - 1u) / blk.grid;     // this block's tiles
     // one trip: the tile after this one sets out while this one is rotated, and is parked behind the trip's work
     auto trip = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
         const bool more = j + 1u < m;
-        if (more) issue_loads(blockIdx.x + (j + 1u) * gridDim.x);
+        if (more) issue_loads(blk.x + (j + 1u) * blk.grid);
         __syncthreads();        // tile j and its sums are parked, and nobody reads buffer (j + 1) & 1 any more
         iteration(rot_tag, search_tag, j, acc_new, acc_old);
         if (more) park((j + 1u) & 1u, (j + 1u) % 3u);
@@ -223,31 +221,51 @@ __global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD)
     else trip(F{}, T{}, m, acc_a, acc_b);
 }
 
+template <int DTYPE, int BITS, int D, bool RAGGED>
+__global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD) void tq_wide_compress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t dl) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    wide_compress_job<DTYPE, BITS, D, RAGGED>(tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2)), TqBlock{blockIdx.x, gridDim.x}, dl, lds);
+}
+
+// keys and values of a layer
+template <int DTYPE, int D, bool RAGGED>
+__global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD) void tq_wide_compress_layer_kernel(TqLayer l, uint32_t dl) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t which = tq_layer_job(l);
+    const TqDevJob job = tq_uniform_job(which ? l.job[1] : l.job[0]);
+    const TqBlock blk = tq_layer_block(l, which);
+    switch (which ? l.bits[1] : l.bits[0]) {
+        case 1: wide_compress_job<DTYPE, 1, D, RAGGED>(job, blk, dl, lds); break;
+        case 2: wide_compress_job<DTYPE, 2, D, RAGGED>(job, blk, dl, lds); break;
+        case 3: wide_compress_job<DTYPE, 3, D, RAGGED>(job, blk, dl, lds); break;
+        case 4: wide_compress_job<DTYPE, 4, D, RAGGED>(job, blk, dl, lds); break;
+        default: wide_compress_job<DTYPE, 8, D, RAGGED>(job, blk, dl, lds); break;
+    }
+}
+
 // decompress: wave w keeps the rows [32w, 32w+32) of Pi^T (leading fp16 term).  The packed bytes of a tile are fetched
 // one tile ahead (every thread the bytes of 16 codes), turned into fp16 centroids through the byte -> centroids table and
 // parked in a double-buffered LDS tile that all waves read as B operands; the scaled, rounded results go through a
 // second LDS tile so that the stores are D*2 contiguous bytes per vector.
 template <int DTYPE, int IPB, int D, bool RAGGED>
-__global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t dl) {
+__device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
     static_assert(DTYPE == TQ_F16 || DTYPE == TQ_BF16, "16-bit outputs");
     using W = Wide<D>;
     constexpr int STEPS = W::STEPS, PIECES = W::PIECES, ROW = W::ROW, THREADS = W::THREADS, WAVES = W::WAVES;
     constexpr int ENTRY = 2 * IPB;                 // bytes of a table entry: the fp16 centroids of one packed byte
     constexpr int RAW = 16 / IPB;                  // packed bytes of a thread's 16 codes: 2, 4, 8, 16
 
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     uint8_t *lds_lut = lds;
     uint8_t (*lds_y)[W::TILE_BYTES] = reinterpret_cast<uint8_t (*)[W::TILE_BYTES]>(lds + 4096);
     uint8_t *lds_out = lds + 4096 + 2 * W::TILE_BYTES;
     float (*lds_norm)[32] = reinterpret_cast<float (*)[32]>(lds + 4096 + 3 * W::TILE_BYTES);       // [2][32]
 
-    const TqDevJob job = tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2));
     uint8_t *out_base = const_cast<uint8_t *>(job.states);
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = tq_uniform32(tid >> 6);
     const uint32_t n = lane & 31u, hk = lane >> 5;
     const uint32_t n_tiles = (job.n_vec + 31u) / 32u;
-    if (blockIdx.x >= n_tiles) return;
+    if (blk.x >= n_tiles) return;
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
     const uint32_t g_bytes = RAGGED ? (dl + IPB - 1u) / IPB : (uint32_t)(D / IPB);      // packed bytes per vector in memory
 
@@ -274,7 +292,7 @@ __global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_decompress_kernel(Tq
         else { const tq_u4 t = tq_gload16(src); raw[0] = t[0]; raw[1] = t[1]; raw[2] = t[2]; raw[3] = t[3]; }
         if (chunk == 0u) norm_bits = tq_gload2(job.vec_norms + slot);
     };
-    issue_loads(blockIdx.x);
+    issue_loads(blk.x);
 
     tq_u4 areg[STEPS];
     {
@@ -336,11 +354,11 @@ __global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_decompress_kernel(Tq
         st_off[k] = st_vec[k] * ROW + (rotated_piece<D>(st_piece[k], st_vec[k]) << 4);
     }
 
-    const uint32_t m = (n_tiles - blockIdx.x + gridDim.x - 1u) / gridDim.x;
+    const uint32_t m = (n_tiles - blk.x + blk.grid - 1u) / blk.grid;
     decode(0u);
     for (uint32_t j = 0; j < m; ++j) {
-        const uint32_t tl = blockIdx.x + j * gridDim.x;
-        if (j + 1u < m) issue_loads(tl + gridDim.x);
+        const uint32_t tl = blk.x + j * blk.grid;
+        if (j + 1u < m) issue_loads(tl + blk.grid);
         __syncthreads();        // tile j is decoded; the output tile of the last iteration has been read
         const uint8_t *ys = lds_y[j & 1u];
         tq_f16v acc = tq_zero16();
@@ -389,39 +407,101 @@ __global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_decompress_kernel(Tq
     }
 }
 
+template <int DTYPE, int IPB, int D, bool RAGGED>
+__global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t dl) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    wide_decompress_job<DTYPE, IPB, D, RAGGED>(tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2)), TqBlock{blockIdx.x, gridDim.x}, dl, lds);
+}
+
+// keys and values of a layer and its window
+template <int DTYPE, int D, bool RAGGED>
+__global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t dl) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t which = tq_layer_job(l);
+    const TqDevJob job = tq_uniform_job(which ? l.job[1] : l.job[0]);
+    const TqBlock blk = tq_layer_block(l, which);
+    tq_with_window(window, [&]() __attribute__((always_inline)) {
+        switch (8 / (which ? l.bits[1] : l.bits[0])) {
+            case 8: wide_decompress_job<DTYPE, 8, D, RAGGED>(job, blk, dl, lds); break;
+            case 4: wide_decompress_job<DTYPE, 4, D, RAGGED>(job, blk, dl, lds); break;
+            case 2: wide_decompress_job<DTYPE, 2, D, RAGGED>(job, blk, dl, lds); break;
+            default: wide_decompress_job<DTYPE, 1, D, RAGGED>(job, blk, dl, lds); break;
+        }
+    });
+}
+
 // ---- host side --------------------------------------------------------------------------
 
 constexpr int MAX_DEVICES = 64;
 std::mutex host_state_mutex;
 
-// Launch of one kernel: blocks of `threads` threads with `lds` bytes of dynamic LDS, as many per compute unit as the
-// runtime says fit (remembered per device in `slots`).
+// Blocks of `threads` threads with `lds` bytes of dynamic LDS that the current device holds at once (what the runtime says fits a
+// compute unit, remembered per device in `slots`, the kernel's own); raises the kernel's LDS limit.
 template <typename K>
-int launch(K kernel, int (&slots)[MAX_DEVICES], uint32_t lds, uint32_t threads, const TqDevJob &job, const tq_job *jobs_dev,
-           int n_jobs, uint32_t max_vec, uint32_t dl, hipStream_t stream) {
+int resident_blocks(K kernel, int (&slots)[MAX_DEVICES], uint32_t lds, uint32_t threads, int &resident) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return (int)e;
     if (dev < 0 || dev >= MAX_DEVICES) return TQ_ERR_NO_DEVICE;
-    int resident;
-    {
-        std::lock_guard<std::mutex> lock(host_state_mutex);
-        if (slots[dev] == 0) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return (int)e;
-            int cus = 0, per_cu = 0;
-            e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-            if (e != hipSuccess) return (int)e;
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, (int)threads, lds);
-            if (e != hipSuccess) return (int)e;
-            slots[dev] = (cus > 0 ? cus : 1) * (per_cu > 0 ? per_cu : 1);
-        }
-        resident = slots[dev];
+    std::lock_guard<std::mutex> lock(host_state_mutex);
+    if (slots[dev] == 0) {
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+        int cus = 0, per_cu = 0;
+        e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e != hipSuccess) return (int)e;
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, (int)threads, lds);
+        if (e != hipSuccess) return (int)e;
+        slots[dev] = (cus > 0 ? cus : 1) * (per_cu > 0 ? per_cu : 1);
     }
+    resident = slots[dev];
+    return 0;
+}
+
+template <typename K>
+int launch(K kernel, int (&slots)[MAX_DEVICES], uint32_t lds, uint32_t threads, const TqDevJob &job, const tq_job *jobs_dev,
+           int n_jobs, uint32_t max_vec, uint32_t dl, hipStream_t stream) {
+    int resident = 0;
+    const int rc = resident_blocks(kernel, slots, lds, threads, resident);
+    if (rc) return rc;
     const uint32_t tiles = (max_vec + 31u) / 32u;
     const uint32_t bx = tq_blocks_per_job(tiles, resident, n_jobs);
     hipLaunchKernelGGL(kernel, dim3(bx, (unsigned)n_jobs, 1), dim3(threads, 1, 1), lds, stream, job, jobs_dev, dl);
     return (int)hipGetLastError();
+}
+
+template <int DTYPE, int D, bool RAGGED>
+int launch_compress_layer(TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, uint32_t dl, hipStream_t s) {
+    static int slots[MAX_DEVICES] = {};
+    int resident = 0;
+    const int rc = resident_blocks(&tq_wide_compress_layer_kernel<DTYPE, D, RAGGED>, slots, Wide<D>::COMPRESS_LDS, Wide<D>::THREADS, resident);
+    if (rc) return rc;
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)resident, cost_k, cost_v);
+    hipLaunchKernelGGL((tq_wide_compress_layer_kernel<DTYPE, D, RAGGED>), dim3(blocks), dim3(Wide<D>::THREADS), Wide<D>::COMPRESS_LDS, s, l, dl);
+    return (int)hipGetLastError();
+}
+template <int DTYPE, int D, bool RAGGED>
+int launch_restore_layer(TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, uint32_t dl, hipStream_t s) {
+    static int slots[MAX_DEVICES] = {};
+    int resident = 0;
+    const int rc = resident_blocks(&tq_wide_restore_layer_kernel<DTYPE, D, RAGGED>, slots, Wide<D>::DECOMPRESS_LDS, Wide<D>::THREADS, resident);
+    if (rc) return rc;
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)resident, cost_k, cost_v);
+    hipLaunchKernelGGL((tq_wide_restore_layer_kernel<DTYPE, D, RAGGED>), dim3(blocks), dim3(Wide<D>::THREADS), Wide<D>::DECOMPRESS_LDS, s, l, w, dl);
+    return (int)hipGetLastError();
+}
+// calls f(D, ragged) as constants
+template <typename F>
+int with_dim(int head_dim, F f) {
+    const int dp = TQ_PADDED_DIM(head_dim);
+    auto pick = [&](auto dim) { return dp != head_dim ? f(dim, std::true_type{}) : f(dim, std::false_type{}); };
+    switch (dp) {
+        case 96: return pick(std::integral_constant<int, 96>{});
+        case 160: return pick(std::integral_constant<int, 160>{});
+        case 192: return pick(std::integral_constant<int, 192>{});
+        case 224: return pick(std::integral_constant<int, 224>{});
+        default: return TQ_ERR_HEAD_DIM;
+    }
 }
 
 template <int DTYPE, int BITS, int D>
@@ -509,4 +589,20 @@ int tq_wide_decompress(int dtype, int bits, int head_dim, const TqDevJob &single
     if (bits < 1 || bits > 8) return TQ_ERR_BITS;
     return dtype == TQ_F16 ? decompress_dim<TQ_F16>(head_dim, bits, single, jobs_dev, n_jobs, max_vec, stream)
                            : decompress_dim<TQ_BF16>(head_dim, bits, single, jobs_dev, n_jobs, max_vec, stream);
+}
+
+int tq_wide_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+    if (!tq_wide_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
+    return with_dim(head_dim, [&](auto dim, auto ragged) {
+        return dtype == TQ_F16 ? launch_compress_layer<TQ_F16, dim.value, ragged.value>(l, n_vec, cost_k, cost_v, (uint32_t)head_dim, stream)
+                               : launch_compress_layer<TQ_BF16, dim.value, ragged.value>(l, n_vec, cost_k, cost_v, (uint32_t)head_dim, stream);
+    });
+}
+
+int tq_wide_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+    if (!tq_wide_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
+    return with_dim(head_dim, [&](auto dim, auto ragged) {
+        return dtype == TQ_F16 ? launch_restore_layer<TQ_F16, dim.value, ragged.value>(l, w, n_vec, cost_k, cost_v, (uint32_t)head_dim, stream)
+                               : launch_restore_layer<TQ_BF16, dim.value, ragged.value>(l, w, n_vec, cost_k, cost_v, (uint32_t)head_dim, stream);
+    });
 }
