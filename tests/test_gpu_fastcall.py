@@ -1,0 +1,155 @@
+"""The eager calls in one step (tqamd_fastcall) against the general path behind them, over the forms that either may be given."""
+import pytest
+import torch
+
+from test_gpu_parity import DEV, bits16, outlier_kv, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+
+
+class _Declines:
+    """An extension module that takes nothing."""
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _general(pkg, monkeypatch, f):
+    with monkeypatch.context() as m:
+        m.setattr(pkg._native, "fast", lambda: _Declines())
+        return f()
+
+
+def _flat(x):
+    if isinstance(x, torch.Tensor):
+        yield x
+    elif isinstance(x, dict):
+        for k in sorted(x):
+            yield from _flat(x[k])
+    elif isinstance(x, (list, tuple)):
+        for y in x:
+            yield from _flat(y)
+    else:
+        yield x
+
+
+def _same(a, b):
+    a, b = list(_flat(a)), list(_flat(b))
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        if isinstance(x, torch.Tensor):
+            assert x.shape == y.shape and x.dtype == y.dtype and x.device == y.device and x.requires_grad == y.requires_grad and torch.equal(x, y)
+        else:
+            assert x == y and type(x) is type(y)
+
+
+def _forms(dim, dtype):
+    x = outlier_kv((2, 3, 41, dim), seed=dim, dtype=dtype).to(DEV)
+    yield "dense", x
+    yield "one token", x[:, :, :1]
+    yield "one row", x[:1, :1]
+    yield "token slice", x[:, :, 3:35]
+    yield "heads last", outlier_kv((2, 41, 3, dim), seed=dim, dtype=dtype).to(DEV).transpose(1, 2)
+    yield "every other token", x[:, :, ::2]
+    yield "every other head", x[:, ::2]
+    yield "broadcast", x[:1].expand(3, 3, 41, dim)
+    yield "wider rows", outlier_kv((2, 3, 41, 2 * dim), seed=dim, dtype=dtype).to(DEV)[..., :dim]
+    yield "odd address", torch.empty(x.numel() + 1, dtype=dtype, device=DEV)[1:].view(x.shape).copy_(x)
+    yield "parameter", torch.nn.Parameter(x.clone())
+    yield "subclass", x.as_subclass(type("Sub", (torch.Tensor,), {}))
+    yield "empty", x[:, :, :0]
+
+
+@pytest.mark.parametrize("dim,bits,dtype", [(128, 4, torch.bfloat16), (128, 6, torch.float32), (64, 3, torch.float16), (80, 2, torch.bfloat16), (256, 8, torch.float16), (45, 1, torch.float32)])
+def test_one_step_codec_calls_equal_the_general_path(pkg, monkeypatch, dim, bits, dtype):
+    comp = pkg.MSECompressor(dim, bits, seed=3, device=DEV)
+    layer = pkg.TurboQuantV3(dim, key_bits=bits, value_bits=2, residual_window=7, layer_idx=8, device=DEV)
+    for name, x in _forms(dim, dtype):
+        if name in ("empty", "subclass"):
+            packed = comp.compress(x)
+            _same([packed[k] for k in ("shape", "idx_pad")], [tuple(x.shape), -dim % (8 // bits)])
+            continue
+        if name == "odd address" and dim % 32 == 0:        # the kernels of these load 16 bytes at a time
+            with pytest.raises((TypeError, RuntimeError)):
+                comp.compress(x)
+            continue
+        packed = comp.compress(x)
+        _same(packed, _general(pkg, monkeypatch, lambda: comp.compress(x)))
+        _same(comp.decompress(packed), _general(pkg, monkeypatch, lambda: comp.decompress(packed)))
+        strided = dict(packed, idx_bytes=packed["idx_bytes"].repeat(1, 1, 1, 2)[..., :packed["idx_bytes"].shape[-1]])
+        _same(comp.decompress(strided), comp.decompress(packed))
+        if x.shape[2] > 7:
+            both = layer.compress_kv(x, x)
+            _same(both, _general(pkg, monkeypatch, lambda: layer.compress_kv(x, x)))
+            _same(layer.decompress_kv(*both), _general(pkg, monkeypatch, lambda: layer.decompress_kv(*both)))
+            other = layer.compress_kv(x, x.contiguous().clone())       # laid out differently where x is not dense
+            _same([c["compressed"] for c in other], [c["compressed"] for c in both])
+
+
+@pytest.mark.parametrize("dim,dtype", [(64, torch.float16), (96, torch.bfloat16), (128, torch.bfloat16), (128, torch.float32), (256, torch.float16), (80, torch.float16)])
+def test_one_step_decode_calls_equal_the_general_path(pkg, monkeypatch, dim, dtype):
+    """update, append and attend over steps that fill the window, move it back and grow the store, new tokens in every layout."""
+    B, H = 2, 2
+    caches = [pkg.V3Cache(6, 2, residual_window=5, n_layers=40) for _ in range(2)]
+    x = outlier_kv((B, H, 300, dim), seed=1, dtype=dtype).to(DEV)
+    swapped = x.transpose(1, 2).contiguous().transpose(1, 2)
+    q = torch.randn(B, 2 * H, 40, dim, generator=torch.Generator().manual_seed(2)).to(dtype).to(DEV)
+    for c in caches:
+        c.append(x[:, :, :260], x[:, :, :260], 8)
+    for t in range(260, 300):
+        src = (x, swapped, x.repeat(1, 1, 1, 2)[..., :dim])[t % 3]
+        k, v = src[:, :, t:t + 1], src[:, :, t - 1:t]
+        qt = q[:, :, t - 260:t - 259]                  # not dense: copied
+        qt = qt.contiguous() if t % 2 else qt
+        step = lambda c: (c.update(k, v, 8) if t % 4 else c.append(k, v, 8), c.attend(qt, 8), c.attend(qt, 8, scale=0.25))  # noqa: E731
+        _same(step(caches[0]), _general(pkg, monkeypatch, lambda: step(caches[1])))
+    a, b = (c._stores[8] for c in caches)
+    assert (a.n_compressed, a.n_recent, a.w0, a.total_seq) == (b.n_compressed, b.n_recent, b.w0, b.total_seq)
+
+
+def test_one_step_calls_refuse_what_the_general_path_refuses(pkg):
+    comp = pkg.MSECompressor(128, 4, seed=3, device=DEV)
+    x = torch.randn(1, 2, 5, 128, device=DEV)
+    packed = comp.compress(x)
+    with pytest.raises(pkg._native.TqError):
+        comp.compress(x.double())
+    with pytest.raises(pkg._native.TqError):
+        comp.compress(x.cpu())
+    comp.bits = 2                                      # the table was built for four
+    with pytest.raises(pkg._native.TqError):
+        comp.compress(x)
+    comp.bits = 4
+    with pytest.raises((RuntimeError, ValueError)):
+        comp.decompress(dict(packed, shape=(1, 2, 6, 128)))
+    cache = pkg.V3Cache(4, 2, residual_window=4, n_layers=40)
+    y = x.bfloat16()
+    cache.append(y, y, 8)
+    for bad in (y[:, :, :2], y[:, :, :1].repeat(2, 1, 1, 1), torch.zeros(1, 3, 1, 128, device=DEV).bfloat16(), y[:, :, :1, :64]):
+        with pytest.raises(ValueError):
+            cache.attend(bad, 8)
+    with pytest.raises(ValueError):
+        cache.append(y[:, :1, :1], y[:, :1, :1], 8)
+    assert cache._stores[8].total_seq == 5
+
+
+@pytest.mark.parametrize("bits,dtype", [(3, torch.bfloat16), (5, torch.float32)])
+def test_one_step_v2_calls_equal_the_general_path(pkg, monkeypatch, bits, dtype):
+    """The codes bit for bit; scores of few queries come from another kernel than the general path's (bound as in
+    test_v2_scores_of_few_queries_equal_those_of_many)."""
+    comp = pkg.TurboQuantCompressorV2(128, bits, seed=5, device=DEV)
+    for name, x in _forms(128, dtype):
+        if name in ("empty", "subclass"):
+            continue
+        packed = comp.compress(x)
+        _same(packed, _general(pkg, monkeypatch, lambda: comp.compress(x)))
+        q = torch.randn(*x.shape[:2], 3, 128, device=DEV)
+        for queries in (q, q.transpose(1, 2).contiguous().transpose(1, 2), q.to(torch.bfloat16), q[:, :, :1], torch.cat((q.new_zeros(1), q.reshape(-1)))[1:].view(q.shape)):
+            a, b = comp.asymmetric_attention_scores(queries, packed), _general(pkg, monkeypatch, lambda: comp.asymmetric_attention_scores(queries, packed))
+            assert a.shape == b.shape and a.dtype == b.dtype
+            scale = queries.double().norm(dim=-1)[..., None] * x.detach().double().norm(dim=-1)[:, :, None, :]
+            assert float(((a.double() - b.double()).abs() / scale.clamp_min(1e-30)).max()) < 3e-5, name

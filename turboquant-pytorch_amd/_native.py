@@ -20,6 +20,9 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libtqamd.so")
+FAST_NAME = "tqamd_fastcall"        # extension module: the eager calls from tensors to the library in one step each
+FAST_PATH = os.path.join(CSRC, FAST_NAME + ".so")
+FAST_SOURCE = "tq_fastcall.cpp"
 SOURCES = ("tq_host.cpp", "tq_compress.hip", "tq_decompress.hip", "tq_anydim.hip", "tq_wide.hip", "tq_attend.hip", "tq_qjl.hip", "tq_qjl_scores.hip",
            "tq_decode.hip", "tq_decode_d64.hip", "tq_decode_d96.hip", "tq_decode_d128_narrow.hip", "tq_decode_d128_wide.hip", "tq_decode_d256.hip")
 HEADERS = ("tq_table.h", "tq_device.h", "tq_anydim.h", "tq_wide.h", "tq_lut.h", "tq_decode.h", "tq_decode_kernel.h", os.path.join("..", "..", "include", "tqamd.h"))
@@ -28,7 +31,7 @@ GPU_ARCH = "gfx950"
 TQ_F32, TQ_F16, TQ_BF16 = 0, 1, 2
 _DTYPE_CODE = {torch.float32: TQ_F32, torch.float16: TQ_F16, torch.bfloat16: TQ_BF16}
 HEAD_DIM = 128
-MAX_QUERY_SCORES = 8    # query tokens a row that tq_qjl_query_scores takes
+MAX_QUERY_SCORES = 8    # query tokens a row that tq_qjl_query_scores takes (tq_fastcall.cpp asks before it calls)
 
 
 class TqError(RuntimeError):
@@ -98,9 +101,26 @@ def _link(objs: Dict[str, str], out_path: str) -> None:
     os.replace(tmp, out_path)
 
 
+def _build_fastcall(force: bool) -> None:
+    """csrc/tqamd_fastcall.so, against the headers and libraries of the installed torch."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    sources = [os.path.join(CSRC, FAST_SOURCE), os.path.join(CSRC, "..", "..", "include", "tqamd.h")]
+    if not force and os.path.exists(FAST_PATH) and os.path.getmtime(FAST_PATH) >= max(map(os.path.getmtime, sources)):
+        return
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
+    tmp = FAST_PATH + ".tmp"
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-isystem" + p for p in cpp_extension.include_paths()),
+          "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(rocm, "include"), sources[0], "-o", tmp,
+          *("-L" + p for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-L" + os.path.join(rocm, "lib"), "-lamdhip64"])
+    os.replace(tmp, FAST_PATH)
+
+
 def build(force: bool = True, verbose: bool = False) -> str:
     """Compile the HIP/C++ sources into csrc/libtqamd.so (cross-compiles without a GPU): one object per source,
-    compiled in parallel, then linked."""
+    compiled in parallel, then linked; and the extension module that calls it."""
+    _build_fastcall(force)
     if not force and os.path.exists(LIB_PATH):
         newest = max(os.path.getmtime(os.path.join(CSRC, f)) for f in SOURCES + HEADERS)
         if os.path.getmtime(LIB_PATH) >= newest:
@@ -247,6 +267,28 @@ def lib() -> ctypes.CDLL:
             getattr(L, name).restype = ci
     _lib = L
     return L
+
+
+_fast = None
+
+
+def fast():
+    """The extension module tqamd_fastcall; raises if it has not been built.  Its functions take what a call has in hand and answer
+    None where the general path has to look at it."""
+    global _fast
+    if _fast is None:
+        from importlib import machinery, util
+        if not os.path.exists(FAST_PATH):
+            raise TqError(f"{FAST_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+        L = lib()
+        loader = machinery.ExtensionFileLoader(FAST_NAME, FAST_PATH)
+        module = util.module_from_spec(util.spec_from_file_location(FAST_NAME, FAST_PATH, loader=loader))
+        loader.exec_module(module)
+        entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend", "tq_qjl_compress", "tq_qjl_query_scores")
+        stream_of = _raw_stream or (lambda index: torch.cuda.current_stream(index).cuda_stream)
+        module.init(tuple(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in entries), stream_of, _workspace, _drop_workspace, _step_scratch, _arrived, _TABLE_TAG)
+        _fast = module
+    return _fast
 
 
 def check(status: int, what: str) -> None:
@@ -528,9 +570,16 @@ def decode_attend(layer: TqDecodeLayer, queries: torch.Tensor, group: int, scale
 
 
 def compress_layer(keys: torch.Tensor, values: torch.Tensor, tokens: int, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int):
-    """The first `tokens` tokens of a layer's keys and values [B,H,S,D] compressed in one call: ((idx_bytes, vec_norms) of the keys,
-    the same of the values), or None where the two are not laid out alike, or not in a form the kernels read in place
+    """The first `tokens` tokens of a layer's keys and values [B,H,S,D] compressed in one call: ((idx_bytes, vec_norms, the tokens behind
+    them) of the keys, the same of the values), or None where the two are not laid out alike, or not in a form the kernels read in place
     (the caller then goes tensor by tensor)."""
+    if keys.is_cuda and not torch.compiler.is_compiling():
+        got = fast().compress_layer(keys, values, tokens, table_k, table_v, bits_k, bits_v)
+        if got is not None:
+            if type(got) is int:
+                check(got, "tq_compress_layer")
+            k_idx, k_nrm, v_idx, v_nrm, k_rest, v_rest = got
+            return (k_idx, k_nrm, k_rest), (v_idx, v_nrm, v_rest)
     shape, stride, dtype, dev = keys.shape, keys.stride(), keys.dtype, keys.device
     if (values.shape != shape or values.stride() != stride or values.dtype != dtype or values.device != dev or dev.type != "cuda"
             or dtype not in _DTYPE_CODE or torch.compiler.is_compiling()):
@@ -565,14 +614,29 @@ def compress_layer(keys: torch.Tensor, values: torch.Tensor, tokens: int, table_
     if rc and ws:
         _drop_workspace(dev, stream)
     check(rc, "tq_compress_layer")
-    return (k_idx, k_nrm), (v_idx, v_nrm)
+    with torch.no_grad():
+        return (k_idx, k_nrm, keys[:, :, tokens:, :]), (v_idx, v_nrm, values[:, :, tokens:, :])
 
 
 def restore_layer(packed_k, packed_v, tokens: int, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int,
-                  k_win: torch.Tensor, v_win: torch.Tensor):
+                  k_win: torch.Tensor, v_win: torch.Tensor, w0: Optional[int] = None, n_win: int = 0):
     """Full-length keys and values [B,H,tokens + n_win,D] in the windows' element type, from packed pairs (idx_bytes [B,H,tokens,G],
     vec_norms [B,H,tokens]: dense, or token slices of one per-row store) and the windows [B,H,n_win,D] behind them, in one
-    call; None where the layout is not one the call takes (the caller then goes step by step)."""
+    call; None where the layout is not one the call takes (the caller then goes step by step).
+    With w0, the pairs are whole per-row stores, of which the first `tokens` slots count, and k_win, v_win whole window buffers, of which
+    the tokens [w0, w0 + n_win) do."""
+    if k_win.is_cuda and not torch.compiler.is_compiling():
+        if w0 is None:
+            got = fast().restore_layer(*packed_k, *packed_v, tokens, table_k, table_v, bits_k, bits_v, k_win, v_win)
+        else:
+            got = fast().restore_store(*packed_k, *packed_v, k_win, v_win, table_k, table_v, bits_k, bits_v, tokens, w0, n_win)
+        if got is not None:
+            if type(got) is int:
+                check(got, "tq_restore_layer")
+            return got
+    if w0 is not None:
+        packed_k, packed_v = (tuple(t[:, :, :tokens] for t in pair) for pair in (packed_k, packed_v))
+        k_win, v_win = k_win[:, :, w0:w0 + n_win], v_win[:, :, w0:w0 + n_win]
     shape, stride, dtype, dev = k_win.shape, k_win.stride(), k_win.dtype, k_win.device
     B, H, n_win, D = shape
     if (v_win.shape != shape or v_win.stride() != stride or v_win.dtype != dtype or v_win.device != dev or dev.type != "cuda"

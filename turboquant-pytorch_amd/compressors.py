@@ -107,11 +107,32 @@ class TurboQuantCompressorV2:
             t = self._s_on[dev] = self.S.to(dev)
         return t
 
-    @torch.no_grad()
+    def _both(self, dev: torch.device) -> torch.Tensor:
+        """Pi^T and sqrt(pi/2)/m S^T one behind the other, made once per device."""
+        st = self._s_on.get(("both", dev))
+        if st is None:
+            with torch.no_grad():
+                m = self.S.shape[0]
+                st = self._s_on[("both", dev)] = torch.stack((self._mse.pi_transposed(dev), self._s(dev).T * (math.sqrt(math.pi / 2) / m))).contiguous()
+        return st
+
     def compress(self, states: torch.Tensor) -> dict:
         """(B, H, S, D) -> {"idx_bytes" u8 [B,H,S,G], "vec_norms" f16 [B,H,S], "sign_bytes" u8 [B,H,S,D/8],
         "residual_norm" f16 [B,H,S], "shape"}.  One call (tq_qjl_compress): a single pass over the input for 16-bit
         elements and MSE codes of up to 4 bits, MSE codes and norms followed by residual signs and norms otherwise."""
+        table, qjl_table = self._mse._tables.get(states.device), self._qjl_tables.get(states.device)
+        if table is not None and qjl_table is not None and states.is_cuda and not torch.compiler.is_compiling():
+            packed = _native.fast().qjl_compress(states, table, qjl_table, self.mse_bits)
+            if packed is not None:
+                if type(packed) is int:
+                    _native.check(packed, "tq_qjl_compress")
+                B, H, S, D = states.shape
+                return {"idx_bytes": packed[0], "vec_norms": packed[1], "sign_bytes": packed[2], "residual_norm": packed[3], "shape": (B, H, S, D)}
+        return self._compress(states)
+
+    @torch.no_grad()
+    def _compress(self, states: torch.Tensor) -> dict:
+        """compress for inputs of any layout."""
         B, H, S, D = states.shape
         _native._require_gpu(states, "states")
         if not states.is_contiguous():
@@ -184,13 +205,26 @@ class TurboQuantCompressorV2:
         signs = (bits.to(torch.int8) * 2 - 1).reshape(B, H, S, -1)[..., :D]
         return {"k_mse": k_mse, "qjl_signs": signs, "residual_norm": compressed["residual_norm"], "shape": (B, H, S, D)}
 
-    @torch.no_grad()
     def asymmetric_attention_scores(self, queries: torch.Tensor, compressed: dict) -> torch.Tensor:
         """<q, k> ~ <q, k_mse> + ||r|| sqrt(pi/2)/m <S q, sign(S r)>  (:124-158): queries (B, H, S_q, D) against a dict
         from compress -> float32 (B, H, S_q, S_k).  Both terms are computed from the packed bytes (the query is
         rotated by Pi for the first and projected by S for the second; neither the reconstruction nor the signs are
         expanded).  A dict in the reference's format (`reference_format`) is accepted too and takes plain matrix
         products."""
+        if queries.is_cuda and "idx_bytes" in compressed and compressed["shape"][3] == _native.HEAD_DIM and not torch.compiler.is_compiling():
+            dev, idx = queries.device, compressed["idx_bytes"]
+            if idx.shape[:3] == compressed["shape"][:3]:       # up to _native.MAX_QUERY_SCORES query tokens in one launch
+                out = _native.fast().qjl_scores(queries, idx, compressed["vec_norms"], compressed["sign_bytes"], compressed["residual_norm"],
+                                                self._mse.table(dev), self._both(dev), self.mse_bits)
+                if out is not None:
+                    if type(out) is int:
+                        _native.check(out, "tq_qjl_query_scores")
+                    return out
+        return self._scores(queries, compressed)
+
+    @torch.no_grad()
+    def _scores(self, queries: torch.Tensor, compressed: dict) -> torch.Tensor:
+        """asymmetric_attention_scores for operands of any layout, any number of query tokens and any head dimension."""
         m = self.S.shape[0]
         corr = math.sqrt(math.pi / 2) / m
         if "idx_bytes" not in compressed:
@@ -213,19 +247,9 @@ class TurboQuantCompressorV2:
             return term1 + corr * ip * compressed["residual_norm"].float().unsqueeze(-2)
         if queries.shape[-1] != D or queries.numel() != B * H * S_q * D:       # the kernels read one query per row of the keys, the reshape below would take any width
             raise ValueError(f"queries {tuple(queries.shape)} do not fit keys {(B, H, S_k, D)}: [{B}, {H}, S_q, {D}] expected")
-        st = self._s_on.get(("both", dev))
-        if st is None:      # Pi^T and sqrt(pi/2)/m S^T one behind the other, made once per device
-            st = self._s_on[("both", dev)] = torch.stack((self._mse.pi_transposed(dev), self._s(dev).T * corr)).contiguous()
+        st = self._both(dev)
         packed = [compressed[k] if compressed[k].is_contiguous() else compressed[k].contiguous()
                   for k in ("idx_bytes", "vec_norms", "sign_bytes", "residual_norm")]
-        if S_q <= _native.MAX_QUERY_SCORES and queries.dtype in _native._DTYPE_CODE and B * H <= 65535:
-            q = queries.contiguous()
-            with _native._on(dev):
-                rc = _native.lib().tq_qjl_query_scores(packed[0].data_ptr(), packed[1].data_ptr(), packed[2].data_ptr(), packed[3].data_ptr(),
-                                                       B * H, S_k, self._mse.table(dev).data_ptr(), st.data_ptr(), D, self.mse_bits,
-                                                       q.data_ptr(), _native._DTYPE_CODE[q.dtype], S_q, out.data_ptr(), _native._stream_handle(dev))
-            _native.check(rc, "tq_qjl_query_scores")
-            return out
         q = queries.float()
         # every query token rotated and projected, in one product: [2, B * H * S_q, D]
         q_both = torch.matmul(q.reshape(1, -1, D), st)

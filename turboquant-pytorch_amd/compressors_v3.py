@@ -111,13 +111,19 @@ class MSECompressor:
             t = self._tables[dev] = _native.upload_table(self._table_host, self.head_dim, self.bits, dev)
         return t
 
-    @torch.no_grad()
     def compress(self, states: torch.Tensor) -> dict:
         """(B, H, S, D) -> {"idx_bytes" u8 [B,H,S,G], "vec_norms" f16 [B,H,S], "shape", "idx_pad"}."""
         B, H, S, D = states.shape
         indices_per_byte = 8 // self.bits
         idx_pad = (indices_per_byte - D % indices_per_byte) % indices_per_byte
-        idx_bytes, vec_norms = _native.call("compress", states, self.table(states.device), self.bits)
+        table = self._tables.get(states.device)
+        packed = _native.fast().compress(states, table, self.bits) if table is not None and states.is_cuda and not torch.compiler.is_compiling() else None
+        if packed is None:
+            with torch.no_grad():
+                packed = _native.call("compress", states, self.table(states.device), self.bits)
+        elif type(packed) is int:
+            _native.check(packed, "tq_compress")
+        idx_bytes, vec_norms = packed
         return {
             "idx_bytes": idx_bytes,
             "vec_norms": vec_norms,
@@ -181,9 +187,21 @@ class MSECompressor:
         out_rot = _native.call("weighted_values", idx_bytes, vec_norms, self.table(idx_bytes.device), self.bits, weights, self.head_dim)
         return torch.matmul(out_rot, self.pi(out_rot.device))
 
-    @torch.no_grad()
     def decompress(self, compressed: dict) -> torch.Tensor:
         """Back to a float32 (B, H, S, D) tensor."""
+        idx_bytes = compressed["idx_bytes"]
+        table = self._tables.get(idx_bytes.device)
+        if table is not None and idx_bytes.is_cuda and not torch.compiler.is_compiling():
+            out = _native.fast().decompress(idx_bytes, compressed["vec_norms"], table, self.bits, compressed["shape"])
+            if out is not None:
+                if type(out) is int:
+                    _native.check(out, "tq_decompress")
+                return out
+        return self._decompress(compressed)
+
+    @torch.no_grad()
+    def _decompress(self, compressed: dict) -> torch.Tensor:
+        """decompress for packed buffers of any layout."""
         B, H, S, D = compressed["shape"]
         width = math.ceil(D / (8 // self.bits))
         idx_bytes = compressed["idx_bytes"].reshape(B, H, S, width)
@@ -246,7 +264,6 @@ class TurboQuantV3:
         self.key_compressor = MSECompressor(head_dim, self.key_bits, seed=seed_base, device=device)
         self.val_compressor = MSECompressor(head_dim, self.value_bits, seed=seed_base + 500, device=device)
 
-    @torch.no_grad()
     def compress_kv(self, keys: torch.Tensor, values: torch.Tensor) -> Tuple[dict, dict]:
         """keys, values (B, H, S, D) -> two dicts with "compressed", "fp16", "shape", "split_at"."""
         B, H, S, D = keys.shape
@@ -264,10 +281,16 @@ class TurboQuantV3:
         if packed is not None:
             return tuple({
                 "compressed": {"idx_bytes": idx, "vec_norms": nrm, "shape": (B, H, split_at, D), "idx_pad": -D % (8 // comp.bits)},
-                "fp16": tensor[:, :, split_at:, :],
+                "fp16": rest,
                 "shape": (B, H, S, D),
                 "split_at": split_at,
-            } for tensor, comp, (idx, nrm) in ((keys, kc, packed[0]), (values, vc, packed[1])))
+            } for comp, (idx, nrm, rest) in ((kc, packed[0]), (vc, packed[1])))
+        return self._compress_by_tensor(keys, values, split_at)
+
+    @torch.no_grad()
+    def _compress_by_tensor(self, keys: torch.Tensor, values: torch.Tensor, split_at: int) -> Tuple[dict, dict]:
+        """compress_kv where the two are not laid out alike, or not as the kernels read them."""
+        B, H, S, D = keys.shape
         out = []
         for tensor, comp in ((keys, self.key_compressor), (values, self.val_compressor)):
             out.append({
@@ -279,14 +302,16 @@ class TurboQuantV3:
             })
         return out[0], out[1]
 
-    @torch.no_grad()
     def decompress_kv(self, compressed_k: dict, compressed_v: dict) -> Tuple[torch.Tensor, torch.Tensor]:
         """-> keys, values (B, H, S, D) in the dtype of the uncompressed window."""
         if compressed_k["compressed"] is None:
             return compressed_k["fp16"], compressed_v["fp16"]
         full = self._restore(compressed_k, compressed_v)
-        if full is not None:
-            return full
+        return full if full is not None else self._restore_by_tensor(compressed_k, compressed_v)
+
+    @torch.no_grad()
+    def _restore_by_tensor(self, compressed_k: dict, compressed_v: dict) -> Tuple[torch.Tensor, torch.Tensor]:
+        """decompress_kv where the dictionaries ask for something else than the call per layer does."""
         out = []
         for c, comp in ((compressed_k, self.key_compressor), (compressed_v, self.val_compressor)):
             B, H, S, D = c["shape"]

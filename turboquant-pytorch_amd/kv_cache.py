@@ -147,8 +147,17 @@ class _LayerStore:
         step is not of that kind or the tensors are not laid out for it; the general path then runs."""
         rw = self.window_tokens
         if (rw == 0 or not (self.one_launch or self.D == _native.HEAD_DIM)
-                or self.n_recent != rw or self.w0 + rw + 1 > self.win_cap or self.n_compressed + 1 > self.capacity
-                or keys.dtype != self.dtype or values.dtype != self.dtype or keys.device != self.device
+                or self.n_recent != rw or self.w0 + rw + 1 > self.win_cap or self.n_compressed + 1 > self.capacity):
+            return False
+        if self.one_launch and keys.is_cuda and not torch.compiler.is_compiling():
+            rc = _native.fast().decode_append(ctypes.addressof(self.record()), keys, values, self.k_win, self.w0, self.w0 + rw, self.n_compressed)
+            if rc is not None:
+                _native.check(rc, "tq_decode_append")
+                self.n_compressed += 1
+                self.w0 += 1
+                self.total_seq += 1
+                return True
+        if (keys.dtype != self.dtype or values.dtype != self.dtype or keys.device != self.device
                 or values.device != self.device or torch.compiler.is_compiling()
                 or keys.shape != (self.B, self.H, 1, self.D) or values.shape != keys.shape):    # the call reads both at the store's geometry
             return False
@@ -280,21 +289,24 @@ class V3Cache:
             st.w0 = 0
         st.extend_window(key_states[:, :, from_new:], value_states[:, :, from_new:])
 
-    @torch.no_grad()
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
                cache_kwargs: Optional[dict] = None) -> Tuple[torch.Tensor, torch.Tensor]:
-        B, H, S_new, D = key_states.shape
-        device = key_states.device
-        st = self._store(key_states, layer_idx)
-        comp = st.comp
-        self._push(st, key_states, value_states)
+        V3Cache.append(self, key_states, value_states, layer_idx)
+        st = self._stores[layer_idx]
         n_c = st.n_compressed
         if n_c and st.dtype == key_states.dtype == value_states.dtype:
-            kc, vc = comp.key_compressor, comp.val_compressor
-            full = _native.restore_layer((st.k_idx[:, :, :n_c], st.k_nrm[:, :, :n_c]), (st.v_idx[:, :, :n_c], st.v_nrm[:, :, :n_c]), n_c,
-                                         kc.table(device), vc.table(device), kc.bits, vc.bits, *st.window())
+            kc, vc, device = st.comp.key_compressor, st.comp.val_compressor, key_states.device
+            full = _native.restore_layer((st.k_idx, st.k_nrm), (st.v_idx, st.v_nrm), n_c, kc.table(device), vc.table(device), kc.bits, vc.bits,
+                                         st.k_win, st.v_win, st.w0, st.n_recent)
             if full is not None:
                 return full
+        return self._full_length(st, key_states, value_states)
+
+    @torch.no_grad()
+    def _full_length(self, st: _LayerStore, key_states: torch.Tensor, value_states: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+        """What `update` returns, step by step."""
+        B, H, S_new, D = key_states.shape
+        device, comp, n_c = key_states.device, st.comp, st.n_compressed
         total = n_c + st.n_recent
         full_k = torch.empty((B, H, total, D), dtype=key_states.dtype, device=device)
         full_v = torch.empty((B, H, total, D), dtype=value_states.dtype, device=device)
@@ -307,13 +319,14 @@ class V3Cache:
             full_v[:, :, n_c:].copy_(vw)
         return full_k, full_v
 
-    @torch.no_grad()
     def append(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int) -> None:
         """`update` without building the full-length tensors: the state afterwards is the same.  For decode
         loops that read the cache through `attend`."""
-        self._push(self._store(key_states, layer_idx), key_states, value_states)
+        st = self._stores.get(layer_idx)
+        if st is None or not st.append_one(key_states, value_states):
+            with torch.no_grad():
+                self._push(self._store(key_states, layer_idx), key_states, value_states)
 
-    @torch.no_grad()
     def attend(self, query_states: torch.Tensor, layer_idx: int, scale: Optional[float] = None,
                fused: Optional[bool] = None) -> torch.Tensor:
         """softmax(scale * q K^T) V of one query token per sequence, [B,Hq,1,D] -> [B,Hq,1,D], over everything
@@ -322,6 +335,19 @@ class V3Cache:
         fused (default: whenever at most 16 query heads share a kv head): one kernel pass over packed keys and
         values with an online softmax per split of the history; otherwise three steps (scores from the packed
         keys, softmax in float32, weighted sum of the packed values).  Window tokens are used as they are."""
+        st = self._stores.get(layer_idx)
+        if st is not None and st.one_launch and st.total_seq and fused is not False and query_states.is_cuda and not torch.compiler.is_compiling():
+            B, Hq, Sq, D = query_states.shape
+            G = Hq // st.H
+            if Sq == 1 and B == st.B and D == st.D and Hq == G * st.H and 1 <= G <= 16 and st.n_recent <= 512:
+                out = self._attend_step(st, query_states, G, D ** -0.5 if scale is None else float(scale))
+                if out is not None:
+                    return out
+        return self._attend(query_states, layer_idx, scale, fused)
+
+    @torch.no_grad()
+    def _attend(self, query_states: torch.Tensor, layer_idx: int, scale: Optional[float], fused: Optional[bool]) -> torch.Tensor:
+        """`attend` for whatever the one-launch step does not take, with every check."""
         st = self._stores.get(layer_idx)
         if st is None or st.total_seq == 0:
             raise ValueError(f"attend: nothing is cached for layer {layer_idx}")
@@ -393,6 +419,10 @@ class V3Cache:
     def _attend_step(st: _LayerStore, query_states: torch.Tensor, G: int, scale: float) -> Optional[torch.Tensor]:
         """The fused path of `attend` in one library call (rotate + window, packed history, merge), with the
         scratch kept per stream.  None when the queries are not laid out for it."""
+        if st.one_launch and query_states.is_cuda:
+            out = _native.fast().decode_attend(ctypes.addressof(st.record()), query_states, st.k_win, scale, st.w0, st.n_recent, st.n_compressed)
+            if out is not None:
+                return out
         B, Hq, _, D = query_states.shape
         if (not query_states.is_contiguous() or query_states.dtype not in _native._DTYPE_CODE or st.k_idx is None
                 or query_states.device != st.device):
