@@ -4,12 +4,10 @@
 //   tq_decode_attend   softmax(scale q K^T) V over the packed history and the uncompressed window, one launch: the queries are
 //                      rotated, the window is attended to and the splits are merged inside the kernel that reads the codes.
 // Few rows: a step is a chain of latencies (tables, query rotation, one or two runs per wave, merge), so launches are what
-// counts; many rows: the main loop, which is bound by the vector and LDS work of the table lookups (counted on this kernel at
-// 512 rows x 16384 tokens: vector instructions take 60 % of the issue slots, the LDS is busy 44 % of the time).
-// Per layer and whole step, six launches / these two (MI355X): 8 rows x 32768 tokens, K4/V2, 4 heads a row 48.9 -> 30.1 us;
-// 512 rows x 16384 tokens 226 -> 212 us, of which attention 200-204; head dimension 64, 32 rows x 6000 tokens, K6/V4 (before:
-// de-quantised to float32 and multiplied by library products) 190 -> 25 us.  Attention alone at 256, 32 rows x 6000 tokens, before /
-// this: K4/V2 307 -> 43 us, K8/V8 344 -> 58 us.
+// counts; many rows: the main loop, which is bound by the vector and LDS work of the table lookups.
+// Per layer and whole step, six launches / these two (MI355X): 8 rows x 32768 tokens, K4/V2, 4 heads a row 48.9 -> 22.5 us;
+// 512 rows x 16384 tokens 226 -> 175 us, of which attention 170; head dimension 64, 32 rows x 6000 tokens, K6/V4 (before:
+// de-quantised to float32 and multiplied by library products) 190 -> 18.7 us.
 // What they compute is what tq_compress and the prepare / partials / merge trio of tq_attend.hip compute (upstream
 // turboquant/generation_test_v2.py:96-135, score definition validate_v3.py:87); at 128 those remain for float32 caches, queries of
 // another type than the cache's and more than 65535 rows.  A value whose norm is infinite in float16 makes its row's results NaN, as there.
@@ -31,71 +29,70 @@ struct AppendArgs {
     int ipb[2];
 };
 
-// Block (32 rows, tensor) of D / 32 waves, one vector per row: wave w produces the rotated coordinates [32 w, 32 w + 32) of
-// the 32 vectors and their codes.  A step has one vector per row, so nothing is shared between blocks or reused: operands, vectors
-// and the quantiser's cells come straight from memory (the cells of a lane's 16 coordinates as 16 loads in flight together)
-// and the launch lasts as long as that chain of loads.  Products and sums run in the order of the kernels that compress whole
-// tensors of this head dimension, so the bytes are theirs.
+// Block (32 rows, tensor, w): one wave, which produces the rotated coordinates [32 w, 32 w + 32) of 32 vectors, one per row, and their
+// codes.  A step has one vector per row, so nothing is reused and the launch lasts as long as its chain of loads: everything a
+// wave reads (vectors, operands, the quantiser's grid, its share of the new tokens) is asked for before anything is waited for, sections of the
+// tables at the places every table has them, and the cells then come from LDS.  A wave each, since four waves of 30 loads share a compute
+// unit's one load pipe, and a launch has few blocks anyway.  (Blocks of D / 32 waves that took the header, the new tokens, the vectors
+// and the cells one after the other / this, append and attend of a layer, us: 8 rows x 32768 tokens at 128 24.7 / 22.5, 32 x 6000 at 64 20.8 / 18.7.)
+// Products and sums run in the order of the kernels that compress
+// whole tensors of this head dimension, so the bytes are theirs.
 template <int D, bool BF>
-__global__ __launch_bounds__(D / 32 * TQ_WAVE) void tq_decode_append_kernel(AppendArgs a) {
-    constexpr int STEPS = D / 16, THREADS = D / 32 * TQ_WAVE;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = tq_uniform32(tid >> 6), which = blockIdx.y;
+__global__ __launch_bounds__(TQ_WAVE) void tq_decode_append_kernel(AppendArgs a) {
+    constexpr int STEPS = D / 16, PIECES = D / 8;
+    constexpr int CELL_LOADS = (D == 128 ? TQ_GRID_COPY_STRIDE(8) : TQ_GRID_LDS_BYTES) / 1024;      // 128: the grids fit two copies at least
+    static_assert(CELL_LOADS * 1024 == (D == 128 ? TQ_GRID_COPY_STRIDE(8) : TQ_GRID_LDS_BYTES), "whole loads of a wave");
+    __shared__ __align__(16) uint8_t lds_grid[CELL_LOADS * 1024];
+    const uint32_t lane = threadIdx.x, which = blockIdx.y, wave = blockIdx.z;
     const uint32_t n = lane & 31u, hk = lane >> 5;
     const uint32_t row0 = blockIdx.x * 32u;
-    const uint8_t *fresh = a.fresh[which];
     uint8_t *win = a.win[which];
-    // the new tokens of the block's rows: 16-byte pieces (another slot than the one read below)
-    for (uint32_t i = tid; i < 32u * (D / 8); i += THREADS) {
-        const uint32_t r = row0 + i / (D / 8), piece = i % (D / 8);
-        if (r < a.rows)
-            tq_gstore16(win + ((size_t)r * a.win_stride + (size_t)a.put * D) * 2u + piece * 16u, tq_gload16(fresh + (size_t)r * a.new_stride[which] * 2u + piece * 16u));
+    // the new tokens, 64 bytes of each row to a wave: to another slot than the one read below
+    tq_u4 fresh[2];
+    uint32_t fresh_row[2];
+    const uint32_t fresh_piece = 4u * wave + (lane & 3u);
+    auto load_fresh = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            fresh_row[i] = row0 + 16u * i + (lane >> 2);
+            fresh[i] = tq_gload16(a.fresh[which] + (size_t)min(fresh_row[i], a.rows - 1u) * a.new_stride[which] * 2u + fresh_piece * 16u);
+        }
+    };
+    auto store_fresh = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (fresh_row[i] < a.rows) tq_gstore16(win + ((size_t)fresh_row[i] * a.win_stride + (size_t)a.put * D) * 2u + fresh_piece * 16u, fresh[i]);
+    };
+    if (!a.compress) {
+        load_fresh();
+        store_fresh();
+        return;
     }
-    if (!a.compress) return;
     const uint8_t *table = a.table[which];
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(table);
     const uint32_t r = min(row0 + n, a.rows - 1u);
     const uint8_t *src = win + ((size_t)r * a.win_stride + (size_t)a.evict * D) * 2u + 16u * hk;
-    const uint8_t *asrc = table + (BF ? hd->off_a_bf16 : hd->off_a_f16) + ((size_t)wave * STEPS * 64u + lane) * 16u;
+    const uint8_t *asrc = table + (BF ? TQ_OFF_A_BF16(D) : TQ_OFF_A_F16) + ((size_t)wave * STEPS * 64u + lane) * 16u;
     const uint32_t step0 = D == 128 ? 2u * wave : 0u;      // the 128-wide kernel starts the contraction at the wave's own quarter
-    tq_u4 x[STEPS];
+    tq_u4 x[STEPS], p[2][STEPS], cells[CELL_LOADS];
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) x[s] = tq_gload16(src + 32 * s);
-    tq_f16v acc = tq_zero16();
-    if constexpr (D == 128) {
-        tq_u4 p[2][STEPS], xs[STEPS];
+    for (int s = 0; s < STEPS; ++s) {
+        const uint32_t sg = D == 128 ? (s + step0) & 7u : (uint32_t)s;
+        x[s] = tq_gload16(src + 32u * sg);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const uint32_t sg = (s + step0) & 7u;
-            p[0][s] = tq_gload16(asrc + (size_t)sg * 1024u);
-            p[1][s] = tq_gload16(asrc + TQ_OPERAND_BYTES_FOR(D) + (size_t)sg * 1024u);
-            xs[s] = tq_gload16(src + 32u * sg);
-        }
-#pragma unroll
-        for (int s = 0; s < STEPS; ++s)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) acc = BF ? mfma_bf16(p[t][s], xs[s], acc) : mfma_f16(p[t][s], xs[s], acc);
-    } else {
-        constexpr int CH = STEPS < 8 ? STEPS : 8;
-        for (int s0 = 0; s0 < STEPS; s0 += CH) {
-            tq_u4 p[2][CH];
-#pragma unroll
-            for (int s = 0; s < CH; ++s) {
-                if (s0 + s < STEPS) {
-                    p[0][s] = tq_gload16(asrc + (size_t)(s0 + s) * 1024u);
-                    p[1][s] = tq_gload16(asrc + TQ_OPERAND_BYTES_FOR(D) + (size_t)(s0 + s) * 1024u);
-                }
-            }
-#pragma unroll
-            for (int s = 0; s < CH; ++s) {
-                if (s0 + s < STEPS) {
-                    const tq_u4 xv = STEPS > CH ? tq_gload16(src + 32u * (s0 + s)) : x[s];
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) acc = BF ? mfma_bf16(p[t][s], xv, acc) : mfma_f16(p[t][s], xv, acc);
-                }
-            }
-        }
+        for (int t = 0; t < 2; ++t) p[t][s] = tq_gload16(asrc + t * TQ_OPERAND_BYTES_FOR(D) + (size_t)sg * 1024u);
     }
+#pragma unroll
+    for (int i = 0; i < CELL_LOADS; ++i) cells[i] = tq_gload16(table + TQ_OFF_GRID(D) + 1024u * i + 16u * lane);
+    load_fresh();
+    const float grid_scale = hd->grid_scale, grid_bias = hd->grid_bias;
+    const uint32_t width = hd->bits;
+    __builtin_amdgcn_sched_barrier(0);
+    tq_f16v acc = tq_zero16();
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc = BF ? mfma_bf16(p[t][s], x[s], acc) : mfma_f16(p[t][s], x[s], acc);
     // ---- sum of squares: lane (n, hk) holds pieces 2 s + hk of its vector
     float ss;
     constexpr int DT = BF ? TQ_BF16 : TQ_F16;
@@ -106,7 +103,8 @@ __global__ __launch_bounds__(D / 32 * TQ_WAVE) void tq_decode_append_kernel(Appe
             share[q] = sumsq8<DT>(x[2 * q + 1], sumsq8<DT>(x[2 * q], 0.f));
             share[q] += __shfl_xor(share[q], 32);
         }
-        ss = (share[0] + share[1]) + (share[2] + share[3]);
+        // share[q] is that of quarter q + w: the pairs (0, 1) and (2, 3) of the vector's quarters
+        ss = wave & 1u ? (share[3] + share[0]) + (share[1] + share[2]) : (share[0] + share[1]) + (share[2] + share[3]);
     } else {
         float even[STEPS], odd[STEPS];
 #pragma unroll
@@ -132,15 +130,18 @@ __global__ __launch_bounds__(D / 32 * TQ_WAVE) void tq_decode_append_kernel(Appe
     const float nrm = tq_norm_from_sumsq(ss);
     float inv = __builtin_amdgcn_rcpf(nrm + 1e-8f);
     if (!BF) inv *= 1.0f / (float)(1 << TQ_F16_PI_SHIFT);
-    const float inv_cell = inv * hd->grid_scale, grid_bias = hd->grid_bias;
+    const float inv_cell = inv * grid_scale;
     // ---- code search: lane (n, hk) holds coordinates 32 w + 16 hk + r
-    const uint8_t *grid = table + hd->off_grid;
+#pragma unroll
+    for (int i = 0; i < CELL_LOADS; ++i) *reinterpret_cast<tq_u4 *>(lds_grid + 1024u * i + 16u * lane) = cells[i];
+    __syncthreads();      // (one wave: the order of its own LDS accesses)
     tq_u2 cell[16];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) cell[q] = tq_gload8(grid + (__float_as_uint(fmaf(acc[q], inv_cell, grid_bias)) & TQ_GRID_ADDR_MASK));
+    for (int q = 0; q < 16; ++q) cell[q] = *reinterpret_cast<const tq_u2 *>(lds_grid + (__float_as_uint(fmaf(acc[q], inv_cell, grid_bias)) & TQ_GRID_ADDR_MASK));
     uint32_t code[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) code[q] = cell[q][1] + (~__float_as_uint(fmaf(acc[q], inv, -__uint_as_float(cell[q][0]))) >> 31);
+    store_fresh();
     if (row0 + n >= a.rows) return;
     const int ipb = a.ipb[which];
     const size_t slot = (size_t)r * a.packed_row_stride;
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(D / 32 * TQ_WAVE) void tq_decode_append_kernel(Appe
         uint32_t w[NW];
 #pragma unroll
         for (int k = 0; k < NW; ++k) w[k] = 0u;
-        const uint32_t width = hd->bits;       // 3-bit codes sit two to a byte, three bits apart
+        // 3-bit codes sit two to a byte, three bits apart
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
             const int byte = q / I, k = q % I;
@@ -181,7 +182,7 @@ bool decode_supported(int head_dim, int bits_k, int bits_v) {
 
 template <int D>
 void launch_append(dim3 grid, hipStream_t s, const AppendArgs &a) {
-    const dim3 block(D / 32 * TQ_WAVE);
+    const dim3 block(TQ_WAVE);
     if (a.bf16) hipLaunchKernelGGL((tq_decode_append_kernel<D, true>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((tq_decode_append_kernel<D, false>), grid, block, 0, s, a);
 }
@@ -323,7 +324,7 @@ extern "C" int tq_decode_append(const tq_decode_layer *layer, const void *k_new,
     a.rows = (uint32_t)rows;
     a.put = (uint32_t)put;
     a.bf16 = layer->dtype == TQ_BF16 ? 1u : 0u;
-    const dim3 grid((unsigned)((rows + 31) / 32), 2, 1);
+    const dim3 grid((unsigned)((rows + 31) / 32), 2, (unsigned)(D / 32));
     const hipStream_t s = static_cast<hipStream_t>(stream);
     switch (D) {
         case 64: launch_append<64>(grid, s, a); break;
