@@ -317,3 +317,23 @@ def test_head_dim_64_in_pairs_equals_the_one_by_one_form(pkg, oracle, bits, dtyp
             want = oracle.NumpyOracle(Pi, cent, bits).decompress(j["idx_bytes"].cpu().numpy().reshape(-1, G), bits16(j["vec_norms"]).reshape(-1))
             err, _ = rel_l2(j["out"].float().cpu().numpy().reshape(-1, D), torch.from_numpy(want).to(j["out"].dtype).float().numpy())
             assert err <= 4e-3, (counts, err)
+
+
+@pytest.mark.parametrize("dim", [80, 144, 176, 208])
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 8])
+def test_ragged_dims_in_chunks_equal_them_by_elements(pkg, dim, bits):
+    """Multiples of 16 that are none of 32 move in whole pieces where everything is aligned, element by element elsewhere: the same bytes
+    and the same values, over full, partial and single tiles of 32 vectors."""
+    layer = pkg.TurboQuantV3(dim, key_bits=bits, value_bits=bits, residual_window=0, layer_idx=8, device=DEV)
+    for (B, H, S), dtype in (((2, 3, 77), torch.float16), ((1, 1, 1), torch.bfloat16), ((1, 4, 64), torch.bfloat16), ((2, 40, 3), torch.float16)):
+        x = outlier_kv((B, H, S, dim), seed=dim + bits, dtype=dtype).to(DEV)
+        shifted = torch.empty(x.numel() + 1, dtype=dtype, device=DEV)[1:].view(x.shape).copy_(x)
+        spaced = torch.nn.functional.pad(x, (0, 3))[..., :dim]
+        k, v = layer.compress_kv(x, x)
+        for other in (shifted, spaced):
+            for a, b in zip((k, v), layer.compress_kv(other, other)):
+                assert torch.equal(a["compressed"]["idx_bytes"], b["compressed"]["idx_bytes"]) and torch.equal(a["compressed"]["vec_norms"], b["compressed"]["vec_norms"])
+        packed = k["compressed"]["idx_bytes"]
+        moved = torch.empty(packed.numel() + 1, dtype=torch.uint8, device=DEV)[1:].view(packed.shape).copy_(packed)
+        k_moved = dict(k, compressed=dict(k["compressed"], idx_bytes=moved))
+        assert torch.equal(layer.decompress_kv(k, v)[0], layer.decompress_kv(k_moved, v)[0])

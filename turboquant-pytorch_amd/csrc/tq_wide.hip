@@ -37,14 +37,29 @@ struct Wide {
     static constexpr uint32_t DECOMPRESS_LDS = 4096 + 3 * TILE_BYTES + 2 * 32 * 4;
 };
 
+// How a head dimension dl fills the D coordinates worked on
+enum Fit {
+    FULL,       // dl == D
+    CHUNKS,     // dl < D in chunks of 16 coordinates, rows, vectors and packed bytes aligned for their pieces: a lane's pieces and codes are
+                // all there or all missing, and every load is one unconditional load of a clamped address
+    ELEMENTS    // dl < D, anything else: element by element and byte by byte where a piece is not whole or not aligned
+};
+// CHUNKS for this job?  (The loads of ELEMENTS sit behind conditions, where the compiler waits for one before it writes the zeros of the
+// other lanes, so nothing is in flight while a tile is worked on: 32 rows x 5873 tokens at 80, 4-bit, keys and values, compress / decompress
+// 40 / 27 us that way, 31 / 23 us this way.)
+__device__ __forceinline__ bool in_chunks(const TqDevJob &job, uint32_t dl, uint32_t packed_bytes) {
+    return dl % 16u == 0u && (((uintptr_t)job.states | (uintptr_t)job.row_stride | (uintptr_t)job.token_stride) & 15u) == 0u &&
+           ((uintptr_t)job.idx_bytes & (uintptr_t)(packed_bytes - 1u)) == 0u;
+}
+
 // position of piece p in row v of a tile
 template <int D>
 __device__ __forceinline__ uint32_t rotated_piece(uint32_t p, uint32_t v) {
     return (p + v) % (uint32_t)Wide<D>::PIECES;
 }
 
-template <int DTYPE, int BITS, int D, bool RAGGED>
-__device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
+template <int DTYPE, int BITS, int D, int FIT>
+__device__ __forceinline__ void wide_compress_tiles(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
     static_assert(DTYPE == TQ_F16 || DTYPE == TQ_BF16, "16-bit inputs");
     using W = Wide<D>;
     constexpr int STEPS = W::STEPS, PIECES = W::PIECES, ROW = W::ROW, THREADS = W::THREADS;
@@ -77,7 +92,9 @@ __device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock b
         for (int l = 0; l < 2; ++l) {
             uint32_t v = tl * 32u + ld_vec[l];
             v = v < job.n_vec ? v : job.n_vec - 1u;
-            if constexpr (RAGGED) {
+            if constexpr (FIT == CHUNKS) {
+                pre[l] = tq_gload16(job.states + tq_vec_offset(job, v) + (ld_piece[l] * 8u < dl ? ld_piece[l] * 16u : 0u));
+            } else if constexpr (FIT == ELEMENTS) {
                 const TQ_GLOBAL uint8_t *src = (const TQ_GLOBAL uint8_t *)job.states + tq_vec_offset(job, v);
                 const uint32_t e0 = ld_piece[l] * 8u;
                 if (e0 + 8u <= dl && (((uintptr_t)src + 2u * e0) & 15u) == 0u) {      // a whole piece at an aligned address
@@ -115,6 +132,7 @@ __device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock b
     auto park = [&](uint32_t b, uint32_t slot) {
 #pragma unroll
         for (int l = 0; l < 2; ++l) {
+            if (FIT == CHUNKS && ld_piece[l] * 8u >= dl) pre[l] = tq_u4{0u, 0u, 0u, 0u};
             *reinterpret_cast<tq_u4 *>(lds_stage[b] + park_off[l]) = pre[l];
             lds_part[slot][ld_vec[l]][ld_piece[l]] = sumsq8<DTYPE>(pre[l], 0.f);
         }
@@ -123,7 +141,7 @@ __device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock b
     uint32_t op_off[STEPS];
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) op_off[s] = n * ROW + (rotated_piece<D>(2u * s + hk, n) << 4);
-    const uint32_t g_bytes = RAGGED ? (dl + IPB - 1u) / IPB : (uint32_t)(D / IPB);      // packed bytes per vector
+    const uint32_t g_bytes = FIT != FULL ? (dl + IPB - 1u) / IPB : (uint32_t)(D / IPB);      // packed bytes per vector
 
     // iteration j: rotate tile j into acc_new, search tile j-1 from acc_old
     auto iteration = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
@@ -163,7 +181,7 @@ __device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock b
                     const tq_u2 cell = *reinterpret_cast<const tq_u2 *>(lds_grid + addr);
                     const float t = fmaf(a, inv, -__uint_as_float(cell[0]));
                     uint32_t code = cell[1] + (~__float_as_uint(t) >> 31);                // base + !(rho < threshold)
-                    if constexpr (RAGGED) code = 32u * wave + 16u * hk + (uint32_t)c < dl ? code : 0u;
+                    if constexpr (FIT == ELEMENTS) code = 32u * wave + 16u * hk + (uint32_t)c < dl ? code : 0u;
                     const int byte = c / IPB, k = c % IPB;                                // most significant code of a byte first
                     words[byte / 4] |= code << (8 * (byte % 4) + BITS * (IPB - 1 - k));
                 }
@@ -172,11 +190,11 @@ __device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock b
         }
         if constexpr (SEARCH) {
             const uint32_t v = (blk.x + (j - 1u) * blk.grid) * 32u + n;
-            if (v < job.n_vec) {
+            if (v < job.n_vec && (FIT != CHUNKS || 32u * wave + 16u * hk < dl)) {
                 const uint32_t slot = tq_packed_slot(job, v);
                 uint8_t *dst = job.idx_bytes + (size_t)slot * g_bytes + (2u * wave + hk) * NB;
                 bool bytewise = false;
-                if constexpr (RAGGED) bytewise = (2u * wave + hk) * NB + NB > g_bytes || ((uintptr_t)dst & (uintptr_t)(NB - 1));
+                if constexpr (FIT == ELEMENTS) bytewise = (2u * wave + hk) * NB + NB > g_bytes || ((uintptr_t)dst & (uintptr_t)(NB - 1));
                 if (bytewise) {
 #pragma unroll
                     for (int b = 0; b < NB; ++b)
@@ -222,6 +240,13 @@ __device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock b
 }
 
 template <int DTYPE, int BITS, int D, bool RAGGED>
+__device__ __forceinline__ void wide_compress_job(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
+    if constexpr (!RAGGED) wide_compress_tiles<DTYPE, BITS, D, FULL>(job, blk, dl, lds);
+    else if (in_chunks(job, dl, 16 / (8 / BITS))) wide_compress_tiles<DTYPE, BITS, D, CHUNKS>(job, blk, dl, lds);
+    else wide_compress_tiles<DTYPE, BITS, D, ELEMENTS>(job, blk, dl, lds);
+}
+
+template <int DTYPE, int BITS, int D, bool RAGGED>
 __global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD) void tq_wide_compress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t dl) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     wide_compress_job<DTYPE, BITS, D, RAGGED>(tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2)), TqBlock{blockIdx.x, gridDim.x}, dl, lds);
@@ -247,8 +272,8 @@ __global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::COMPRESS_WAVES_PER_SIMD)
 // one tile ahead (every thread the bytes of 16 codes), turned into fp16 centroids through the byte -> centroids table and
 // parked in a double-buffered LDS tile that all waves read as B operands; the scaled, rounded results go through a
 // second LDS tile so that the stores are D*2 contiguous bytes per vector.
-template <int DTYPE, int IPB, int D, bool RAGGED>
-__device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
+template <int DTYPE, int IPB, int D, int FIT>
+__device__ __forceinline__ void wide_decompress_tiles(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
     static_assert(DTYPE == TQ_F16 || DTYPE == TQ_BF16, "16-bit outputs");
     using W = Wide<D>;
     constexpr int STEPS = W::STEPS, PIECES = W::PIECES, ROW = W::ROW, THREADS = W::THREADS, WAVES = W::WAVES;
@@ -267,7 +292,7 @@ __device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock
     const uint32_t n_tiles = (job.n_vec + 31u) / 32u;
     if (blk.x >= n_tiles) return;
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
-    const uint32_t g_bytes = RAGGED ? (dl + IPB - 1u) / IPB : (uint32_t)(D / IPB);      // packed bytes per vector in memory
+    const uint32_t g_bytes = FIT != FULL ? (dl + IPB - 1u) / IPB : (uint32_t)(D / IPB);      // packed bytes per vector in memory
 
     // a thread's share of a tile: codes [16 c, 16 c + 16) of vector dv, c = tid % (2 WAVES)
     const uint32_t dv = tid / (2u * WAVES), chunk = tid % (2u * WAVES);
@@ -277,9 +302,9 @@ __device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock
         uint32_t v = tl * 32u + dv;
         v = v < job.n_vec ? v : job.n_vec - 1u;
         const uint32_t slot = tq_packed_slot(job, v);
-        const uint8_t *src = job.idx_bytes + (size_t)slot * g_bytes + chunk * RAW;
+        const uint8_t *src = job.idx_bytes + (size_t)slot * g_bytes + (FIT != CHUNKS || 16u * chunk < dl ? chunk * RAW : 0u);
         bool bytewise = false;
-        if constexpr (RAGGED) bytewise = chunk * RAW + RAW > g_bytes || ((uintptr_t)src & (uintptr_t)(RAW - 1));
+        if constexpr (FIT == ELEMENTS) bytewise = chunk * RAW + RAW > g_bytes || ((uintptr_t)src & (uintptr_t)(RAW - 1));
         if (bytewise) {     // byte by byte; past the vector's last byte: zero (never decoded)
 #pragma unroll
             for (int q = 0; q < 4; ++q) raw[q] = 0u;
@@ -327,7 +352,7 @@ __device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock
                 h[4 * byte] = c[0]; h[4 * byte + 1] = c[1]; h[4 * byte + 2] = c[2]; h[4 * byte + 3] = c[3];
             }
         }
-        if constexpr (RAGGED) {     // coordinates the vector does not have contribute nothing
+        if constexpr (FIT == ELEMENTS) {     // coordinates the vector does not have contribute nothing (CHUNKS: their operands are zero, the centroids finite)
 #pragma unroll
             for (int k = 0; k < 16; ++k)
                 if (16u * chunk + (uint32_t)k >= dl) h[k / 2] &= (k & 1) ? 0x0000ffffu : 0xffff0000u;
@@ -391,10 +416,10 @@ __device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock
             const uint32_t v = tl * 32u + st_vec[k];
             if (v >= job.n_vec) continue;
             uint8_t *dst = out_base + tq_vec_offset(job, v) + st_piece[k] * 16u;
-            if constexpr (RAGGED) {
+            if constexpr (FIT != FULL) {
                 const uint32_t e0 = st_piece[k] * 8u;
                 if (e0 >= dl) continue;
-                if (e0 + 8u > dl || ((uintptr_t)dst & 15u)) {       // element by element
+                if (FIT == ELEMENTS && (e0 + 8u > dl || ((uintptr_t)dst & 15u))) {       // element by element
 #pragma unroll
                     for (uint32_t e = 0; e < 8u; ++e)
                         if (e0 + e < dl) *reinterpret_cast<TQ_GLOBAL uint16_t *>((TQ_GLOBAL uint8_t *)dst + 2u * e) = (uint16_t)(val[e / 2] >> (16 * (e & 1)));
@@ -405,6 +430,13 @@ __device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock
         }
         if (j + 1u < m) decode((j + 1u) & 1u);
     }
+}
+
+template <int DTYPE, int IPB, int D, bool RAGGED>
+__device__ __forceinline__ void wide_decompress_job(const TqDevJob &job, TqBlock blk, uint32_t dl, uint8_t *lds) {
+    if constexpr (!RAGGED) wide_decompress_tiles<DTYPE, IPB, D, FULL>(job, blk, dl, lds);
+    else if (in_chunks(job, dl, 16 / IPB)) wide_decompress_tiles<DTYPE, IPB, D, CHUNKS>(job, blk, dl, lds);
+    else wide_decompress_tiles<DTYPE, IPB, D, ELEMENTS>(job, blk, dl, lds);
 }
 
 template <int DTYPE, int IPB, int D, bool RAGGED>
