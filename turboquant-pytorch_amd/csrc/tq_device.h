@@ -162,6 +162,42 @@ __device__ __forceinline__ uint32_t tq_packed_slot(const TqDevJob &job, uint32_t
     return row * job.packed_row_stride + (v - row * job.tokens);
 }
 
+// A block's walk over tiles of 32 consecutive vectors, a fixed number of tiles at a time: row and token of the tile's first vector are
+// carried along on the scalar unit, and a lane's vector is one comparison further on.  (A 32-bit division per address is some 25
+// vector instructions, several of them at a quarter of the rate: three of them were a third of a trip of the 96-wide compress kernel.)
+struct TqTileWalk {
+    uint32_t v, row, tok, step, step_row, step_tok;
+    __device__ __forceinline__ TqTileWalk(const TqDevJob &job, uint32_t tile, uint32_t tiles_per_step) {
+        v = tile * 32u;
+        row = tq_uniform32(v / job.tokens);
+        tok = v - row * job.tokens;
+        step = tiles_per_step * 32u;
+        step_row = tq_uniform32(step / job.tokens);
+        step_tok = step - step_row * job.tokens;
+    }
+    __device__ __forceinline__ void next(const TqDevJob &job) {
+        v += step;
+        row += step_row;
+        tok += step_tok;
+        if (tok >= job.tokens) {
+            tok -= job.tokens;
+            ++row;
+        }
+    }
+    // byte offset in `states` of vector i < 32 of the tile, own = i * token_stride + what the lane adds; a tile in rows of fewer
+    // than 32 tokens may hold several row ends
+    __device__ __forceinline__ long long offset(const TqDevJob &job, uint32_t i, long long own) const {
+        const long long base = (long long)row * job.row_stride + (long long)tok * job.token_stride;
+        if (job.tokens < 32u) return tq_vec_offset(job, v + i) + own - (long long)i * job.token_stride;
+        return base + own + (tok + i >= job.tokens ? job.row_stride - (long long)job.tokens * job.token_stride : 0ll);
+    }
+    // the same for the packed slot
+    __device__ __forceinline__ uint32_t slot(const TqDevJob &job, uint32_t i) const {
+        if (job.tokens < 32u) return tq_packed_slot(job, v + i);
+        return row * job.packed_row_stride + tok + i + (tok + i >= job.tokens ? job.packed_row_stride - job.tokens : 0u);
+    }
+};
+
 // Global-memory accessors (explicit address space: plain pointers read from a descriptor
 // would otherwise be accessed with flat instructions, which also occupy the LDS counter).
 __device__ __forceinline__ tq_u4 tq_gload16(const uint8_t *p) {
