@@ -479,18 +479,20 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
 
     // loads of a tile: piece i = l * 512 + tid of the tile's 1024 is piece i % 32 of vector i / 32, so that the 32 pieces
-    // of a vector sit in 32 consecutive lanes; vectors past the end re-read the job's last one (never stored)
+    // of a vector sit in 32 consecutive lanes; vectors past the end read the tile's first piece (never stored)
     const uint32_t ld_vec = tid >> 5, ld_piece = tid & 31u;
+    const long long ld_own = (long long)ld_vec * job.token_stride + ld_piece * 16u;
     tq_u4 pre[2];
-    auto issue_loads = [&](uint32_t tl) {
+    auto issue_loads = [&](const TqTileWalk &t) {
 #pragma unroll
         for (int l = 0; l < 2; ++l) {
-            uint32_t v = tl * 32u + l * 16u + ld_vec;
-            v = v < job.n_vec ? v : job.n_vec - 1u;
-            pre[l] = tq_gload16(job.states + tq_vec_offset(job, v) + ld_piece * 16u);
+            const uint32_t i = l * 16u + ld_vec;
+            const bool there = t.v + i < job.n_vec;
+            pre[l] = tq_gload16(job.states + t.offset(job, there ? i : 0u, there ? ld_own + 16ll * l * job.token_stride : 0ll));
         }
     };
-    issue_loads(blk.x);
+    TqTileWalk ahead(job, blk.x, blk.grid), done = ahead;      // of the tile fetched next, of the tile searched next
+    issue_loads(ahead);
 
     tq_u4 areg[2][STEPS];
     {
@@ -556,9 +558,8 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
             if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (SEARCH) {
-            const uint32_t v = (blk.x + (j - 1u) * blk.grid) * 32u + n;
-            if (v < job.n_vec) {
-                const uint32_t slot = tq_packed_slot(job, v);
+            if (done.v + n < job.n_vec) {
+                const uint32_t slot = done.slot(job, n);
                 uint8_t *dst = job.idx_bytes + (size_t)slot * g_bytes + (2u * wave + hk) * NB;
                 if constexpr (NB == 2) tq_gstore2(reinterpret_cast<uint16_t *>(dst), (uint16_t)words[0]);
                 else if constexpr (NB == 4) *reinterpret_cast<TQ_GLOBAL uint32_t *>((TQ_GLOBAL uint8_t *)dst) = words[0];
@@ -569,6 +570,7 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
                     tq_gstore2(job.vec_norms + slot, __builtin_bit_cast(uint16_t, hn));
                 }
             }
+            done.next(job);
         }
     };
 
@@ -576,7 +578,10 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
     // one trip: the tile after this one sets out while this one is rotated, and is parked behind the trip's work
     auto trip = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
         const bool more = j + 1u < m;
-        if (more) issue_loads(blk.x + (j + 1u) * blk.grid);
+        if (more) {
+            ahead.next(job);
+            issue_loads(ahead);
+        }
         __syncthreads();        // tile j and its sums are parked, and nobody reads buffer (j + 1) & 1 any more
         iteration(rot_tag, search_tag, j, acc_new, acc_old);
         if (more) park((j + 1u) & 1u, (j + 1u) % 3u);
@@ -653,10 +658,8 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
     const uint32_t dv = tid >> 3, chunk = tid & 7u;
     uint32_t raw[RW];
     uint16_t norm_bits = 0;
-    auto issue_loads = [&](uint32_t tl) {
-        uint32_t v = tl * 32u + dv;
-        v = v < job.n_vec ? v : job.n_vec - 1u;
-        const uint32_t slot = tq_packed_slot(job, v);
+    auto issue_loads = [&](const TqTileWalk &t) {
+        const uint32_t slot = t.slot(job, t.v + dv < job.n_vec ? dv : 0u);      // (past the end: the tile's first vector again)
         const uint8_t *src = job.idx_bytes + (size_t)slot * g_bytes + chunk * RAW;
         if constexpr (RW == 1) raw[0] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src);
         else if constexpr (RW == 2) { const tq_u2 t = tq_gload8(src); raw[0] = t[0]; raw[1] = t[1]; }
@@ -670,7 +673,8 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
         }
         if (chunk == 0u) norm_bits = tq_gload2(job.vec_norms + slot);
     };
-    issue_loads(blk.x);
+    TqTileWalk ahead(job, blk.x, blk.grid), here = ahead;      // of the tile fetched next, of the tile stored
+    issue_loads(ahead);
 
     tq_u4 areg[2][STEPS];       // row tiles 2w, 2w + 1
     {
@@ -718,11 +722,14 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
     const uint32_t op_base = n * (D * 2) + (((hk << 3) ^ (n & 31u)) << 4);
     auto op_step = [](int s) { return (uint32_t)((((2 * (s & 1)) << 3) | (s >> 1)) << 4); };
 
+    const long long st_own = (long long)(tid >> 5) * job.token_stride + (tid & 31u) * 16u;      // of the stores below
     const uint32_t m = (n_tiles - blk.x + blk.grid - 1u) / blk.grid;
     decode(0u);
     for (uint32_t j = 0; j < m; ++j) {
-        const uint32_t tl = blk.x + j * blk.grid;
-        if (j + 1u < m) issue_loads(tl + blk.grid);
+        if (j + 1u < m) {
+            ahead.next(job);
+            issue_loads(ahead);
+        }
         __syncthreads();        // tile j is decoded; the output tile of the last iteration has been read
         const uint8_t *ys = lds_y[j & 1u];
         tq_f16v acc[2] = {tq_zero16(), tq_zero16()};
@@ -758,9 +765,9 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
         for (int k = 0; k < 4; ++k) {       // 1024 pieces, 256 threads: piece i % 32 of vector i / 32, 512 contiguous bytes per vector
             const uint32_t i = k * 256u + tid, vl = i >> 5, p = i & 31u;
             const tq_u4 val = *reinterpret_cast<const tq_u4 *>(lds_out + vl * (D * 2) + ((p ^ (vl & 31u)) << 4));
-            const uint32_t v = tl * 32u + vl;
-            if (v < job.n_vec) tq_gstore16_stream(out_base + tq_vec_offset(job, v) + p * 16u, val);
+            if (here.v + vl < job.n_vec) tq_gstore16_stream(out_base + here.offset(job, vl, st_own + 8ll * k * job.token_stride), val);
         }
+        here.next(job);
         if (j + 1u < m) decode((j + 1u) & 1u);
     }
 }
