@@ -39,7 +39,7 @@ struct AppendArgs {
 // whole tensors of this head dimension, so the bytes are theirs.
 template <int D, bool BF>
 __global__ __launch_bounds__(TQ_WAVE) void tq_decode_append_kernel(AppendArgs a) {
-    constexpr int STEPS = D / 16, PIECES = D / 8;
+    constexpr int STEPS = D / 16;
     constexpr int CELL_LOADS = (D == 128 ? TQ_GRID_COPY_STRIDE(8) : TQ_GRID_LDS_BYTES) / 1024;      // 128: the grids fit two copies at least
     static_assert(CELL_LOADS * 1024 == (D == 128 ? TQ_GRID_COPY_STRIDE(8) : TQ_GRID_LDS_BYTES), "whole loads of a wave");
     __shared__ __align__(16) uint8_t lds_grid[CELL_LOADS * 1024];
