@@ -23,7 +23,7 @@ __device__ __forceinline__ void split_f16x8(tq_u4 v, tq_u4 &hi, tq_u4 &lo) {
 
 // Records of a row with several splits travel between blocks past the caches that are not shared (stores and loads of device
 // scope), so that nothing has to be written back or invalidated around the arrival counter: with fences there a step of
-// 8 rows x 32768 tokens took 32.0 us and now 30.0, one of 32 rows x 6000 tokens, 64 wide, 27.3 and now 24.7.  A row with one split keeps
+// 8 rows x 32768 tokens took 32.0 us with fences and 30.0 this way when it was made, one of 32 rows x 6000 tokens, 64 wide, 27.3 and 24.7.  A row with one split keeps
 // its records in its own block: they stay cached (512 rows x 16384 tokens: 2 % longer otherwise).
 // No release and acquire of the language stand behind this order, all accesses are relaxed: it rests on the hardware, where a
 // store of device scope counts in vmcnt until every compute unit sees it, and on both sides going through put_record and
