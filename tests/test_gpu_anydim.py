@@ -337,3 +337,22 @@ def test_ragged_dims_in_chunks_equal_them_by_elements(pkg, dim, bits):
         moved = torch.empty(packed.numel() + 1, dtype=torch.uint8, device=DEV)[1:].view(packed.shape).copy_(packed)
         k_moved = dict(k, compressed=dict(k["compressed"], idx_bytes=moved))
         assert torch.equal(layer.decompress_kv(k, v)[0], layer.decompress_kv(k_moved, v)[0])
+
+
+@pytest.mark.parametrize("dim", [80, 90, 96, 160, 192, 224, 256])
+def test_rows_that_end_at_every_place_of_a_tile(pkg, dim):
+    """A tile of 32 vectors lies in one row, holds a row's end, several of them (rows of fewer than 32 tokens) or the job's: the bytes
+    and values of token slices (a row stride of their own) equal those of the same vectors laid end to end, nothing else is written."""
+    comp = pkg.MSECompressor(dim, 4, seed=3, device=DEV)
+    for rows in (1, 3, 40):
+        for tokens in (1, 5, 31, 32, 33, 63, 64, 65, 97):
+            big = outlier_kv((1, rows, tokens + 3, dim), seed=tokens, dtype=torch.float16).to(DEV)
+            part = big[:, :, 2:2 + tokens]
+            packed, dense = comp.compress(part), comp.compress(part.contiguous())
+            for name in ("idx_bytes", "vec_norms"):
+                assert torch.equal(packed[name], dense[name]), (rows, tokens, name)
+            out, want = torch.full_like(big, 7.0), torch.empty_like(part, memory_format=torch.contiguous_format)
+            comp.decompress_into(dense, out[:, :, 2:2 + tokens])
+            comp.decompress_into(dense, want)
+            assert torch.equal(out[:, :, 2:2 + tokens], want), (rows, tokens)
+            assert bool((out[:, :, :2] == 7).all()) and bool((out[:, :, 2 + tokens:] == 7).all()), (rows, tokens)

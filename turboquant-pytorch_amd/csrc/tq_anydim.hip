@@ -487,8 +487,7 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
 #pragma unroll
         for (int l = 0; l < 2; ++l) {
             const uint32_t i = l * 16u + ld_vec;
-            const bool there = t.v + i < job.n_vec;
-            pre[l] = tq_gload16(job.states + t.offset(job, there ? i : 0u, there ? ld_own + 16ll * l * job.token_stride : 0ll));
+            pre[l] = tq_gload16(job.states + t.offset(job, i, ld_own + 16ll * l * job.token_stride));
         }
     };
     TqTileWalk ahead(job, blk.x, blk.grid), done = ahead;      // of the tile fetched next, of the tile searched next
@@ -659,7 +658,7 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
     uint32_t raw[RW];
     uint16_t norm_bits = 0;
     auto issue_loads = [&](const TqTileWalk &t) {
-        const uint32_t slot = t.slot(job, t.v + dv < job.n_vec ? dv : 0u);      // (past the end: the tile's first vector again)
+        const uint32_t slot = t.slot(job, dv);
         const uint8_t *src = job.idx_bytes + (size_t)slot * g_bytes + chunk * RAW;
         if constexpr (RW == 1) raw[0] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src);
         else if constexpr (RW == 2) { const tq_u2 t = tq_gload8(src); raw[0] = t[0]; raw[1] = t[1]; }

@@ -184,17 +184,34 @@ struct TqTileWalk {
             ++row;
         }
     }
-    // byte offset in `states` of vector i < 32 of the tile, own = i * token_stride + what the lane adds; a tile in rows of fewer
-    // than 32 tokens may hold several row ends
+    // Whole: all 32 vectors exist and lie in one row.  Looked at first (uniform), so that a tile costs one addition per address; the empty asm
+    // keeps the rest behind a branch.  (As selects in every tile: dense job lists, which need none of it, 2 to 6 % slower, 24 tensors of 8 x 4099
+    // tokens at 160, 2-bit, restore 75 / 80 us without and with them; here 76.  A branch on jobs of one row alone left layers 3 to 10 % slower.)
+    __device__ __forceinline__ bool whole(const TqDevJob &job) const { return tok + 32u <= job.tokens; }
+    // Byte offset in `states` of vector i < 32 of the tile, own = i * token_stride + what the lane adds.  A vector that the job does not
+    // have: the first byte of the tile.  A tile in rows of fewer than 32 tokens may hold several row ends.
     __device__ __forceinline__ long long offset(const TqDevJob &job, uint32_t i, long long own) const {
         const long long base = (long long)row * job.row_stride + (long long)tok * job.token_stride;
-        if (job.tokens < 32u) return tq_vec_offset(job, v + i) + own - (long long)i * job.token_stride;
-        return base + own + (tok + i >= job.tokens ? job.row_stride - (long long)job.tokens * job.token_stride : 0ll);
+        long long off = base + own;
+        if (!whole(job)) {
+            asm volatile("");
+            if (job.tokens < 32u) off = tq_vec_offset(job, v + i) + own - (long long)i * job.token_stride;
+            else if (tok + i >= job.tokens) off += job.row_stride - (long long)job.tokens * job.token_stride;
+            if (v + i >= job.n_vec) off = base;
+        }
+        return off;
     }
     // the same for the packed slot
     __device__ __forceinline__ uint32_t slot(const TqDevJob &job, uint32_t i) const {
-        if (job.tokens < 32u) return tq_packed_slot(job, v + i);
-        return row * job.packed_row_stride + tok + i + (tok + i >= job.tokens ? job.packed_row_stride - job.tokens : 0u);
+        const uint32_t first = row * job.packed_row_stride + tok;
+        uint32_t s = first + i;
+        if (!whole(job)) {
+            asm volatile("");
+            if (job.tokens < 32u) s = tq_packed_slot(job, v + i);
+            else if (tok + i >= job.tokens) s += job.packed_row_stride - job.tokens;
+            if (v + i >= job.n_vec) s = first;
+        }
+        return s;
     }
 };
 

@@ -93,10 +93,9 @@ __device__ __forceinline__ void wide_compress_tiles(const TqDevJob &job, TqBlock
     auto issue_loads = [&](const TqTileWalk &t) {
 #pragma unroll
         for (int l = 0; l < 2; ++l) {
-            const bool there = t.v + ld_vec[l] < job.n_vec;
-            const uint8_t *piece = job.states + t.offset(job, there ? ld_vec[l] : 0u, there ? ld_own[l] : 0ll);
+            const uint8_t *piece = job.states + t.offset(job, ld_vec[l], ld_own[l]);
             if constexpr (FIT == ELEMENTS) {
-                const uint32_t e0 = there ? ld_piece[l] * 8u : 0u;
+                const uint32_t e0 = t.v + ld_vec[l] < job.n_vec ? ld_piece[l] * 8u : 0u;
                 const TQ_GLOBAL uint8_t *src = (const TQ_GLOBAL uint8_t *)piece - 2u * e0;
                 if (e0 + 8u <= dl && (((uintptr_t)src + 2u * e0) & 15u) == 0u) {      // a whole piece at an aligned address
                     pre[l] = *reinterpret_cast<const TQ_GLOBAL tq_u4 *>(src + 2u * e0);
@@ -304,7 +303,7 @@ __device__ __forceinline__ void wide_decompress_tiles(const TqDevJob &job, TqBlo
     uint32_t raw[4] = {0u, 0u, 0u, 0u};
     uint16_t norm_bits = 0;
     auto issue_loads = [&](const TqTileWalk &t) {
-        const uint32_t slot = t.slot(job, t.v + dv < job.n_vec ? dv : 0u);      // (past the end: the tile's first vector again)
+        const uint32_t slot = t.slot(job, dv);
         const uint8_t *src = job.idx_bytes + (size_t)slot * g_bytes + (FIT != CHUNKS || 16u * chunk < dl ? chunk * RAW : 0u);
         bool bytewise = false;
         if constexpr (FIT == ELEMENTS) bytewise = chunk * RAW + RAW > g_bytes || ((uintptr_t)src & (uintptr_t)(RAW - 1));
