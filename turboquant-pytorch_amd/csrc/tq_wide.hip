@@ -34,6 +34,10 @@ struct Wide {
     // compress: quantiser grid | two tiles | per-piece sums of squares of three tiles
     static constexpr uint32_t COMPRESS_LDS = TQ_GRID_LDS_BYTES + 2 * TILE_BYTES + 3 * 32 * PIECES * 4;
     // decompress: byte -> centroids table | two tiles of centroids | output tile | norms of two tiles
+    // waves per SIMD the restore of a layer is compiled for: as many as the per-tensor kernel has.  Left alone its five bodies and the piece
+    // of the window took 136 registers at 224, where a block is seven waves and one instead of two were resident (8 x 16384 tokens, K4/V2, no
+    // window: per tensor 41 us, 44.5 that way, 40.0 this way), and four waves instead of five at 96
+    static constexpr int RESTORE_WAVES_PER_SIMD = D == 96 ? 5 : 4;
     static constexpr uint32_t DECOMPRESS_LDS = 4096 + 3 * TILE_BYTES + 2 * 32 * 4;
 };
 
@@ -454,7 +458,7 @@ __global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_decompress_kernel(Tq
 
 // keys and values of a layer and its window
 template <int DTYPE, int D, bool RAGGED>
-__global__ __launch_bounds__(Wide<D>::THREADS) void tq_wide_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t dl) {
+__global__ __launch_bounds__(Wide<D>::THREADS, Wide<D>::RESTORE_WAVES_PER_SIMD) void tq_wide_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t dl) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t which = tq_layer_job(l);
     const TqDevJob job = tq_uniform_job(which ? l.job[1] : l.job[0]);
