@@ -633,7 +633,7 @@ def restore_layer(packed_k, packed_v, tokens: int, table_k: torch.Tensor, table_
         if got is not None:
             if type(got) is int:
                 check(got, "tq_restore_layer")
-            return got
+            return got or None      # False: no call takes such a window
     if w0 is not None:
         packed_k, packed_v = (tuple(t[:, :, :tokens] for t in pair) for pair in (packed_k, packed_v))
         k_win, v_win = k_win[:, :, w0:w0 + n_win], v_win[:, :, w0:w0 + n_win]

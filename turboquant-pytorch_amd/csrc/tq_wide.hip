@@ -34,7 +34,7 @@ struct Wide {
     // compress: quantiser grid | two tiles | per-piece sums of squares of three tiles
     static constexpr uint32_t COMPRESS_LDS = TQ_GRID_LDS_BYTES + 2 * TILE_BYTES + 3 * 32 * PIECES * 4;
     // decompress: byte -> centroids table | two tiles of centroids | output tile | norms of two tiles
-    // waves per SIMD the restore of a layer is compiled for: as many as the per-tensor kernel has.  Left alone its five bodies and the piece
+    // waves per SIMD the restore of a layer is compiled for: as many as the per-tensor kernel has.  Left alone its bodies and the piece
     // of the window took 136 registers at 224, where a block is seven waves and one instead of two were resident (8 x 16384 tokens, K4/V2, no
     // window: per tensor 41 us, 44.5 that way, 40.0 this way), and four waves instead of five at 96
     static constexpr int RESTORE_WAVES_PER_SIMD = D == 96 ? 5 : 4;
