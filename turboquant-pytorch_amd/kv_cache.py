@@ -272,8 +272,6 @@ class V3Cache:
         """Bookkeeping of generation_test_v2.py:96-126: the uncompressed tokens are (window ++ new); all but
         the last `residual_window` of them are compressed for good, the rest is the new window."""
         S_new = key_states.shape[2]
-        if S_new == 1 and st.append_one(key_states, value_states):
-            return
         st.total_seq += S_new
         rw = self.residual_window
         recent = st.n_recent + S_new
