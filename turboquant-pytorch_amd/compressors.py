@@ -211,9 +211,11 @@ class TurboQuantCompressorV2:
         rotated by Pi for the first and projected by S for the second; neither the reconstruction nor the signs are
         expanded).  A dict in the reference's format (`reference_format`) is accepted too and takes plain matrix
         products."""
-        if queries.is_cuda and "idx_bytes" in compressed and compressed["shape"][3] == _native.HEAD_DIM and not torch.compiler.is_compiling():
+        # few query tokens: one launch
+        if (queries.size(-2) <= _native.MAX_QUERY_SCORES and queries.is_cuda and "idx_bytes" in compressed
+                and compressed["shape"][3] == _native.HEAD_DIM and not torch.compiler.is_compiling()):
             dev, idx = queries.device, compressed["idx_bytes"]
-            if idx.shape[:3] == compressed["shape"][:3]:       # up to _native.MAX_QUERY_SCORES query tokens in one launch
+            if idx.shape[:3] == compressed["shape"][:3]:
                 out = _native.fast().qjl_scores(queries, idx, compressed["vec_norms"], compressed["sign_bytes"], compressed["residual_norm"],
                                                 self._mse.table(dev), self._both(dev), self.mse_bits)
                 if out is not None:
