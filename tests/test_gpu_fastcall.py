@@ -153,3 +153,11 @@ def test_one_step_v2_calls_equal_the_general_path(pkg, monkeypatch, bits, dtype)
             assert a.shape == b.shape and a.dtype == b.dtype
             scale = queries.double().norm(dim=-1)[..., None] * x.detach().double().norm(dim=-1)[:, :, None, :]
             assert float(((a.double() - b.double()).abs() / scale.clamp_min(1e-30)).max()) < 3e-5, name
+
+
+def test_v2_scores_of_a_negated_view(pkg):
+    """A tensor whose sign torch keeps as a flag is read with that sign."""
+    comp = pkg.TurboQuantCompressorV2(128, 3, seed=5, device=DEV)
+    packed = comp.compress(outlier_kv((1, 2, 70, 128), seed=1, dtype=torch.bfloat16).to(DEV))
+    q = torch.randn(1, 2, 3, 128, generator=torch.Generator().manual_seed(2)).to(DEV)
+    assert torch.equal(comp.asymmetric_attention_scores(torch._neg_view(q), packed), comp.asymmetric_attention_scores(-q, packed))

@@ -44,7 +44,7 @@ struct Raised {};        // a Python exception is set
 inline const at::Tensor *tensor(PyObject *o) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
-    return t.has_storage() && t.layout() == at::kStrided && t.is_cuda() ? &t : nullptr;
+    return t.has_storage() && t.layout() == at::kStrided && t.is_cuda() && !t.is_neg() ? &t : nullptr;      // (neg: memory holds the values without their sign)
 }
 inline long long integer(PyObject *o) {
     const long long v = PyLong_AsLongLong(o);
