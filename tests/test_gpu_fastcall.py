@@ -155,6 +155,26 @@ def test_one_step_v2_calls_equal_the_general_path(pkg, monkeypatch, bits, dtype)
             assert float(((a.double() - b.double()).abs() / scale.clamp_min(1e-30)).max()) < 3e-5, name
 
 
+def test_allocations_that_fail_raise_torchs_own_error(pkg):
+    """A caller that frees memory and tries again on torch.cuda.OutOfMemoryError gets that error from every call."""
+    comp = pkg.MSECompressor(128, 1, seed=3, device=DEV)
+    layer = pkg.TurboQuantV3(128, key_bits=1, value_bits=1, residual_window=0, layer_idx=8, device=DEV)
+    x = torch.zeros(1, 8, 1 << 16, 128, dtype=torch.bfloat16, device=DEV)
+    packed, both = comp.compress(x), layer.compress_kv(x, x)
+    big = torch.zeros(1, 8, 1 << 20, 16, dtype=torch.uint8, device=DEV)
+    many = {"idx_bytes": big, "vec_norms": torch.zeros(big.shape[:3], dtype=torch.float16, device=DEV), "shape": (*big.shape[:3], 128), "idx_pad": 0}
+    wide = tuple(dict(b, compressed=many, shape=(1, 8, 1 << 20, 128), split_at=1 << 20) for b in both)
+    torch.cuda.empty_cache()
+    try:
+        torch.cuda.set_per_process_memory_fraction(1e-6)        # nothing can be added to what is held
+        for call in (lambda: comp.decompress(many), lambda: layer.decompress_kv(*wide)):
+            with pytest.raises(torch.cuda.OutOfMemoryError):
+                call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert comp.decompress(packed).shape == x.shape
+
+
 def test_v2_scores_of_a_negated_view(pkg):
     """A tensor whose sign torch keeps as a flag is read with that sign."""
     comp = pkg.TurboQuantCompressorV2(128, 3, seed=5, device=DEV)

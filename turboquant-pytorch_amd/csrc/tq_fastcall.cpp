@@ -5,6 +5,7 @@
 // Every function answers None where the arguments are not plain tensors laid out as its kernel reads them (other types and subclasses, a
 // device that is not the current one, strides, alignment, a stream that is being captured where that matters): the caller then takes its
 // general path, which copies, falls back or raises.  A status other than 0 comes back as an integer.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -402,22 +403,22 @@ PyObject *qjl_scores(PyObject *const *a) {
     return THPVariable_Wrap(out);
 }
 
-// No exception leaves a function, and none records gradients.
+// No exception leaves a function, and none records gradients.  Errors of torch's (no memory, a device error) become the Python exceptions
+// that its own functions raise.
 template <PyObject *(*F)(PyObject *const *), int N>
 PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != N) {
         PyErr_Format(PyExc_TypeError, "expected %d arguments, got %zd", N, n);
         return nullptr;
     }
+    HANDLE_TH_ERRORS
     try {
         c10::NoGradGuard no_grad;
         return F(args);
     } catch (const Raised &) {
         return nullptr;
-    } catch (const std::exception &e) {
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
     }
+    END_HANDLE_TH_ERRORS
 }
 
 // init(addresses of the entry points in the order of Entries, raw_stream, workspace, drop_workspace, scratch, arrived, tag)
