@@ -776,3 +776,27 @@ def test_host_side_of_the_abi_under_sanitizers(tmp_path):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0")      # (the HIP runtime keeps its own allocations until exit)
     run = subprocess.run([exe], capture_output=True, text=True, timeout=300, env=env)
     assert run.returncode == 0 and run.stdout.strip() == "ok", run.stdout + run.stderr[-3000:]
+
+
+def test_extension_built_against_something_else_is_not_used(pkg, monkeypatch):
+    """tqamd_fastcall takes Python objects for the tensors of the torch it was compiled against, and addresses of the library for entry points
+    of its header: of another torch, interpreter or library it is refused, with how to build it."""
+    native = pkg._native
+    monkeypatch.setattr(native, "_fast", None)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "0.0.1")
+        with pytest.raises(native.TqError, match="build"):
+            native.fast()
+    with monkeypatch.context() as m:
+        library = native.lib()
+
+        class Newer:
+            tq_abi_version = staticmethod(lambda: library.tq_abi_version() + 1)
+
+            def __getattr__(self, name):
+                return getattr(library, name)
+
+        m.setattr(native, "lib", lambda: Newer())
+        with pytest.raises(native.TqError, match="build"):
+            native.fast()
+    assert native.fast() is native.fast()

@@ -12,6 +12,7 @@ import ctypes
 import os
 import shutil
 import subprocess
+import sysconfig
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -21,7 +22,6 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libtqamd.so")
 FAST_NAME = "tqamd_fastcall"        # extension module: the eager calls from tensors to the library in one step each
-FAST_PATH = os.path.join(CSRC, FAST_NAME + ".so")
 FAST_SOURCE = "tq_fastcall.cpp"
 SOURCES = ("tq_host.cpp", "tq_compress.hip", "tq_decompress.hip", "tq_anydim.hip", "tq_wide.hip", "tq_attend.hip", "tq_qjl.hip", "tq_qjl_scores.hip",
            "tq_decode.hip", "tq_decode_d64.hip", "tq_decode_d96.hip", "tq_decode_d128_narrow.hip", "tq_decode_d128_wide.hip", "tq_decode_d256.hip")
@@ -101,20 +101,29 @@ def _link(objs: Dict[str, str], out_path: str) -> None:
     os.replace(tmp, out_path)
 
 
+def _fast_path() -> str:
+    """The extension module's file, named for the interpreter and the torch it is compiled against: loaded into others it would read their
+    objects as what they are not."""
+    return os.path.join(CSRC, f"{FAST_NAME}.{sysconfig.get_config_var('SOABI')}.torch-{torch.__version__}.so")
+
+
 def _build_fastcall(force: bool) -> None:
-    """csrc/tqamd_fastcall.so, against the headers and libraries of the installed torch."""
-    import sysconfig
+    """csrc/tqamd_fastcall.*.so, against the headers and libraries of the installed torch; in place of those built for others."""
     from torch.utils import cpp_extension
+    path = _fast_path()
     sources = [os.path.join(CSRC, FAST_SOURCE), os.path.join(CSRC, "..", "..", "include", "tqamd.h")]
-    if not force and os.path.exists(FAST_PATH) and os.path.getmtime(FAST_PATH) >= max(map(os.path.getmtime, sources)):
+    if not force and os.path.exists(path) and os.path.getmtime(path) >= max(map(os.path.getmtime, sources)):
         return
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
-    tmp = FAST_PATH + ".tmp"
+    tmp = path + ".tmp"
     _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-isystem" + p for p in cpp_extension.include_paths()),
           "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(rocm, "include"), sources[0], "-o", tmp,
           *("-L" + p for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-L" + os.path.join(rocm, "lib"), "-lamdhip64"])
-    os.replace(tmp, FAST_PATH)
+    os.replace(tmp, path)
+    for name in os.listdir(CSRC):
+        if name.startswith(FAST_NAME + ".") and name.endswith(".so") and name != os.path.basename(path):
+            os.remove(os.path.join(CSRC, name))
 
 
 def build(force: bool = True, verbose: bool = False) -> str:
@@ -273,17 +282,24 @@ _fast = None
 
 
 def fast():
-    """The extension module tqamd_fastcall; raises if it has not been built.  Its functions take what a call has in hand and answer
-    None where the general path has to look at it."""
+    """The extension module tqamd_fastcall; raises if it has not been built for this interpreter, torch and library (the general path
+    would serve its calls, several times slower, and nobody would know).  Its functions take what a call has in hand and answer None
+    where the general path has to look at it."""
     global _fast
     if _fast is None:
         from importlib import machinery, util
-        if not os.path.exists(FAST_PATH):
-            raise TqError(f"{FAST_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+        path, how = _fast_path(), "build it with `python -c 'import __graft_entry__ as g; g.build()'`"
+        if not os.path.exists(path):
+            raise TqError(f"{path} is missing: {how}")
         L = lib()
-        loader = machinery.ExtensionFileLoader(FAST_NAME, FAST_PATH)
-        module = util.module_from_spec(util.spec_from_file_location(FAST_NAME, FAST_PATH, loader=loader))
-        loader.exec_module(module)
+        loader = machinery.ExtensionFileLoader(FAST_NAME, path)
+        try:
+            module = util.module_from_spec(util.spec_from_file_location(FAST_NAME, path, loader=loader))
+            loader.exec_module(module)
+        except ImportError as e:
+            raise TqError(f"{path} cannot be loaded ({e}): {how}") from e
+        if module.abi_version != L.tq_abi_version():
+            raise TqError(f"{path} was built for version {module.abi_version} of the library, this is {L.tq_abi_version()}: {how}")
         entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend", "tq_qjl_compress", "tq_qjl_query_scores")
         stream_of = _raw_stream or (lambda index: torch.cuda.current_stream(index).cuda_stream)
         module.init(tuple(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in entries), stream_of, _workspace, _drop_workspace, _step_scratch, _arrived, _TABLE_TAG)

@@ -455,4 +455,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "tqamd_fastcall", nullptr, -1, meth
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_tqamd_fastcall(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_tqamd_fastcall(void) {
+    PyObject *m = PyModule_Create(&module);
+    if (m && PyModule_AddIntConstant(m, "abi_version", TQ_ABI_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}
