@@ -413,8 +413,8 @@ int tq_attend_step(const void *queries, int q_dtype, long long rows, int group, 
  * tq_decode_append: as tq_append_token (same bytes as tq_compress with rows x 1 token).
  * tq_decode_attend: softmax(scale * q K^T) V of one query token per head ([rows, group, head_dim], group <= 16) over the first
  *   `tokens` packed slots of every row and its window slots win_first .. win_first + n_win - 1 (n_win <= 512; not both
- *   empty).  scratch: tq_decode_scratch_floats() float32 values (scratch_size: how many there are; TQ_ERR_CAPACITY if
- *   too few), arrived: `rows` counters, zero before the first use and left zero by every launch that completes; neither
+ *   empty).  scratch: tq_decode_scratch_floats() float32 values at a multiple of 4 bytes (scratch_size: how many there are;
+ *   TQ_ERR_CAPACITY if too few; one of them is there to begin at a multiple of 8), arrived: `rows` counters, zero before the first use and left zero by every launch that completes; neither
  *   is shared by launches that can overlap in time.
  * tq_decode_supported: 1 if these calls take the combination, 0 otherwise.
  */

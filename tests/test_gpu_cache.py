@@ -3,6 +3,8 @@ streaming cache built on it, against the dense kernels, the CPU oracle and the b
 the reference's generation-time cache (generation_test_v2.py:80-165)."""
 import copy
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -833,6 +835,23 @@ def test_decode_attention_with_heads_side_by_side(pkg, dim, bits):
             ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
             err = float((cache.attend(q, 8).double().reshape(ref.shape) - ref).norm() / ref.norm())
             assert err < (1.5e-3 if dim == 128 else 3.5e-4), (rows, tokens, group, err)
+
+
+def test_decode_attention_with_scratch_at_any_float(pkg):
+    """Scratch that begins at an odd multiple of 4 bytes gives the same bytes, and nothing is written outside of it."""
+    native = pkg._native
+    cache = pkg.V3Cache(4, 2, residual_window=40, n_layers=40)
+    x = torch.randn(2, 2, 1500, 128, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)
+    cache.append(x, x, 8)
+    st, q = cache._stores[8], torch.randn(2, 8, 1, 128, generator=torch.Generator().manual_seed(2)).bfloat16().to(DEV)
+    floats = native.lib().tq_decode_scratch_floats(4, 4, 128, st.n_compressed, st.n_recent)
+    counters, want = torch.zeros(4, dtype=torch.int32, device=DEV), cache.attend(q, 8)
+    for start in (4, 5):
+        scratch, out = torch.full((floats + 16,), 7.0, device=DEV), torch.empty_like(q)
+        assert (scratch.data_ptr() + 4 * start) % 8 == 4 * (start % 2)
+        native.check(native.lib().tq_decode_attend(ctypes.addressof(st.record()), q.data_ptr(), 4, 128 ** -0.5, st.w0, st.n_recent, st.n_compressed, scratch.data_ptr() + 4 * start,
+                                                   floats, counters.data_ptr(), out.data_ptr(), native._stream_handle(q.device)), "tq_decode_attend")
+        assert torch.equal(out, want) and bool((scratch[:start] == 7).all()) and bool((scratch[start + floats:] == 7).all())
 
 
 @pytest.mark.parametrize("dim,tokens,window", [(64, 34000, 260), (96, 17000, 40), (128, 70000, 128), (256, 20000, 5)])

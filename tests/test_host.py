@@ -800,3 +800,15 @@ def test_extension_built_against_something_else_is_not_used(pkg, monkeypatch):
         with pytest.raises(native.TqError, match="build"):
             native.fast()
     assert native.fast() is native.fast()
+
+
+def test_decode_attend_counts_the_float_that_aligns_its_scratch(pkg):
+    """Records are written and exchanged between blocks 8 bytes at a time: scratch at an odd multiple of 4 loses its first float, which
+    tq_decode_scratch_floats includes.  (Nothing is launched: the scratch is always one float short.)"""
+    native = pkg._native
+    layer = native.TqDecodeLayer(4096, 4096, 4096, 4096, 4096, 4096, 4096, 4096, 4096, 1 << 20, 1024, 8, 128, native.TQ_BF16, 4, 2)
+    floats = native.lib().tq_decode_scratch_floats(8, 4, 128, 1000, 128)
+    assert floats % 2 == 1          # records are of 130 floats
+    attend = lambda scratch, size: native.lib().tq_decode_attend(ctypes.addressof(layer), 4096, 4, 1.0, 0, 128, 1000, scratch, size, 4096, 4096, None)  # noqa: E731
+    assert attend(4096 + 4, floats - 1) == native.ERR_CAPACITY and attend(4096, floats - 2) == native.ERR_CAPACITY
+    assert attend(4096 + 2, floats) == native.ERR_ALIGN

@@ -237,7 +237,7 @@ extern "C" int tq_decode_supported(int head_dim, int dtype, int bits_k, int bits
 
 extern "C" long long tq_decode_scratch_floats(long long rows, int group, int head_dim, long long tokens, long long n_win) {
     if (rows < 0 || rows > 65535 || group < 1 || group > MAX_GROUP || tokens < 0 || n_win < 0 || n_win > MAX_WINDOW) return TQ_ERR_SIZE;
-    return scratch_floats(rows, group, head_dim, decode_splits(rows, tokens), n_win);
+    return scratch_floats(rows, group, head_dim, decode_splits(rows, tokens), n_win) + 1;      // (see tq_decode_attend)
 }
 
 extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
@@ -255,6 +255,8 @@ extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *querie
     if (tokens > (layer->packed_row_stride ? layer->packed_row_stride : (rows == 1 ? tokens : 0))) return TQ_ERR_SIZE;
     if (((uintptr_t)queries & 15u) || ((uintptr_t)scratch & 3u) || ((uintptr_t)arrived & 3u) || ((uintptr_t)out & 1u)) return TQ_ERR_ALIGN;
     const int splits = decode_splits(rows, tokens);
+    // records are stored and exchanged between blocks in pairs of floats, 8 bytes at a time
+    if ((uintptr_t)scratch & 4u) { ++scratch; --scratch_size; }
     if (scratch_size < scratch_floats(rows, group, D, splits, n_win)) return TQ_ERR_CAPACITY;
     TqDecodeArgs a;
     a.queries = static_cast<const uint8_t *>(queries);
