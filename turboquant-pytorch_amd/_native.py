@@ -23,9 +23,11 @@ CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libtqamd.so")
 FAST_NAME = "tqamd_fastcall"        # extension module: the eager calls from tensors to the library in one step each
 FAST_SOURCE = "tq_fastcall.cpp"
-SOURCES = ("tq_host.cpp", "tq_compress.hip", "tq_decompress.hip", "tq_anydim.hip", "tq_wide.hip", "tq_attend.hip", "tq_qjl.hip", "tq_qjl_scores.hip",
-           "tq_decode.hip", "tq_decode_d64.hip", "tq_decode_d96.hip", "tq_decode_d128_narrow.hip", "tq_decode_d128_wide.hip", "tq_decode_d256.hip")
-HEADERS = ("tq_table.h", "tq_device.h", "tq_anydim.h", "tq_wide.h", "tq_lut.h", "tq_decode.h", "tq_decode_kernel.h", os.path.join("..", "..", "include", "tqamd.h"))
+# (the ones that take longest to compile first)
+SOURCES = ("tq_decode_d256.hip", "tq_decode_d96.hip", "tq_decode_d64.hip", "tq_decode_d128_narrow.hip", "tq_decode_d128_wide.hip", "tq_compress.hip", "tq_decompress.hip",
+           "tq_wide_d224.hip", "tq_wide_d192.hip", "tq_wide_d160.hip", "tq_wide_d96.hip", "tq_anydim.hip", "tq_attend.hip", "tq_qjl.hip",
+           "tq_qjl_scores.hip", "tq_decode.hip", "tq_wide.hip", "tq_host.cpp")
+HEADERS = ("tq_table.h", "tq_device.h", "tq_anydim.h", "tq_wide.h", "tq_wide_kernel.h", "tq_lut.h", "tq_decode.h", "tq_decode_kernel.h", os.path.join("..", "..", "include", "tqamd.h"))
 GPU_ARCH = "gfx950"
 
 TQ_F32, TQ_F16, TQ_BF16 = 0, 1, 2

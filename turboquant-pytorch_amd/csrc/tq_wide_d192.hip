@@ -1,0 +1,3 @@
+#include "tq_wide_kernel.h"
+
+TQ_WIDE_DEFINE(192)
