@@ -197,14 +197,16 @@ int tq_decompress_batched(const tq_job *jobs_host, const tq_job *jobs_dev, int n
                           int head_dim, void *workspace, void *stream);
 
 /*
- * Keys and values of one layer in one call.
- * tq_compress_layer: two tq_compress calls on tensors of one layout, into dense packed buffers.
+ * Keys and values of one layer in one call, where the kernels allow it (head_dim 128, 64 in pairs, 256 and 65-96, 129-224 in 16-bit elements)
+ * in one launch, in which both are worked on at the same time.
+ * tq_compress_layer: what two tq_compress calls do on tensors of one layout, into dense packed buffers.
  * tq_restore_layer: the full-length keys and values [batch, heads, tokens + n_win, head_dim] (dense) of a layer whose first `tokens`
  *   tokens are packed (packed_row_stride as for tq_decompress) and whose last n_win (0 or more) are kept as they are, in the
  *   output's element type: head h of sequence b of k_win / v_win starts at element b * win_batch_stride + h * win_head_stride,
  *   its tokens follow one another.  With a window, its addresses and strides, the outputs' and the rows' lengths in bytes are
  *   multiples of 16 (TQ_ERR_ALIGN otherwise); at most 65535 rows.
- * The workspace is that of tq_decompress, used by the launches of the call one after the other.
+ * The workspace is that of tq_decompress, tq_workspace_bytes(1) bytes: keys and values draw from a pair of counters each, in the two halves of
+ * it, so all of its bytes are zero before the call, not the first counters alone, and all are zero after it.
  */
 int tq_compress_layer(const void *keys, const void *values, int dtype, long long rows, long long tokens, long long row_stride, long long token_stride,
                       const void *table_k, const void *table_v, int head_dim, int bits_k, int bits_v, uint8_t *k_idx, uint16_t *k_norms,

@@ -316,12 +316,12 @@ struct WindowTile {
 //     each (WindowTile);
 //   * the waves' sums meet in LDS; with several splits per row the block that arrives last at the row's counter merges the
 //     records of all splits and of the window, rotates the value sums back and stores the result.
-// With few rows that is a chain of latencies, and what keeps it short (8 rows x 32768 tokens, K4/V2, 4 heads, 22 splits; clock stamps
-// of a launch before / after): all loads of the start issued at once in the order of their use, tables found without their header, queries
+// With few rows that is a chain of latencies, and what keeps it short (8 rows x 32768 tokens, K4/V2, 4 heads; clock stamps of a launch in 22
+// splits, which the rule of then took, before / after; it takes 32 now): all loads of the start issued at once in the order of their use, tables found without their header, queries
 // rotated by 4.2 / 2.5 us; the window's values loaded with its keys and its sums stored without a branch for each, 7.0 / 4.5; the block's
 // tokens dealt out evenly; records merged with one trip to memory and a code of a few hundred bytes (code that runs once is fetched from
 // the L2 as it goes: 1 us for 2.4 KiB of it), rows of Pi_v under way before the block knows that it needs them, last arrival to result 5.5 / 3.4.
-// Whole step of 32 layers 948 -> 778 us; 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
+// Whole step of 32 layers 948 -> 778 us (734 since the append asks for all of its loads at once, see tq_decode.hip); 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
 // The matrix products have 16 columns and a row of the cache seldom 16 query heads.  C blocks of 16 tokens share them (C = 4 for up to 4
 // heads, 2 for up to 8): every block's scores are computed for the heads repeated C times, a lane keeps those of its own column's
 // block, and the weights of the other blocks are zeros in its column of the value product.  The softmax of a token then costs 1 / C

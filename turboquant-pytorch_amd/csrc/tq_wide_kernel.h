@@ -52,7 +52,8 @@ enum Fit {
 };
 // CHUNKS for this job?  (The loads of ELEMENTS sit behind conditions, where the compiler waits for one before it writes the zeros of the
 // other lanes, so nothing is in flight while a tile is worked on: 32 rows x 5873 tokens at 80, 4-bit, keys and values, compress / decompress
-// 40 / 27 us that way, 31 / 23 us this way, 28.6 / 21.9 us with TqTileWalk instead of a division an address.)
+// 40 / 27 us that way, 31 / 23 us this way, 28.6 / 21.9 us with TqTileWalk instead of a division an address, 26.5 /
+// 21.1 us since that looks for whole tiles first.)
 __device__ __forceinline__ bool in_chunks(const TqDevJob &job, uint32_t dl, uint32_t packed_bytes) {
     return dl % 16u == 0u && (((uintptr_t)job.states | (uintptr_t)job.row_stride | (uintptr_t)job.token_stride) & 15u) == 0u &&
            ((uintptr_t)job.idx_bytes & (uintptr_t)(packed_bytes - 1u)) == 0u;
