@@ -356,3 +356,33 @@ def test_rows_that_end_at_every_place_of_a_tile(pkg, dim):
             comp.decompress_into(dense, want)
             assert torch.equal(out[:, :, 2:2 + tokens], want), (rows, tokens)
             assert bool((out[:, :, :2] == 7).all()) and bool((out[:, :, 2 + tokens:] == 7).all()), (rows, tokens)
+
+
+@pytest.mark.parametrize("bits,dtype", [(4, torch.bfloat16), (2, torch.float16), (8, torch.float32), (1, torch.bfloat16)])
+@pytest.mark.parametrize("rows,tokens", [((1, 1), 1), ((1, 1), 63), ((1, 1), 8191), ((1, 3), 63), ((1, 3), 65), ((2, 2), 127), ((2, 3), 2079)])
+def test_head_dim_64_rows_that_end_in_half_a_pair(pkg, bits, dtype, rows, tokens):
+    """De-quantising rows of an odd number of 64-wide vectors: bit for bit what rows of one vector more give, and nothing beyond the
+    last vector is written; packed rows at even and odd slots, the last one ending where the store ends, and whole layers with a window."""
+    D, G = 64, 64 // (8 // bits)
+    comp = pkg.MSECompressor(D, bits, seed=5, device=DEV)
+    x = outlier_kv(rows + (tokens + 1, D), seed=tokens + bits, dtype=dtype).to(DEV)
+    packed = comp.compress(x)
+    even = torch.empty(rows + (tokens + 1, D), dtype=dtype, device=DEV)
+    comp.decompress_packed(packed["idx_bytes"], packed["vec_norms"], even)
+    want = even[:, :, :tokens]
+    for cap in (tokens, tokens + 1, tokens + 2):
+        idx = torch.zeros(rows + (cap, G), dtype=torch.uint8, device=DEV)
+        nrm = torch.zeros(rows + (cap,), dtype=torch.float16, device=DEV)
+        idx[:, :, :tokens] = packed["idx_bytes"][:, :, :tokens]
+        nrm[:, :, :tokens] = packed["vec_norms"][:, :, :tokens]
+        out = torch.full(rows + (tokens + 2, D), 3.0, dtype=dtype, device=DEV)
+        comp.decompress_packed(idx[:, :, :tokens], nrm[:, :, :tokens], out[:, :, :tokens])
+        assert torch.equal(out[:, :, :tokens], want) and (out[:, :, tokens:] == 3.0).all(), cap
+        if cap > tokens:
+            for n_win in (0, 5):
+                win = torch.randn(rows + (n_win, D), device=DEV).to(dtype)
+                part = (idx[:, :, :tokens], nrm[:, :, :tokens])
+                got = pkg._native.restore_layer(part, part, tokens, comp.table(), comp.table(), bits, bits, win, win)
+                assert got is not None
+                for t in got:
+                    assert torch.equal(t[:, :, :tokens], want) and torch.equal(t[:, :, tokens:], win), (cap, n_win)

@@ -61,8 +61,8 @@ __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
 }
 
 // One block's share of a job; `counter`: the job's two counters, or NULL; lds: decompress_lds_bytes.
-template <int DTYPE, int IPB>
-__device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk, uint32_t *counter, uint32_t paired, uint8_t *lds, uint32_t (&tk)[3]) {
+template <int DTYPE, int IPB, bool PAIRED>
+__device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk, uint32_t *counter, uint8_t *lds, uint32_t (&tk)[3]) {
     using T = OutTraits<DTYPE>;
     constexpr int ELEM = T::ELEM;
     constexpr int VEC_BYTES = TQ_HEAD_DIM * ELEM;   // 256 or 512
@@ -72,9 +72,14 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     constexpr int VEC_PER_STORE = 64 / PIECES;
     constexpr int NB = 64 / IPB;                    // packed bytes per lane
     constexpr int NW = NB / 4;                      // dwords per lane: 2, 4, 8, 16
-
-    // paired: the job's vectors are 64 wide; two neighbours are one 128-wide row here (diag(Pi, Pi)^T from the table's pair
-    // section).  Lane half hk decodes and produces the second vector of the pair; only its norm is its own.
+    
+    // PAIRED: the job's vectors are 64 wide; two neighbours are one 128-wide row here (diag(Pi, Pi)^T from the table's pair
+    // section).  Lane half hk decodes and produces the second vector of the pair; only its norm is its own.  Packed slots count
+    // 64-wide vectors.  Where a row ends in half a pair (job.odd) its second half reads the first one again and is not stored.
+    // (Odd rows used to go through the kernel of any dimension, a launch each for keys, values and window: eight layers of a decode step
+    // of 8 rows of 18940 tokens, odd and even in turn, 188 -> 144 us.  Kernels of their own for pairs: with both kinds of rows in one,
+    // small launches of 128-wide vectors took 2 % longer.)
+    constexpr uint32_t VSHIFT = PAIRED ? 1u : 0u;
     uint8_t *out_base = const_cast<uint8_t *>(job.states);
 
     const uint32_t tid = threadIdx.x;
@@ -113,7 +118,7 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
         constexpr int NT = T::WAVES * TQ_WAVE;
         constexpr int A_TRIPS = TQ_OPERAND_BYTES / 16 / NT;
         static_assert(A_TRIPS * NT * 16 == TQ_OPERAND_BYTES, "whole trips");
-        const uint8_t *a_src = job.table + (paired ? hd->off_pair_at_f16 : hd->off_at_f16);
+        const uint8_t *a_src = job.table + (PAIRED ? hd->off_pair_at_f16 : hd->off_at_f16);
         tq_u4 v[A_TRIPS];
 #pragma unroll
         for (int k = 0; k < A_TRIPS; ++k) v[k] = tq_gload16(a_src + 16u * (tid + k * NT));
@@ -146,13 +151,12 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
         const uint32_t row = one_row ? 0u : v0 / job.tokens;
         const uint32_t tok = v0 - row * job.tokens;
         o.out_base = (long long)row * job.row_stride + (long long)tok * job.token_stride;
-        o.slot_base = one_row ? tok : row * job.packed_row_stride + tok;
-        o.in_row = one_row ? 32u : job.tokens - tok;
+        o.slot_base = row * job.packed_row_stride + (tok << VSHIFT);
+        o.in_row = job.tokens - tok;
         return o;
     };
     // jump of the output offset / packed slot from the last vector of a row to the first of the next
     const long long row_wrap = job.row_stride - (long long)job.tokens * job.token_stride;
-    const uint32_t slot_wrap = job.packed_row_stride - job.tokens;
     uint32_t st_off[NSTORE];   // byte offset of this lane's piece of store j relative to the tile's first vector
 #pragma unroll
     for (int j = 0; j < NSTORE; ++j) st_off[j] = (j * VEC_PER_STORE + st_vec) * (uint32_t)job.token_stride + st_piece * 16u;
@@ -160,19 +164,22 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     uint32_t raw[NW];
     uint16_t norm_bits = 0;
     // this lane's half vector of tile `tl` (FULL: all 32 vectors of the tile exist, nothing is predicated)
-    auto issue_loads = [&](auto full_tag, auto fast_tag, uint32_t tl) {
+    auto issue_loads = [&](auto full_tag, auto fast_tag, auto odd_tag, uint32_t tl) {
         constexpr bool FULL = decltype(full_tag)::value;
         constexpr bool FAST = decltype(fast_tag)::value;
+        constexpr bool ODD = decltype(odd_tag)::value;
         const bool ok = FULL || tl * 32u + n < job.n_vec;
         const uint32_t vl = ok ? n : 0u;
-        uint32_t slot;
+        uint32_t slot, half = hk;
         if constexpr (FAST) {
             const Origin o = origin_of(tl);
-            slot = o.slot_base + vl + (vl >= o.in_row ? slot_wrap : 0u);
+            slot = o.slot_base + (vl << VSHIFT) + (vl >= o.in_row ? job.packed_row_stride - (job.tokens << VSHIFT) : 0u);
+            if (ODD && vl + 1u == o.in_row) half = 0u;
         } else {   // rows shorter than a tile: the general formula
-            slot = tq_packed_slot(job, tl * 32u + vl);
+            const uint32_t row = (tl * 32u + vl) / job.tokens;
+            slot = row * job.packed_row_stride + ((tl * 32u + vl - row * job.tokens) << VSHIFT);
         }
-        const uint8_t *src = job.idx_bytes + (size_t)slot * (2 * NB) + hk * NB;
+        const uint8_t *src = job.idx_bytes + (size_t)slot * ((2 * NB) >> VSHIFT) + half * NB;
         if constexpr (NW == 2) {
             const tq_u2 t = tq_gload8(src);
             raw[0] = t[0]; raw[1] = t[1];
@@ -184,11 +191,11 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
                 for (int i = 0; i < 4; ++i) raw[4 * q + i] = t[i];
             }
         }
-        norm_bits = tq_gload2(job.vec_norms + (paired ? 2u * (size_t)slot + hk : (size_t)slot));
+        norm_bits = tq_gload2(job.vec_norms + (size_t)slot + (PAIRED ? half : 0u));
     };
 
     // one tile: decode + rotate + scale + transpose + store
-    auto process = [&](auto full_tag, auto fast_tag, uint32_t tl, const uint32_t (&cur)[NW], float nrm) {
+    auto process = [&](auto full_tag, auto fast_tag, auto odd_tag, uint32_t tl, const uint32_t (&cur)[NW], float nrm) {
         constexpr bool FULL = decltype(full_tag)::value;
         constexpr bool FAST = decltype(fast_tag)::value;
         // ---- x_hat[64h + 16t + r] = sum_j y[j] * Pi[j][.]   (un-scaled)
@@ -260,7 +267,8 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
 #pragma unroll
             for (int j = 0; j < NSTORE; ++j) {
                 const uint32_t vl = j * VEC_PER_STORE + st_vec;
-                if (FULL || tl * 32u + vl < job.n_vec)
+                const bool whole = !decltype(odd_tag)::value || vl + 1u != o.in_row || st_piece < (uint32_t)PIECES / 2u;
+                if ((FULL || tl * 32u + vl < job.n_vec) && whole)
                     tq_gstore16_stream(base + st_off[j] + (vl >= o.in_row ? row_wrap : 0ll), val[j]);
             }
         } else {
@@ -278,10 +286,10 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     // leaves the stores in flight (s_waitcnt vmcnt(#stores)) instead of draining them every iteration.
     // The loop runs once per ticket of the block, the same number of times in every wave (the barrier).
     const uint32_t n_full = job.n_vec / 32u;
-    auto run = [&](auto fast_tag) {
+    auto run = [&](auto fast_tag, auto odd_tag) {
         uint32_t cur[NW];
         float nrm = 0.f;
-        if (tile < n_full) issue_loads(std::true_type{}, fast_tag, tile);
+        if (tile < n_full) issue_loads(std::true_type{}, fast_tag, odd_tag, tile);
         stage_tables();
         if (tile < n_full) {
 #pragma unroll
@@ -295,9 +303,9 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
             const uint32_t nbase = tk[s_next];             // written before the previous barrier
             const uint32_t next = nbase + wave;
             if (tile < n_full) {
-                issue_loads(std::true_type{}, fast_tag, next < n_full ? next : tile);
+                issue_loads(std::true_type{}, fast_tag, odd_tag, next < n_full ? next : tile);
                 asm volatile("" ::: "memory");          // the prefetch stays ahead of the tile's work
-                process(std::true_type{}, fast_tag, tile, cur, nrm);
+                process(std::true_type{}, fast_tag, odd_tag, tile, cur, nrm);
                 // take the prefetched registers here, behind the stores: the wait for them then sits inside
                 // the loop body, where the number of younger stores is known
 #pragma unroll
@@ -309,11 +317,11 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
                 asm volatile("" : "+v"(nb));
                 nrm = half_bits_to_float((uint16_t)nb);
             } else if (tile == n_full && n_full < n_tiles) {   // the partial last tile of the job
-                issue_loads(std::false_type{}, fast_tag, tile);
+                issue_loads(std::false_type{}, fast_tag, odd_tag, tile);
                 uint32_t part[NW];
 #pragma unroll
                 for (int i = 0; i < NW; ++i) part[i] = raw[i];
-                process(std::false_type{}, fast_tag, tile, part, half_bits_to_float(norm_bits));
+                process(std::false_type{}, fast_tag, odd_tag, tile, part, half_bits_to_float(norm_bits));
             }
             if (tid == 0) tk[s_fresh] = fresh;             // last read two barriers ago (three slots, not two: the first
             __syncthreads();                               // ticket is read after a barrier that this write could overtake)
@@ -323,7 +331,9 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
             s_fresh = s_fresh == 2u ? 0u : s_fresh + 1u;
         }
     };
-    if (fast) run(std::true_type{}); else run(std::false_type{});
+    if (!fast) run(std::false_type{}, std::false_type{});
+    else if (PAIRED && job.odd) run(std::true_type{}, std::bool_constant<PAIRED>{});
+    else run(std::true_type{}, std::false_type{});
 
     // Every ticket this block drew has been answered (the values went through LDS) before it reports itself
     // done, so the block that finds all others done knows that nobody touches the counters again in this
@@ -337,29 +347,29 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     }
 }
 
-template <int DTYPE, int IPB>
-__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace, uint32_t paired) {
+template <int DTYPE, int IPB, bool PAIRED>
+__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tk[3];
-    const TqDevJob job = tq_pair_job(tq_load_job(job0, jobs, blockIdx.y, OutTraits<DTYPE>::ELEM), paired != 0u);
-    decompress_job<DTYPE, IPB>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr, paired, lds, tk);
+    const TqDevJob job = tq_pair_rows(tq_load_job(job0, jobs, blockIdx.y, OutTraits<DTYPE>::ELEM), PAIRED);
+    decompress_job<DTYPE, IPB, PAIRED>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr, lds, tk);
 }
 
 // keys and values of a layer and its window; the two jobs' counters share one job's record of the workspace
-template <int DTYPE>
-__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t *workspace, uint32_t paired) {
+template <int DTYPE, bool PAIRED>
+__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t *workspace) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tk[3];
     const uint32_t which = tq_layer_job(l);
-    const TqDevJob job = tq_pair_job(which ? l.job[1] : l.job[0], paired != 0u);
+    const TqDevJob job = tq_pair_rows(which ? l.job[1] : l.job[0], PAIRED);
     const TqBlock blk = tq_layer_block(l, which);
     uint32_t *counter = workspace ? workspace + which * (TQ_WORKSPACE_BYTES_PER_JOB / 8) : nullptr;
     tq_with_window(window, [&]() __attribute__((always_inline)) {
         switch (8 / (which ? l.bits[1] : l.bits[0])) {
-            case 8: decompress_job<DTYPE, 8>(job, blk, counter, paired, lds, tk); break;
-            case 4: decompress_job<DTYPE, 4>(job, blk, counter, paired, lds, tk); break;
-            case 2: decompress_job<DTYPE, 2>(job, blk, counter, paired, lds, tk); break;
-            default: decompress_job<DTYPE, 1>(job, blk, counter, paired, lds, tk); break;
+            case 8: decompress_job<DTYPE, 8, PAIRED>(job, blk, counter, lds, tk); break;
+            case 4: decompress_job<DTYPE, 4, PAIRED>(job, blk, counter, lds, tk); break;
+            case 2: decompress_job<DTYPE, 2, PAIRED>(job, blk, counter, lds, tk); break;
+            default: decompress_job<DTYPE, 1, PAIRED>(job, blk, counter, lds, tk); break;
         }
     });
 }
@@ -428,59 +438,59 @@ int allow_lds(const void *kernel, size_t lds, bool (&configured)[MAX_DEVICES]) {
     return 0;
 }
 
-template <int DTYPE, int IPB>
-int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *workspace, bool paired,
-                      hipStream_t stream) {
+template <int DTYPE, int IPB, bool PAIRED>
+int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *workspace, hipStream_t stream) {
     using T = OutTraits<DTYPE>;
     int cus = 0;
     int rc = device_cus(cus);
     if (rc) return rc;
     constexpr size_t lds = decompress_lds_bytes<DTYPE>();
     static bool configured[MAX_DEVICES] = {};
-    rc = allow_lds(reinterpret_cast<const void *>(&tq_decompress_kernel<DTYPE, IPB>), lds, configured);
+    rc = allow_lds(reinterpret_cast<const void *>(&tq_decompress_kernel<DTYPE, IPB, PAIRED>), lds, configured);
     if (rc) return rc;
     const uint32_t want = (max_tiles + T::WAVES - 1) / T::WAVES;
     const uint32_t bx = tq_blocks_per_job(want, cus, n_jobs);
     dim3 grid(bx, (unsigned)n_jobs, 1), block(T::WAVES * TQ_WAVE, 1, 1);
     // tickets pay off once every block has several to draw; below that the fixed assignment starts sooner
     uint32_t *counters = want >= 4u * bx ? static_cast<uint32_t *>(workspace) : nullptr;
-    hipLaunchKernelGGL((tq_decompress_kernel<DTYPE, IPB>), grid, block, lds, stream, job, jobs_dev, counters, paired ? 1u : 0u);
+    hipLaunchKernelGGL((tq_decompress_kernel<DTYPE, IPB, PAIRED>), grid, block, lds, stream, job, jobs_dev, counters);
     return (int)hipGetLastError();
 }
 
-template <int DTYPE>
-int launch_layer(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, void *workspace, bool paired, hipStream_t stream) {
+template <int DTYPE, bool PAIRED>
+int launch_layer(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, void *workspace, hipStream_t stream) {
     using T = OutTraits<DTYPE>;
     int cus = 0;
     int rc = device_cus(cus);
     if (rc) return rc;
     constexpr size_t lds = decompress_lds_bytes<DTYPE>();
     static bool configured[MAX_DEVICES] = {};
-    rc = allow_lds(reinterpret_cast<const void *>(&tq_restore_layer_kernel<DTYPE>), lds, configured);
+    rc = allow_lds(reinterpret_cast<const void *>(&tq_restore_layer_kernel<DTYPE, PAIRED>), lds, configured);
     if (rc) return rc;
     const uint32_t want = (tiles + T::WAVES - 1) / T::WAVES;
     const uint32_t blocks = tq_layer_blocks(l, want, (uint32_t)cus, cost_k, cost_v);
     uint32_t *counters = 2u * want >= 4u * blocks ? static_cast<uint32_t *>(workspace) : nullptr;      // as in launch_decompress
-    hipLaunchKernelGGL((tq_restore_layer_kernel<DTYPE>), dim3(blocks), dim3(T::WAVES * TQ_WAVE), lds, stream, l, window, counters, paired ? 1u : 0u);
+    hipLaunchKernelGGL((tq_restore_layer_kernel<DTYPE, PAIRED>), dim3(blocks), dim3(T::WAVES * TQ_WAVE), lds, stream, l, window, counters);
     return (int)hipGetLastError();
 }
 
-template <int DTYPE>
-int dispatch_bits(int bits, const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *ws, bool paired, hipStream_t s) {
+template <int DTYPE, bool PAIRED>
+int dispatch_bits(int bits, const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *ws, hipStream_t s) {
     switch (8 / bits) {
-        case 8: return launch_decompress<DTYPE, 8>(job, jobs_dev, n_jobs, max_tiles, ws, paired, s);
-        case 4: return launch_decompress<DTYPE, 4>(job, jobs_dev, n_jobs, max_tiles, ws, paired, s);
-        case 2: return launch_decompress<DTYPE, 2>(job, jobs_dev, n_jobs, max_tiles, ws, paired, s);
-        case 1: return launch_decompress<DTYPE, 1>(job, jobs_dev, n_jobs, max_tiles, ws, paired, s);
+        case 8: return launch_decompress<DTYPE, 8, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case 4: return launch_decompress<DTYPE, 4, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case 2: return launch_decompress<DTYPE, 2, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case 1: return launch_decompress<DTYPE, 1, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
         default: return TQ_ERR_BITS;
     }
 }
 
-int dispatch(int dtype, int bits, const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *ws, bool paired, hipStream_t s) {
+template <bool PAIRED>
+int dispatch(int dtype, int bits, const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *ws, hipStream_t s) {
     switch (dtype) {
-        case TQ_F32: return dispatch_bits<TQ_F32>(bits, job, jobs_dev, n_jobs, max_tiles, ws, paired, s);
-        case TQ_F16: return dispatch_bits<TQ_F16>(bits, job, jobs_dev, n_jobs, max_tiles, ws, paired, s);
-        case TQ_BF16: return dispatch_bits<TQ_BF16>(bits, job, jobs_dev, n_jobs, max_tiles, ws, paired, s);
+        case TQ_F32: return dispatch_bits<TQ_F32, PAIRED>(bits, job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case TQ_F16: return dispatch_bits<TQ_F16, PAIRED>(bits, job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case TQ_BF16: return dispatch_bits<TQ_BF16, PAIRED>(bits, job, jobs_dev, n_jobs, max_tiles, ws, s);
         default: return TQ_ERR_DTYPE;
     }
 }
@@ -531,11 +541,11 @@ extern "C" int tq_decompress(const uint8_t *idx_bytes, const uint16_t *vec_norms
     job.packed_row_stride = (uint32_t)(packed_row_stride ? packed_row_stride : tokens);
     job.row_stride = row_stride * elem_bytes(out_dtype);
     job.token_stride = token_stride * elem_bytes(out_dtype);
-    if (head_dim == TQ_HEAD_DIM / 2 && tq_pairable(rows, tokens, token_stride, packed_row_stride, head_dim, idx_bytes))
-        return dispatch(out_dtype, bits, job, nullptr, 1, (uint32_t)((n_vec / 2 + 31) / 32), workspace, true, static_cast<hipStream_t>(stream));
+    if (tq_pairable_rows(rows, tokens, token_stride, head_dim, idx_bytes))
+        return dispatch<true>(out_dtype, bits, job, nullptr, 1, (uint32_t)((tq_pairs(rows, tokens) + 31) / 32), workspace, static_cast<hipStream_t>(stream));
     if (head_dim != TQ_HEAD_DIM)     // the run-time-dimension kernel assigns its tiles statically: no counters
         return tq_anydim_decompress(out_dtype, bits, head_dim, job, nullptr, 1, (uint32_t)n_vec, static_cast<hipStream_t>(stream));
-    return dispatch(out_dtype, bits, job, nullptr, 1, (uint32_t)((n_vec + 31) / 32), workspace, false, static_cast<hipStream_t>(stream));
+    return dispatch<false>(out_dtype, bits, job, nullptr, 1, (uint32_t)((n_vec + 31) / 32), workspace, static_cast<hipStream_t>(stream));
 }
 
 namespace {
@@ -574,7 +584,7 @@ extern "C" int tq_restore_layer(const uint8_t *k_idx, const uint16_t *k_norms, c
     if (!rc) rc = check_job(v_out, dtype, r, t, rs, head_dim, table_v, head_dim, bits_v, v_idx, v_norms, packed_row_stride, &n_vec);
     if (rc) return rc;
     if ((uintptr_t)workspace & 63u) return TQ_ERR_ALIGN;
-    const bool paired = tq_pairable(r, t, head_dim, packed_row_stride, head_dim, k_idx) && tq_pairable(r, t, head_dim, packed_row_stride, head_dim, v_idx);
+    const bool paired = tq_pairable_rows(r, t, head_dim, head_dim, k_idx) && tq_pairable_rows(r, t, head_dim, head_dim, v_idx);
     const long long off = tokens * head_dim * elem;
     if ((head_dim == TQ_HEAD_DIM || paired || tq_anydim_layer_supported(head_dim, dtype)) && 2 * rows * (run / 16) < 0xffffffffll) {
         TqLayer l{};
@@ -607,11 +617,15 @@ extern "C" int tq_restore_layer(const uint8_t *k_idx, const uint16_t *k_norms, c
         const uint32_t cost_k = (uint32_t)tq_vector_bytes(head_dim, (int)elem, bits_k), cost_v = (uint32_t)tq_vector_bytes(head_dim, (int)elem, bits_v);
         const hipStream_t s = static_cast<hipStream_t>(stream);
         if (head_dim != TQ_HEAD_DIM && !paired) return tq_anydim_restore_layer(dtype, head_dim, l, w, (uint32_t)n_vec, cost_k, cost_v, s);
-        const uint32_t tiles = (uint32_t)(((paired ? n_vec / 2 : n_vec) + 31) / 32);
+        const uint32_t tiles = (uint32_t)(((paired ? tq_pairs(r, t) : n_vec) + 31) / 32);
+        auto launch = [&](auto type_tag) {
+            constexpr int T = decltype(type_tag)::value;
+            return paired ? launch_layer<T, true>(l, w, tiles, cost_k, cost_v, workspace, s) : launch_layer<T, false>(l, w, tiles, cost_k, cost_v, workspace, s);
+        };
         switch (dtype) {
-            case TQ_F32: return launch_layer<TQ_F32>(l, w, tiles, cost_k, cost_v, workspace, paired, s);
-            case TQ_F16: return launch_layer<TQ_F16>(l, w, tiles, cost_k, cost_v, workspace, paired, s);
-            default: return launch_layer<TQ_BF16>(l, w, tiles, cost_k, cost_v, workspace, paired, s);
+            case TQ_F32: return launch(std::integral_constant<int, TQ_F32>{});
+            case TQ_F16: return launch(std::integral_constant<int, TQ_F16>{});
+            default: return launch(std::integral_constant<int, TQ_BF16>{});
         }
     }
     rc = tq_decompress(k_idx, k_norms, packed_row_stride, r, t, table_k, head_dim, bits_k, k_out, dtype, rs, head_dim, workspace, stream);
@@ -633,9 +647,10 @@ extern "C" long long tq_workspace_bytes(int n_jobs) {
 }
 
 namespace {
-// Argument checks of a batch; max_vec = vectors of its largest job (0: nothing to launch).
+// Argument checks of a batch; max_vec = vectors (paired: pairs) of its largest job (0: nothing to launch).
 int check_batch(const tq_job *jobs_host, int n_jobs, int head_dim, long long *max_vec, bool *paired) {
     *max_vec = 0;
+    long long max_pairs = 0;
     *paired = head_dim == TQ_HEAD_DIM / 2;       // 64-wide vectors in pairs, if every job of the launch allows it
     for (int i = 0; i < n_jobs; ++i) {
         const tq_job &j = jobs_host[i];
@@ -647,8 +662,10 @@ int check_batch(const tq_job *jobs_host, int n_jobs, int head_dim, long long *ma
                                  head_dim, j.bits, j.idx_bytes, j.vec_norms, j.packed_row_stride, &n_vec);
         if (rc) return rc;
         if (n_vec > *max_vec) *max_vec = n_vec;
-        if (n_vec && !tq_pairable(j.rows, j.tokens, j.token_stride, j.packed_row_stride, head_dim, j.idx_bytes)) *paired = false;
+        if (n_vec && tq_pairs(j.rows, j.tokens) > max_pairs) max_pairs = tq_pairs(j.rows, j.tokens);
+        if (n_vec && !tq_pairable_rows(j.rows, j.tokens, j.token_stride, head_dim, j.idx_bytes)) *paired = false;
     }
+    if (*paired) *max_vec = max_pairs;
     return TQ_OK;
 }
 
@@ -656,13 +673,13 @@ int launch_batch(const tq_job *jobs_host, const tq_job *jobs_dev, int n_jobs, in
                  void *workspace, void *stream) {
     TqDevJob none{};
     if (paired)
-        return dispatch(jobs_host[0].dtype, jobs_host[0].bits, none, jobs_dev, n_jobs, (uint32_t)((max_vec / 2 + 31) / 32),
-                        workspace, true, static_cast<hipStream_t>(stream));
+        return dispatch<true>(jobs_host[0].dtype, jobs_host[0].bits, none, jobs_dev, n_jobs, (uint32_t)((max_vec + 31) / 32),
+                        workspace, static_cast<hipStream_t>(stream));
     if (head_dim != TQ_HEAD_DIM)
         return tq_anydim_decompress(jobs_host[0].dtype, jobs_host[0].bits, head_dim, none, jobs_dev, n_jobs, (uint32_t)max_vec,
                                     static_cast<hipStream_t>(stream));
-    return dispatch(jobs_host[0].dtype, jobs_host[0].bits, none, jobs_dev, n_jobs, (uint32_t)((max_vec + 31) / 32),
-                    workspace, false, static_cast<hipStream_t>(stream));
+    return dispatch<false>(jobs_host[0].dtype, jobs_host[0].bits, none, jobs_dev, n_jobs, (uint32_t)((max_vec + 31) / 32),
+                    workspace, static_cast<hipStream_t>(stream));
 }
 }  // namespace
 

@@ -30,6 +30,7 @@ struct TqDevJob {
     uint32_t packed_row_stride;  // packed slots per row (>= tokens)
     long long row_stride;    // bytes
     long long token_stride;  // bytes
+    uint32_t odd = 0;        // rows of pairs whose last pair has no second vector (tq_pair_rows)
 };
 
 __device__ __forceinline__ TqDevJob tq_load_job(const TqDevJob &single, const tq_job *jobs, uint32_t index, int elem_bytes) {
@@ -145,6 +146,19 @@ __device__ __forceinline__ TqDevJob tq_uniform_job(const TqDevJob &j) {
     u.row_stride = (long long)tq_uniform64((uint64_t)j.row_stride);
     u.token_stride = (long long)tq_uniform64((uint64_t)j.token_stride);
     return u;
+}
+
+// tq_pair_job for the kernels that de-quantise, which take any number of tokens a row: the last pair of an odd one has no second vector
+// (job.odd), and packed slots stay those of 64-wide vectors (a row may start at an odd one).
+__device__ __forceinline__ TqDevJob tq_pair_rows(TqDevJob j, bool paired) {
+    if (paired && j.n_vec) {
+        const uint32_t rows = tq_uniform32(j.n_vec / j.tokens);      // (a division is vector work: what follows from it stays scalar this way)
+        j.odd = j.tokens & 1u;
+        j.tokens = (j.tokens + 1u) >> 1;
+        j.n_vec = rows * j.tokens;
+        j.token_stride <<= 1;
+    }
+    return j;
 }
 
 // Byte offset of vector v inside `states`.
@@ -480,6 +494,14 @@ static inline bool tq_pairable(long long rows, long long tokens, long long token
     return head_dim == TQ_HEAD_DIM / 2 && tokens > 0 && (tokens & 1) == 0 && token_stride == head_dim && (packed_row_stride & 1) == 0 &&
            ((uintptr_t)idx_bytes & 15u) == 0;      // (the 128-wide kernels move packed bytes 16 at a time)
 }
+
+// For de-quantising, rows of any length: the last pair of an odd row is half a pair (tq_pair_rows).  Rows of fewer than 32 pairs may
+// end several times in a tile, which the kernel follows for whole pairs only.
+static inline bool tq_pairable_rows(long long rows, long long tokens, long long token_stride, int head_dim, const void *idx_bytes) {
+    return head_dim == TQ_HEAD_DIM / 2 && tokens > 0 && token_stride == head_dim && ((uintptr_t)idx_bytes & 15u) == 0 &&
+           ((tokens & 1) == 0 || rows == 1 || tokens >= 63);
+}
+static inline long long tq_pairs(long long rows, long long tokens) { return rows * ((tokens + 1) / 2); }
 
 // Alignment the packed codes need: 16 bytes for the 128-wide kernels; the kernels of the other head dimensions move them
 // in pieces no larger than the largest power of two that divides a vector's packed bytes (a token slice of a store of
