@@ -230,3 +230,19 @@ def test_v2_scores_of_few_queries_equal_those_of_many(pkg, bits, dtype):
             assert few.shape == (1, rows, n, tokens)
             err = float(((few.double() - many[:, :, :n].double()).abs() / scale[:, :, :n]).max())
             assert err < 3e-5, (rows, tokens, n, err)
+
+
+@pytest.mark.parametrize("bits,dtype", [(3, torch.bfloat16), (2, torch.float16), (5, torch.bfloat16), (4, torch.float16)])
+@pytest.mark.parametrize("n", [32, 33, 63, 64, 65, 2047, 20001])
+def test_v2_keys_of_any_number_do_not_depend_on_their_tile(pkg, bits, dtype, n):
+    """The last tile of a ragged job starts at the 32nd vector from its end: the same bytes as those vectors compressed alone, and the
+    vectors before them as in a job of whole tiles."""
+    comp = pkg.TurboQuantCompressorV2(128, bits, seed=42, device=DEV)
+    x = torch.randn((1, 1, n, 128), generator=torch.Generator().manual_seed(n)).to(dtype).to(DEV)
+    whole = comp.compress(x)
+    for part in (slice(n - 32, n), slice(0, n // 32 * 32)):
+        alone = comp.compress(x[:, :, part].contiguous())
+        for key, value in alone.items():
+            if torch.is_tensor(value):
+                got = whole[key].reshape(n, -1)[part]
+                assert torch.equal(got, value.reshape(got.shape)), (key, part)
