@@ -449,7 +449,7 @@ __global__ __launch_bounds__(MAX_WAVES *TQ_WAVE, 2) void tq_anydim_decompress_ke
 }
 
 // ====================================================================================================================
-// Head dimension 256 with 16-bit elements: the rotation resident in registers, as in the 128-wide kernels.
+// Head dimension 256 (compress: 16-bit elements): the rotation resident in registers, as in the 128-wide kernels.
 //
 // compress: a block is eight waves that share tiles of 32 vectors (16 KiB); wave w keeps the 32 rows [32w, 32w+32) of
 // Pi as MFMA A operands for all 16 steps of the contraction, two 16-bit terms (128 registers).  A tile is fetched with
@@ -629,12 +629,14 @@ __global__ __launch_bounds__(512, 1) void tq_d256_compress_layer_kernel(TqLayer 
 // operands for all 16 steps (the leading fp16 term: 128 registers).  The packed bytes of a tile are fetched one tile
 // ahead (every thread the bytes of 32 codes), turned into fp16 centroids through the byte -> centroids table and parked
 // in a double-buffered swizzled LDS tile that all four waves read as B operands; the scaled, rounded results go through
-// a second LDS tile so that the stores are 512 contiguous bytes per vector.
+// a second LDS tile so that the stores are 512 (float32: 1024) contiguous bytes per vector.  float32 outputs (what
+// MSECompressor.decompress returns) went through the kernel of any dimension, whose lanes store 16 bytes of 32 vectors at a time:
+// compress and restore of 231912 bf16 vectors, 4-bit, 174 -> 123 us (restore 119 -> 45); of 8000 25.3 -> 13.0.
 template <int DTYPE, int IPB>
 __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock blk, uint8_t *lds) {
-    static_assert(DTYPE == TQ_F16 || DTYPE == TQ_BF16, "16-bit outputs");
-    constexpr int D = 256, STEPS = D / 16;
+    constexpr int D = 256, STEPS = D / 16, ELEM = DTYPE == TQ_F32 ? 4 : 2;
     constexpr int TILE_BYTES = 32 * D * 2;
+    constexpr uint32_t VEC_BYTES = D * ELEM, PIECES = VEC_BYTES / 16, VEC_PER_STORE = 256u / PIECES;     // of the output
     constexpr int ENTRY = 2 * IPB;                 // bytes of a table entry: the fp16 centroids of one packed byte
     constexpr int RAW = 32 / IPB;                  // packed bytes of a thread's 32 codes: 4, 8, 16, 32
     constexpr int RW = RAW / 4;                    // as dwords
@@ -642,7 +644,7 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
     uint8_t *lds_lut = lds;
     uint8_t (*lds_y)[TILE_BYTES] = reinterpret_cast<uint8_t (*)[TILE_BYTES]>(lds + 4096);
     uint8_t *lds_out = lds + 4096 + 2 * TILE_BYTES;
-    float (*lds_norm)[32] = reinterpret_cast<float (*)[32]>(lds + 4096 + 3 * TILE_BYTES);       // [2][32]
+    float (*lds_norm)[32] = reinterpret_cast<float (*)[32]>(lds_out + 32 * VEC_BYTES);       // [2][32]
 
     uint8_t *out_base = const_cast<uint8_t *>(job.states);
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -721,7 +723,7 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
     const uint32_t op_base = n * (D * 2) + (((hk << 3) ^ (n & 31u)) << 4);
     auto op_step = [](int s) { return (uint32_t)((((2 * (s & 1)) << 3) | (s >> 1)) << 4); };
 
-    const long long st_own = (long long)(tid >> 5) * job.token_stride + (tid & 31u) * 16u;      // of the stores below
+    const long long st_own = (long long)(tid / PIECES) * job.token_stride + (tid % PIECES) * 16u;      // of the stores below
     const uint32_t m = (n_tiles - blk.x + blk.grid - 1u) / blk.grid;
     decode(0u);
     for (uint32_t j = 0; j < m; ++j) {
@@ -738,33 +740,37 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
             acc[0] = mfma_f16(areg[0][s], b, acc[0]);
             acc[1] = mfma_f16(areg[1][s], b, acc[1]);
         }
-        // lane (n, hk) holds elements 32 t + 16 hk + r of vector n for its row tiles t = 2w, 2w + 1: pieces 4 t + 2 hk + c
+        // lane (n, hk) holds elements 32 t + 16 hk + r of vector n for its row tiles t = 2w, 2w + 1: ELEM consecutive pieces of 16 bytes
         const float nrm = lds_norm[j & 1u][n];
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
+            for (int c = 0; c < ELEM; ++c) {
                 tq_u4 o;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float x0 = acc[t][8 * c + 2 * e] * nrm, x1 = acc[t][8 * c + 2 * e + 1] * nrm;
-                    if constexpr (DTYPE == TQ_F16) {
-                        const tq_half2 hh = {(_Float16)x0, (_Float16)x1};
-                        o[e] = __builtin_bit_cast(uint32_t, hh);
+                    if constexpr (DTYPE == TQ_F32) {
+                        o[e] = __float_as_uint(acc[t][4 * c + e] * nrm);
                     } else {
-                        const tq_bf2 hh = {(__bf16)x0, (__bf16)x1};
-                        o[e] = __builtin_bit_cast(uint32_t, hh);
+                        const float x0 = acc[t][8 * c + 2 * e] * nrm, x1 = acc[t][8 * c + 2 * e + 1] * nrm;
+                        if constexpr (DTYPE == TQ_F16) {
+                            const tq_half2 hh = {(_Float16)x0, (_Float16)x1};
+                            o[e] = __builtin_bit_cast(uint32_t, hh);
+                        } else {
+                            const tq_bf2 hh = {(__bf16)x0, (__bf16)x1};
+                            o[e] = __builtin_bit_cast(uint32_t, hh);
+                        }
                     }
                 }
-                const uint32_t piece = 4u * (2u * wave + t) + 2u * hk + c;
-                *reinterpret_cast<tq_u4 *>(lds_out + n * (D * 2) + ((piece ^ (n & 31u)) << 4)) = o;
+                const uint32_t piece = (2u * (2u * wave + t) + hk) * ELEM + c;
+                *reinterpret_cast<tq_u4 *>(lds_out + n * VEC_BYTES + ((piece ^ (n & 31u)) << 4)) = o;
             }
         __syncthreads();        // the output tile is complete
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {       // 1024 pieces, 256 threads: piece i % 32 of vector i / 32, 512 contiguous bytes per vector
-            const uint32_t i = k * 256u + tid, vl = i >> 5, p = i & 31u;
-            const tq_u4 val = *reinterpret_cast<const tq_u4 *>(lds_out + vl * (D * 2) + ((p ^ (vl & 31u)) << 4));
-            if (here.v + vl < job.n_vec) tq_gstore16_stream(out_base + here.offset(job, vl, st_own + 8ll * k * job.token_stride), val);
+        for (uint32_t k = 0; k < 32u / VEC_PER_STORE; ++k) {       // 256 threads: piece i % PIECES of vector i / PIECES
+            const uint32_t vl = k * VEC_PER_STORE + tid / PIECES, p = tid % PIECES;
+            const tq_u4 val = *reinterpret_cast<const tq_u4 *>(lds_out + vl * VEC_BYTES + ((p ^ (vl & 31u)) << 4));
+            if (here.v + vl < job.n_vec) tq_gstore16_stream(out_base + here.offset(job, vl, st_own + (long long)(VEC_PER_STORE * k) * job.token_stride), val);
         }
         here.next(job);
         if (j + 1u < m) decode((j + 1u) & 1u);
@@ -774,7 +780,7 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
 template <int DTYPE, int IPB>
 __global__ __launch_bounds__(256, 2) void tq_d256_decompress_kernel(TqDevJob job0, const tq_job *jobs) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    d256_decompress_job<DTYPE, IPB>(tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, 2)), TqBlock{blockIdx.x, gridDim.x}, lds);
+    d256_decompress_job<DTYPE, IPB>(tq_uniform_job(tq_load_job(job0, jobs, blockIdx.y, DTYPE == TQ_F32 ? 4 : 2)), TqBlock{blockIdx.x, gridDim.x}, lds);
 }
 
 // keys and values of a layer and its window
@@ -846,7 +852,8 @@ int launch(K kernel, uint32_t (&raised)[MAX_DEVICES], L lds_for, uint32_t nt_max
 
 // 256-wide kernels: threads per block, blocks per compute unit, bytes of dynamic LDS
 struct D256Compress { static constexpr uint32_t THREADS = 512, RESIDENT = 1, LDS = TQ_GRID_LDS_BYTES + 2u * 32u * 256u * 2u + 3u * 32u * 4u; };
-struct D256Decompress { static constexpr uint32_t THREADS = 256, RESIDENT = 2, LDS = 4096u + 3u * 32u * 256u * 2u + 2u * 32u * 4u; };
+template <int DTYPE>
+struct D256Decompress { static constexpr uint32_t THREADS = 256, RESIDENT = 2, LDS = 4096u + (2u * 2u + (DTYPE == TQ_F32 ? 4u : 2u)) * 32u * 256u + 2u * 32u * 4u; };
 
 // Blocks the current device holds at once; raises the kernel's LDS limit, once per device (`raised` is the kernel's own).
 template <typename S, typename K>
@@ -886,10 +893,10 @@ template <int DTYPE>
 int launch_d256_restore_layer(TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
     static bool raised[MAX_DEVICES] = {};
     int slots = 0;
-    const int rc = d256_slots<D256Decompress>(&tq_d256_restore_layer_kernel<DTYPE>, raised, slots);
+    const int rc = d256_slots<D256Decompress<DTYPE>>(&tq_d256_restore_layer_kernel<DTYPE>, raised, slots);
     if (rc) return rc;
     const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)slots, cost_k, cost_v);
-    hipLaunchKernelGGL((tq_d256_restore_layer_kernel<DTYPE>), dim3(blocks), dim3(D256Decompress::THREADS), D256Decompress::LDS, stream, l, w);
+    hipLaunchKernelGGL((tq_d256_restore_layer_kernel<DTYPE>), dim3(blocks), dim3(D256Decompress<DTYPE>::THREADS), D256Decompress<DTYPE>::LDS, stream, l, w);
     return (int)hipGetLastError();
 }
 
@@ -926,11 +933,9 @@ int compress_bits(int bits, const TqDevJob &job, const tq_job *jobs_dev, int n_j
 
 template <int DTYPE, int IPB>
 int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_vec, uint32_t d, hipStream_t s) {
-    if constexpr (DTYPE != TQ_F32) {
-        if (d == 256u) {
-            static bool raised256[MAX_DEVICES] = {};
-            return launch_d256<D256Decompress>(&tq_d256_decompress_kernel<DTYPE, IPB>, raised256, job, jobs_dev, n_jobs, max_vec, s);
-        }
+    if (d == 256u) {
+        static bool raised256[MAX_DEVICES] = {};
+        return launch_d256<D256Decompress<DTYPE>>(&tq_d256_decompress_kernel<DTYPE, IPB>, raised256, job, jobs_dev, n_jobs, max_vec, s);
     }
     const uint32_t dp = TQ_PADDED_DIM(d);
     if (dp != d) {
