@@ -870,6 +870,22 @@ def test_decode_attention_merges_many_splits(pkg, dim, tokens, window):
         assert err < (1.5e-3 if dim == 128 else 3.5e-4), (group, err)
 
 
+@pytest.mark.parametrize("dim,bits", [(64, (6, 4)), (96, (4, 2)), (128, (4, 2)), (256, (8, 4)), (256, (4, 2))])
+@pytest.mark.parametrize("rows,tokens,window", [(1, 200, 128), (2, 400, 33), (1, 700, 512), (3, 1500, 128), (1, 6000, 128), (1, 9000, 128), (40, 1300, 100), (300, 70, 128)])
+def test_decode_attention_deals_out_window_and_history(pkg, dim, bits, rows, tokens, window):
+    """Tiles of the window against splits of the history: fewer, as many and more of them, splits with and without a tile, groups on both
+    sides of what is merged in one go, against float64 over the store as the kernel holds it.  Bounds as in test_decode_attention_merges_many_splits."""
+    g = torch.Generator().manual_seed(dim + tokens)
+    cache = pkg.V3Cache(bits[0], bits[1], residual_window=window, n_layers=40)
+    k, v = (torch.randn(1, rows, tokens + window, dim, generator=g).half().to(DEV) for _ in range(2))
+    cache.append(k, v, 8)
+    for group in (1, 4, 7, 16):
+        q = 2 * torch.randn(1, rows * group, 1, dim, generator=g).half().to(DEV)
+        ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
+        err = float((cache.attend(q, 8).double().reshape(ref.shape) - ref).norm() / ref.norm())
+        assert err < (1.5e-3 if dim == 128 else 3.5e-4), (group, err)
+
+
 @pytest.mark.parametrize("dim", [64, 96, 128, 256])
 @pytest.mark.parametrize("bits", [(4, 2), (8, 3), (6, 4)])
 def test_one_launch_append_stores_the_bytes_of_compress(pkg, dim, bits):

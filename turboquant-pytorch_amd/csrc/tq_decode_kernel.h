@@ -321,7 +321,11 @@ struct WindowTile {
 // rotated by 4.2 / 2.5 us; the window's values loaded with its keys and its sums stored without a branch for each, 7.0 / 4.5; the block's
 // tokens dealt out evenly; records merged with one trip to memory and a code of a few hundred bytes (code that runs once is fetched from
 // the L2 as it goes: 1 us for 2.4 KiB of it), rows of Pi_v under way before the block knows that it needs them, last arrival to result 5.5 / 3.4.
-// Whole step of 32 layers 948 -> 778 us (734 since the append asks for all of its loads at once, see tq_decode.hip); 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
+// A tile of the window used to stand before the block's barrier: everybody in it waited 2.3 us (256 wide 4.4) for the wave that had it, and the row for the
+// block.  It is finished behind the barrier now, and its block takes 64 tokens less (see tq_decode_attend); records are merged without loops around their
+// loads.  us a step of eight layers, append and attend: 8 rows x 32768 tokens 170 -> 164; 64 wide, 32 x 6000, K6/V4 146 -> 130; 96 wide, 2 x 8574
+// 130 -> 118; 256 wide, 8 x 9906, K3/V2 291 -> 262; 512 x 16384 1366 -> 1354.
+// Before that, whole step of 32 layers 948 -> 778 us (734 since the append asks for all of its loads at once, see tq_decode.hip); 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
 // The matrix products have 16 columns and a row of the cache seldom 16 query heads.  C blocks of 16 tokens share them (C = 4 for up to 4
 // heads, 2 for up to 8): every block's scores are computed for the heads repeated C times, a lane keeps those of its own column's
 // block, and the weights of the other blocks are zeros in its column of the value product.  The softmax of a token then costs 1 / C
@@ -364,7 +368,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     constexpr int QROW = D + 4;                          // rotated queries in LDS, floats per head
     constexpr int ROTP = DTHREADS / (D / 4) >= 16 ? 16 : DTHREADS / (D / 4);     // parts of the contraction when rotating back
     constexpr int ROTK = D / ROTP;                       // rows of Pi_v per part
-    constexpr int RG = C == 4 ? 4 : 8;                   // heads rotated back at a time
+    constexpr int RG = 4;                                // heads rotated back at a time (8: twice the work where a row has 4, at 256 3.4 us for 2.0)
     static_assert(DW * AREA >= 2 * MAX_GROUP * D * 4 && ROTP * RG * D * 4 <= 65536, "LDS areas too small");
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds_lut[65536];      // (the strictest alignment: lies at address 0, where no base has to be added)
@@ -386,8 +390,10 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     const uint32_t head = n16 % HEADS, cls = n16 / HEADS;
     const bool live = head < G;
 
-    const uint32_t t_begin = min(a.tokens, split * a.chunk);
-    const uint32_t t_end = min(a.tokens, t_begin + a.chunk);
+    const uint32_t win_tiles = (a.n_win + WIN_TILE - 1u) / WIN_TILE;     // tile w goes to the block of split w % splits
+    // (a split that has a tile of the window takes win_cost tokens less, see tq_decode_attend)
+    const uint32_t t_begin = min(a.tokens, split * a.chunk - min(split, win_tiles) * a.win_cost);
+    const uint32_t t_end = min(a.tokens, (split + 1u) * a.chunk - min(split + 1u, win_tiles) * a.win_cost);
     const size_t slot0 = (size_t)row * a.packed_row_stride;
     uint8_t *vcodes = lds_area[wave];
     // Runs of a wave: in every whole round of the block one of RUN tokens; what is left of the block's tokens is dealt out evenly, in
@@ -457,7 +463,6 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     // ---- start: loads in the order in which their data is used, nothing waits for what it does not need.  Tables, then the operands of
     // the query rotation (the first waves) or a tile of the window (from the last wave down), then the first run; a wave that has no run
     // reads the row's first token (of a row without history, what the host put there instead).
-    const uint32_t win_tiles = (a.n_win + WIN_TILE - 1u) / WIN_TILE;     // tile w goes to the block of split w % splits
     uint32_t wt = DW - 1u - wave;
     TQ_GLOBAL float *wrec = (TQ_GLOBAL float *)a.win_part + (size_t)row * win_tiles * G * PART;
     if (tid < (uint32_t)DW) lds_trips[tid] = 0u;
@@ -475,6 +480,16 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         table_k.store(lds_lut, tid);
         table_v.store(lds_lut + 128, tid);
     };
+    // The barrier stands where rotated queries and tables are complete.  What is left of the window comes behind it: its waves, and nobody
+    // else, begin their runs later.
+    auto window = [&](auto bf_tag) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (; split + wt * splits < win_tiles; wt += DW) {
+            WindowTile<D, decltype(bf_tag)::value> w;
+            w.load(a, row, split + wt * splits, lane);
+            w.finish(a, wrec + (size_t)(split + wt * splits) * G * PART, splits > 1u, lane);
+        }
+    };
     auto start = [&](auto bf_tag) __attribute__((always_inline)) {
         constexpr bool BF = decltype(bf_tag)::value;
         if (wave < (uint32_t)TILES) {
@@ -482,24 +497,23 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
             r.load(a.queries + (size_t)row * G * D * 2u, G, a.table_k, wave, lane);
             first_run();
             r.finish(&lds_qrot[0][0], QROW, a.scale, wave, lane);
+            // (256 wide a tile takes several runs' time, and where every split has one or more it is better spent together: 128 rows x 4000
+            // tokens, K8/V8, 8 heads, eight layers 809 us, behind the barrier 857)
+            if (D == 256 && win_tiles > splits) window(bf_tag);
+            __syncthreads();
         } else if (split + wt * splits < win_tiles) {
             WindowTile<D, BF> w;
             w.load(a, row, split + wt * splits, lane);
             first_run();
+            __syncthreads();
             w.finish(a, wrec + (size_t)(split + wt * splits) * G * PART, splits > 1u, lane);
             wt += DW;
         } else {
             first_run();
-        }
-#pragma unroll 1
-        for (; split + wt * splits < win_tiles; wt += DW) {
-            WindowTile<D, BF> w;
-            w.load(a, row, split + wt * splits, lane);
-            w.finish(a, wrec + (size_t)(split + wt * splits) * G * PART, splits > 1u, lane);
+            __syncthreads();
         }
     };
-    if (a.bf16) start(std::true_type{}); else start(std::false_type{});
-    __syncthreads();
+    if (a.bf16) { start(std::true_type{}); window(std::true_type{}); } else { start(std::false_type{}); window(std::false_type{}); }
 
     // ---- B operand of the score product: fp16 of q * 2^(10 - e), e = binary exponent of the head's largest magnitude.  At 256 with
     // 8-bit codes on either side registers run out (28 spilled with 8-bit keys and values): the low term, the same in every wave, lies
@@ -540,12 +554,10 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
 #pragma unroll
             for (int k = 0; k < QREG; ++k) qb[k][s] = __builtin_bit_cast(tq_u4, term[k]);
 #pragma unroll
-            for (int k = QREG; k < QT; ++k)         // the same in every wave
-                if (wave == 0u) lds_q[(k - QREG) * SK + s][lane] = __builtin_bit_cast(tq_u4, term[k]);
+            for (int k = QREG; k < QT; ++k)         // the same in every wave, and each writes it: none waits for another
+                lds_q[(k - QREG) * SK + s][lane] = __builtin_bit_cast(tq_u4, term[k]);
         }
     }
-    if constexpr (QT > QREG) __syncthreads();
-
     const uint32_t slot_k = RepLut<IPBK>::lane_offset(lane), slot_v = 128u + RepLut<IPBV>::lane_offset(lane);
     tq_f4v acc[NC];          // weighted value sums: register r = column 4 q4 + r of the scores (head and block of tokens), c = coordinate value_coord(n16, c)
 #pragma unroll
@@ -859,8 +871,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     // do, thread 0 may count the block as done, see put_record)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    // rows of Pi_v for the rotation back: thread (four columns, part) takes ROTK of them.  Loaded while the counter is asked whether
-    // they are needed (all blocks but one of a row load them for nothing: 4 D^2 bytes from the L2); wave 0, which asks, afterwards.
+    // rows of Pi_v for the rotation back: thread (four columns, part) takes ROTK of them, loaded behind the records that it has to wait for
     const uint32_t rc = (tid % (D / 4)) * 4u, rp = tid / (D / 4);
     tq_u4 pv[ROTK];
     auto load_pv = [&]() __attribute__((always_inline)) {
@@ -868,7 +879,6 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
 #pragma unroll
         for (int k = 0; k < ROTK; ++k) pv[k] = tq_gload16(src + k * (D * 4));
     };
-    if (wave) load_pv();
     if (splits > 1u) {
         if (tid == 0u) {
             const bool last = __hip_atomic_fetch_add(a.arrived + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1u;
@@ -878,69 +888,45 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         __syncthreads();
         if (!lds_last) return;
     }
-    if (!wave) load_pv();
     float *ysum = reinterpret_cast<float *>(&lds_area[0][0]);     // [head][D]: sums in the rotated space
     float *wsum = ysum + MAX_GROUP * D;                           // [head][D]: the window's, plain
-    // One trip to memory where few records meet: references and sums of exp of a head's records (a lane each) and the sums (four columns
-    // a lane, every fourth record; the quarters of a wave are added in registers) are under way together.  Little code: it runs once
-    // and is fetched for the first time (33 loads a lane, written out: 2.0 us from the first to the last of them, now 0.4).
+    // Where few records meet there is one trip to memory: references and sums of exp of a head's records (a lane each), the sums (four columns
+    // a lane, every fourth record; the quarters of a wave are added in registers) and the rows of Pi_v, which are needed last, are under way
+    // together.  No loop holds a load there: behind one the compiler waits for everything in flight, the rows of Pi_v among it (32 rows x 6000
+    // tokens, 64 wide, from the last arrival to merged sums: 1.9 us with loops, now 1.4).  What is left grows with the records: one compute unit reads
+    // what other dies wrote at some 27 KB/us (8 rows x 32768, 66 KB: 2.4 us; 256 wide, 8 x 9906, 120 KB and 256 KB of Pi_v: 5.2).  Little code: it runs once and is fetched for the first time
+    // (33 loads a lane, written out: 2.0 us from the first to the last of them, now 0.4).
     auto merge = [&](auto across_tag) __attribute__((always_inline)) {
         constexpr bool ACROSS = decltype(across_tag)::value;
-        constexpr int YB = 8;                                         // records a lane has under way
         const uint32_t step = G * PART, nrec = splits + win_tiles;    // (a row's records lie within 4.5 MiB)
         const Records part(a.partial + (size_t)row * splits * step, splits * step), wpart(a.win_part + (size_t)row * win_tiles * step, win_tiles * step);
         // weights of the records: exp(reference - largest reference of the head)
         float *wgt = reinterpret_cast<float *>(lds_lut);              // [head][splits, then window tiles: each up to a multiple of 4, zeros behind]
         const uint32_t wfirst = (splits + 3u) / 4u * 4u, wrow = wfirst + (win_tiles + 3u) / 4u * 4u;
         auto place = [&](uint32_t s) { return s < splits ? s : wfirst + s - splits; };
-        auto head_of = [&](uint32_t s, uint32_t g) { return s < splits ? part.load2<ACROSS>(s * step + g * PART) : wpart.load2<ACROSS>((s - splits) * step + g * PART); };
-        tq_u2 ml = {0u, 0u};
-        tq_u4 y[YB], w;
-        if (wave < G && lane < nrec) ml = head_of(lane, wave);
-        auto fetch = [&](uint32_t off, uint32_t s0) __attribute__((always_inline)) {
+        auto fetch = [&](auto &y, uint32_t off, uint32_t s0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int s = 0; s < YB; ++s) y[s] = part.load4<ACROSS>((s0 + 4u * s + q4) * step + off);
+            for (int s = 0; s < (int)(sizeof(y) / sizeof(y[0])); ++s) y[s] = part.load4<ACROSS>((s0 + 4u * s + q4) * step + off);
         };
-        const uint32_t col = (wave * 16u + n16) * 4u;                 // + DTHREADS: further heads
-        fetch(col / D * PART + 2u + col % D, 0u);
-        w = wpart.load4<ACROSS>(q4 * step + col / D * PART + 2u + col % D);
-        for (uint32_t g = wave; g < G; g += DW) {
-            if (g != wave && lane < nrec) ml = head_of(lane, g);
-            float m = lane < nrec ? __uint_as_float(ml[0]) : -3.0e38f;
-            for (uint32_t s = lane + 64u; s < nrec; s += 64u) m = fmaxf(m, __uint_as_float(head_of(s, g)[0]));
-            m = reduce_wave(m, OpMax());
-            for (uint32_t s = lane; s < wrow; s += 64u) wgt[g * wrow + s] = 0.f;      // (the LDS serves a wave in order)
-            asm volatile("" ::: "memory");
-            float den = 0.f;
-            for (uint32_t s = lane; s < nrec; s += 64u) {
-                const tq_u2 r = s == lane ? ml : head_of(s, g);
-                const float f = __expf(__uint_as_float(r[0]) - m);
-                wgt[g * wrow + place(s)] = f;
-                den = fmaf(f, __uint_as_float(r[1]), den);
-            }
-            den = reduce_wave(den, OpAdd());
-            if (lane == 0u) lds_den[g] = den;
-        }
-        __syncthreads();
-        for (uint32_t p = col; p < G * D; p += DTHREADS) {
-            const uint32_t g = p / D, off = g * PART + 2u + p % D;
-            const float *f = wgt + g * wrow + q4;
-            float ys[4] = {0.f, 0.f, 0.f, 0.f}, ws[4] = {0.f, 0.f, 0.f, 0.f};
-            for (uint32_t s0 = 0; s0 < splits; s0 += 4 * YB) {
-                if (p != col || s0) fetch(off, s0);
+        float ys[4], ws[4];
+        auto add_records = [&](const auto &y, const float *f, uint32_t s0) __attribute__((always_inline)) {
 #pragma unroll
-                for (int s = 0; s < YB; ++s) {
-                    if (s0 + 4u * s >= splits) break;     // (uniform)
-                    const float fs = f[s0 + 4 * s];       // (zero for what lies past the last record)
+            for (int s = 0; s < (int)(sizeof(y) / sizeof(y[0])); ++s) {
+                if (s0 + 4u * s >= splits) break;     // (uniform)
+                const float fs = f[s0 + 4 * s];       // (zero for what lies past the last record)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) ys[c] = fmaf(fs, __uint_as_float(y[s][c]), ys[c]);
-                }
+                for (int c = 0; c < 4; ++c) ys[c] = fmaf(fs, __uint_as_float(y[s][c]), ys[c]);
             }
-            for (uint32_t s0 = 0; s0 < win_tiles; s0 += 4u) {
-                if (p != col || s0) w = wpart.load4<ACROSS>((s0 + q4) * step + off);
+        };
+        auto add_window = [&](tq_u4 w, float f) __attribute__((always_inline)) {
 #pragma unroll
-                for (int c = 0; c < 4; ++c) ws[c] = fmaf(f[wfirst + s0], __uint_as_float(w[c]), ws[c]);
-            }
+            for (int c = 0; c < 4; ++c) ws[c] = fmaf(f, __uint_as_float(w[c]), ws[c]);
+        };
+        auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) ys[c] = ws[c] = 0.f;
+        };
+        auto put_sums = [&](uint32_t p) __attribute__((always_inline)) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 ys[c] = reduce_rows(ys[c], OpAdd());
@@ -950,7 +936,109 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 *reinterpret_cast<float4 *>(ysum + p) = make_float4(ys[0], ys[1], ys[2], ys[3]);
                 *reinterpret_cast<float4 *>(wsum + p) = make_float4(ws[0], ws[1], ws[2], ws[3]);
             }
+        };
+        const uint32_t col = (wave * 16u + n16) * 4u;                 // + DTHREADS: further heads
+        // references and sums of exp of head g's records, R x 64 of them, a lane each (of either kind: where there is none of one it reads as zero)
+        auto load_heads = [&](auto &ml, uint32_t g) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < (int)(sizeof(ml) / sizeof(ml[0])); ++k) {
+                const uint32_t s = 64u * k + lane;
+                const tq_u2 hs = part.load2<ACROSS>(s * step + g * PART), hw = wpart.load2<ACROSS>((s - splits) * step + g * PART);
+                ml[k] = s < splits ? hs : hw;
+            }
+        };
+        auto weigh = [&](const auto &ml, uint32_t g) __attribute__((always_inline)) {
+            constexpr int R = sizeof(ml) / sizeof(ml[0]);
+            float m = -3.0e38f, den = 0.f;
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const uint32_t s = 64u * k + lane;
+                if (s < nrec) m = fmaxf(m, __uint_as_float(ml[k][0]));
+                if (s < wrow) wgt[g * wrow + s] = 0.f;       // (the LDS serves a wave in order)
+            }
+            m = reduce_wave(m, OpMax());
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const uint32_t s = 64u * k + lane;
+                if (s < nrec) {
+                    const float f = __expf(__uint_as_float(ml[k][0]) - m);
+                    wgt[g * wrow + place(s)] = f;
+                    den = fmaf(f, __uint_as_float(ml[k][1]), den);
+                }
+            }
+            den = reduce_wave(den, OpAdd());
+            if (lane == 0u) lds_den[g] = den;
+        };
+        auto few = [&](auto passes) __attribute__((always_inline)) {
+            constexpr int N = decltype(passes)::value;                // of 512 columns
+            tq_u4 y[N][8], w[N];
+            tq_u2 ml[1];
+            load_heads(ml, wave);
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const uint32_t p = col + k * DTHREADS, off = p / D * PART + 2u + p % D;
+                fetch(y[k], off, 0u);
+                w[k] = wpart.load4<ACROSS>(q4 * step + off);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (N <= 2) load_pv();                          // (more columns leave no registers for them yet)
+            if (wave < G) weigh(ml, wave);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const uint32_t p = col + k * DTHREADS;
+                if (p >= G * D) break;
+                const float *f = wgt + p / D * wrow + q4;
+                clear();
+                add_records(y[k], f, 0u);
+                if (win_tiles) add_window(w[k], f[wfirst]);
+                put_sums(p);
+            }
+            if constexpr (N > 2) load_pv();
+            __syncthreads();
+        };
+        if (G <= (uint32_t)DW && splits <= 32u && win_tiles <= 4u) {
+            if (G * D <= (uint32_t)DTHREADS) { few(std::integral_constant<int, 1>{}); return; }
+            if constexpr (DW * D > DTHREADS) {
+                if (G * D <= 2u * DTHREADS) { few(std::integral_constant<int, 2>{}); return; }
+            }
+            if constexpr (DW * D > 2 * DTHREADS) { few(std::integral_constant<int, 4>{}); return; }
         }
+        tq_u4 y[8], w;
+        tq_u2 ml[(MAX_SPLITS + MAX_WINDOW / WIN_TILE + 63) / 64];
+        load_heads(ml, wave);
+        fetch(y, col / D * PART + 2u + col % D, 0u);
+        w = wpart.load4<ACROSS>(q4 * step + col / D * PART + 2u + col % D);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (D <= 128) load_pv();
+        for (uint32_t g = wave; g < G; g += DW) {
+            if (g != wave) load_heads(ml, g);
+            weigh(ml, g);
+        }
+        __syncthreads();
+        for (uint32_t p = col; p < G * D; p += DTHREADS) {
+            const uint32_t g = p / D, off = g * PART + 2u + p % D;
+            const float *f = wgt + g * wrow + q4;
+            if (p != col) {
+                fetch(y, off, 0u);
+                w = wpart.load4<ACROSS>(q4 * step + off);
+            }
+            clear();
+            for (uint32_t s0 = 0;;) {       // the next 32 records under way (past the last one: zeros) while these are added
+                tq_u4 z[8];
+                fetch(z, off, s0 + 32u);
+                add_records(y, f, s0);
+                s0 += 32u;
+                if (s0 >= splits) break;
+#pragma unroll
+                for (int s = 0; s < 8; ++s) y[s] = z[s];
+            }
+            if (win_tiles) add_window(w, f[wfirst]);
+            for (uint32_t s0 = 4u; s0 < win_tiles; s0 += 4u) add_window(wpart.load4<ACROSS>((s0 + q4) * step + off), f[wfirst + s0]);
+            put_sums(p);
+        }
+        if constexpr (D > 128) load_pv();
         __syncthreads();
     };
     if (splits > 1u) merge(std::true_type{}); else merge(std::false_type{});
