@@ -741,3 +741,21 @@ def test_compressor_on_the_cpu_follows_the_tensors(pkg):
     assert k.shape == x.shape and torch.equal(k[:, :, -8:], x[:, :, -8:])
     with pytest.raises(Exception):
         host.compress(x.cpu())
+
+
+@pytest.mark.parametrize("dim,bits", [(128, 4), (128, 8), (128, 1), (64, 3)])
+@pytest.mark.parametrize("rows,tokens", [(1, 1), (1, 16384), (1, 16385), (3, 16415), (2, 49200), (5, 40), (300, 33)])
+def test_float32_vectors_do_not_depend_on_the_size_of_their_job(pkg, dim, bits, rows, tokens):
+    """Float32 vectors in one call, rows that lie apart among them, against the same vectors a thousand at a time (blocks of one tile on the
+    way there, blocks of fewer waves on the way back): the same bytes, and the same float32 results."""
+    comp = pkg.MSECompressor(dim, bits, seed=42, device=DEV)
+    wide = torch.randn(1, rows, tokens + 8, dim, generator=torch.Generator().manual_seed(tokens)).to(DEV)
+    x = wide[:, :, :tokens]
+    whole = comp.compress(x)
+    out = comp.decompress(whole)
+    for r in {0, rows - 1}:
+        for t in range(0, tokens, 1000):
+            part = comp.compress(x[:, r:r + 1, t:t + 1000].contiguous())
+            for key in ("idx_bytes", "vec_norms"):
+                assert torch.equal(part[key], whole[key][:, r:r + 1, t:t + 1000]), (key, r, t)
+            assert torch.equal(comp.decompress(part), out[:, r:r + 1, t:t + 1000]), (r, t)

@@ -55,7 +55,7 @@ namespace {
 template <int DTYPE> struct InTraits;
 template <> struct InTraits<TQ_F16> { static constexpr int ELEM = 2, TERMS = 2, MIN_WAVES = TQ_C16_WAVES; };
 template <> struct InTraits<TQ_BF16> { static constexpr int ELEM = 2, TERMS = 2, MIN_WAVES = TQ_C16_WAVES; };
-// fp32 input keeps three rotation terms resident and stages 16 KiB tiles
+// fp32 input keeps three rotation terms resident and stages tiles as three bf16 terms, 24 KiB
 template <> struct InTraits<TQ_F32> { static constexpr int ELEM = 4, TERMS = 3, MIN_WAVES = 2; };
 
 constexpr int CWAVES = TQ_TILES;        // waves per block = MFMA row tiles
@@ -80,10 +80,10 @@ struct CompressLds {
     static constexpr int ELEM = InTraits<DTYPE>::ELEM;
     static constexpr int RING = ELEM == 2 ? TQ_RING : 2;     // staged tiles
     using Grid = uint8_t[TQ_GRID_LDS_BYTES];
-    using Stage = uint8_t[RING][32 * TQ_HEAD_DIM * ELEM];
+    using Stage = uint8_t[RING][32 * TQ_HEAD_DIM * (ELEM == 2 ? 2 : 6)];
     using Part = float[2][32][4];      // sum of squares of the tile's vectors, one share per wave (pipelined path)
     using Ss = float[2][32];           // the same, whole (16-bit inputs)
-    using Ssh = float[2][32][2];       // the same per half of a row (rows that are pairs of 64-wide vectors)
+    using Ssh = float[ELEM == 2 ? 2 : 3][32][2];       // the same per half of a row (rows that are pairs of 64-wide vectors; fp32 inputs)
     using Tk = uint32_t[4];            // ticket k of the block sits in slot k % 4 (counter mode only)
     static __device__ __forceinline__ Grid &grid() { __shared__ __attribute__((aligned(16))) Grid a; return a; }
     static __device__ __forceinline__ Stage &stage() { __shared__ __attribute__((aligned(1024))) Stage a; return a; }
@@ -105,6 +105,7 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     constexpr int PIECES = VEC_BYTES / 16;             // 16-byte pieces per vector
     constexpr int VEC_PER_LOAD = 64 / PIECES;          // vectors covered by one load instruction
     constexpr int NB = P::NB, NW = P::NW;
+    constexpr int TERM = 32 * TQ_HEAD_DIM * 2;         // one bf16 term of a staged tile of fp32 inputs
 
     constexpr int RING = CompressLds<DTYPE>::RING;
     auto &lds_grid = CompressLds<DTYPE>::grid();
@@ -165,7 +166,6 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     // ---- this wave's quarter of the rotation, resident for the whole kernel.  Wave w walks the 16-input
     // steps of the contraction in the order 2w, 2w+1, ... (mod 8): its first two steps then cover inputs
     // [32w, 32w+32), the share of the vector whose squares it sums in the pipelined path.
-    // (fp32 inputs sum their squares while they walk the steps, every wave over the whole vector: same order in all waves)
     const uint32_t step0 = ELEM == 2 ? 2u * wave : 0u;
     tq_u4 areg[T::TERMS][TQ_STEPS];
     // Rotation operands into registers and the quantiser grid into LDS (one copy per code position, base pre-shifted).
@@ -210,8 +210,8 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     // LDS offset of this lane's piece of load j (computed where it is used: these paths are not the hot one)
     auto st_off = [&](int j) {
         const uint32_t vl = (wave * NLOAD + j) * VEC_PER_LOAD + ld_vec;
-        const uint32_t swz = (ELEM == 2) ? (vl & 15u) : ((vl & 15u) << 1);
-        return vl * VEC_BYTES + ((ld_piece ^ swz) << 4);
+        if constexpr (ELEM == 2) return vl * VEC_BYTES + ((ld_piece ^ (vl & 15u)) << 4);
+        else return vl * (VEC_BYTES / 2) + (((ld_piece >> 1) ^ (vl & 15u)) << 4) + (ld_piece & 1u) * 8u;      // of a term: four of its values
     };
 
     tq_u4 pre[NLOAD];
@@ -236,11 +236,13 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
         constexpr int N = decltype(n_tag)::value;
         return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x110 + N, 0xf, 0xf, true));
     };
-    auto park = [&](uint32_t b, const tq_u4 (&src)[NLOAD]) {
+    // fp32 inputs are split into their terms here, once (by the waves that read the operands it took four times as many vector
+    // instructions as everything else together); their squares are summed per half of a row, the 16 lanes of a DPP row, in slot `slot`.
+    auto park = [&](uint32_t b, uint32_t slot, const tq_u4 (&src)[NLOAD]) {
         uint8_t *stage = lds_stage[b];
-#pragma unroll
-        for (int j = 0; j < NLOAD; ++j) *reinterpret_cast<tq_u4 *>(stage + st_off(j)) = src[j];
         if constexpr (ELEM == 2) {
+#pragma unroll
+            for (int j = 0; j < NLOAD; ++j) *reinterpret_cast<tq_u4 *>(stage + st_off(j)) = src[j];
 #pragma unroll
             for (int j = 0; j < NLOAD; ++j) {
                 const float own = sumsq8<DTYPE>(src[j], 0.f);
@@ -251,40 +253,58 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
                 if ((lane & 15u) == 15u) lds_ss[b][(wave * NLOAD + j) * VEC_PER_LOAD + ld_vec] = total;
                 if ((lane & 7u) == 7u) lds_ssh[b][(wave * NLOAD + j) * VEC_PER_LOAD + ld_vec][(lane >> 3) & 1u] = pair;   // pieces 0..7, 8..15
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NLOAD; ++j) {
+                tq_u2 t[3];
+                float ss = 0.f;
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {      // x = its three terms exactly: every term a truncation, every remainder exact
+                    uint32_t r[2][3];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const float x = __uint_as_float(src[j][2 * d + i]);
+                        const float r1 = x - __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+                        const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+                        ss = fmaf(x, x, ss);
+                        r[i][0] = __float_as_uint(x); r[i][1] = __float_as_uint(r1); r[i][2] = __float_as_uint(r2);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) t[k][d] = __builtin_amdgcn_perm(r[1][k], r[0][k], 0x07060302u);
+                }
+#pragma unroll
+                for (int k = 0; k < 3; ++k) *reinterpret_cast<tq_u2 *>(stage + k * TERM + st_off(j)) = t[k];
+                auto add_rotated = [&](auto n_tag) {
+                    ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x120 + decltype(n_tag)::value, 0xf, 0xf, true));
+                };
+                add_rotated(std::integral_constant<int, 8>{});
+                add_rotated(std::integral_constant<int, 4>{});
+                add_rotated(std::integral_constant<int, 2>{});
+                add_rotated(std::integral_constant<int, 1>{});
+                if ((lane & 15u) == 0u) lds_ssh[slot][(wave * NLOAD + j) * VEC_PER_LOAD + ld_vec][(lane >> 4) & 1u] = ss;
+            }
         }
     };
 
     // ---- the three stages of a tile ---------------------------------------------------------
     // (1) rotation step s of the tile parked in `stage`: acc[r] += sum over 16 inputs of
-    //     Pi[32w + 16h + r][k] * x_n[k]  (raw, unnormalised); fp32 inputs also sum their squares here
-    auto rotate_step = [&](const uint8_t *stage, int s, tq_f16v &acc, float &ss0, float &ss1) {
+    //     Pi[32w + 16h + r][k] * x_n[k]  (raw, unnormalised)
+    auto rotate_step = [&](const uint8_t *stage, int s, tq_f16v &acc) {
         const uint32_t sg = ((uint32_t)s + step0) & 7u;   // the step of the contraction that areg[.][s] belongs to
+        const uint8_t *at = stage + n * (TQ_HEAD_DIM * 2) + (((2u * sg + hk) ^ (n & 15u)) << 4);
         if constexpr (ELEM == 2) {
-            const uint32_t piece = 2u * sg + hk;
-            const tq_u4 bop = *reinterpret_cast<const tq_u4 *>(stage + n * VEC_BYTES + ((piece ^ (n & 15u)) << 4));
+            const tq_u4 bop = *reinterpret_cast<const tq_u4 *>(at);
 #pragma unroll
             for (int term = 0; term < T::TERMS; ++term)
                 acc = (DTYPE == TQ_F16) ? mfma_f16(areg[term][s], bop, acc) : mfma_bf16(areg[term][s], bop, acc);
         } else {
-            const uint32_t piece = 2u * (2u * sg + hk);
-            const uint32_t swz = (n & 15u) << 1;
-            const uint8_t *row = stage + n * VEC_BYTES;
-            const tq_u4 q0 = *reinterpret_cast<const tq_u4 *>(row + ((piece ^ swz) << 4));
-            const tq_u4 q1 = *reinterpret_cast<const tq_u4 *>(row + (((piece + 1u) ^ swz) << 4));
-            float x[8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { x[i] = __uint_as_float(q0[i]); x[4 + i] = __uint_as_float(q1[i]); }
-            if (!paired || (sg >> 2) == half) {      // (a half row: the four steps that cover it)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) { if (i & 1) ss1 = fmaf(x[i], x[i], ss1); else ss0 = fmaf(x[i], x[i], ss0); }
-            }
-            tq_u4 xt[3];
-            split_f32x8(x, xt[0], xt[1], xt[2]);
             // all products whose weight is >= 2^-24 of the leading one: (x term i, Pi term j), i + j <= 2
 #pragma unroll
-            for (int i = 0; i < 3; ++i)
+            for (int i = 0; i < 3; ++i) {
+                const tq_u4 bop = *reinterpret_cast<const tq_u4 *>(at + i * TERM);
 #pragma unroll
-                for (int term = 0; term + i < 3; ++term) acc = mfma_bf16(areg[term][s], xt[i], acc);
+                for (int term = 0; term + i < 3; ++term) acc = mfma_bf16(areg[term][s], bop, acc);
+            }
         }
     };
 
@@ -299,15 +319,9 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
         sc.inv_cell = sc.inv * grid_scale;   // grid_scale is a power of two: exact
         return sc;
     };
-    auto scale_of = [&](uint32_t b, float ss0, float ss1) {
-        float ss;
-        if constexpr (ELEM == 2) {
-            ss = paired ? lds_ssh[b][n][half] : lds_ss[b][n];
-        } else {
-            ss = ss0 + ss1;                 // both lanes of a vector hold half of the squares
-            ss += __shfl_xor(ss, 32);
-        }
-        return scale_from_ss(ss);
+    auto scale_of = [&](uint32_t slot) {
+        if constexpr (ELEM == 2) return scale_from_ss(paired ? lds_ssh[slot][n][half] : lds_ss[slot][n]);
+        else return scale_from_ss(paired ? lds_ssh[slot][n][half] : lds_ssh[slot][n][0] + lds_ssh[slot][n][1]);
     };
 
     // (3) code search + packing.  Lane (n, hk) of wave w holds coordinates 32w + 16hk + r.
@@ -352,10 +366,9 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     // Leaves the lane's packed words in `words` and the vector's norm in `nrm`.
     auto compute = [&](uint32_t b, uint32_t (&words)[NW], float &nrm) {
         tq_f16v acc = tq_zero16();
-        float ss0 = 0.f, ss1 = 0.f;
 #pragma unroll
-        for (int s = 0; s < TQ_STEPS; ++s) rotate_step(lds_stage[b], s, acc, ss0, ss1);
-        const Scale sc = scale_of(b, ss0, ss1);
+        for (int s = 0; s < TQ_STEPS; ++s) rotate_step(lds_stage[b], s, acc);
+        const Scale sc = scale_of(b);
         Search z;
         search_begin(z);
 #pragma unroll
@@ -390,7 +403,7 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     float nrm;
     // (the pipelined path addresses a tile's vectors with 32-bit offsets from a scalar base: the stride limit of ticket_job)
     const bool pipelined = ticket_job && tile < n_full;
-    if (!pipelined) load_tables();
+    if (!pipelined && (ELEM == 2 || tile >= n_full)) load_tables();
     if (pipelined) {
         if constexpr (ELEM == 2) {
             // Jobs with 16-bit elements (the KV-cache case): a software pipeline over this block's full
@@ -672,28 +685,107 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
             buf = 0u;
         }
     } else if (!ticket_job && tile < n_full) {
-        // General case (fp32 elements, rows of fewer than 32 tokens or too far apart).  Iteration k: start the
-        // loads of tile k+1, barrier (publishes buffer k, and everyone has finished reading buffer
-        // k-1), compute and store tile k, then park tile k+1 into the other buffer.  Loads, stores
-        // and the wait for the loads sit in one straight line, unpredicated: s_waitcnt vmcnt(#stores).
-        issue_loads(std::true_type{}, tile);
-        park(0, pre);
-        while (tile < n_full) {
-            const uint32_t next = tile + tile_stride;
-            issue_loads(std::true_type{}, next < n_full ? next : tile);
+        if constexpr (ELEM == 2) {
+            // General case (rows of fewer than 32 tokens or too far apart).  Iteration k: start the
+            // loads of tile k+1, barrier (publishes buffer k, and everyone has finished reading buffer
+            // k-1), compute and store tile k, then park tile k+1 into the other buffer.  Loads, stores
+            // and the wait for the loads sit in one straight line, unpredicated: s_waitcnt vmcnt(#stores).
+            issue_loads(std::true_type{}, tile);
+            park(0u, 0u, pre);
+            while (tile < n_full) {
+                const uint32_t next = tile + tile_stride;
+                issue_loads(std::true_type{}, next < n_full ? next : tile);
+                __syncthreads();
+                compute(buf, words, nrm);
+                const uint32_t slot = tq_packed_slot(job, tile * 32u + n);
+                store(job.idx_bytes + (size_t)slot * (8 * NB) + lane_slot, job.vec_norms + norm_slot(slot), words, nrm);
+                buf ^= 1u;
+                park(buf, buf, pre);
+                tile = next;
+            }
+        } else {
+            // fp32 elements, any rows: the same with the search of tile k-1 between the matrix instructions of tile k, from the other
+            // accumulator set (sums of squares wait in three slots).  Six bf16 products a step keep the matrix pipe busy for a third of the
+            // time, set-up and the first tile take another 4 us; the rest are waits of two waves a SIMD, the rotation's three terms leave no
+            // registers for a third (nor for loads two tiles ahead: 32.5 us, spilled).  131168 vectors, 4-bit: 34.8 us while every wave
+            // split the whole tile into its terms, now 29.8.
+            const uint32_t m = (n_full - tile + tile_stride - 1u) / tile_stride;      // this block's full tiles
+            auto only_one = [&]() __attribute__((always_inline)) {          // a small job: nothing to overlap
+                issue_loads(std::true_type{}, tile);
+                load_tables();
+                park(0u, 0u, pre);
+                __syncthreads();
+                compute(0u, words, nrm);
+                const uint32_t slot = tq_packed_slot(job, tile * 32u + n);
+                store(job.idx_bytes + (size_t)slot * (8 * NB) + lane_slot, job.vec_norms + norm_slot(slot), words, nrm);
+            };
+            auto several = [&]() __attribute__((always_inline)) {
+                TqTileWalk ahead(job, tile, tile_stride), done = ahead;
+                long long own[NLOAD];
+#pragma unroll
+                for (int j = 0; j < NLOAD; ++j) own[j] = (long long)((wave * NLOAD + j) * VEC_PER_LOAD + ld_vec) * job.token_stride + ld_piece * 16u;
+                auto issue = [&]() {
+#pragma unroll
+                    for (int j = 0; j < NLOAD; ++j) pre[j] = tq_gload16(job.states + ahead.offset(job, (wave * NLOAD + j) * VEC_PER_LOAD + ld_vec, own[j]));
+                };
+                auto trip = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
+                    constexpr bool ROT = decltype(rot_tag)::value, SEARCH = decltype(search_tag)::value;
+                    const bool more = ROT && j + 1u < m;
+                    if (more) {
+                        ahead.next(job);
+                        issue();
+                    }
+                    __syncthreads();        // tile j and its sums are parked, and nobody reads buffer (j + 1) & 1 any more
+                    const uint8_t *stage = lds_stage[j & 1u];
+                    Scale sc{};
+                    if constexpr (SEARCH) sc = scale_of((j + 2u) % 3u);       // tile j-1 sits in slot (j-1) % 3
+                    if constexpr (ROT) acc_new = tq_zero16();
+                    Search z;
+                    search_begin(z);
+#pragma unroll
+                    for (int s = 0; s < TQ_STEPS; ++s) {
+                        if constexpr (ROT) rotate_step(stage, s, acc_new);
+                        if constexpr (SEARCH) {
+                            search_coord(z, 2 * s, acc_old, sc);
+                            search_coord(z, 2 * s + 1, acc_old, sc);
+                        }
+                    }
+                    if constexpr (SEARCH) {
+                        search_end(z, words);
+                        const uint32_t slot = done.slot(job, n);
+                        store(job.idx_bytes + (size_t)slot * (8 * NB) + lane_slot, job.vec_norms + norm_slot(slot), words, sc.nrm);
+                        done.next(job);
+                    }
+                    if (more) park((j + 1u) & 1u, (j + 1u) % 3u, pre);
+                };
+                using Y = std::true_type;
+                using N = std::false_type;
+                tq_f16v acc_a, acc_b;       // tiles with an even index rotate into acc_a, the others into acc_b
+                issue();
+                load_tables();
+                park(0u, 0u, pre);
+                trip(Y{}, N{}, 0u, acc_a, acc_a);
+                uint32_t j = 1;
+                for (; j + 1u < m; j += 2u) {
+                    trip(Y{}, Y{}, j, acc_b, acc_a);
+                    trip(Y{}, Y{}, j + 1u, acc_a, acc_b);
+                }
+                if (j < m) {
+                    trip(Y{}, Y{}, j, acc_b, acc_a);
+                    ++j;
+                }
+                if (m & 1u) trip(N{}, Y{}, m, acc_b, acc_a);        // the last tile's codes
+                else trip(N{}, Y{}, m, acc_a, acc_b);
+            };
+            if (m == 1u) only_one(); else several();
+            tile += m * tile_stride;
             __syncthreads();
-            compute(buf, words, nrm);
-            const uint32_t slot = tq_packed_slot(job, tile * 32u + n);
-            store(job.idx_bytes + (size_t)slot * (8 * NB) + lane_slot, job.vec_norms + norm_slot(slot), words, nrm);
-            buf ^= 1u;
-            park(buf, pre);
-            tile = next;
         }
     }
     // the partial last tile of the job, if this block is the one whose turn it is
     if (tile == n_full && n_full < n_tiles) {
         issue_loads(std::false_type{}, tile);
-        park(buf, pre);
+        park(buf, buf, pre);
         __syncthreads();
         compute(buf, words, nrm);
         const uint32_t v = tile * 32u + n;

@@ -43,17 +43,18 @@ static __device__ __align__(256) uint32_t scratch[TQ_NOALLOC_MAX_JOBS * (TQ_WORK
 
 namespace {
 
-template <int DTYPE> struct OutTraits;
-template <> struct OutTraits<TQ_F16> { static constexpr int ELEM = 2, WAVES = 8; };
-template <> struct OutTraits<TQ_BF16> { static constexpr int ELEM = 2, WAVES = 8; };
-template <> struct OutTraits<TQ_F32> { static constexpr int ELEM = 4, WAVES = 4; };
+// Waves of a block.  Pi^T is staged once a block and one block is resident per compute unit, so eight; jobs that do not give each wave of
+// such blocks a tile are spread over more compute units by blocks of four.
+constexpr int MANY = 8, FEW = 4;
+// HALVES: parts of a tile that a wave transposes and stores one after the other; eight waves' whole tiles of 32-bit outputs and Pi^T do not fit the LDS
+template <int DTYPE, int W> struct OutTraits { static constexpr int ELEM = DTYPE == TQ_F32 ? 4 : 2, WAVES = W, HALVES = ELEM == 4 && W == MANY ? 2 : 1; };
 
 constexpr int LUT_LDS_BYTES = 4096;
 
-template <int DTYPE>
+template <int DTYPE, int W>
 constexpr size_t decompress_lds_bytes() {
-    using T = OutTraits<DTYPE>;
-    return (size_t)TQ_OPERAND_BYTES + LUT_LDS_BYTES + (size_t)T::WAVES * 32 * TQ_HEAD_DIM * T::ELEM;
+    using T = OutTraits<DTYPE, W>;
+    return (size_t)TQ_OPERAND_BYTES + LUT_LDS_BYTES + (size_t)T::WAVES * 32 * TQ_HEAD_DIM * T::ELEM / T::HALVES;
 }
 
 __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
@@ -61,13 +62,14 @@ __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
 }
 
 // One block's share of a job; `counter`: the job's two counters, or NULL; lds: decompress_lds_bytes.
-template <int DTYPE, int IPB, bool PAIRED>
+template <int DTYPE, int IPB, bool PAIRED, int W>
 __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk, uint32_t *counter, uint8_t *lds, uint32_t (&tk)[3]) {
-    using T = OutTraits<DTYPE>;
+    using T = OutTraits<DTYPE, W>;
     constexpr int ELEM = T::ELEM;
     constexpr int VEC_BYTES = TQ_HEAD_DIM * ELEM;   // 256 or 512
-    constexpr int STAGE = 32 * VEC_BYTES;
-    constexpr int NSTORE = STAGE / 1024;            // 16-byte stores per lane per tile
+    constexpr int HALVES = T::HALVES;
+    constexpr int STAGE = 32 * VEC_BYTES / HALVES;  // a wave's part of the LDS
+    constexpr int NSTORE = 32 * VEC_BYTES / 1024;   // 16-byte stores per lane per tile
     constexpr int PIECES = VEC_BYTES / 16;          // 16-byte pieces per vector: 16 or 32
     constexpr int VEC_PER_STORE = 64 / PIECES;
     constexpr int NB = 64 / IPB;                    // packed bytes per lane
@@ -157,9 +159,10 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     };
     // jump of the output offset / packed slot from the last vector of a row to the first of the next
     const long long row_wrap = job.row_stride - (long long)job.tokens * job.token_stride;
-    uint32_t st_off[NSTORE];   // byte offset of this lane's piece of store j relative to the tile's first vector
+    constexpr int NOFF = ELEM == 2 ? NSTORE : 1;      // (32-bit outputs: the rest is added where it is used, on the scalar unit)
+    uint32_t st_off[NOFF];   // byte offset of this lane's piece of store j relative to the tile's first vector
 #pragma unroll
-    for (int j = 0; j < NSTORE; ++j) st_off[j] = (j * VEC_PER_STORE + st_vec) * (uint32_t)job.token_stride + st_piece * 16u;
+    for (int j = 0; j < NOFF; ++j) st_off[j] = (j * VEC_PER_STORE + st_vec) * (uint32_t)job.token_stride + st_piece * 16u;
 
     uint32_t raw[NW];
     uint16_t norm_bits = 0;
@@ -242,41 +245,44 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
                     const uint32_t piece = 8u * hk + 2u * t + c;
                     *reinterpret_cast<tq_u4 *>(stage + n * VEC_BYTES + ((piece ^ (n & 15u)) << 4)) = o;
                 }
-        } else {
-#pragma unroll
-            for (int t = 0; t < TQ_TILES; ++t)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {  // four 16-byte pieces of 4 floats per MFMA tile
-                    tq_u4 o;
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) o[d] = __float_as_uint(acc[t][4 * c + d] * nrm);
-                    const uint32_t piece = 16u * hk + 4u * t + c;
-                    *reinterpret_cast<tq_u4 *>(stage + n * VEC_BYTES + ((piece ^ n) << 4)) = o;
-                }
         }
-        tq_u4 val[NSTORE];
+        constexpr uint32_t PART = 32 / HALVES;   // vectors
+        auto stage_part = [&](uint32_t h) {      // 32-bit outputs: vectors [PART h, PART h + PART)
+            if (n / PART == h) {
 #pragma unroll
-        for (int j = 0; j < NSTORE; ++j) {
-            const uint32_t vl = j * VEC_PER_STORE + st_vec;
-            const uint32_t swz = (ELEM == 2) ? (vl & 15u) : vl;
-            val[j] = *reinterpret_cast<const tq_u4 *>(stage + vl * VEC_BYTES + ((st_piece ^ swz) << 4));
-        }
-        if constexpr (FAST) {
-            const Origin o = origin_of(tl);
-            uint8_t *base = out_base + o.out_base;
+                for (int t = 0; t < TQ_TILES; ++t)
 #pragma unroll
-            for (int j = 0; j < NSTORE; ++j) {
+                    for (int c = 0; c < 4; ++c) {  // four 16-byte pieces of 4 floats per MFMA tile
+                        tq_u4 o;
+#pragma unroll
+                        for (int d = 0; d < 4; ++d) o[d] = __float_as_uint(acc[t][4 * c + d] * nrm);
+                        const uint32_t piece = 16u * hk + 4u * t + c;
+                        *reinterpret_cast<tq_u4 *>(stage + n % PART * VEC_BYTES + ((piece ^ n) << 4)) = o;
+                    }
+            }
+        };
+        // (32-bit outputs: a half is stored before the next one is staged, or registers run out)
+        constexpr int PER_HALF = NSTORE / HALVES;
+        const Origin o = FAST ? origin_of(tl) : Origin{};
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) {
+            if constexpr (ELEM == 4) stage_part(h);
+            tq_u4 val[PER_HALF];
+#pragma unroll
+            for (int k = 0; k < PER_HALF; ++k) {
+                const uint32_t vl = (h * PER_HALF + k) * VEC_PER_STORE + st_vec;
+                const uint32_t swz = (ELEM == 2) ? (vl & 15u) : vl;
+                val[k] = *reinterpret_cast<const tq_u4 *>(stage + vl % PART * VEC_BYTES + ((st_piece ^ swz) << 4));
+            }
+#pragma unroll
+            for (int k = 0; k < PER_HALF; ++k) {
+                const int j = h * PER_HALF + k;
                 const uint32_t vl = j * VEC_PER_STORE + st_vec;
                 const bool whole = !decltype(odd_tag)::value || vl + 1u != o.in_row || st_piece < (uint32_t)PIECES / 2u;
-                if ((FULL || tl * 32u + vl < job.n_vec) && whole)
-                    tq_gstore16_stream(base + st_off[j] + (vl >= o.in_row ? row_wrap : 0ll), val[j]);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < NSTORE; ++j) {
-                const uint32_t vl = j * VEC_PER_STORE + st_vec;
-                if (FULL || tl * 32u + vl < job.n_vec)
-                    tq_gstore16_stream(out_base + tq_vec_offset(job, tl * 32u + vl) + st_piece * 16u, val[j]);
+                if ((FULL || tl * 32u + vl < job.n_vec) && whole) {
+                    if constexpr (FAST) tq_gstore16_stream(out_base + o.out_base + (ELEM == 2 ? 0ll : (long long)(j * VEC_PER_STORE) * job.token_stride) + st_off[ELEM == 2 ? j : 0] + (vl >= o.in_row ? row_wrap : 0ll), val[k]);
+                    else tq_gstore16_stream(out_base + tq_vec_offset(job, tl * 32u + vl) + st_piece * 16u, val[k]);
+                }
             }
         }
     };
@@ -347,17 +353,17 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     }
 }
 
-template <int DTYPE, int IPB, bool PAIRED>
-__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace) {
+template <int DTYPE, int IPB, bool PAIRED, int W>
+__global__ __launch_bounds__(W *TQ_WAVE) void tq_decompress_kernel(TqDevJob job0, const tq_job *jobs, uint32_t *workspace) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tk[3];
-    const TqDevJob job = tq_pair_rows(tq_load_job(job0, jobs, blockIdx.y, OutTraits<DTYPE>::ELEM), PAIRED);
-    decompress_job<DTYPE, IPB, PAIRED>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr, lds, tk);
+    const TqDevJob job = tq_pair_rows(tq_load_job(job0, jobs, blockIdx.y, OutTraits<DTYPE, W>::ELEM), PAIRED);
+    decompress_job<DTYPE, IPB, PAIRED, W>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr, lds, tk);
 }
 
 // keys and values of a layer and its window; the two jobs' counters share one job's record of the workspace
-template <int DTYPE, bool PAIRED>
-__global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t *workspace) {
+template <int DTYPE, bool PAIRED, int W>
+__global__ __launch_bounds__(W *TQ_WAVE) void tq_restore_layer_kernel(TqLayer l, TqWindowCopy window, uint32_t *workspace) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tk[3];
     const uint32_t which = tq_layer_job(l);
@@ -366,10 +372,10 @@ __global__ __launch_bounds__(OutTraits<DTYPE>::WAVES *TQ_WAVE) void tq_restore_l
     uint32_t *counter = workspace ? workspace + which * (TQ_WORKSPACE_BYTES_PER_JOB / 8) : nullptr;
     tq_with_window(window, [&]() __attribute__((always_inline)) {
         switch (8 / (which ? l.bits[1] : l.bits[0])) {
-            case 8: decompress_job<DTYPE, 8, PAIRED>(job, blk, counter, lds, tk); break;
-            case 4: decompress_job<DTYPE, 4, PAIRED>(job, blk, counter, lds, tk); break;
-            case 2: decompress_job<DTYPE, 2, PAIRED>(job, blk, counter, lds, tk); break;
-            default: decompress_job<DTYPE, 1, PAIRED>(job, blk, counter, lds, tk); break;
+            case 8: decompress_job<DTYPE, 8, PAIRED, W>(job, blk, counter, lds, tk); break;
+            case 4: decompress_job<DTYPE, 4, PAIRED, W>(job, blk, counter, lds, tk); break;
+            case 2: decompress_job<DTYPE, 2, PAIRED, W>(job, blk, counter, lds, tk); break;
+            default: decompress_job<DTYPE, 1, PAIRED, W>(job, blk, counter, lds, tk); break;
         }
     });
 }
@@ -438,49 +444,61 @@ int allow_lds(const void *kernel, size_t lds, bool (&configured)[MAX_DEVICES]) {
     return 0;
 }
 
-template <int DTYPE, int IPB, bool PAIRED>
-int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *workspace, hipStream_t stream) {
-    using T = OutTraits<DTYPE>;
-    int cus = 0;
-    int rc = device_cus(cus);
-    if (rc) return rc;
-    constexpr size_t lds = decompress_lds_bytes<DTYPE>();
+template <int DTYPE, int IPB, bool PAIRED, int W>
+int launch_decompress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, int cus, void *workspace, hipStream_t stream) {
+    using T = OutTraits<DTYPE, W>;
+    constexpr size_t lds = decompress_lds_bytes<DTYPE, W>();
     static bool configured[MAX_DEVICES] = {};
-    rc = allow_lds(reinterpret_cast<const void *>(&tq_decompress_kernel<DTYPE, IPB, PAIRED>), lds, configured);
+    const int rc = allow_lds(reinterpret_cast<const void *>(&tq_decompress_kernel<DTYPE, IPB, PAIRED, W>), lds, configured);
     if (rc) return rc;
     const uint32_t want = (max_tiles + T::WAVES - 1) / T::WAVES;
     const uint32_t bx = tq_blocks_per_job(want, cus, n_jobs);
     dim3 grid(bx, (unsigned)n_jobs, 1), block(T::WAVES * TQ_WAVE, 1, 1);
     // tickets pay off once every block has several to draw; below that the fixed assignment starts sooner
     uint32_t *counters = want >= 4u * bx ? static_cast<uint32_t *>(workspace) : nullptr;
-    hipLaunchKernelGGL((tq_decompress_kernel<DTYPE, IPB, PAIRED>), grid, block, lds, stream, job, jobs_dev, counters);
+    hipLaunchKernelGGL((tq_decompress_kernel<DTYPE, IPB, PAIRED, W>), grid, block, lds, stream, job, jobs_dev, counters);
+    return (int)hipGetLastError();
+}
+
+template <int DTYPE, bool PAIRED, int W>
+int launch_layer_of(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, int cus, void *workspace, hipStream_t stream) {
+    using T = OutTraits<DTYPE, W>;
+    constexpr size_t lds = decompress_lds_bytes<DTYPE, W>();
+    static bool configured[MAX_DEVICES] = {};
+    const int rc = allow_lds(reinterpret_cast<const void *>(&tq_restore_layer_kernel<DTYPE, PAIRED, W>), lds, configured);
+    if (rc) return rc;
+    const uint32_t want = (tiles + T::WAVES - 1) / T::WAVES;
+    const uint32_t blocks = tq_layer_blocks(l, want, (uint32_t)cus, cost_k, cost_v);
+    uint32_t *counters = 2u * want >= 4u * blocks ? static_cast<uint32_t *>(workspace) : nullptr;      // as in launch_decompress
+    hipLaunchKernelGGL((tq_restore_layer_kernel<DTYPE, PAIRED, W>), dim3(blocks), dim3(T::WAVES * TQ_WAVE), lds, stream, l, window, counters);
     return (int)hipGetLastError();
 }
 
 template <int DTYPE, bool PAIRED>
 int launch_layer(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, void *workspace, hipStream_t stream) {
-    using T = OutTraits<DTYPE>;
     int cus = 0;
-    int rc = device_cus(cus);
+    const int rc = device_cus(cus);
     if (rc) return rc;
-    constexpr size_t lds = decompress_lds_bytes<DTYPE>();
-    static bool configured[MAX_DEVICES] = {};
-    rc = allow_lds(reinterpret_cast<const void *>(&tq_restore_layer_kernel<DTYPE, PAIRED>), lds, configured);
+    return 2ull * tiles <= FEW * (unsigned long long)cus ? launch_layer_of<DTYPE, PAIRED, FEW>(l, window, tiles, cost_k, cost_v, cus, workspace, stream)
+                                                         : launch_layer_of<DTYPE, PAIRED, MANY>(l, window, tiles, cost_k, cost_v, cus, workspace, stream);
+}
+
+template <int DTYPE, int IPB, bool PAIRED>
+int launch_either(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *ws, hipStream_t s) {
+    int cus = 0;
+    const int rc = device_cus(cus);
     if (rc) return rc;
-    const uint32_t want = (tiles + T::WAVES - 1) / T::WAVES;
-    const uint32_t blocks = tq_layer_blocks(l, want, (uint32_t)cus, cost_k, cost_v);
-    uint32_t *counters = 2u * want >= 4u * blocks ? static_cast<uint32_t *>(workspace) : nullptr;      // as in launch_decompress
-    hipLaunchKernelGGL((tq_restore_layer_kernel<DTYPE, PAIRED>), dim3(blocks), dim3(T::WAVES * TQ_WAVE), lds, stream, l, window, counters);
-    return (int)hipGetLastError();
+    return (unsigned long long)n_jobs * max_tiles <= FEW * (unsigned long long)cus ? launch_decompress<DTYPE, IPB, PAIRED, FEW>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s)
+                                                                                   : launch_decompress<DTYPE, IPB, PAIRED, MANY>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s);
 }
 
 template <int DTYPE, bool PAIRED>
 int dispatch_bits(int bits, const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_tiles, void *ws, hipStream_t s) {
     switch (8 / bits) {
-        case 8: return launch_decompress<DTYPE, 8, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
-        case 4: return launch_decompress<DTYPE, 4, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
-        case 2: return launch_decompress<DTYPE, 2, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
-        case 1: return launch_decompress<DTYPE, 1, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case 8: return launch_either<DTYPE, 8, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case 4: return launch_either<DTYPE, 4, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case 2: return launch_either<DTYPE, 2, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
+        case 1: return launch_either<DTYPE, 1, PAIRED>(job, jobs_dev, n_jobs, max_tiles, ws, s);
         default: return TQ_ERR_BITS;
     }
 }
