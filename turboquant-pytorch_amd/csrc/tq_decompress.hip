@@ -43,10 +43,12 @@ static __device__ __align__(256) uint32_t scratch[TQ_NOALLOC_MAX_JOBS * (TQ_WORK
 
 namespace {
 
-// Waves of a block.  Pi^T is staged once a block and one block is resident per compute unit, so eight; jobs that do not give each wave of
-// such blocks a tile are spread over more compute units by blocks of four.
-constexpr int MANY = 8, FEW = 4;
-// HALVES: parts of a tile that a wave transposes and stores one after the other; eight waves' whole tiles of 32-bit outputs and Pi^T do not fit the LDS
+// Waves of a block: one block is resident per compute unit (Pi^T is staged once a block), so eight, two to a SIMD.  32-bit outputs of up to
+// six tiles a compute unit go out faster from blocks of four, which spread over twice as many compute units (MSECompressor.compress and
+// decompress, eight waves / four, us: 3920 vectors, bf16, 6-bit 12.5 / 11.5; 32800, 4-bit 15.7 / 15.3; 48000 18.2 / 18.2; 131168, float32 45.5 / 48.5).
+constexpr int MANY = 8, FEW = 4, FEW_TILES = 6;
+// HALVES: parts of a tile that a wave transposes and stores one after the other.  Whole tiles of 32-bit outputs of eight waves and Pi^T do not fit the LDS; blocks of
+// four waves, which held them whole, left a wave alone on its SIMD (131168 vectors: 20.6 us, this way 16.8).
 template <int DTYPE, int W> struct OutTraits { static constexpr int ELEM = DTYPE == TQ_F32 ? 4 : 2, WAVES = W, HALVES = ELEM == 4 && W == MANY ? 2 : 1; };
 
 constexpr int LUT_LDS_BYTES = 4096;
@@ -159,7 +161,7 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     };
     // jump of the output offset / packed slot from the last vector of a row to the first of the next
     const long long row_wrap = job.row_stride - (long long)job.tokens * job.token_stride;
-    constexpr int NOFF = ELEM == 2 ? NSTORE : 1;      // (32-bit outputs: the rest is added where it is used, on the scalar unit)
+    constexpr int NOFF = HALVES == 1 ? NSTORE : 1;    // (where registers are short the rest is added where it is used, on the scalar unit)
     uint32_t st_off[NOFF];   // byte offset of this lane's piece of store j relative to the tile's first vector
 #pragma unroll
     for (int j = 0; j < NOFF; ++j) st_off[j] = (j * VEC_PER_STORE + st_vec) * (uint32_t)job.token_stride + st_piece * 16u;
@@ -280,7 +282,7 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
                 const uint32_t vl = j * VEC_PER_STORE + st_vec;
                 const bool whole = !decltype(odd_tag)::value || vl + 1u != o.in_row || st_piece < (uint32_t)PIECES / 2u;
                 if ((FULL || tl * 32u + vl < job.n_vec) && whole) {
-                    if constexpr (FAST) tq_gstore16_stream(out_base + o.out_base + (ELEM == 2 ? 0ll : (long long)(j * VEC_PER_STORE) * job.token_stride) + st_off[ELEM == 2 ? j : 0] + (vl >= o.in_row ? row_wrap : 0ll), val[k]);
+                    if constexpr (FAST) tq_gstore16_stream(out_base + o.out_base + (NOFF > 1 ? 0ll : (long long)(j * VEC_PER_STORE) * job.token_stride) + st_off[NOFF > 1 ? j : 0] + (vl >= o.in_row ? row_wrap : 0ll), val[k]);
                     else tq_gstore16_stream(out_base + tq_vec_offset(job, tl * 32u + vl) + st_piece * 16u, val[k]);
                 }
             }
@@ -479,8 +481,9 @@ int launch_layer(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint32_
     int cus = 0;
     const int rc = device_cus(cus);
     if (rc) return rc;
-    return 2ull * tiles <= FEW * (unsigned long long)cus ? launch_layer_of<DTYPE, PAIRED, FEW>(l, window, tiles, cost_k, cost_v, cus, workspace, stream)
-                                                         : launch_layer_of<DTYPE, PAIRED, MANY>(l, window, tiles, cost_k, cost_v, cus, workspace, stream);
+    if constexpr (DTYPE == TQ_F32)
+        if (2ull * tiles <= FEW_TILES * (unsigned long long)cus) return launch_layer_of<DTYPE, PAIRED, FEW>(l, window, tiles, cost_k, cost_v, cus, workspace, stream);
+    return launch_layer_of<DTYPE, PAIRED, MANY>(l, window, tiles, cost_k, cost_v, cus, workspace, stream);
 }
 
 template <int DTYPE, int IPB, bool PAIRED>
@@ -488,8 +491,9 @@ int launch_either(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint3
     int cus = 0;
     const int rc = device_cus(cus);
     if (rc) return rc;
-    return (unsigned long long)n_jobs * max_tiles <= FEW * (unsigned long long)cus ? launch_decompress<DTYPE, IPB, PAIRED, FEW>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s)
-                                                                                   : launch_decompress<DTYPE, IPB, PAIRED, MANY>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s);
+    if constexpr (DTYPE == TQ_F32)
+        if ((unsigned long long)n_jobs * max_tiles <= FEW_TILES * (unsigned long long)cus) return launch_decompress<DTYPE, IPB, PAIRED, FEW>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s);
+    return launch_decompress<DTYPE, IPB, PAIRED, MANY>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s);
 }
 
 template <int DTYPE, bool PAIRED>
