@@ -512,8 +512,14 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
             const uint32_t v = l * 16u + ld_vec;
             *reinterpret_cast<tq_u4 *>(lds_stage[b] + v * (D * 2) + ((ld_piece ^ (v & 31u)) << 4)) = pre[l];
             float s = sumsq8<DTYPE>(pre[l], 0.f);
-#pragma unroll
-            for (int m = 1; m < 32; m <<= 1) s += __shfl_xor(s, m);
+            // the butterfly over lanes 1, 2, 4, 8 and 16 apart (from the third step on the lanes of a group agree, and a mirror does)
+            auto add = [&](auto ctrl) { s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), decltype(ctrl)::value, 0xf, 0xf, true)); };
+            add(std::integral_constant<int, 0xb1>{});
+            add(std::integral_constant<int, 0x4e>{});
+            add(std::integral_constant<int, 0x141>{});
+            add(std::integral_constant<int, 0x140>{});
+            const auto two = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+            s = __uint_as_float(two[0]) + __uint_as_float(two[1]);
             if (ld_piece == 0u) lds_ss[slot][v] = s;
         }
     };
@@ -522,7 +528,7 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
     const uint32_t g_bytes = D / IPB;
 
     // iteration j: rotate tile j into acc_new, search tile j-1 from acc_old
-    auto iteration = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
+    auto iteration = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old, auto between) {
         constexpr bool ROT = decltype(rot_tag)::value, SEARCH = decltype(search_tag)::value;
         const uint8_t *stage = lds_stage[j & 1u];
         float nrm = 0.f, inv = 0.f, inv_cell = 0.f;
@@ -555,6 +561,7 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
             // keep the steps in this order: with all 16 operand reads and table lookups hoisted to the top the kernel
             // runs out of registers (the rotation alone holds 128)
             if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+            if (s == STEPS / 2 - 1) between();
         }
         if constexpr (SEARCH) {
             if (done.v + n < job.n_vec) {
@@ -574,20 +581,28 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
     };
 
     const uint32_t m = (n_tiles - blk.x + blk.grid - 1u) / blk.grid;     // this block's tiles
-    // one trip: the tile after this one sets out while this one is rotated, and is parked behind the trip's work
+    // One trip: half-way through it the tile after this one, which set out half-way through the last trip, is parked and the one after that
+    // sets out.  (Behind the trip's work, with the eight waves of the compute unit's one block in step, nothing ran beside the park, whose sums went
+    // through the LDS besides: keys and values of 8 x 16256 tokens, K4/V2, 80 us, this way 77.)
     auto trip = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
-        const bool more = j + 1u < m;
-        if (more) {
-            ahead.next(job);
-            issue_loads(ahead);
-        }
         __syncthreads();        // tile j and its sums are parked, and nobody reads buffer (j + 1) & 1 any more
-        iteration(rot_tag, search_tag, j, acc_new, acc_old);
-        if (more) park((j + 1u) & 1u, (j + 1u) % 3u);
+        iteration(rot_tag, search_tag, j, acc_new, acc_old, [&]() __attribute__((always_inline)) {
+            if (j + 1u < m) {
+                park((j + 1u) & 1u, (j + 1u) % 3u);
+                if (j + 2u < m) {
+                    ahead.next(job);
+                    issue_loads(ahead);
+                }
+            }
+        });
     };
     using T = std::true_type;
     using F = std::false_type;
     park(0u, 0u);
+    if (m > 1u) {
+        ahead.next(job);
+        issue_loads(ahead);
+    }
     tq_f16v acc_a, acc_b;       // tiles with an even index rotate into acc_a, the others into acc_b
     trip(T{}, F{}, 0u, acc_a, acc_a);
     uint32_t j = 1;
