@@ -102,9 +102,9 @@ __global__ __launch_bounds__(MAX_WAVES *TQ_WAVE, 2) void tq_anydim_compress_kern
     const uint32_t term_halves = GV * row_halves;    // one staged term
 
     const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
-    const uint8_t *a_src = job.table + (DTYPE == TQ_F16 ? hd->off_a_f16 : hd->off_a_bf16);
+    const uint8_t *a_src = job.table + (DTYPE == TQ_F16 ? TQ_OFF_A_F16 : TQ_OFF_A_BF16(d));
     const uint32_t a_term = TQ_OPERAND_BYTES_FOR(d);
-    tq_copy_to_lds(lds_grid, job.table + hd->off_grid, hd->grid_cells * 8u, tid, nthreads);
+    tq_stage_in_lds<TQ_GRID_LDS_BYTES, MAX_WAVES * TQ_WAVE>(lds_grid, job.table + TQ_OFF_GRID(d), tid);
     const float grid_scale = hd->grid_scale, grid_bias = hd->grid_bias;
     const uint32_t g_bytes = (dl + IPB - 1u) / IPB;  // packed bytes per vector
 
@@ -305,9 +305,8 @@ __global__ __launch_bounds__(MAX_WAVES *TQ_WAVE, 2) void tq_anydim_decompress_ke
     float *norms = reinterpret_cast<float *>(lds + 4096);
     uint16_t *ys = reinterpret_cast<uint16_t *>(norms + GV);
 
-    const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
-    const uint8_t *a_src = job.table + hd->off_at_f16;      // the leading fp16 term of Pi^T, as in the 128-wide kernel
-    tq_copy_to_lds(lds_lut, job.table + hd->off_lut, 256u * ENTRY, tid, nthreads);
+    const uint8_t *a_src = job.table + TQ_OFF_AT_F16(d);     // the leading fp16 term of Pi^T, as in the 128-wide kernel
+    tq_copy_to_lds(lds_lut, job.table + TQ_OFF_LUT(d), 256u * ENTRY, tid, nthreads);
 
     auto load_a = [&](uint32_t rb, uint32_t s) { return tq_gload16(a_src + (((size_t)rb * steps + s) * 64u + lane) * 16u); };
 
@@ -495,14 +494,14 @@ __device__ __forceinline__ void d256_compress_job(const TqDevJob &job, TqBlock b
 
     tq_u4 areg[2][STEPS];
     {
-        const uint8_t *src = job.table + (DTYPE == TQ_F16 ? hd->off_a_f16 : hd->off_a_bf16);
+        const uint8_t *src = job.table + (DTYPE == TQ_F16 ? TQ_OFF_A_F16 : TQ_OFF_A_BF16(D));
 #pragma unroll
         for (int term = 0; term < 2; ++term)
 #pragma unroll
             for (int s = 0; s < STEPS; ++s)
                 areg[term][s] = tq_gload16(src + (size_t)term * TQ_OPERAND_BYTES_FOR(D) + (((size_t)wave * STEPS + s) * 64 + lane) * 16);
     }
-    tq_copy_to_lds(lds_grid, job.table + hd->off_grid, hd->grid_cells * 8u, tid, 512u);
+    tq_stage_in_lds<TQ_GRID_LDS_BYTES, 512>(lds_grid, job.table + TQ_OFF_GRID(D), tid);
     const float grid_scale = hd->grid_scale, grid_bias = hd->grid_bias;
 
     // park the prefetched tile in buffer b and leave the vectors' sums of squares in slot `slot`
@@ -667,7 +666,6 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
     const uint32_t n = lane & 31u, hk = lane >> 5;
     const uint32_t n_tiles = (job.n_vec + 31u) / 32u;
     if (blk.x >= n_tiles) return;
-    const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
     const uint32_t g_bytes = D / IPB;
 
     // a thread's share of a tile: codes [32 c, 32 c + 32) of vector dv, c = tid % 8
@@ -694,14 +692,14 @@ __device__ __forceinline__ void d256_decompress_job(const TqDevJob &job, TqBlock
 
     tq_u4 areg[2][STEPS];       // row tiles 2w, 2w + 1
     {
-        const uint8_t *src = job.table + hd->off_at_f16;
+        const uint8_t *src = job.table + TQ_OFF_AT_F16(D);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int s = 0; s < STEPS; ++s)
                 areg[t][s] = tq_gload16(src + (((size_t)(2u * wave + t) * STEPS + s) * 64 + lane) * 16);
     }
-    tq_copy_to_lds(lds_lut, job.table + hd->off_lut, 256u * ENTRY, tid, 256u);
+    tq_stage_in_lds<256 * ENTRY, 256>(lds_lut, job.table + TQ_OFF_LUT(D), tid);
     __syncthreads();
 
     // the prefetched bytes -> 32 fp16 centroids = pieces 4 chunk .. 4 chunk + 3 of row dv of buffer b

@@ -170,10 +170,16 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     tq_u4 areg[T::TERMS][TQ_STEPS];
     // Rotation operands into registers and the quantiser grid into LDS (one copy per code position, base pre-shifted).
     // Every cell is fetched once and written to all its copies; the fetches of a thread are issued together.
-    // Called once per block: behind the first tile loads on the pipelined path, so that their latencies overlap.
+    // Called once per block: behind the first tile loads on the pipelined path, so that their latencies overlap.  Sections are taken where every
+    // table has them: the table's header in front was a trip to memory of its own (16 rows of 3968
+    // tokens, K6/V4, compress and restore, which does the same: 32.0 -> 31.3 us).
     auto load_tables = [&]() {
-        const uint8_t *src = job.table + (paired ? (DTYPE == TQ_F16 ? hd->off_pair_a_f16 : hd->off_pair_a_bf16)
-                                                 : (DTYPE == TQ_F16 ? hd->off_a_f16 : hd->off_a_bf16));
+        const uint8_t *src = job.table + (DTYPE == TQ_F16 ? TQ_OFF_A_F16 : TQ_OFF_A_BF16(TQ_HEAD_DIM));
+        uint32_t grid = TQ_OFF_GRID(TQ_HEAD_DIM);
+        if (paired) {      // (tables of 64-wide vectors: the pairs' section lies behind sections of the width)
+            src = job.table + (DTYPE == TQ_F16 ? hd->off_pair_a_f16 : hd->off_pair_a_bf16);
+            grid = TQ_OFF_GRID(TQ_HEAD_DIM / 2);
+        }
 #pragma unroll
         for (int term = 0; term < T::TERMS; ++term)
 #pragma unroll
@@ -181,8 +187,8 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
                 areg[term][s] = tq_gload16(src + (size_t)term * TQ_OPERAND_BYTES +
                                            (((size_t)wave * TQ_STEPS + ((s + step0) & 7u)) * 64 + lane) * 16);
         constexpr int CELL_TRIPS = (TQ_GRID_MAX_CELLS(BITS) + CTHREADS - 1) / CTHREADS;
-        const uint32_t cells = hd->grid_cells;
-        const uint8_t *gsrc = job.table + hd->off_grid;
+        constexpr uint32_t cells = TQ_GRID_MAX_CELLS(BITS);      // (a table has room for as many: how many it uses need not be known)
+        const uint8_t *gsrc = job.table + grid;
         tq_u2 cell[CELL_TRIPS];
 #pragma unroll
         for (int k = 0; k < CELL_TRIPS; ++k) {

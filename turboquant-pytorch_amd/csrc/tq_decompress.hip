@@ -122,14 +122,14 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
         constexpr int NT = T::WAVES * TQ_WAVE;
         constexpr int A_TRIPS = TQ_OPERAND_BYTES / 16 / NT;
         static_assert(A_TRIPS * NT * 16 == TQ_OPERAND_BYTES, "whole trips");
-        const uint8_t *a_src = job.table + (PAIRED ? hd->off_pair_at_f16 : hd->off_at_f16);
+        const uint8_t *a_src = job.table + (PAIRED ? hd->off_pair_at_f16 : TQ_OFF_AT_F16(TQ_HEAD_DIM));
         tq_u4 v[A_TRIPS];
 #pragma unroll
         for (int k = 0; k < A_TRIPS; ++k) v[k] = tq_gload16(a_src + 16u * (tid + k * NT));
         if (tid == 0) tk[1] = draw();
 #pragma unroll
         for (int k = 0; k < A_TRIPS; ++k) reinterpret_cast<tq_u4 *>(lds_a)[tid + k * NT] = v[k];
-        tq_copy_to_lds(lds_lut, job.table + hd->off_lut, 256u * 2u * IPB, tid, NT);
+        tq_copy_to_lds(lds_lut, job.table + TQ_OFF_LUT(PAIRED ? TQ_HEAD_DIM / 2 : TQ_HEAD_DIM), 256u * 2u * IPB, tid, NT);
         __syncthreads();
     };
 

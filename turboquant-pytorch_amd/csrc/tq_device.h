@@ -265,6 +265,19 @@ __device__ __forceinline__ void tq_copy_to_lds(uint8_t *dst, const uint8_t *src,
     for (uint32_t i = tid; i < bytes / 16; i += nthreads) d[i] = tq_gload16(src + 16u * i);
 }
 
+// The same for a size and a number of threads known beforehand: all fetches of a thread under way together.
+template <uint32_t BYTES, uint32_t NT>
+__device__ __forceinline__ void tq_stage_in_lds(uint8_t *dst, const uint8_t *src, uint32_t tid) {
+    constexpr uint32_t PIECES = BYTES / 16u, TRIPS = (PIECES + NT - 1u) / NT;
+    static_assert(BYTES % 16u == 0u, "whole pieces");
+    tq_u4 v[TRIPS];
+#pragma unroll
+    for (uint32_t k = 0; k < TRIPS; ++k) v[k] = tq_gload16(src + 16u * min(tid + k * NT, PIECES - 1u));
+#pragma unroll
+    for (uint32_t k = 0; k < TRIPS; ++k)
+        if ((k + 1u) * NT <= PIECES || tid + k * NT < PIECES) reinterpret_cast<tq_u4 *>(dst)[tid + k * NT] = v[k];
+}
+
 __device__ __forceinline__ tq_f16v tq_zero16() {
     tq_f16v z;
 #pragma unroll

@@ -382,7 +382,7 @@ __global__ __launch_bounds__(QTHREADS, 2) void tq_qjl_fused_kernel(TqQjlDevJob j
     const uint32_t step0 = 2u * wave;
     tq_u4 areg[2][TQ_STEPS], mreg[2][TQ_STEPS];
     {
-        const uint8_t *src = job.table + (DTYPE == TQ_F16 ? hd->off_a_f16 : hd->off_a_bf16);
+        const uint8_t *src = job.table + (DTYPE == TQ_F16 ? TQ_OFF_A_F16 : TQ_OFF_A_BF16(TQ_HEAD_DIM));
         const uint8_t *msrc = job.qjl_table + qh->off_m;
 #pragma unroll
         for (int term = 0; term < 2; ++term)
@@ -393,8 +393,8 @@ __global__ __launch_bounds__(QTHREADS, 2) void tq_qjl_fused_kernel(TqQjlDevJob j
             }
     }
     {   // quantiser grid: one copy per position of a code in a word, base pre-shifted (as in the compress kernel)
-        const uint32_t cells = hd->grid_cells;
-        const uint8_t *gsrc = job.table + hd->off_grid;
+        constexpr uint32_t cells = TQ_GRID_MAX_CELLS(BITS);
+        const uint8_t *gsrc = job.table + TQ_OFF_GRID(TQ_HEAD_DIM);
         for (uint32_t q = tid; q < cells; q += QTHREADS) {
             const tq_u2 cell = tq_gload8(gsrc + 8u * q);
 #pragma unroll

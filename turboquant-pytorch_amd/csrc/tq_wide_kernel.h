@@ -123,14 +123,14 @@ __device__ __forceinline__ void wide_compress_tiles(const TqDevJob &job, TqBlock
 
     tq_u4 areg[2][STEPS];
     {
-        const uint8_t *src = job.table + (DTYPE == TQ_F16 ? hd->off_a_f16 : hd->off_a_bf16);
+        const uint8_t *src = job.table + (DTYPE == TQ_F16 ? TQ_OFF_A_F16 : TQ_OFF_A_BF16(D));
 #pragma unroll
         for (int term = 0; term < 2; ++term)
 #pragma unroll
             for (int s = 0; s < STEPS; ++s)
                 areg[term][s] = tq_gload16(src + (size_t)term * TQ_OPERAND_BYTES_FOR(D) + (((size_t)wave * STEPS + s) * 64 + lane) * 16);
     }
-    tq_copy_to_lds(lds_grid, job.table + hd->off_grid, hd->grid_cells * 8u, tid, (uint32_t)THREADS);
+    tq_stage_in_lds<TQ_GRID_LDS_BYTES, THREADS>(lds_grid, job.table + TQ_OFF_GRID(D), tid);
     const float grid_scale = hd->grid_scale, grid_bias = hd->grid_bias;
 
     // park the prefetched tile in buffer b and leave the pieces' sums of squares in slot `slot`
@@ -302,7 +302,6 @@ __device__ __forceinline__ void wide_decompress_tiles(const TqDevJob &job, TqBlo
     const uint32_t n = lane & 31u, hk = lane >> 5;
     const uint32_t n_tiles = (job.n_vec + 31u) / 32u;
     if (blk.x >= n_tiles) return;
-    const TqTableHeader *hd = reinterpret_cast<const TqTableHeader *>(job.table);
     const uint32_t g_bytes = FIT != FULL ? (dl + IPB - 1u) / IPB : (uint32_t)(D / IPB);      // packed bytes per vector in memory
 
     // a thread's share of a tile: codes [16 c, 16 c + 16) of vector dv, c = tid % (2 WAVES)
@@ -331,11 +330,11 @@ __device__ __forceinline__ void wide_decompress_tiles(const TqDevJob &job, TqBlo
 
     tq_u4 areg[STEPS];
     {
-        const uint8_t *src = job.table + hd->off_at_f16;
+        const uint8_t *src = job.table + TQ_OFF_AT_F16(D);
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) areg[s] = tq_gload16(src + (((size_t)wave * STEPS + s) * 64 + lane) * 16);
     }
-    tq_copy_to_lds(lds_lut, job.table + hd->off_lut, 256u * ENTRY, tid, (uint32_t)THREADS);
+    tq_stage_in_lds<256 * ENTRY, THREADS>(lds_lut, job.table + TQ_OFF_LUT(D), tid);
     __syncthreads();
 
     // the prefetched bytes -> 16 fp16 centroids = pieces 2 chunk, 2 chunk + 1 of row dv of buffer b.  In this tile the even
