@@ -250,7 +250,7 @@ int tq_qjl_signs(const void *states, int dtype, long long n_vec, long long token
  * writes).  The n_vec vectors lie token_stride elements apart; all four outputs are dense ([n_vec, G], [n_vec],
  * [n_vec, 16], [n_vec]).  For 16-bit inputs and codes of up to TQ_QJL_ONE_PASS_MAX_BITS bits the vectors are read once, by a
  * kernel that works on the residual in rotated coordinates ((Pi x)[k] - ||x|| centroid(code_k), projected by S Pi^T
- * from the table of tq_qjl_table_build); float32 inputs, wider codes and the last n_vec % 32 vectors of a job take
+ * from the table of tq_qjl_table_build); float32 inputs, wider codes and jobs of fewer than 32 vectors take
  * tq_compress followed by tq_qjl_signs.  Both forms write the same codes and norms; their sign bits agree wherever a
  * projection is further than 1e-5 of |S row| |residual| from zero.
  * The batched form is one launch for many (layer) jobs that share dtype and mse_bits; `jobs_dev` is a device copy of the
