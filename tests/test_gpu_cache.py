@@ -1159,6 +1159,21 @@ def test_large_layers_equal_the_calls_per_tensor(pkg, dim, dtype):
         assert all(torch.equal(a, b) for a, b in zip(comp.decompress_kv(*packed), full))
 
 
+@pytest.mark.parametrize("dim,dtype,tokens", [(128, torch.bfloat16, 2048), (128, torch.float16, 4096), (128, torch.bfloat16, 4097), (128, torch.bfloat16, 8191),
+                                              (128, torch.float32, 3000), (64, torch.float16, 8193), (64, torch.bfloat16, 6001), (96, torch.bfloat16, 4500), (256, torch.float16, 1027)])
+def test_layers_of_a_few_tiles_a_block_equal_the_calls_per_tensor(pkg, dim, dtype, tokens):
+    """Sizes about those at which the blocks of a layer launch, a few tiles each, are dealt out to keys and values by bytes or in halves."""
+    g = torch.Generator().manual_seed(tokens)
+    k, v = (torch.randn(1, 16, tokens, dim, generator=g).to(dtype).to(DEV) for _ in range(2))
+    comp = pkg.TurboQuantV3(dim, key_bits=8, value_bits=2, residual_window=0, layer_idx=8, device=DEV)
+    packed = comp.compress_kv(k, v)
+    full = comp.decompress_kv(*packed)
+    for c, x, got, out in zip((comp.key_compressor, comp.val_compressor), (k, v), packed, full):
+        want = c.compress(x)
+        assert torch.equal(got["compressed"]["idx_bytes"], want["idx_bytes"]) and torch.equal(got["compressed"]["vec_norms"], want["vec_norms"])
+        assert torch.equal(out, c.decompress(want).to(out.dtype))
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_update_restores_the_layer_as_the_calls_per_tensor_do(pkg, monkeypatch, dim):
     """V3Cache.update from a per-row store (packed slots between the rows) and a window that moves through its buffer."""

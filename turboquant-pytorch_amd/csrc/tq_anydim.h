@@ -11,5 +11,5 @@ int tq_anydim_decompress(int dtype, int bits, int head_dim, const TqDevJob &sing
                          uint32_t max_vec, hipStream_t stream);
 // keys and values of a layer in one launch (TqLayer: everything but `split` filled in): 16-bit elements, head dimensions with kernels of their own
 bool tq_anydim_layer_supported(int head_dim, int dtype);
-int tq_anydim_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream);
-int tq_anydim_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream);
+int tq_anydim_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, hipStream_t stream);
+int tq_anydim_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, hipStream_t stream);

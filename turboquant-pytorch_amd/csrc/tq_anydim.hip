@@ -893,22 +893,22 @@ int launch_d256(K kernel, bool (&raised)[MAX_DEVICES], const TqDevJob &job, cons
     return (int)hipGetLastError();
 }
 template <int DTYPE>
-int launch_d256_compress_layer(TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+int launch_d256_compress_layer(TqLayer &l, uint32_t n_vec, hipStream_t stream) {
     static bool raised[MAX_DEVICES] = {};
     int slots = 0;
     const int rc = d256_slots<D256Compress>(&tq_d256_compress_layer_kernel<DTYPE>, raised, slots);
     if (rc) return rc;
-    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)slots, cost_k, cost_v);
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)slots);
     hipLaunchKernelGGL((tq_d256_compress_layer_kernel<DTYPE>), dim3(blocks), dim3(D256Compress::THREADS), D256Compress::LDS, stream, l);
     return (int)hipGetLastError();
 }
 template <int DTYPE>
-int launch_d256_restore_layer(TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+int launch_d256_restore_layer(TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, hipStream_t stream) {
     static bool raised[MAX_DEVICES] = {};
     int slots = 0;
     const int rc = d256_slots<D256Decompress<DTYPE>>(&tq_d256_restore_layer_kernel<DTYPE>, raised, slots);
     if (rc) return rc;
-    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)slots, cost_k, cost_v);
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)slots);
     hipLaunchKernelGGL((tq_d256_restore_layer_kernel<DTYPE>), dim3(blocks), dim3(D256Decompress<DTYPE>::THREADS), D256Decompress<DTYPE>::LDS, stream, l, w);
     return (int)hipGetLastError();
 }
@@ -1008,14 +1008,14 @@ bool tq_anydim_layer_supported(int head_dim, int dtype) {
     return tq_wide_supported(head_dim, dtype) || (head_dim == 256 && (dtype == TQ_F16 || dtype == TQ_BF16));
 }
 
-int tq_anydim_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+int tq_anydim_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, hipStream_t stream) {
     if (!tq_anydim_layer_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
-    if (head_dim != 256) return tq_wide_compress_layer(dtype, head_dim, l, n_vec, cost_k, cost_v, stream);
-    return dtype == TQ_F16 ? launch_d256_compress_layer<TQ_F16>(l, n_vec, cost_k, cost_v, stream) : launch_d256_compress_layer<TQ_BF16>(l, n_vec, cost_k, cost_v, stream);
+    if (head_dim != 256) return tq_wide_compress_layer(dtype, head_dim, l, n_vec, stream);
+    return dtype == TQ_F16 ? launch_d256_compress_layer<TQ_F16>(l, n_vec, stream) : launch_d256_compress_layer<TQ_BF16>(l, n_vec, stream);
 }
 
-int tq_anydim_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+int tq_anydim_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, hipStream_t stream) {
     if (!tq_anydim_layer_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
-    if (head_dim != 256) return tq_wide_restore_layer(dtype, head_dim, l, w, n_vec, cost_k, cost_v, stream);
-    return dtype == TQ_F16 ? launch_d256_restore_layer<TQ_F16>(l, w, n_vec, cost_k, cost_v, stream) : launch_d256_restore_layer<TQ_BF16>(l, w, n_vec, cost_k, cost_v, stream);
+    if (head_dim != 256) return tq_wide_restore_layer(dtype, head_dim, l, w, n_vec, stream);
+    return dtype == TQ_F16 ? launch_d256_restore_layer<TQ_F16>(l, w, n_vec, stream) : launch_d256_restore_layer<TQ_BF16>(l, w, n_vec, stream);
 }

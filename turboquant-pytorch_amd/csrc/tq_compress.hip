@@ -906,7 +906,7 @@ int launch_compress(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uin
 }
 
 template <int DTYPE>
-int launch_layer(TqLayer &l, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, void *workspace, bool paired, hipStream_t stream) {
+int launch_layer(TqLayer &l, uint32_t tiles, void *workspace, bool paired, hipStream_t stream) {
     DeviceInfo info;
     int rc = query_device(info);
     if (rc) return rc;
@@ -915,12 +915,12 @@ int launch_layer(TqLayer &l, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, v
     rc = resident_blocks(tq_compress_layer_kernel<DTYPE>, info, resident_on, resident);
     if (rc) return rc;
     const uint32_t slots = (uint32_t)(info.cus * resident);
-    uint32_t blocks = tq_layer_blocks(l, tiles, slots, cost_k, cost_v), tshift = 0;
+    uint32_t blocks = tq_layer_blocks(l, tiles, slots), tshift = 0;
     uint32_t *counters = nullptr;
     if (workspace && InTraits<DTYPE>::ELEM == 2 && TQ_COMPRESS_TICKET_SHIFT > 0) {       // as in launch_compress
         const uint32_t tickets = (tiles + (1u << TQ_COMPRESS_TICKET_SHIFT) - 1u) >> TQ_COMPRESS_TICKET_SHIFT;
         if (2u * tickets >= 4u * slots) {
-            blocks = tq_layer_blocks(l, tickets, slots, cost_k, cost_v);
+            blocks = tq_layer_blocks(l, tickets, slots);
             tshift = TQ_COMPRESS_TICKET_SHIFT;
             counters = static_cast<uint32_t *>(workspace);
         }
@@ -1030,14 +1030,13 @@ extern "C" int tq_compress_layer(const void *keys, const void *values, int dtype
             job.token_stride = token_stride * eb;
             l.bits[i] = i ? bits_v : bits_k;
         }
-        const uint32_t cost_k = (uint32_t)tq_vector_bytes(head_dim, eb, bits_k), cost_v = (uint32_t)tq_vector_bytes(head_dim, eb, bits_v);
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        if (head_dim != TQ_HEAD_DIM && !paired) return tq_anydim_compress_layer(dtype, head_dim, l, (uint32_t)n_vec, cost_k, cost_v, s);
+        if (head_dim != TQ_HEAD_DIM && !paired) return tq_anydim_compress_layer(dtype, head_dim, l, (uint32_t)n_vec, s);
         const uint32_t tiles = (uint32_t)(((paired ? n_vec / 2 : n_vec) + 31) / 32);
         switch (dtype) {
-            case TQ_F32: return launch_layer<TQ_F32>(l, tiles, cost_k, cost_v, workspace, paired, s);
-            case TQ_F16: return launch_layer<TQ_F16>(l, tiles, cost_k, cost_v, workspace, paired, s);
-            default: return launch_layer<TQ_BF16>(l, tiles, cost_k, cost_v, workspace, paired, s);
+            case TQ_F32: return launch_layer<TQ_F32>(l, tiles, workspace, paired, s);
+            case TQ_F16: return launch_layer<TQ_F16>(l, tiles, workspace, paired, s);
+            default: return launch_layer<TQ_BF16>(l, tiles, workspace, paired, s);
         }
     }
     rc = tq_compress(keys, dtype, rows, tokens, row_stride, token_stride, table_k, head_dim, bits_k, k_idx, k_norms, 0, workspace, stream);

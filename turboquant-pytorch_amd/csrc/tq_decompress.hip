@@ -470,8 +470,8 @@ int launch_layer_of(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint
     const int rc = allow_lds(reinterpret_cast<const void *>(&tq_restore_layer_kernel<DTYPE, PAIRED, W>), lds, configured);
     if (rc) return rc;
     const uint32_t want = (tiles + T::WAVES - 1) / T::WAVES;
-    const uint32_t blocks = tq_layer_blocks(l, want, (uint32_t)cus, cost_k, cost_v);
-    uint32_t *counters = 2u * want >= 4u * blocks ? static_cast<uint32_t *>(workspace) : nullptr;      // as in launch_decompress
+    uint32_t *counters = 2ull * want >= 4ull * (uint32_t)cus ? static_cast<uint32_t *>(workspace) : nullptr;      // as in launch_decompress
+    const uint32_t blocks = tq_layer_blocks(l, want, (uint32_t)cus, cost_k, cost_v, counters == nullptr);
     hipLaunchKernelGGL((tq_restore_layer_kernel<DTYPE, PAIRED, W>), dim3(blocks), dim3(T::WAVES * TQ_WAVE), lds, stream, l, window, counters);
     return (int)hipGetLastError();
 }
@@ -638,7 +638,7 @@ extern "C" int tq_restore_layer(const uint8_t *k_idx, const uint16_t *k_norms, c
         }
         const uint32_t cost_k = (uint32_t)tq_vector_bytes(head_dim, (int)elem, bits_k), cost_v = (uint32_t)tq_vector_bytes(head_dim, (int)elem, bits_v);
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        if (head_dim != TQ_HEAD_DIM && !paired) return tq_anydim_restore_layer(dtype, head_dim, l, w, (uint32_t)n_vec, cost_k, cost_v, s);
+        if (head_dim != TQ_HEAD_DIM && !paired) return tq_anydim_restore_layer(dtype, head_dim, l, w, (uint32_t)n_vec, s);
         const uint32_t tiles = (uint32_t)(((paired ? tq_pairs(r, t) : n_vec) + 31) / 32);
         auto launch = [&](auto type_tag) {
             constexpr int T = decltype(type_tag)::value;

@@ -55,7 +55,7 @@ struct TqBlock {
 };
 
 // Keys and values of a layer in one launch (plain calls of tq_compress_layer and tq_restore_layer): blocks [0, split) work on the
-// keys, the others on the values, each with the body of its own code width; blocks are dealt out by the bytes a vector costs.
+// keys, the others on the values, each with the body of its own code width.
 // A launch of its own for each paid for start and drain twice, with half the chip idle at the seam.  us a layer, compress + restore, two
 // launches each way and one for the window / one and one: 8 x 32640 tokens, bf16, K4/V2 95 / 81; 16 x 3968, fp16, K6/V4 44.5 / 35.5; 8 x 16256, 256 wide
 // 140 / 132; 32 x 5873, 80 wide 76 / 63.
@@ -69,12 +69,25 @@ __device__ __forceinline__ TqBlock tq_layer_block(const TqLayer &l, uint32_t whi
     return which ? TqBlock{blockIdx.x - l.split, gridDim.x - l.split} : TqBlock{blockIdx.x, l.split};
 }
 // Blocks of such a launch: as many as are resident at once (`slots`), at most `want` for either job, one each at least; sets l.split.
-static inline uint32_t tq_layer_blocks(TqLayer &l, uint32_t want, uint32_t slots, uint32_t cost_k, uint32_t cost_v) {
+// Halves by default: rotation and search (256 and the dimensions of tq_wide_kernel.h: decoding as well) take as long for every code width.  Dealt out by
+// the bytes of a vector, K4/V2 at 128 gave the keys 53 % of the blocks, and the values' blocks were the last by as much.  us a compress, by bytes /
+// halves: 8 x 32640 tokens, K4/V2 48.9 / 47.5; 16 x 3968, K6/V4 18.0 / 17.6; 16 x 20000, K8/V2 61.2 / 59.3; 256 wide, 8 x 9000, K8/V2 46.5 / 42.7; 80
+// wide, 32 x 5873, K4/V2 25.2 / 24.5; 64 wide, 8 x 60000, K4/V2 43.6 / 42.7.  A restore: 256 wide, 8 x 9000, K8/V2 27.4 / 25.9; 80 wide, as before, 19.5 / 18.5.
+// Costs: the 128-wide restore, whose time follows the bytes (16 x 20000, K8/V2 39.2 by bytes, 41.1 in halves).  Where blocks of its small jobs take a
+// few tiles each, fixed beforehand (`fixed`), whole tiles count: halves if the costlier job's last block is done sooner that way (16 x 3968, K6/V4: three
+// tiles for some waves by bytes, 11.8; two for all in halves, 10.7).
+static inline uint32_t tq_layer_blocks(TqLayer &l, uint32_t want, uint32_t slots, uint32_t cost_k = 1u, uint32_t cost_v = 1u, bool fixed = false) {
     uint32_t total = want < slots / 2u ? 2u * want : slots;
     if (total < 2u) total = 2u;
+    auto last = [&](uint32_t blocks, uint32_t cost) { return (unsigned long long)((want + blocks - 1u) / blocks) * cost; };
+    auto longest = [&](uint32_t k) {
+        const unsigned long long a = last(k, cost_k), b = last(total - k, cost_v);
+        return a > b ? a : b;
+    };
     uint32_t k = (uint32_t)((unsigned long long)total * cost_k / (cost_k + cost_v));
     if (k < 1u) k = 1u;
     if (k > total - 1u) k = total - 1u;
+    if (fixed && longest(total / 2u) < longest(k)) k = total / 2u;
     uint32_t v = total - k;
     if (k > want) k = want;
     if (v > want) v = want;

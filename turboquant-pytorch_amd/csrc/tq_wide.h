@@ -10,8 +10,8 @@ int tq_wide_compress(int dtype, int bits, int head_dim, const TqDevJob &single, 
 int tq_wide_decompress(int dtype, int bits, int head_dim, const TqDevJob &single, const tq_job *jobs_dev, int n_jobs,
                        uint32_t max_vec, hipStream_t stream);
 // keys and values of a layer in one launch (TqLayer: everything but `split` filled in)
-int tq_wide_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream);
-int tq_wide_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream);
+int tq_wide_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, hipStream_t stream);
+int tq_wide_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, hipStream_t stream);
 
 // The same for one padded dimension each (tq_wide_d96.hip ... tq_wide_d224.hip), `dl` of whose coordinates a vector has; arguments checked above.
 #define TQ_WIDE_DECLARE(D)                                                                                                                       \
@@ -19,8 +19,8 @@ int tq_wide_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCop
                               hipStream_t s);                                                                                                   \
     int tq_wide_decompress_d##D(int dtype, int bits, uint32_t dl, const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint32_t max_vec,     \
                                 hipStream_t s);                                                                                                 \
-    int tq_wide_compress_layer_d##D(int dtype, uint32_t dl, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t s);        \
-    int tq_wide_restore_layer_d##D(int dtype, uint32_t dl, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v,  \
+    int tq_wide_compress_layer_d##D(int dtype, uint32_t dl, TqLayer &l, uint32_t n_vec, hipStream_t s);        \
+    int tq_wide_restore_layer_d##D(int dtype, uint32_t dl, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec,  \
                                    hipStream_t s);
 TQ_WIDE_DECLARE(96)
 TQ_WIDE_DECLARE(160)

@@ -32,24 +32,24 @@ int tq_wide_decompress(int dtype, int bits, int head_dim, const TqDevJob &single
     }
 }
 
-int tq_wide_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+int tq_wide_compress_layer(int dtype, int head_dim, TqLayer &l, uint32_t n_vec, hipStream_t stream) {
     if (!tq_wide_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
     const uint32_t dl = (uint32_t)head_dim;
     switch (TQ_PADDED_DIM(head_dim)) {
-        case 96: return tq_wide_compress_layer_d96(dtype, dl, l, n_vec, cost_k, cost_v, stream);
-        case 160: return tq_wide_compress_layer_d160(dtype, dl, l, n_vec, cost_k, cost_v, stream);
-        case 192: return tq_wide_compress_layer_d192(dtype, dl, l, n_vec, cost_k, cost_v, stream);
-        default: return tq_wide_compress_layer_d224(dtype, dl, l, n_vec, cost_k, cost_v, stream);
+        case 96: return tq_wide_compress_layer_d96(dtype, dl, l, n_vec, stream);
+        case 160: return tq_wide_compress_layer_d160(dtype, dl, l, n_vec, stream);
+        case 192: return tq_wide_compress_layer_d192(dtype, dl, l, n_vec, stream);
+        default: return tq_wide_compress_layer_d224(dtype, dl, l, n_vec, stream);
     }
 }
 
-int tq_wide_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t stream) {
+int tq_wide_restore_layer(int dtype, int head_dim, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, hipStream_t stream) {
     if (!tq_wide_supported(head_dim, dtype)) return TQ_ERR_HEAD_DIM;
     const uint32_t dl = (uint32_t)head_dim;
     switch (TQ_PADDED_DIM(head_dim)) {
-        case 96: return tq_wide_restore_layer_d96(dtype, dl, l, w, n_vec, cost_k, cost_v, stream);
-        case 160: return tq_wide_restore_layer_d160(dtype, dl, l, w, n_vec, cost_k, cost_v, stream);
-        case 192: return tq_wide_restore_layer_d192(dtype, dl, l, w, n_vec, cost_k, cost_v, stream);
-        default: return tq_wide_restore_layer_d224(dtype, dl, l, w, n_vec, cost_k, cost_v, stream);
+        case 96: return tq_wide_restore_layer_d96(dtype, dl, l, w, n_vec, stream);
+        case 160: return tq_wide_restore_layer_d160(dtype, dl, l, w, n_vec, stream);
+        case 192: return tq_wide_restore_layer_d192(dtype, dl, l, w, n_vec, stream);
+        default: return tq_wide_restore_layer_d224(dtype, dl, l, w, n_vec, stream);
     }
 }

@@ -516,22 +516,22 @@ int launch(K kernel, int (&slots)[MAX_DEVICES], uint32_t lds, uint32_t threads, 
 }
 
 template <int DTYPE, int D, bool RAGGED>
-int launch_compress_layer(TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, uint32_t dl, hipStream_t s) {
+int launch_compress_layer(TqLayer &l, uint32_t n_vec, uint32_t dl, hipStream_t s) {
     static int slots[MAX_DEVICES] = {};
     int resident = 0;
     const int rc = resident_blocks(&tq_wide_compress_layer_kernel<DTYPE, D, RAGGED>, slots, Wide<D>::COMPRESS_LDS, Wide<D>::THREADS, resident);
     if (rc) return rc;
-    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)resident, cost_k, cost_v);
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)resident);
     hipLaunchKernelGGL((tq_wide_compress_layer_kernel<DTYPE, D, RAGGED>), dim3(blocks), dim3(Wide<D>::THREADS), Wide<D>::COMPRESS_LDS, s, l, dl);
     return (int)hipGetLastError();
 }
 template <int DTYPE, int D, bool RAGGED>
-int launch_restore_layer(TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, uint32_t dl, hipStream_t s) {
+int launch_restore_layer(TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t dl, hipStream_t s) {
     static int slots[MAX_DEVICES] = {};
     int resident = 0;
     const int rc = resident_blocks(&tq_wide_restore_layer_kernel<DTYPE, D, RAGGED>, slots, Wide<D>::DECOMPRESS_LDS, Wide<D>::THREADS, resident);
     if (rc) return rc;
-    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)resident, cost_k, cost_v);
+    const uint32_t blocks = tq_layer_blocks(l, (n_vec + 31u) / 32u, (uint32_t)resident);
     hipLaunchKernelGGL((tq_wide_restore_layer_kernel<DTYPE, D, RAGGED>), dim3(blocks), dim3(Wide<D>::THREADS), Wide<D>::DECOMPRESS_LDS, s, l, w, dl);
     return (int)hipGetLastError();
 }
@@ -590,18 +590,18 @@ int decompress_bits(int bits, const TqDevJob &job, const tq_job *jobs_dev, int n
         return dtype == TQ_F16 ? decompress_bits<TQ_F16, D>(bits, job, jobs_dev, n_jobs, max_vec, dl, s)                                         \
                                : decompress_bits<TQ_BF16, D>(bits, job, jobs_dev, n_jobs, max_vec, dl, s);                                       \
     }                                                                                                                                            \
-    int tq_wide_compress_layer_d##D(int dtype, uint32_t dl, TqLayer &l, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v, hipStream_t s) {       \
+    int tq_wide_compress_layer_d##D(int dtype, uint32_t dl, TqLayer &l, uint32_t n_vec, hipStream_t s) {       \
         if (dl != (uint32_t)D)                                                                                                                   \
-            return dtype == TQ_F16 ? launch_compress_layer<TQ_F16, D, true>(l, n_vec, cost_k, cost_v, dl, s)                                     \
-                                   : launch_compress_layer<TQ_BF16, D, true>(l, n_vec, cost_k, cost_v, dl, s);                                   \
-        return dtype == TQ_F16 ? launch_compress_layer<TQ_F16, D, false>(l, n_vec, cost_k, cost_v, dl, s)                                        \
-                               : launch_compress_layer<TQ_BF16, D, false>(l, n_vec, cost_k, cost_v, dl, s);                                      \
+            return dtype == TQ_F16 ? launch_compress_layer<TQ_F16, D, true>(l, n_vec, dl, s)                                     \
+                                   : launch_compress_layer<TQ_BF16, D, true>(l, n_vec, dl, s);                                   \
+        return dtype == TQ_F16 ? launch_compress_layer<TQ_F16, D, false>(l, n_vec, dl, s)                                        \
+                               : launch_compress_layer<TQ_BF16, D, false>(l, n_vec, dl, s);                                      \
     }                                                                                                                                            \
-    int tq_wide_restore_layer_d##D(int dtype, uint32_t dl, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec, uint32_t cost_k, uint32_t cost_v,  \
+    int tq_wide_restore_layer_d##D(int dtype, uint32_t dl, TqLayer &l, const TqWindowCopy &w, uint32_t n_vec,  \
                                    hipStream_t s) {                                                                                             \
         if (dl != (uint32_t)D)                                                                                                                   \
-            return dtype == TQ_F16 ? launch_restore_layer<TQ_F16, D, true>(l, w, n_vec, cost_k, cost_v, dl, s)                                   \
-                                   : launch_restore_layer<TQ_BF16, D, true>(l, w, n_vec, cost_k, cost_v, dl, s);                                 \
-        return dtype == TQ_F16 ? launch_restore_layer<TQ_F16, D, false>(l, w, n_vec, cost_k, cost_v, dl, s)                                      \
-                               : launch_restore_layer<TQ_BF16, D, false>(l, w, n_vec, cost_k, cost_v, dl, s);                                    \
+            return dtype == TQ_F16 ? launch_restore_layer<TQ_F16, D, true>(l, w, n_vec, dl, s)                                   \
+                                   : launch_restore_layer<TQ_BF16, D, true>(l, w, n_vec, dl, s);                                 \
+        return dtype == TQ_F16 ? launch_restore_layer<TQ_F16, D, false>(l, w, n_vec, dl, s)                                      \
+                               : launch_restore_layer<TQ_BF16, D, false>(l, w, n_vec, dl, s);                                    \
     }
