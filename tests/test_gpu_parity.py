@@ -759,3 +759,30 @@ def test_float32_vectors_do_not_depend_on_the_size_of_their_job(pkg, dim, bits, 
             for key in ("idx_bytes", "vec_norms"):
                 assert torch.equal(part[key], whole[key][:, r:r + 1, t:t + 1000]), (key, r, t)
             assert torch.equal(comp.decompress(part), out[:, r:r + 1, t:t + 1000]), (r, t)
+
+
+@pytest.mark.parametrize("dim", [128, 64])
+@pytest.mark.parametrize("tokens", [640, 20010, 70002])
+def test_float32_norms_come_from_one_order_of_additions(pkg, dim, tokens):
+    """The squares of a float32 vector are added in one order whatever the size of the call: chains over the even and the odd elements of
+    either half of the 16-element steps, the two of a half first, then the halves.  One large element and small ones whose squares it
+    swallows make the order visible: sums about M^2, M half-way between two float16 norms.  Sums within four units of M^2 are left out:
+    the square root behind them is good to two float32 units, half as many units of the sum each."""
+    rng = np.random.default_rng(dim + tokens)
+    m = 1.0 + 2.0 ** -11
+    x = rng.integers(2896, 4096, (tokens, dim)) * 2.0 ** -24          # squares of 2^-25 to 2^-24 in 24 bits
+    x[np.arange(tokens), rng.integers(0, 16, tokens)] = m - rng.integers(0, dim // 4, tokens) * 2.0 ** -23
+    x = x.astype(np.float32)
+    steps = x.reshape(tokens, dim // 16, 2, 4, 2).astype(np.float64)
+    chain = np.zeros((tokens, 2, 2), dtype=np.float32)
+    for s in range(dim // 16):
+        for i in range(4):
+            chain = (steps[:, s, :, i] ** 2 + chain).astype(np.float32)      # (exact in float64: a fused multiply-add)
+    half = chain[..., 0] + chain[..., 1]
+    ss = (half[:, 0] + half[:, 1]).astype(np.float64)
+    clear = np.abs(ss - m * m) > 4 * 2.0 ** -23
+    assert clear.mean() > 0.5 and 0.1 < (ss > m * m).mean() < 0.95
+    want = np.where(ss > m * m, 1.0 + 2.0 ** -10, 1.0)
+    comp = pkg.MSECompressor(dim, 4, seed=42, device=DEV)
+    got = comp.compress(torch.from_numpy(x).to(DEV).view(1, 1, tokens, dim))["vec_norms"].cpu().numpy().reshape(-1).astype(np.float64)
+    assert (got[clear] == want[clear]).all(), int((got[clear] != want[clear]).sum())

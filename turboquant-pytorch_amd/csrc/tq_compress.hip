@@ -209,27 +209,35 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     };
     const float grid_scale = hd->grid_scale, grid_bias = hd->grid_bias;
 
-    const uint32_t ld_vec = lane / PIECES, ld_piece = lane % PIECES;  // role in the coalesced loads
+    // Role in the loads, 16 bytes a lane.  16-bit inputs: piece ld_piece of vector ld_vec of every four.  fp32 inputs: eight lanes share a
+    // vector; lane (vk, vq) has the eight elements of half vk of steps 2 vq and 2 vq + 1, pieces ld_piece + {0, 1, 4, 5} (see park).
+    const uint32_t vk = (lane >> 2) & 1u, vq = lane & 3u;
+    const uint32_t ld_vec = ELEM == 2 ? lane / PIECES : lane >> 3, ld_piece = ELEM == 2 ? lane % PIECES : 8u * vq + 2u * vk;
     const uint32_t n = lane & 31u, hk = lane >> 5;                    // role in the MFMA: column, half
     const uint32_t half = wave >> 1;                                  // paired rows: the 64-wide vector this wave's coordinates belong to
 
-    // LDS offset of this lane's piece of load j (computed where it is used: these paths are not the hot one)
+    // LDS offset of this lane's piece of load j of 16-bit inputs (computed where it is used: these paths are not the hot one)
     auto st_off = [&](int j) {
         const uint32_t vl = (wave * NLOAD + j) * VEC_PER_LOAD + ld_vec;
-        if constexpr (ELEM == 2) return vl * VEC_BYTES + ((ld_piece ^ (vl & 15u)) << 4);
-        else return vl * (VEC_BYTES / 2) + (((ld_piece >> 1) ^ (vl & 15u)) << 4) + (ld_piece & 1u) * 8u;      // of a term: four of its values
+        return vl * VEC_BYTES + ((ld_piece ^ (vl & 15u)) << 4);
     };
 
     tq_u4 pre[NLOAD];
     // loads of this wave's quarter of tile `tl`, generic addressing (any strides, tail clamped)
+    auto load_vector = [&](const uint8_t *at) {      // fp32 inputs
+#pragma unroll
+        for (int j = 0; j < NLOAD; ++j) pre[j] = tq_gload16(at + (j / 2) * 64 + (j % 2) * 16);
+    };
     auto issue_loads = [&](auto full_tag, uint32_t tl) {
         constexpr bool FULL = decltype(full_tag)::value;
         const uint32_t v0 = tl * 32u + (wave * NLOAD) * VEC_PER_LOAD + ld_vec;
 #pragma unroll
-        for (int j = 0; j < NLOAD; ++j) {
+        for (int j = 0; j < (ELEM == 2 ? NLOAD : 1); ++j) {
             uint32_t v = v0 + j * VEC_PER_LOAD;
             if (!FULL) v = v < job.n_vec ? v : job.n_vec - 1u;   // tail: re-read the last vector, never stored
-            pre[j] = tq_gload16(job.states + tq_vec_offset(job, v) + ld_piece * 16u);
+            const uint8_t *at = job.states + tq_vec_offset(job, v) + ld_piece * 16u;
+            if constexpr (ELEM == 2) pre[j] = tq_gload16(at);
+            else load_vector(at);
         }
     };
 
@@ -243,7 +251,11 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
         return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x110 + N, 0xf, 0xf, true));
     };
     // fp32 inputs are split into their terms here, once (by the waves that read the operands it took four times as many vector
-    // instructions as everything else together); their squares are summed per half of a row, the 16 lanes of a DPP row, in slot `slot`.
+    // instructions as everything else together).  Their squares are added in the order in which those waves walked a vector, which fixes the
+    // last bit of the norm and with it the codes next to a boundary: four chains, over the even and the odd elements of either half (hk) of
+    // the steps 0..7.  The eight lanes of a vector, two steps of a half each, hand the chains on from lane to lane.  The sum ends up in
+    // element 1 of slot `slot`; pairs of 64-wide vectors, four steps each, use both.  (131168 vectors, 4-bit: 31.5 us.  Squares added by lanes
+    // of whole loads, in an order of their own, 30.9; in this order from such loads, pieces exchanged through the LDS, 3 us more.)
     auto park = [&](uint32_t b, uint32_t slot, const tq_u4 (&src)[NLOAD]) {
         uint8_t *stage = lds_stage[b];
         if constexpr (ELEM == 2) {
@@ -260,34 +272,48 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
                 if ((lane & 7u) == 7u) lds_ssh[b][(wave * NLOAD + j) * VEC_PER_LOAD + ld_vec][(lane >> 3) & 1u] = pair;   // pieces 0..7, 8..15
             }
         } else {
+            static_assert(NLOAD == 4 && VEC_PER_LOAD == 2, "eight vectors a wave, four pieces a lane");
+            const bool first = vq == 0u || (paired && vq == 2u);
+            auto handed_on = [&](float s) {      // from the lane before it in its quad
+                const float t = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x90, 0xf, 0xf, true));
+                return first ? 0.f : t;
+            };
+            float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-            for (int j = 0; j < NLOAD; ++j) {
-                tq_u2 t[3];
-                float ss = 0.f;
+            for (int turn = 0; turn < 4; ++turn) {      // (after turn t the chains are right up to lane t of the quad)
+                if (turn) {
+                    s0 = handed_on(s0);
+                    s1 = handed_on(s1);
+                }
 #pragma unroll
-                for (int d = 0; d < 2; ++d) {      // x = its three terms exactly: every term a truncation, every remainder exact
+                for (int i = 0; i < 16; i += 2) {
+                    const tq_u4 &p = src[i / 4];
+                    const float e = __uint_as_float(p[i % 4]), o = __uint_as_float(p[i % 4 + 1]);
+                    s0 = fmaf(e, e, s0);
+                    s1 = fmaf(o, o, s1);
+                }
+            }
+            const float one = s0 + s1, both = one + row_shr(one, std::integral_constant<int, 4>{});       // at vk == 1
+            if (vk == 1u && (vq & 1u)) lds_ssh[slot][wave * 8u + ld_vec][vq >> 1] = both;
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                tq_u4 t[3];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {      // x = its three terms exactly: every term a truncation, every remainder exact
                     uint32_t r[2][3];
 #pragma unroll
                     for (int i = 0; i < 2; ++i) {
-                        const float x = __uint_as_float(src[j][2 * d + i]);
-                        const float r1 = x - __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+                        const float f = __uint_as_float(src[2 * a + d / 2][d % 2 * 2 + i]);
+                        const float r1 = f - __uint_as_float(__float_as_uint(f) & 0xffff0000u);
                         const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
-                        ss = fmaf(x, x, ss);
-                        r[i][0] = __float_as_uint(x); r[i][1] = __float_as_uint(r1); r[i][2] = __float_as_uint(r2);
+                        r[i][0] = __float_as_uint(f); r[i][1] = __float_as_uint(r1); r[i][2] = __float_as_uint(r2);
                     }
 #pragma unroll
                     for (int k = 0; k < 3; ++k) t[k][d] = __builtin_amdgcn_perm(r[1][k], r[0][k], 0x07060302u);
                 }
+                const uint32_t vl = wave * 8u + ld_vec, at = vl * (TQ_HEAD_DIM * 2) + (((4u * vq + 2u * a + vk) ^ (vl & 15u)) << 4);
 #pragma unroll
-                for (int k = 0; k < 3; ++k) *reinterpret_cast<tq_u2 *>(stage + k * TERM + st_off(j)) = t[k];
-                auto add_rotated = [&](auto n_tag) {
-                    ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x120 + decltype(n_tag)::value, 0xf, 0xf, true));
-                };
-                add_rotated(std::integral_constant<int, 8>{});
-                add_rotated(std::integral_constant<int, 4>{});
-                add_rotated(std::integral_constant<int, 2>{});
-                add_rotated(std::integral_constant<int, 1>{});
-                if ((lane & 15u) == 0u) lds_ssh[slot][(wave * NLOAD + j) * VEC_PER_LOAD + ld_vec][(lane >> 4) & 1u] = ss;
+                for (int k = 0; k < 3; ++k) *reinterpret_cast<tq_u4 *>(stage + k * TERM + at) = t[k];
             }
         }
     };
@@ -327,7 +353,7 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
     };
     auto scale_of = [&](uint32_t slot) {
         if constexpr (ELEM == 2) return scale_from_ss(paired ? lds_ssh[slot][n][half] : lds_ss[slot][n]);
-        else return scale_from_ss(paired ? lds_ssh[slot][n][half] : lds_ssh[slot][n][0] + lds_ssh[slot][n][1]);
+        else return scale_from_ss(lds_ssh[slot][n][paired ? half : 1u]);
     };
 
     // (3) code search + packing.  Lane (n, hk) of wave w holds coordinates 32w + 16hk + r.
@@ -713,8 +739,8 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
             // fp32 elements, any rows: the same with the search of tile k-1 between the matrix instructions of tile k, from the other
             // accumulator set (sums of squares wait in three slots).  Six bf16 products a step keep the matrix pipe busy for a third of the
             // time, set-up and the first tile take another 4 us; the rest are waits of two waves a SIMD, the rotation's three terms leave no
-            // registers for a third (nor for loads two tiles ahead: 32.5 us, spilled).  131168 vectors, 4-bit: 34.8 us while every wave
-            // split the whole tile into its terms, now 29.8.
+            // registers for a third (nor for loads two tiles ahead: 32.5 us, spilled).  131168 vectors, 4-bit: 34.6 us while every wave
+            // split the whole tile into its terms, now 31.5.
             const uint32_t m = (n_full - tile + tile_stride - 1u) / tile_stride;      // this block's full tiles
             auto only_one = [&]() __attribute__((always_inline)) {          // a small job: nothing to overlap
                 issue_loads(std::true_type{}, tile);
@@ -727,13 +753,9 @@ __device__ __forceinline__ void compress_job(const TqDevJob &job, TqBlock blk, u
             };
             auto several = [&]() __attribute__((always_inline)) {
                 TqTileWalk ahead(job, tile, tile_stride), done = ahead;
-                long long own[NLOAD];
-#pragma unroll
-                for (int j = 0; j < NLOAD; ++j) own[j] = (long long)((wave * NLOAD + j) * VEC_PER_LOAD + ld_vec) * job.token_stride + ld_piece * 16u;
-                auto issue = [&]() {
-#pragma unroll
-                    for (int j = 0; j < NLOAD; ++j) pre[j] = tq_gload16(job.states + ahead.offset(job, (wave * NLOAD + j) * VEC_PER_LOAD + ld_vec, own[j]));
-                };
+                const uint32_t first = wave * 8u + ld_vec;
+                const long long own = (long long)first * job.token_stride + ld_piece * 16u;
+                auto issue = [&]() { load_vector(job.states + ahead.offset(job, first, own)); };
                 auto trip = [&](auto rot_tag, auto search_tag, uint32_t j, tq_f16v &acc_new, const tq_f16v &acc_old) {
                     constexpr bool ROT = decltype(rot_tag)::value, SEARCH = decltype(search_tag)::value;
                     const bool more = ROT && j + 1u < m;
