@@ -887,6 +887,28 @@ def test_decode_attention_deals_out_window_and_history(pkg, dim, bits, rows, tok
 
 
 @pytest.mark.parametrize("dim", [64, 96, 128, 256])
+@pytest.mark.parametrize("rows,tokens", [(2, 1000), (4, 6000), (8, 20000), (40, 1300)])
+def test_decode_attention_sums_the_history_alike_whatever_the_window_holds(pkg, dim, rows, tokens):
+    """Windows of no weight at all, logits below -1000: bit for bit what the history gives without one, whatever their size.  (Histories cut
+    by what the window takes came out rounded another way: 8e-4 at 128.)"""
+    g = torch.Generator().manual_seed(dim + tokens)
+    k, v = (torch.randn(1, rows, tokens, dim, generator=g).half().to(DEV) for _ in range(2))
+    q = torch.randn(1, rows * 8, 1, dim, generator=g)
+    q[..., 0] = 8.0
+    q = q.half().to(DEV)
+    want = None
+    for window in (0, 16, 100, 128, 500):
+        far = torch.zeros(1, rows, window, dim)
+        far[..., 0] = -250.0 * dim ** 0.5
+        part = torch.randn(1, rows, window, dim, generator=g).half().to(DEV)
+        cache = pkg.V3Cache(4, 2, residual_window=window, n_layers=40)
+        cache.append(torch.cat([k, far.half().to(DEV)], 2), torch.cat([v, part], 2), 8)
+        got = cache.attend(q, 8)
+        want = got if want is None else want
+        assert torch.equal(got, want), (window, float((got.double() - want.double()).norm() / want.double().norm()))
+
+
+@pytest.mark.parametrize("dim", [64, 96, 128, 256])
 @pytest.mark.parametrize("bits", [(4, 2), (8, 3), (6, 4)])
 def test_one_launch_append_stores_the_bytes_of_compress(pkg, dim, bits):
     """tq_decode_append against MSECompressor.compress on the evicted tokens (1 to 70 rows: full and partial tiles of rows)."""

@@ -15,7 +15,7 @@ struct TqDecodeArgs {
     uint8_t *out;                    // [rows, group, D]
     long long win_stride;
     float scale;
-    uint32_t tokens, packed_row_stride, group, chunk, win_cost, n_win, bf16;       // split s: chunk tokens, less win_cost if it has a tile of the window
+    uint32_t tokens, packed_row_stride, group, chunk, n_win, bf16;
 };
 
 namespace {

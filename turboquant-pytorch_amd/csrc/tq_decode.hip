@@ -275,14 +275,7 @@ extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *querie
     a.tokens = (uint32_t)tokens;
     a.packed_row_stride = (uint32_t)layer->packed_row_stride;
     a.group = (uint32_t)group;
-    // A tile of the window takes its wave 2.3 us (256 wide: 4.4), about as long as a run of 64 tokens: a split that has one gets that much less of
-    // the history, where no split has two.  (Clock stamps, 8 rows x 32768 tokens, last wave of a block out of its loop: 9.6 us in the median block, 11.5 in those
-    // with a tile without this, 10.4 with it.)
-    const long long win_tiles = (n_win + WIN_TILE - 1) / WIN_TILE;
-    constexpr long long WIN_COST = 64;
-    auto chunk = [&](long long cost) { return ((tokens + win_tiles * cost + splits - 1) / splits + 15) / 16 * 16; };
-    a.win_cost = splits > 1 && win_tiles <= splits && chunk(WIN_COST) >= WIN_COST ? (uint32_t)WIN_COST : 0u;
-    a.chunk = (uint32_t)chunk(a.win_cost);
+    a.chunk = (uint32_t)(((tokens + splits - 1) / splits + 15) / 16 * 16);
     a.n_win = (uint32_t)n_win;
     a.bf16 = layer->dtype == TQ_BF16 ? 1u : 0u;
     if (!tokens) {       // no history: the loads that every wave starts with find the tables instead, and nothing is done with them

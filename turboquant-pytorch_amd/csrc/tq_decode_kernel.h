@@ -322,7 +322,7 @@ struct WindowTile {
 // tokens dealt out evenly; records merged with one trip to memory and a code of a few hundred bytes (code that runs once is fetched from
 // the L2 as it goes: 1 us for 2.4 KiB of it), rows of Pi_v under way before the block knows that it needs them, last arrival to result 5.5 / 3.4.
 // A tile of the window used to stand before the block's barrier: everybody in it waited 2.3 us (256 wide 4.4) for the wave that had it, and the row for the
-// block.  It is finished behind the barrier now, and its block takes 64 tokens less (see tq_decode_attend); records are merged without loops around their
+// block.  It is finished behind the barrier now; records are merged without loops around their
 // loads.  us a step of eight layers, append and attend: 8 rows x 32768 tokens 170 -> 164; 64 wide, 32 x 6000, K6/V4 146 -> 130; 96 wide, 2 x 8574
 // 130 -> 118; 256 wide, 8 x 9906, K3/V2 291 -> 262; 512 x 16384 1366 -> 1354.
 // Before that, whole step of 32 layers 948 -> 778 us (734 since the append asks for all of its loads at once, see tq_decode.hip); 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
@@ -391,9 +391,9 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     const bool live = head < G;
 
     const uint32_t win_tiles = (a.n_win + WIN_TILE - 1u) / WIN_TILE;     // tile w goes to the block of split w % splits
-    // (a split that has a tile of the window takes win_cost tokens less, see tq_decode_attend)
-    const uint32_t t_begin = min(a.tokens, split * a.chunk - min(split, win_tiles) * a.win_cost);
-    const uint32_t t_end = min(a.tokens, (split + 1u) * a.chunk - min(split + 1u, win_tiles) * a.win_cost);
+    // (the same cut of the history whatever the window holds: a sum in other parts is another rounding)
+    const uint32_t t_begin = min(a.tokens, split * a.chunk);
+    const uint32_t t_end = min(a.tokens, t_begin + a.chunk);
     const size_t slot0 = (size_t)row * a.packed_row_stride;
     uint8_t *vcodes = lds_area[wave];
     // Runs of a wave: in every whole round of the block one of RUN tokens; what is left of the block's tokens is dealt out evenly, in
