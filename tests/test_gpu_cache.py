@@ -886,6 +886,22 @@ def test_decode_attention_deals_out_window_and_history(pkg, dim, bits, rows, tok
         assert err < (1.5e-3 if dim == 128 else 3.5e-4), (group, err)
 
 
+@pytest.mark.parametrize("dim,bits", [(64, (6, 4)), (96, (4, 2)), (128, (4, 2)), (128, (8, 4)), (256, (4, 2))])
+@pytest.mark.parametrize("rows,tokens,window", [(1, 150, 32), (2, 1500, 128), (1, 9000, 128), (1, 16000, 160)])
+def test_decode_attention_of_any_number_of_heads(pkg, dim, bits, rows, tokens, window):
+    """Heads that end at every place of what a wave weighs, a pass merges and is rotated back, against float64 over the store as the kernel
+    holds it; one split, up to 32, 64 and more records.  Bounds as in test_decode_attention_merges_many_splits."""
+    g = torch.Generator().manual_seed(dim + tokens)
+    cache = pkg.V3Cache(bits[0], bits[1], residual_window=window, n_layers=40)
+    k, v = (torch.randn(1, rows, tokens + window, dim, generator=g).half().to(DEV) for _ in range(2))
+    cache.append(k, v, 8)
+    for group in (2, 3, 5, 6, 8, 9, 10, 11, 12, 13, 15, 16):
+        q = 2 * torch.randn(1, rows * group, 1, dim, generator=g).half().to(DEV)
+        ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
+        err = float((cache.attend(q, 8).double().reshape(ref.shape) - ref).norm() / ref.norm())
+        assert err < (1.5e-3 if dim == 128 else 3.5e-4), (group, err)
+
+
 @pytest.mark.parametrize("dim", [64, 96, 128, 256])
 @pytest.mark.parametrize("rows,tokens", [(2, 1000), (4, 6000), (8, 20000), (40, 1300)])
 def test_decode_attention_sums_the_history_alike_whatever_the_window_holds(pkg, dim, rows, tokens):

@@ -368,8 +368,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     constexpr int QROW = D + 4;                          // rotated queries in LDS, floats per head
     constexpr int ROTP = DTHREADS / (D / 4) >= 16 ? 16 : DTHREADS / (D / 4);     // parts of the contraction when rotating back
     constexpr int ROTK = D / ROTP;                       // rows of Pi_v per part
-    constexpr int RG = 4;                                // heads rotated back at a time (8: twice the work where a row has 4, at 256 3.4 us for 2.0)
-    static_assert(DW * AREA >= 2 * MAX_GROUP * D * 4 && ROTP * RG * D * 4 <= 65536, "LDS areas too small");
+    static_assert(DW * AREA >= 2 * MAX_GROUP * D * 4, "LDS area too small");
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds_lut[65536];      // (the strictest alignment: lies at address 0, where no base has to be added)
     __shared__ __attribute__((aligned(16))) uint8_t lds_area[DW][AREA];
@@ -1042,9 +1041,13 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         __syncthreads();
     };
     if (splits > 1u) merge(std::true_type{}); else merge(std::false_type{});
-    // out = (ysum @ Pi_v + wsum) / den, RG heads at a time
+    // out = (ysum @ Pi_v + wsum) / den, eight heads at a time as long as more than four are left, then four: eight are twice the work where a
+    // row has four (at 256 3.4 us for 2.0), and every pass costs two barriers (all in fours / this, 4 rows x 6000 tokens, us: 64 wide, 16 heads
+    // 18.8 / 18.1, 8 heads 13.5 / 13.2; 128 wide 25.6 / 25.1, 17.9 / 17.7)
     float *parts = reinterpret_cast<float *>(lds_lut);            // [part][RG][D]
-    for (uint32_t g0 = 0; g0 < G; g0 += RG) {
+    auto rotate_back = [&](auto heads, uint32_t g0) __attribute__((always_inline)) {
+        constexpr int RG = decltype(heads)::value;
+        static_assert(ROTP * RG * D * 4 <= 65536, "LDS area too small");
         float x[RG][4];
 #pragma unroll
         for (int g = 0; g < RG; ++g)
@@ -1077,7 +1080,11 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
             if (a.bf16) { const __bf16 h = (__bf16)v; *o = __builtin_bit_cast(uint16_t, h); }
             else { const _Float16 h = (_Float16)v; *o = __builtin_bit_cast(uint16_t, h); }
         }
-    }
+    };
+    uint32_t g0 = 0;
+    if constexpr (C != 4)
+        for (; G - g0 > 4u && g0 < G; g0 += 8u) rotate_back(std::integral_constant<int, 8>{}, g0);
+    if (g0 < G) rotate_back(std::integral_constant<int, 4>{}, g0);
 }
 
 template <int D, int IPBK, int IPBV>
