@@ -895,6 +895,9 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     // tokens, 64 wide, from the last arrival to merged sums: 1.9 us with loops, now 1.4).  What is left grows with the records: one compute unit reads
     // what other dies wrote at some 27 KB/us (8 rows x 32768, 66 KB: 2.4 us; 256 wide, 8 x 9906, 120 KB and 256 KB of Pi_v: 5.2).  Little code: it runs once and is fetched for the first time
     // (33 loads a lane, written out: 2.0 us from the first to the last of them, now 0.4).
+    // Two heads a wave where a row has more than eight: they went through the loops of `many` (16 heads, 32 rows x 6000 tokens, us: 64 wide
+    // 20.4, this way 18.2, 128 wide 28.7 / 25.8).  `many` takes the references with as few loads as there are records for, and asks for a further 32
+    // records only where there are any (2 rows x 20000 tokens, about 40 splits, 128 wide, 8 heads 21.9 / 20.9, 16 heads 29.7 / 27.3).
     auto merge = [&](auto across_tag) __attribute__((always_inline)) {
         constexpr bool ACROSS = decltype(across_tag)::value;
         const uint32_t step = G * PART, nrec = splits + win_tiles;    // (a row's records lie within 4.5 MiB)
@@ -971,9 +974,11 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         };
         auto few = [&](auto passes) __attribute__((always_inline)) {
             constexpr int N = decltype(passes)::value;                // of 512 columns
+            constexpr int H = C == 1 ? 2 : 1;                         // heads a wave weighs
             tq_u4 y[N][8], w[N];
-            tq_u2 ml[1];
-            load_heads(ml, wave);
+            tq_u2 ml[H][1];
+#pragma unroll
+            for (int h = 0; h < H; ++h) load_heads(ml[h], wave + h * DW);
 #pragma unroll
             for (int k = 0; k < N; ++k) {
                 const uint32_t p = col + k * DTHREADS, off = p / D * PART + 2u + p % D;
@@ -982,7 +987,9 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (N <= 2) load_pv();                          // (more columns leave no registers for them yet)
-            if (wave < G) weigh(ml, wave);
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+                if (wave + h * DW < G) weigh(ml[h], wave + h * DW);
             __syncthreads();
 #pragma unroll
             for (int k = 0; k < N; ++k) {
@@ -997,48 +1004,55 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
             if constexpr (N > 2) load_pv();
             __syncthreads();
         };
-        if (G <= (uint32_t)DW && splits <= 32u && win_tiles <= 4u) {
-            if (G * D <= (uint32_t)DTHREADS) { few(std::integral_constant<int, 1>{}); return; }
-            if constexpr (DW * D > DTHREADS) {
+        if (splits <= 32u && win_tiles <= 4u) {      // (launched for at most HEADS heads, HEADS = 16 for 9 at least, see launch_decode)
+            constexpr int LEAST = C == 1 ? 9 : 1;
+            if constexpr (LEAST * D <= DTHREADS) {
+                if (G * D <= (uint32_t)DTHREADS) { few(std::integral_constant<int, 1>{}); return; }
+            }
+            if constexpr (HEADS * D > DTHREADS && LEAST * D <= 2 * DTHREADS) {
                 if (G * D <= 2u * DTHREADS) { few(std::integral_constant<int, 2>{}); return; }
             }
-            if constexpr (DW * D > 2 * DTHREADS) { few(std::integral_constant<int, 4>{}); return; }
+            if constexpr (HEADS * D > 2 * DTHREADS && HEADS * D <= 4 * DTHREADS) { few(std::integral_constant<int, 4>{}); return; }
         }
-        tq_u4 y[8], w;
-        tq_u2 ml[(MAX_SPLITS + MAX_WINDOW / WIN_TILE + 63) / 64];
-        load_heads(ml, wave);
-        fetch(y, col / D * PART + 2u + col % D, 0u);
-        w = wpart.load4<ACROSS>(q4 * step + col / D * PART + 2u + col % D);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (D <= 128) load_pv();
-        for (uint32_t g = wave; g < G; g += DW) {
-            if (g != wave) load_heads(ml, g);
-            weigh(ml, g);
-        }
-        __syncthreads();
-        for (uint32_t p = col; p < G * D; p += DTHREADS) {
-            const uint32_t g = p / D, off = g * PART + 2u + p % D;
-            const float *f = wgt + g * wrow + q4;
-            if (p != col) {
-                fetch(y, off, 0u);
-                w = wpart.load4<ACROSS>(q4 * step + off);
+        auto many = [&](auto reads) __attribute__((always_inline)) {      // of 64 records' references each
+            tq_u4 y[8], w;
+            tq_u2 ml[decltype(reads)::value];
+            load_heads(ml, wave);
+            fetch(y, col / D * PART + 2u + col % D, 0u);
+            w = wpart.load4<ACROSS>(q4 * step + col / D * PART + 2u + col % D);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (D <= 128) load_pv();
+            for (uint32_t g = wave; g < G; g += DW) {
+                if (g != wave) load_heads(ml, g);
+                weigh(ml, g);
             }
-            clear();
-            for (uint32_t s0 = 0;;) {       // the next 32 records under way (past the last one: zeros) while these are added
-                tq_u4 z[8];
-                fetch(z, off, s0 + 32u);
-                add_records(y, f, s0);
-                s0 += 32u;
-                if (s0 >= splits) break;
+            __syncthreads();
+            for (uint32_t p = col; p < G * D; p += DTHREADS) {
+                const uint32_t g = p / D, off = g * PART + 2u + p % D;
+                const float *f = wgt + g * wrow + q4;
+                if (p != col) {
+                    fetch(y, off, 0u);
+                    w = wpart.load4<ACROSS>(q4 * step + off);
+                }
+                clear();
+                uint32_t s0 = 0;
+                for (; s0 + 32u < splits; s0 += 32u) {       // the next 32 records under way while these are added
+                    tq_u4 z[8];
+                    fetch(z, off, s0 + 32u);
+                    add_records(y, f, s0);
 #pragma unroll
-                for (int s = 0; s < 8; ++s) y[s] = z[s];
+                    for (int s = 0; s < 8; ++s) y[s] = z[s];
+                }
+                add_records(y, f, s0);
+                if (win_tiles) add_window(w, f[wfirst]);
+                for (uint32_t t = 4u; t < win_tiles; t += 4u) add_window(wpart.load4<ACROSS>((t + q4) * step + off), f[wfirst + t]);
+                put_sums(p);
             }
-            if (win_tiles) add_window(w, f[wfirst]);
-            for (uint32_t s0 = 4u; s0 < win_tiles; s0 += 4u) add_window(wpart.load4<ACROSS>((s0 + q4) * step + off), f[wfirst + s0]);
-            put_sums(p);
-        }
-        if constexpr (D > 128) load_pv();
-        __syncthreads();
+            if constexpr (D > 128) load_pv();
+            __syncthreads();
+        };
+        if (wrow <= 64u) many(std::integral_constant<int, 1>{});
+        else many(std::integral_constant<int, (MAX_SPLITS + MAX_WINDOW / WIN_TILE + 63) / 64>{});
     };
     if (splits > 1u) merge(std::true_type{}); else merge(std::false_type{});
     // out = (ysum @ Pi_v + wsum) / den, eight heads at a time as long as more than four are left, then four: eight are twice the work where a
