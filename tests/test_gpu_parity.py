@@ -786,3 +786,30 @@ def test_float32_norms_come_from_one_order_of_additions(pkg, dim, tokens):
     comp = pkg.MSECompressor(dim, 4, seed=42, device=DEV)
     got = comp.compress(torch.from_numpy(x).to(DEV).view(1, 1, tokens, dim))["vec_norms"].cpu().numpy().reshape(-1).astype(np.float64)
     assert (got[clear] == want[clear]).all(), int((got[clear] != want[clear]).sum())
+
+
+@pytest.mark.parametrize("dim,bits", [(128, 4), (128, 8), (64, 2), (64, 1)])
+@pytest.mark.parametrize("tiles", [1023, 1024, 1025, 2048, 2049, 3073, 8191, 8193])
+def test_float32_results_do_not_depend_on_the_size_of_the_blocks(pkg, dim, bits, tiles):
+    """Restores to float32 on either side of where blocks of four and of eight waves take turns (rounds of 4 x 256 tiles): the same values as
+    the same vectors in calls of a few tiles, alone, in a list and as a layer with a window."""
+    comp = pkg.MSECompressor(dim, bits, seed=42, device=DEV)
+    n = tiles * 32 * (128 // dim) - 5
+    x = outlier_kv((1, 1, 4096, dim), seed=dim + bits, dtype=torch.float32).to(DEV)
+    few = comp.compress(x)
+    back = comp.decompress(few)
+    repeat = lambda t: t.repeat((1, 1, -(-n // 4096)) + (1,) * (t.dim() - 3))[:, :, :n].contiguous()  # noqa: E731
+    packed = {"idx_bytes": repeat(few["idx_bytes"]), "vec_norms": repeat(few["vec_norms"])}
+    want = repeat(back)
+    out = torch.empty((1, 1, n, dim), device=DEV)
+    comp.decompress_packed(packed["idx_bytes"], packed["vec_norms"], out)
+    assert torch.equal(out, want)
+    out.zero_()
+    jobs = [{"states": out[:, :, a:b], "idx_bytes": packed["idx_bytes"][:, :, a:b], "vec_norms": packed["vec_norms"][:, :, a:b], "table": comp.table(), "bits": bits}
+            for a, b in ((0, n // 64 * 32), (n // 64 * 32, n))]
+    pkg._native.JobList(jobs, torch.device(DEV)).decompress()
+    assert torch.equal(out, want)
+    half, win = n // 2, torch.randn((1, 1, 5, dim), device=DEV)
+    part = (packed["idx_bytes"][:, :, :half], packed["vec_norms"][:, :, :half])
+    for got in pkg._native.restore_layer(part, part, half, comp.table(), comp.table(), bits, bits, win, win):
+        assert torch.equal(got[:, :, :half], want[:, :, :half]) and torch.equal(got[:, :, half:], win)

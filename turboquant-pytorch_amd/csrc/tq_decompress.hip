@@ -43,10 +43,9 @@ static __device__ __align__(256) uint32_t scratch[TQ_NOALLOC_MAX_JOBS * (TQ_WORK
 
 namespace {
 
-// Waves of a block: one block is resident per compute unit (Pi^T is staged once a block), so eight, two to a SIMD.  32-bit outputs of up to
-// six tiles a compute unit go out faster from blocks of four, which spread over twice as many compute units (MSECompressor.compress and
-// decompress, eight waves / four, us: 3920 vectors, bf16, 6-bit 12.5 / 11.5; 32800, 4-bit 15.7 / 15.3; 48000 18.2 / 18.2; 131168, float32 45.5 / 48.5).
-constexpr int MANY = 8, FEW = 4, FEW_TILES = 6;
+// Waves of a block: one block is resident per compute unit (Pi^T is staged once a block), so eight, two to a SIMD; 32-bit outputs of some
+// numbers of tiles are faster in blocks of four (blocks_of_four).
+constexpr int MANY = 8, FEW = 4;
 // HALVES: parts of a tile that a wave transposes and stores one after the other.  Whole tiles of 32-bit outputs of eight waves and Pi^T do not fit the LDS; blocks of
 // four waves, which held them whole, left a wave alone on its SIMD (131168 vectors: 20.6 us, this way 16.8).
 template <int DTYPE, int W> struct OutTraits { static constexpr int ELEM = DTYPE == TQ_F32 ? 4 : 2, WAVES = W, HALVES = ELEM == 4 && W == MANY ? 2 : 1; };
@@ -476,13 +475,23 @@ int launch_layer_of(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint
     return (int)hipGetLastError();
 }
 
+// 32-bit outputs, `tiles` in all.  A round of blocks of eight waves takes about as long as two of blocks of four, so where the last round of eight
+// would be half empty at best, four waves save half a round; over many rounds that is little, and tickets (launch_decompress) save more.
+// Blocks of four take no tickets (131072 vectors, 4-bit, 20.4 us with; a captured call, which has none, 15.4).  MSECompressor.decompress, bf16 inputs, 4-bit, us, blocks of four up to six tiles a
+// compute unit / this rule: 41600 vectors 9.0 / 8.1; 96000 13.5 / 11.9; 160000 19.9 / 17.3; 224000 25.0 / 22.7; 2-bit 96000 12.6 / 11.7, 8-bit 15.0 / 13.3; 64
+// wide 192000 13.7 / 12.1; lists of 32 tensors of 3000 15.2 / 12.3.
+bool blocks_of_four(unsigned long long tiles, int cus) {
+    const unsigned long long round = FEW * (unsigned long long)cus;
+    return tiles < 8u * round && (tiles + round - 1) / round % 2u == 1u;
+}
+
 template <int DTYPE, bool PAIRED>
 int launch_layer(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint32_t cost_k, uint32_t cost_v, void *workspace, hipStream_t stream) {
     int cus = 0;
     const int rc = device_cus(cus);
     if (rc) return rc;
     if constexpr (DTYPE == TQ_F32)
-        if (2ull * tiles <= FEW_TILES * (unsigned long long)cus) return launch_layer_of<DTYPE, PAIRED, FEW>(l, window, tiles, cost_k, cost_v, cus, workspace, stream);
+        if (blocks_of_four(2ull * tiles, cus)) return launch_layer_of<DTYPE, PAIRED, FEW>(l, window, tiles, cost_k, cost_v, cus, nullptr, stream);
     return launch_layer_of<DTYPE, PAIRED, MANY>(l, window, tiles, cost_k, cost_v, cus, workspace, stream);
 }
 
@@ -492,7 +501,7 @@ int launch_either(const TqDevJob &job, const tq_job *jobs_dev, int n_jobs, uint3
     const int rc = device_cus(cus);
     if (rc) return rc;
     if constexpr (DTYPE == TQ_F32)
-        if ((unsigned long long)n_jobs * max_tiles <= FEW_TILES * (unsigned long long)cus) return launch_decompress<DTYPE, IPB, PAIRED, FEW>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s);
+        if (blocks_of_four((unsigned long long)n_jobs * max_tiles, cus)) return launch_decompress<DTYPE, IPB, PAIRED, FEW>(job, jobs_dev, n_jobs, max_tiles, cus, nullptr, s);
     return launch_decompress<DTYPE, IPB, PAIRED, MANY>(job, jobs_dev, n_jobs, max_tiles, cus, ws, s);
 }
 
