@@ -63,7 +63,7 @@ __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
 }
 
 // One block's share of a job; `counter`: the job's two counters, or NULL; lds: decompress_lds_bytes.
-template <int DTYPE, int IPB, bool PAIRED, int W>
+template <int DTYPE, int IPB, bool PAIRED, int W, bool LAYER>
 __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk, uint32_t *counter, uint8_t *lds, uint32_t (&tk)[3]) {
     using T = OutTraits<DTYPE, W>;
     constexpr int ELEM = T::ELEM;
@@ -160,7 +160,9 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     };
     // jump of the output offset / packed slot from the last vector of a row to the first of the next
     const long long row_wrap = job.row_stride - (long long)job.tokens * job.token_stride;
-    constexpr int NOFF = HALVES == 1 ? NSTORE : 1;    // (where registers are short the rest is added where it is used, on the scalar unit)
+    // (where registers are short the rest is added where it is used, on the scalar unit: 32-bit outputs of eight waves, and of the layer
+    // kernels, which hold the bodies of all widths: layer of 8 x 6000 float32, K8/V4 16.4 us with all offsets kept, this way 14.0)
+    constexpr int NOFF = ELEM == 2 || (HALVES == 1 && !LAYER) ? NSTORE : 1;
     uint32_t st_off[NOFF];   // byte offset of this lane's piece of store j relative to the tile's first vector
 #pragma unroll
     for (int j = 0; j < NOFF; ++j) st_off[j] = (j * VEC_PER_STORE + st_vec) * (uint32_t)job.token_stride + st_piece * 16u;
@@ -359,7 +361,7 @@ __global__ __launch_bounds__(W *TQ_WAVE) void tq_decompress_kernel(TqDevJob job0
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t tk[3];
     const TqDevJob job = tq_pair_rows(tq_load_job(job0, jobs, blockIdx.y, OutTraits<DTYPE, W>::ELEM), PAIRED);
-    decompress_job<DTYPE, IPB, PAIRED, W>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr, lds, tk);
+    decompress_job<DTYPE, IPB, PAIRED, W, false>(job, TqBlock{blockIdx.x, gridDim.x}, workspace ? workspace + blockIdx.y * (TQ_WORKSPACE_BYTES_PER_JOB / 4) : nullptr, lds, tk);
 }
 
 // keys and values of a layer and its window; the two jobs' counters share one job's record of the workspace
@@ -373,10 +375,10 @@ __global__ __launch_bounds__(W *TQ_WAVE) void tq_restore_layer_kernel(TqLayer l,
     uint32_t *counter = workspace ? workspace + which * (TQ_WORKSPACE_BYTES_PER_JOB / 8) : nullptr;
     tq_with_window(window, [&]() __attribute__((always_inline)) {
         switch (8 / (which ? l.bits[1] : l.bits[0])) {
-            case 8: decompress_job<DTYPE, 8, PAIRED, W>(job, blk, counter, lds, tk); break;
-            case 4: decompress_job<DTYPE, 4, PAIRED, W>(job, blk, counter, lds, tk); break;
-            case 2: decompress_job<DTYPE, 2, PAIRED, W>(job, blk, counter, lds, tk); break;
-            default: decompress_job<DTYPE, 1, PAIRED, W>(job, blk, counter, lds, tk); break;
+            case 8: decompress_job<DTYPE, 8, PAIRED, W, true>(job, blk, counter, lds, tk); break;
+            case 4: decompress_job<DTYPE, 4, PAIRED, W, true>(job, blk, counter, lds, tk); break;
+            case 2: decompress_job<DTYPE, 2, PAIRED, W, true>(job, blk, counter, lds, tk); break;
+            default: decompress_job<DTYPE, 1, PAIRED, W, true>(job, blk, counter, lds, tk); break;
         }
     });
 }
