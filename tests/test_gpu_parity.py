@@ -789,7 +789,7 @@ def test_float32_norms_come_from_one_order_of_additions(pkg, dim, tokens):
 
 
 @pytest.mark.parametrize("dim,bits", [(128, 4), (128, 8), (64, 2), (64, 1)])
-@pytest.mark.parametrize("tiles", [1023, 1024, 1025, 2048, 2049, 3073, 8191, 8193])
+@pytest.mark.parametrize("tiles", [1023, 1025, 1536, 1537, 2048, 2049, 3585, 8191, 8193])
 def test_float32_results_do_not_depend_on_the_size_of_the_blocks(pkg, dim, bits, tiles):
     """Restores to float32 on either side of where blocks of four and of eight waves take turns (rounds of 4 x 256 tiles): the same values as
     the same vectors in calls of a few tiles, alone, in a list and as a layer with a window."""

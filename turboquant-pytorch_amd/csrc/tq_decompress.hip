@@ -477,14 +477,15 @@ int launch_layer_of(TqLayer &l, const TqWindowCopy &window, uint32_t tiles, uint
     return (int)hipGetLastError();
 }
 
-// 32-bit outputs, `tiles` in all.  A round of blocks of eight waves takes about as long as two of blocks of four, so where the last round of eight
-// would be half empty at best, four waves save half a round; over many rounds that is little, and tickets (launch_decompress) save more.
-// Blocks of four take no tickets (131072 vectors, 4-bit, 20.4 us with; a captured call, which has none, 15.4).  MSECompressor.decompress, bf16 inputs, 4-bit, us, blocks of four up to six tiles a
-// compute unit / this rule: 41600 vectors 9.0 / 8.1; 96000 13.5 / 11.9; 160000 19.9 / 17.3; 224000 25.0 / 22.7; 2-bit 96000 12.6 / 11.7, 8-bit 15.0 / 13.3; 64
-// wide 192000 13.7 / 12.1; lists of 32 tensors of 3000 15.2 / 12.3.
+// 32-bit outputs, `tiles` in all.  A round of blocks of eight waves takes a little less than two of blocks of four, so eight are faster where
+// both end with the same round filled by no more than half; else fours save what is left empty of the last round, or no less than eights. Over
+// many rounds that is little, and tickets (launch_decompress) save more; blocks of four take none (131072 vectors, 4-bit, 20.4 us with; a
+// captured call, which has none, 15.4).  MSECompressor.decompress, bf16 inputs, 4-bit, us, blocks of four up to six tiles a compute unit / this
+// rule: 41600 vectors 9.0 / 8.1; 64000 9.7 / 9.7; 96000 13.5 / 11.9; 128000 15.2 / 14.6; 160000 19.9 / 17.3; 224000 25.0 / 22.7; 252800 26.3 / 25.2; 2-bit 96000
+// 12.6 / 11.7; 8-bit 15.0 / 13.3; 64 wide 192000 13.7 / 12.1; lists of 32 tensors of 3000 15.2 / 12.3; layers of 8 x 8000, 64 wide, K4/V2 11.2 / 10.2.
 bool blocks_of_four(unsigned long long tiles, int cus) {
-    const unsigned long long round = FEW * (unsigned long long)cus;
-    return tiles < 8u * round && (tiles + round - 1) / round % 2u == 1u;
+    const unsigned long long round = FEW * (unsigned long long)cus, last = tiles % (2u * round);
+    return tiles < 8u * round && (last <= round || 2u * last > 3u * round);
 }
 
 template <int DTYPE, bool PAIRED>
