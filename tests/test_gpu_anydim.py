@@ -254,10 +254,11 @@ def test_v3_orchestration_and_cache_at_head_dim_64(pkg, oracle):
 @pytest.mark.parametrize("bits,dtype", [(4, torch.bfloat16), (2, torch.float16), (8, torch.float32), (3, torch.bfloat16)])
 def test_head_dim_64_in_pairs_equals_the_one_by_one_form(pkg, oracle, bits, dtype):
     """64-wide vectors go through the 128-wide kernels two at a time (as rows rotated by diag(Pi, Pi)) whenever every
-    row of the job holds an even number of tokens that lie 64 elements apart; otherwise one by one through the
-    run-time-dimension kernels.  Both forms against the oracle, and against each other: the same codes (outside the
-    boundary window), norms within one fp16 unit, the same de-quantised values; dense tensors, token slices of a
-    preallocated store at even and odd offsets, job lists that mix both kinds."""
+    row of the job holds an even number of tokens that lie 64 elements apart; otherwise they are compressed one by one
+    by the run-time-dimension kernels (de-quantised in pairs all the same where rows of an odd number have 63 tokens at least).  Both forms
+    against the oracle, and against each other: the same codes (outside the boundary window), norms within one fp16
+    unit, the same de-quantised values; dense tensors, token slices of a preallocated store at even and odd offsets, job
+    lists that mix both kinds."""
     native = pkg._native
     D = 64
     comp = pkg.MSECompressor(D, bits, seed=11 + bits, device=DEV)
@@ -386,3 +387,61 @@ def test_head_dim_64_rows_that_end_in_half_a_pair(pkg, bits, dtype, rows, tokens
                 assert got is not None
                 for t in got:
                     assert torch.equal(t[:, :, :tokens], want) and torch.equal(t[:, :, tokens:], win), (cap, n_win)
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 8])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_head_dim_64_short_even_rows_at_odd_slots(pkg, bits, dtype):
+    """Rows of an even number of 64-wide vectors, fewer than a tile of pairs, in a store of an odd capacity: every second row starts at an
+    odd slot.  Bit for bit what the dense call gives."""
+    D, G = 64, 64 // (8 // bits)
+    comp = pkg.MSECompressor(D, bits, seed=5, device=DEV)
+    for tokens in (2, 6, 30, 62):
+        packed = comp.compress(outlier_kv((3, 5, tokens, D), seed=tokens + bits, dtype=dtype).to(DEV))
+        want = torch.empty((3, 5, tokens, D), dtype=dtype, device=DEV)
+        comp.decompress_packed(packed["idx_bytes"], packed["vec_norms"], want)
+        idx = torch.zeros((3, 5, tokens + 1, G), dtype=torch.uint8, device=DEV)
+        nrm = torch.zeros((3, 5, tokens + 1), dtype=torch.float16, device=DEV)
+        idx[:, :, :tokens], nrm[:, :, :tokens] = packed["idx_bytes"], packed["vec_norms"]
+        out = torch.full((3, 5, tokens + 2, D), 3.0, dtype=dtype, device=DEV)
+        comp.decompress_packed(idx[:, :, :tokens], nrm[:, :, :tokens], out[:, :, :tokens])
+        assert torch.equal(out[:, :, :tokens], want) and bool((out[:, :, tokens:] == 3.0).all()), tokens
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_head_dim_64_restored_one_by_one(pkg, bits, dtype):
+    """What still goes through the run-time-dimension kernel at 64: several rows of an odd number of less than 63 tokens, and tokens that lie
+    apart.  Against the pairs: the products are the same, the sums are of 64 terms in another order (2^-24 each), and a 16-bit result may
+    round to the neighbour."""
+    D, tol = 64, {torch.float32: 64 * 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    comp = pkg.MSECompressor(D, bits, seed=5, device=DEV)
+    for rows, tokens, apart in ((3, 61, 0), (40, 33, 0), (7, 1, 0), (3, 64, 32), (2, 347, 8), (1, 5, 64)):
+        packed = comp.compress(outlier_kv((1, rows, tokens, D), seed=tokens + bits, dtype=dtype).to(DEV))
+        want = torch.empty((1, rows, tokens, D), dtype=dtype, device=DEV)       # dense: one row of rows * tokens vectors, in pairs
+        comp.decompress_packed(packed["idx_bytes"], packed["vec_norms"], want)
+        out = torch.full((1, rows, tokens + 3, D + apart), 3.0, dtype=dtype, device=DEV)
+        comp.decompress_packed(packed["idx_bytes"], packed["vec_norms"], out[:, :, 1:1 + tokens, :D])
+        got = out[:, :, 1:1 + tokens, :D].double()
+        err = float((got - want.double()).norm() / want.double().norm())
+        assert err <= tol, (rows, tokens, apart, err)
+        assert bool((out[:, :, :1] == 3).all()) and bool((out[:, :, 1 + tokens:] == 3).all()) and bool((out[..., D:] == 3).all()), (rows, tokens, apart)
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("rows,tokens", [(1, 31), (3, 33), (40, 5), (40, 65), (7, 97), (3000, 31), (8000, 5), (20000, 1), (2000, 33)])
+def test_float32_rows_that_end_at_every_place_of_a_tile(pkg, dim, rows, tokens):
+    """Float32 token slices of a larger tensor, in and out: tiles with a row's end, several of them or the job's, one and many tiles a block.
+    The bytes and values of the same vectors laid end to end, nothing else is written.  (64: even rows, which go in pairs both ways.)"""
+    tokens += tokens % 2 if dim == 64 else 0
+    comp = pkg.MSECompressor(dim, 4, seed=3, device=DEV)
+    big = torch.randn(1, rows, tokens + 3, dim, generator=torch.Generator(device=DEV).manual_seed(tokens), device=DEV)
+    part = big[:, :, 2:2 + tokens]
+    packed, dense = comp.compress(part), comp.compress(part.contiguous())
+    for name in ("idx_bytes", "vec_norms"):
+        assert torch.equal(packed[name], dense[name]), name
+    out, want = torch.full_like(big, 7.0), torch.empty_like(part, memory_format=torch.contiguous_format)
+    comp.decompress_into(dense, out[:, :, 2:2 + tokens])
+    comp.decompress_into(dense, want)
+    assert torch.equal(out[:, :, 2:2 + tokens], want)
+    assert bool((out[:, :, :2] == 7).all()) and bool((out[:, :, 2 + tokens:] == 7).all())

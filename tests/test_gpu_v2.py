@@ -152,7 +152,7 @@ def test_v2_one_pass_form_against_the_two_kernel_form(pkg, oracle, bits, dtype):
     within 1e-5 of |S row| |residual| of zero, residual norms within one fp16 unit; single call and batched list."""
     import ctypes
     native = pkg._native
-    L, n = 3, 4096 + 32 * 7 + 11                 # full tiles for the one-pass kernel, a ragged end for the other form
+    L, n = 3, 4096 + 32 * 7 + 11                 # whole tiles and a ragged last one
     comps = [pkg.TurboQuantCompressorV2(128, bits, seed=31 * l + bits, device=DEV) for l in range(L)]
     xs = [outlier_kv((1, 1, n, 128), seed=300 + l, dtype=dtype).to(DEV) for l in range(L)]
     packed = [c.empty_packed(1, 1, n, DEV) for c in comps]
@@ -246,3 +246,21 @@ def test_v2_keys_of_any_number_do_not_depend_on_their_tile(pkg, bits, dtype, n):
             if torch.is_tensor(value):
                 got = whole[key].reshape(n, -1)[part]
                 assert torch.equal(got, value.reshape(got.shape)), (key, part)
+
+
+@pytest.mark.parametrize("bits,dtype", [(3, torch.bfloat16), (5, torch.float16), (3, torch.float32)])
+def test_v2_job_lists_of_any_sizes_equal_single_calls(pkg, bits, dtype):
+    """Jobs below, at and above the 32 vectors from which the one-pass kernel takes them, in one list: byte for byte what a call each gives."""
+    comp = pkg.TurboQuantCompressorV2(128, bits, seed=42, device=DEV)
+    xs = [torch.randn((1, 1, n, 128), generator=torch.Generator().manual_seed(n)).to(dtype).to(DEV) for n in (31, 4331, 1, 0, 32, 33, 2, 64, 63, 1000)]
+    names = ("idx_bytes", "vec_norms", "sign_bytes", "residual_norm")
+    packed = [comp.empty_packed(1, 1, x.shape[2], DEV) for x in xs]
+    for p in packed:
+        for k in names:
+            p[k].fill_(0x55 if p[k].dtype == torch.uint8 else 3.0)
+    pkg._native.QjlJobList([comp.job(x, p) for x, p in zip(xs, packed)], torch.device(DEV)).compress()
+    for x, p in zip(xs, packed):
+        if x.numel():
+            alone = comp.compress(x)
+            for k in names:
+                assert torch.equal(alone[k].view(torch.uint8), p[k].view(torch.uint8)), (x.shape[2], k)
