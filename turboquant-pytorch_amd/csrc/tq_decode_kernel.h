@@ -320,11 +320,10 @@ struct WindowTile {
 // splits, which the rule of then took, before / after; it takes 32 now): all loads of the start issued at once in the order of their use, tables found without their header, queries
 // rotated by 4.2 / 2.5 us; the window's values loaded with its keys and its sums stored without a branch for each, 7.0 / 4.5; the block's
 // tokens dealt out evenly; records merged with one trip to memory and a code of a few hundred bytes (code that runs once is fetched from
-// the L2 as it goes: 1 us for 2.4 KiB of it), rows of Pi_v under way before the block knows that it needs them, last arrival to result 5.5 / 3.4.
+// the L2 as it goes: 1 us for 2.4 KiB of it), last arrival to result 5.5 / 3.4.
 // A tile of the window used to stand before the block's barrier: everybody in it waited 2.3 us (256 wide 4.4) for the wave that had it, and the row for the
-// block.  It is finished behind the barrier now; records are merged without loops around their
-// loads.  us a step of eight layers, append and attend: 8 rows x 32768 tokens 170 -> 164; 64 wide, 32 x 6000, K6/V4 146 -> 130; 96 wide, 2 x 8574
-// 130 -> 118; 256 wide, 8 x 9906, K3/V2 291 -> 262; 512 x 16384 1366 -> 1354.
+// block.  It is finished behind the barrier now; records are merged without loops around their loads.  us a layer, 4 heads, K4/V2: 8 rows x 32768
+// tokens 21.0 -> 20.3; 4 x 6000 16.4 -> 15.0; 64 wide, 32 x 6000 15.8 -> 14.8; 256 wide, 8 x 16384 35.3 -> 33.0.
 // Before that, whole step of 32 layers 948 -> 778 us (734 since the append asks for all of its loads at once, see tq_decode.hip); 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
 // The matrix products have 16 columns and a row of the cache seldom 16 query heads.  C blocks of 16 tokens share them (C = 4 for up to 4
 // heads, 2 for up to 8): every block's scores are computed for the heads repeated C times, a lane keeps those of its own column's

@@ -80,7 +80,7 @@ __device__ __forceinline__ void decompress_job(const TqDevJob &job, TqBlock blk,
     // section).  Lane half hk decodes and produces the second vector of the pair; only its norm is its own.  Packed slots count
     // 64-wide vectors.  Where a row ends in half a pair (job.odd) its second half reads the first one again and is not stored.
     // (Odd rows used to go through the kernel of any dimension, a launch each for keys, values and window: eight layers of a decode step
-    // of 8 rows of 18940 tokens, odd and even in turn, 188 -> 144 us.  Kernels of their own for pairs: with both kinds of rows in one,
+    // of 8 rows of 18940 tokens, odd and even in turn, 188 -> 140 us.  Kernels of their own for pairs: with both kinds of rows in one,
     // small launches of 128-wide vectors took 2 % longer.)
     constexpr uint32_t VSHIFT = PAIRED ? 1u : 0u;
     uint8_t *out_base = const_cast<uint8_t *>(job.states);
