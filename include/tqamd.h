@@ -418,6 +418,8 @@ int tq_attend_step(const void *queries, int q_dtype, long long rows, int group, 
  *   empty).  scratch: tq_decode_scratch_floats() float32 values at a multiple of 4 bytes (scratch_size: how many there are;
  *   TQ_ERR_CAPACITY if too few; one of them is there to begin at a multiple of 8), arrived: `rows` counters, zero before the first use and left zero by every launch that completes; neither
  *   is shared by launches that can overlap in time.
+ * tq_decode_attend_spread: the same with n_arrived >= rows counters (TQ_ERR_CAPACITY if fewer): from 32 * rows on every row
+ *   has a line of memory to itself, which few rows with many blocks each finish sooner with.
  * tq_decode_supported: 1 if these calls take the combination, 0 otherwise.
  */
 typedef struct tq_decode_layer {
@@ -436,6 +438,9 @@ int tq_decode_supported(int head_dim, int dtype, int bits_k, int bits_v);
 long long tq_decode_scratch_floats(long long rows, int group, int head_dim, long long tokens, long long n_win);
 int tq_decode_attend(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
                      long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, void *out, void *stream);
+int tq_decode_attend_spread(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
+                            long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, long long n_arrived, void *out,
+                            void *stream);
 int tq_decode_append(const tq_decode_layer *layer, const void *k_new, const void *v_new, long long k_new_stride, long long v_new_stride,
                      long long evict, long long put, long long packed_slot, void *stream);
 

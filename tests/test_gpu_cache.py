@@ -854,6 +854,23 @@ def test_decode_attention_with_scratch_at_any_float(pkg):
         assert torch.equal(out, want) and bool((scratch[:start] == 7).all()) and bool((scratch[start + floats:] == 7).all())
 
 
+@pytest.mark.parametrize("n_arrived", [5, 9, 10, 63, 64, 159, 160, 1000])
+def test_decode_attention_with_counters_at_any_spread(pkg, n_arrived):
+    """5 rows whose arrival counters lie 1 to 32 apart, by how many there are: the same bytes, all counters zero again, none touched past the last."""
+    native = pkg._native
+    cache = pkg.V3Cache(4, 2, residual_window=40, n_layers=40)
+    x = torch.randn(1, 5, 1500, 128, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)
+    cache.append(x, x, 8)
+    st, q = cache._stores[8], torch.randn(1, 20, 1, 128, generator=torch.Generator().manual_seed(2)).bfloat16().to(DEV)
+    floats = native.lib().tq_decode_scratch_floats(5, 4, 128, st.n_compressed, st.n_recent)
+    scratch, counters, out, want = torch.empty(floats, device=DEV), torch.zeros(n_arrived + 8, dtype=torch.int32, device=DEV), torch.empty_like(q), cache.attend(q, 8)
+    counters[n_arrived:] = 7
+    for _ in range(2):
+        native.check(native.lib().tq_decode_attend_spread(ctypes.addressof(st.record()), q.data_ptr(), 4, 128 ** -0.5, st.w0, st.n_recent, st.n_compressed, scratch.data_ptr(), floats,
+                                                          counters.data_ptr(), n_arrived, out.data_ptr(), native._stream_handle(q.device)), "tq_decode_attend_spread")
+        assert torch.equal(out, want) and not bool(counters[:n_arrived].any()) and bool((counters[n_arrived:] == 7).all())
+
+
 @pytest.mark.parametrize("dim,tokens,window", [(64, 34000, 260), (96, 17000, 40), (128, 70000, 128), (256, 20000, 5)])
 def test_decode_attention_merges_many_splits(pkg, dim, tokens, window):
     """One row over many blocks: more records than a lane has under way at a time (32) and than a wave has lanes, several windows' tiles

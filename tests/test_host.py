@@ -812,3 +812,11 @@ def test_decode_attend_counts_the_float_that_aligns_its_scratch(pkg):
     attend = lambda scratch, size: native.lib().tq_decode_attend(ctypes.addressof(layer), 4096, 4, 1.0, 0, 128, 1000, scratch, size, 4096, 4096, None)  # noqa: E731
     assert attend(4096 + 4, floats - 1) == native.ERR_CAPACITY and attend(4096, floats - 2) == native.ERR_CAPACITY
     assert attend(4096 + 2, floats) == native.ERR_ALIGN
+
+
+def test_decode_attend_spread_wants_a_counter_for_every_row(pkg):
+    native = pkg._native
+    layer = native.TqDecodeLayer(*([4096] * 9), 128 * 128, 2000, 8, 128, native.TQ_BF16, 4, 2)
+    size = native.lib().tq_decode_scratch_floats(8, 4, 128, 1000, 128)
+    attend = lambda n_arrived: native.lib().tq_decode_attend_spread(ctypes.addressof(layer), 4096, 4, 1.0, 0, 128, 1000, 4096, size, 4096, n_arrived, 4096, None)  # noqa: E731
+    assert attend(7) == native.ERR_CAPACITY and attend(0) == native.ERR_CAPACITY

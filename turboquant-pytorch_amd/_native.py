@@ -212,7 +212,7 @@ EXPORTS = (
     "tq_qjl_compress", "tq_qjl_compress_batched", "tq_qjl_scores", "tq_qjl_query_scores",
     "tq_scores", "tq_weighted_values", "tq_weighted_values_splits", "tq_attend_partials", "tq_attend_splits",
     "tq_attend_prepare", "tq_attend_merge", "tq_append_token", "tq_attend_step",
-    "tq_decode_supported", "tq_decode_scratch_floats", "tq_decode_attend", "tq_decode_append",
+    "tq_decode_supported", "tq_decode_scratch_floats", "tq_decode_attend", "tq_decode_attend_spread", "tq_decode_append",
     "tq_compress_layer", "tq_restore_layer",
 )
 
@@ -270,6 +270,7 @@ def lib() -> ctypes.CDLL:
     L.tq_decode_scratch_floats.restype = ll
     L.tq_decode_scratch_floats.argtypes = [ll, ci, ci, ll, ll]
     L.tq_decode_attend.argtypes = [vp, vp, ci, ctypes.c_float, ll, ll, ll, vp, ll, vp, vp, vp]
+    L.tq_decode_attend_spread.argtypes = [vp, vp, ci, ctypes.c_float, ll, ll, ll, vp, ll, vp, ll, vp, vp]
     L.tq_decode_append.argtypes = [vp, vp, vp, ll, ll, ll, ll, ll, vp]
     L.tq_compress_layer.argtypes = [vp, vp, ci, ll, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, vp, vp, vp, vp]
     L.tq_restore_layer.argtypes = [vp, vp, vp, vp, ll, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, ll, ll, ll, vp, vp, ci, vp, vp]
@@ -302,7 +303,7 @@ def fast():
             raise TqError(f"{path} cannot be loaded ({e}): {how}") from e
         if module.abi_version != L.tq_abi_version():
             raise TqError(f"{path} was built for version {module.abi_version} of the library, this is {L.tq_abi_version()}: {how}")
-        entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend", "tq_qjl_compress", "tq_qjl_query_scores")
+        entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend_spread", "tq_qjl_compress", "tq_qjl_query_scores")
         stream_of = _raw_stream or (lambda index: torch.cuda.current_stream(index).cuda_stream)
         module.init(tuple(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in entries), stream_of, _workspace, _drop_workspace, _step_scratch, _arrived, _TABLE_TAG)
         _fast = module
@@ -553,11 +554,12 @@ _arrived: Dict[Tuple[int, int], torch.Tensor] = {}
 
 def arrival_counters(device: torch.device, stream: int, rows: int) -> torch.Tensor:
     """The counters through which the blocks of a row find out in tq_decode_attend which of them comes last: one zeroed
-    buffer per (device, stream), on the terms of `_workspace`.  (Never asked for while a graph is being captured.)"""
+    buffer per (device, stream), on the terms of `_workspace`.  (Never asked for while a graph is being captured.)  32 KiB at least: up to 256
+    rows have a line of memory each, which tq_decode_attend_spread makes use of."""
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     buf = _arrived.get(key)
     if buf is None or buf.numel() < rows:
-        buf = _arrived[key] = torch.zeros(max(rows, 1024), dtype=torch.int32, device=device)
+        buf = _arrived[key] = torch.zeros(max(rows, 8192), dtype=torch.int32, device=device)
     return buf
 
 

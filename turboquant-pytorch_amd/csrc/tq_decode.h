@@ -11,11 +11,11 @@ struct TqDecodeArgs {
     const uint8_t *k_win, *v_win;    // row r, token t at element r * win_stride + t * D
     float *partial;                  // [rows, splits, group, D + 2]: reference score, sum of exp, D sums in the rotated value space
     float *win_part;                 // [rows, window tiles, group, D + 2]: the same over 32 window tokens, sums in the plain space
-    uint32_t *arrived;               // [rows] blocks of the row that are done; zero before and after every launch (splits > 1)
+    uint32_t *arrived;               // row r: [r * arrived_stride] blocks of the row that are done; zero before and after every launch (splits > 1)
     uint8_t *out;                    // [rows, group, D]
     long long win_stride;
     float scale;
-    uint32_t tokens, packed_row_stride, group, chunk, n_win, bf16;
+    uint32_t tokens, packed_row_stride, group, chunk, n_win, bf16, arrived_stride;
 };
 
 namespace {

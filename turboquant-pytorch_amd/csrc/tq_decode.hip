@@ -240,8 +240,9 @@ extern "C" long long tq_decode_scratch_floats(long long rows, int group, int hea
     return scratch_floats(rows, group, head_dim, decode_splits(rows, tokens), n_win) + 1;      // (see tq_decode_attend)
 }
 
-extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
-                                long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, void *out, void *stream) {
+extern "C" int tq_decode_attend_spread(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
+                                       long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, long long n_arrived, void *out,
+                                       void *stream) {
     const int rc = check_layer(layer);
     if (rc) return rc;
     const int D = layer->head_dim;
@@ -257,7 +258,7 @@ extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *querie
     const int splits = decode_splits(rows, tokens);
     // records are stored and exchanged between blocks in pairs of floats, 8 bytes at a time
     if ((uintptr_t)scratch & 4u) { ++scratch; --scratch_size; }
-    if (scratch_size < scratch_floats(rows, group, D, splits, n_win)) return TQ_ERR_CAPACITY;
+    if (scratch_size < scratch_floats(rows, group, D, splits, n_win) || n_arrived < rows) return TQ_ERR_CAPACITY;
     TqDecodeArgs a;
     a.queries = static_cast<const uint8_t *>(queries);
     a.k_idx = layer->k_idx; a.v_idx = layer->v_idx; a.k_norms = layer->k_norms; a.v_norms = layer->v_norms;
@@ -269,6 +270,10 @@ extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *querie
     a.partial = scratch;
     a.win_part = scratch + (size_t)rows * splits * group * (D + 2);
     a.arrived = arrived;
+    // A counter of its own to every line of 128 bytes where there are enough of them (closer together where there are fewer): the blocks
+    // that finish together would otherwise queue at one line, an atomic about every 14 ns.
+    a.arrived_stride = 32u;
+    while (a.arrived_stride > 1u && (long long)a.arrived_stride * rows > n_arrived) a.arrived_stride >>= 1;
     a.out = static_cast<uint8_t *>(out);
     a.win_stride = layer->win_stride;
     a.scale = scale;
@@ -292,6 +297,11 @@ extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *querie
         case 128: return ik >= 4 ? tq_decode_launch_d128_narrow(ik, iv, grid, s, a) : tq_decode_launch_d128_wide(ik, iv, grid, s, a);
         default: return tq_decode_launch_d256(ik, iv, grid, s, a);
     }
+}
+
+extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
+                                long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, void *out, void *stream) {
+    return tq_decode_attend_spread(layer, queries, group, scale, win_first, n_win, tokens, scratch, scratch_size, arrived, layer ? layer->rows : 0, out, stream);
 }
 
 extern "C" int tq_decode_append(const tq_decode_layer *layer, const void *k_new, const void *v_new, long long k_new_stride, long long v_new_stride,

@@ -879,8 +879,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     };
     if (splits > 1u) {
         if (tid == 0u) {
-            const bool last = __hip_atomic_fetch_add(a.arrived + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1u;
-            if (last) __hip_atomic_store(a.arrived + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const bool last = __hip_atomic_fetch_add(a.arrived + (size_t)row * a.arrived_stride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1u;
+            if (last) __hip_atomic_store(a.arrived + (size_t)row * a.arrived_stride, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             lds_last = last ? 1u : 0u;
         }
         __syncthreads();

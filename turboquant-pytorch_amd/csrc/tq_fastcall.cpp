@@ -28,7 +28,7 @@ struct Entries {
     decltype(&tq_compress_layer) compress_layer;
     decltype(&tq_restore_layer) restore_layer;
     decltype(&tq_decode_append) decode_append;
-    decltype(&tq_decode_attend) decode_attend;
+    decltype(&tq_decode_attend_spread) decode_attend;
     decltype(&tq_qjl_compress) qjl_compress;
     decltype(&tq_qjl_query_scores) qjl_query_scores;
 } lib{};
@@ -355,7 +355,7 @@ PyObject *decode_attend(PyObject *const *a) {
     NEED(counters.numel() >= rows);
     at::Tensor out = empty(q.sizes(), q.scalar_type(), q);
     const int rc = launch(lib.decode_attend, reinterpret_cast<const tq_decode_layer *>(integer(a[0])), (const void *)address(q), (int)(Hq / H), (float)scale, integer(a[4]), n_win,
-                          integer(a[6]), (float *)address(buf), (long long)buf.numel(), (uint32_t *)address(counters), (void *)address(out), s.raw());
+                          integer(a[6]), (float *)address(buf), (long long)buf.numel(), (uint32_t *)address(counters), (long long)counters.numel(), (void *)address(out), s.raw());
     NEED(rc == 0);           // (a buffer that is too small, or an argument the library refuses: nothing was launched)
     return THPVariable_Wrap(out);
 }
