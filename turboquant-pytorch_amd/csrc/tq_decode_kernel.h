@@ -364,6 +364,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     constexpr int P_SHIFT = 14 - SLACK_LOG2;             // p * 2^P_SHIFT * (value norm / 2^ev_ref < 2) <= 2^15 fits fp16
     constexpr int HR = D == 256 && C == 1 ? 8 : HEADS;   // heads per round of the merge through LDS
     constexpr int AREA = VBYTES > HR * PART * 4 ? VBYTES : HR * PART * 4;    // per wave: staged value codes, later its sums
+    constexpr bool EARLY_PV = D <= 128 && C > 1;         // rows of Pi_v asked for by every block that may be the last (see there)
     constexpr int QROW = D + 4;                          // rotated queries in LDS, floats per head
     constexpr int ROTP = DTHREADS / (D / 4) >= 16 ? 16 : DTHREADS / (D / 4);     // parts of the contraction when rotating back
     constexpr int ROTK = D / ROTP;                       // rows of Pi_v per part
@@ -869,7 +870,10 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     // do, thread 0 may count the block as done, see put_record)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    // rows of Pi_v for the rotation back: thread (four columns, part) takes ROTK of them, loaded behind the records that it has to wait for
+    // Rows of Pi_v for the rotation back: thread (four columns, part) takes ROTK of them.  Where registers allow they are asked for right behind
+    // the atomic, by every block, so that they arrive while its answer is on its way and only the records are left to wait for: 8 rows x
+    // 32768 tokens, from the last block's count to merged sums 2.9 -> 2.3 us (the other blocks drop them: 64 KB of the L2 each at 128).
+    // At 256 (four times as much) and for more than eight heads they are loaded behind the records.
     const uint32_t rc = (tid % (D / 4)) * 4u, rp = tid / (D / 4);
     tq_u4 pv[ROTK];
     auto load_pv = [&]() __attribute__((always_inline)) {
@@ -878,8 +882,15 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
         for (int k = 0; k < ROTK; ++k) pv[k] = tq_gload16(src + k * (D * 4));
     };
     if (splits > 1u) {
+        uint32_t before = 0u;
+        if (tid == 0u) before = __hip_atomic_fetch_add(a.arrived + (size_t)row * a.arrived_stride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if constexpr (EARLY_PV) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_pv();
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (tid == 0u) {
-            const bool last = __hip_atomic_fetch_add(a.arrived + (size_t)row * a.arrived_stride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1u;
+            const bool last = before == splits - 1u;
             if (last) __hip_atomic_store(a.arrived + (size_t)row * a.arrived_stride, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             lds_last = last ? 1u : 0u;
         }
@@ -985,7 +996,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 w[k] = wpart.load4<ACROSS>(q4 * step + off);
             }
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (N <= 2) load_pv();                          // (more columns leave no registers for them yet)
+            if constexpr (N <= 2 && !(ACROSS && EARLY_PV)) load_pv();                          // (more columns leave no registers for them yet)
 #pragma unroll
             for (int h = 0; h < H; ++h)
                 if (wave + h * DW < G) weigh(ml[h], wave + h * DW);
@@ -1000,7 +1011,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 if (win_tiles) add_window(w[k], f[wfirst]);
                 put_sums(p);
             }
-            if constexpr (N > 2) load_pv();
+            if constexpr (N > 2 && !(ACROSS && EARLY_PV)) load_pv();
             __syncthreads();
         };
         if (splits <= 32u && win_tiles <= 4u) {      // (launched for at most HEADS heads, HEADS = 16 for 9 at least, see launch_decode)
@@ -1020,7 +1031,7 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
             fetch(y, col / D * PART + 2u + col % D, 0u);
             w = wpart.load4<ACROSS>(q4 * step + col / D * PART + 2u + col % D);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (D <= 128) load_pv();
+            if constexpr (D <= 128 && !(ACROSS && EARLY_PV)) load_pv();
             for (uint32_t g = wave; g < G; g += DW) {
                 if (g != wave) load_heads(ml, g);
                 weigh(ml, g);
