@@ -854,6 +854,25 @@ def test_decode_attention_with_scratch_at_any_float(pkg):
         assert torch.equal(out, want) and bool((scratch[:start] == 7).all()) and bool((scratch[start + floats:] == 7).all())
 
 
+@pytest.mark.parametrize("dim,bits", [(64, (6, 4)), (64, (2, 8)), (96, (4, 2)), (96, (8, 8)), (128, (4, 2)), (128, (1, 1)), (128, (8, 8)), (256, (4, 2)), (256, (8, 4))])
+def test_decode_attention_of_a_layer_on_either_side_of_streaming(pkg, dim, bits):
+    """A layer of 8 MiB of packed codes and norms is read with other loads than one a token short of it: one row, the last tokens of a run
+    and of the store among them.  Against float64 over the store as the kernel holds it, bounds as in test_decode_attention_with_heads_side_by_side; the
+    many tokens of about equal weight leave results of 0.01, where float16 still rounds to 2^-11 of a value."""
+    g = torch.Generator().manual_seed(dim + bits[0])
+    per_token = dim // (8 // bits[0]) + dim // (8 // bits[1]) + 4
+    least = -(-(8 << 20) // (2 * per_token))          # tokens of two rows from which on a layer is streamed
+    for tokens in (least - 1, least, least + 33):
+        cache = pkg.V3Cache(bits[0], bits[1], residual_window=3, n_layers=40)
+        k, v = (torch.randn(1, 2, tokens + 3, dim, generator=g).half().to(DEV) for _ in range(2))
+        cache.append(k, v, 8)
+        for group in (1, 5, 16):
+            q = 2 * torch.randn(1, 2 * group, 1, dim, generator=g).half().to(DEV)
+            ref = _exact_attention(cache._stores[8], q, dim ** -0.5)
+            err = float((cache.attend(q, 8).double().reshape(ref.shape) - ref).norm() / ref.norm())
+            assert err < (1.5e-3 if dim == 128 else 3.5e-4), (tokens, group, err)
+
+
 @pytest.mark.parametrize("n_arrived", [5, 9, 10, 63, 64, 159, 160, 1000])
 def test_decode_attention_with_counters_at_any_spread(pkg, n_arrived):
     """5 rows whose arrival counters lie 1 to 32 apart, by how many there are: the same bytes, all counters zero again, none touched past the last."""

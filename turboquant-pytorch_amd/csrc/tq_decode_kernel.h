@@ -339,7 +339,7 @@ struct WindowTile {
 //     reference weight times the largest value norm's binade, a grid of 2^-34 of that below (the smaller SLACK_LOG2, the finer).
 //     Two terms on a grid of 2^-30 lost up to 2^-8 of weights around 2^-22 of the reference, a short history behind one token
 //     that takes nearly everything.  The third one costs 4 to 5 % where rows are many (96 wide, 512 rows x 8000 tokens: 102 -> 107 us).
-template <int D, int IPBK, int IPBV, int C>
+template <int D, int IPBK, int IPBV, int C, bool STREAM>
 __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArgs a) {
     static_assert(DTHREADS == LUT_THREADS, "threads that stage the tables");
     constexpr int QT = D != 128 || IPBK == 1 ? 2 : 1;    // fp16 terms of a rotated query
@@ -412,6 +412,9 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     uint16_t kn_raw, vn_raw;
     // n_tok >= 1: what lies past the last token is read as that token.  One form for whole and partial runs: with a branch between two
     // the registers are merged behind it, and that waits for the loads just issued.
+    auto load16 = [](const uint8_t *p) __attribute__((always_inline)) { return STREAM ? tq_gload16_stream(p) : tq_gload16(p); };
+    auto load8 = [](const uint8_t *p) __attribute__((always_inline)) { return STREAM ? tq_gload8_stream(p) : tq_gload8(p); };
+    auto load4 = [](const uint8_t *p) __attribute__((always_inline)) { return STREAM ? tq_gload4_stream(p) : tq_gload4(p); };
     auto issue_keys = [&](uint32_t t0, uint32_t n_tok) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < SUB; ++u)
@@ -422,20 +425,20 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 if constexpr (KB % 16 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 16; ++p) {
-                        const tq_u4 v = tq_gload16(src + 16 * p);
+                        const tq_u4 v = load16(src + 16 * p);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) kraw[u][b][4 * p + i] = v[i];
                     }
                 } else if constexpr (KB % 8 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 8; ++p) {
-                        const tq_u2 v = tq_gload8(src + 8 * p);
+                        const tq_u2 v = load8(src + 8 * p);
                         kraw[u][b][2 * p] = v[0]; kraw[u][b][2 * p + 1] = v[1];
                     }
                 } else if constexpr (KB % 4 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 4; ++p)
-                        kraw[u][b][p] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)src + 4 * p);
+                        kraw[u][b][p] = load4(src + 4 * p);
                 } else {
                     static_assert(KB % 2 == 0, "key bytes of a lane");
                     uint32_t h[KB / 2];
@@ -451,8 +454,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
 #pragma unroll
         for (int p = 0; p < NVP; ++p) {
             const uint32_t piece = min(p * 64u + lane, min((uint32_t)VPIECES, n_tok * (GBV / VPB)) - 1u);
-            if constexpr (VPB == 16) vpiece[p] = tq_gload16(vsrc + piece * 16u);
-            else { const tq_u2 v = tq_gload8(vsrc + piece * 8u); vpiece[p][0] = v[0]; vpiece[p][1] = v[1]; }
+            if constexpr (VPB == 16) vpiece[p] = load16(vsrc + piece * 16u);
+            else { const tq_u2 v = load8(vsrc + piece * 8u); vpiece[p][0] = v[0]; vpiece[p][1] = v[1]; }
         }
         const uint32_t own = min(lane, n_tok - 1u);       // (lanes past the end: see trip)
         kn_raw = tq_gload2(a.k_norms + slot0 + t0 + own);
@@ -1111,18 +1114,24 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     if (g0 < G) rotate_back(std::integral_constant<int, 4>{}, g0);
 }
 
+// STREAM: what decides is whether the history can still lie in the last-level cache (256 MB) when the next step comes for it.  A layer of 8 MiB is
+// taken for one that does not: 32 of them fill it, and so do the weights that a model reads between two steps.  Read with the
+// non-temporal hint, what is used once no longer drives out what every block of the next launch reads (tables, operands, code), and few rows start and
+// merge sooner.  us a pass without / with it, 128 wide unless stated: 32 layers of 8 x 32768 tokens 669 / 635, 16 of 32 x 6000 at 64 276 / 264, 24
+// of 128 x 4182 642 / 620, 8 of 512 x 16384 1378 / 1355.  Caches that fit lose by it: 32 of 2 x 8738 476 / 484, 16 of 8 x 6289 270 / 280.
+template <int D, int IPBK, int IPBV, int C>
+int launch_decode(dim3 grid, hipStream_t s, const TqDecodeArgs &a) {
+    const uint64_t bytes = (uint64_t)grid.y * a.tokens * (D / IPBK + D / IPBV + 4);
+    if (bytes >= 8u << 20) hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, C, true>), grid, dim3(DTHREADS), 0, s, a);
+    else hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, C, false>), grid, dim3(DTHREADS), 0, s, a);
+    return (int)hipGetLastError();
+}
 template <int D, int IPBK, int IPBV>
 int launch_decode(dim3 grid, hipStream_t s, const TqDecodeArgs &a) {
-    const dim3 block(DTHREADS);
     if constexpr (decode_run(D, IPBK, IPBV) == 64) {
-        if (a.group <= 4u) {
-            hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, 4>), grid, block, 0, s, a);
-            return (int)hipGetLastError();
-        }
+        if (a.group <= 4u) return launch_decode<D, IPBK, IPBV, 4>(grid, s, a);
     }
-    if (a.group <= 8u) hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, 2>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, 1>), grid, block, 0, s, a);
-    return (int)hipGetLastError();
+    return a.group <= 8u ? launch_decode<D, IPBK, IPBV, 2>(grid, s, a) : launch_decode<D, IPBK, IPBV, 1>(grid, s, a);
 }
 template <int D, int IPBK>
 int launch_decode(int ipbv, dim3 grid, hipStream_t s, const TqDecodeArgs &a) {

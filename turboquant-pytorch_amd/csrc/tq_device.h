@@ -253,6 +253,19 @@ __device__ __forceinline__ tq_u2 tq_gload8(const uint8_t *p) {
 __device__ __forceinline__ uint16_t tq_gload2(const uint16_t *p) {
     return *((const TQ_GLOBAL uint16_t *)p);
 }
+__device__ __forceinline__ uint32_t tq_gload4(const uint8_t *p) {
+    return *reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)p);
+}
+// Loads of what a launch reads once (the packed history of a decode step), with the non-temporal hint: when it pays, see launch_decode.
+__device__ __forceinline__ tq_u4 tq_gload16_stream(const uint8_t *p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const TQ_GLOBAL tq_u4 *>((const TQ_GLOBAL uint8_t *)p));
+}
+__device__ __forceinline__ tq_u2 tq_gload8_stream(const uint8_t *p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const TQ_GLOBAL tq_u2 *>((const TQ_GLOBAL uint8_t *)p));
+}
+__device__ __forceinline__ uint32_t tq_gload4_stream(const uint8_t *p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const TQ_GLOBAL uint32_t *>((const TQ_GLOBAL uint8_t *)p));
+}
 // Streaming store for bulk output that this launch does not read again (the de-quantised tensors): the
 // non-temporal hint keeps it out of the last-level cache.  Measured on the Llama-3-8B 32K workload: the 4- and
 // 8-bit decompress launches 4-5 % faster (436 -> 413 us, 340 -> 327 us), and packed codes that fit the
