@@ -121,7 +121,7 @@ def _build_fastcall(force: bool) -> None:
     _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-isystem" + p for p in cpp_extension.include_paths()),
           "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(rocm, "include"), sources[0], "-o", tmp,
-          *("-L" + p for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-L" + os.path.join(rocm, "lib"), "-lamdhip64"])
+          *("-L" + p for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-L" + os.path.join(rocm, "lib"), "-lamdhip64"])
     os.replace(tmp, path)
     for name in os.listdir(CSRC):
         if name.startswith(FAST_NAME + ".") and name.endswith(".so") and name != os.path.basename(path):
@@ -304,8 +304,7 @@ def fast():
         if module.abi_version != L.tq_abi_version():
             raise TqError(f"{path} was built for version {module.abi_version} of the library, this is {L.tq_abi_version()}: {how}")
         entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend_spread", "tq_qjl_compress", "tq_qjl_query_scores")
-        stream_of = _raw_stream or (lambda index: torch.cuda.current_stream(index).cuda_stream)
-        module.init(tuple(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in entries), stream_of, _workspace, _drop_workspace, _step_scratch, _arrived, _TABLE_TAG)
+        module.init(tuple(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in entries), _workspace, _drop_workspace, _step_scratch, _arrived, _TABLE_TAG)
         _fast = module
     return _fast
 
@@ -598,8 +597,7 @@ def compress_layer(keys: torch.Tensor, values: torch.Tensor, tokens: int, table_
         if got is not None:
             if type(got) is int:
                 check(got, "tq_compress_layer")
-            k_idx, k_nrm, v_idx, v_nrm, k_rest, v_rest = got
-            return (k_idx, k_nrm, k_rest), (v_idx, v_nrm, v_rest)
+            return got
     shape, stride, dtype, dev = keys.shape, keys.stride(), keys.dtype, keys.device
     if (values.shape != shape or values.stride() != stride or values.dtype != dtype or values.device != dev or dev.type != "cuda"
             or dtype not in _DTYPE_CODE or torch.compiler.is_compiling()):
@@ -639,14 +637,16 @@ def compress_layer(keys: torch.Tensor, values: torch.Tensor, tokens: int, table_
 
 
 def restore_layer(packed_k, packed_v, tokens: int, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int,
-                  k_win: torch.Tensor, v_win: torch.Tensor, w0: Optional[int] = None, n_win: int = 0):
+                  k_win: torch.Tensor, v_win: torch.Tensor, w0: Optional[int] = None, n_win: int = 0, shapes=None):
     """Full-length keys and values [B,H,tokens + n_win,D] in the windows' element type, from packed pairs (idx_bytes [B,H,tokens,G],
     vec_norms [B,H,tokens]: dense, or token slices of one per-row store) and the windows [B,H,n_win,D] behind them, in one
     call; None where the layout is not one the call takes (the caller then goes step by step).
     With w0, the pairs are whole per-row stores, of which the first `tokens` slots count, and k_win, v_win whole window buffers, of which
-    the tokens [w0, w0 + n_win) do."""
+    the tokens [w0, w0 + n_win) do.  `shapes`: what the results' and the pairs' shapes have to be (None where they are not)."""
     if k_win.is_cuda and not torch.compiler.is_compiling():
-        if w0 is None:
+        if shapes is not None:
+            got = fast().restore_dicts(*packed_k, *packed_v, tokens, table_k, table_v, bits_k, bits_v, k_win, v_win, *shapes)
+        elif w0 is None:
             got = fast().restore_layer(*packed_k, *packed_v, tokens, table_k, table_v, bits_k, bits_v, k_win, v_win)
         else:
             got = fast().restore_store(*packed_k, *packed_v, k_win, v_win, table_k, table_v, bits_k, bits_v, tokens, w0, n_win)
@@ -654,6 +654,10 @@ def restore_layer(packed_k, packed_v, tokens: int, table_k: torch.Tensor, table_
             if type(got) is int:
                 check(got, "tq_restore_layer")
             return got or None      # False: no call takes such a window
+    if shapes is not None:
+        B, H, S, D = shapes[0]
+        if k_win.shape != (B, H, S - tokens, D) or shapes[1] != (B, H, tokens, D):
+            return None
     if w0 is not None:
         packed_k, packed_v = (tuple(t[:, :, :tokens] for t in pair) for pair in (packed_k, packed_v))
         k_win, v_win = k_win[:, :, w0:w0 + n_win], v_win[:, :, w0:w0 + n_win]

@@ -116,8 +116,8 @@ class MSECompressor:
         B, H, S, D = states.shape
         indices_per_byte = 8 // self.bits
         idx_pad = (indices_per_byte - D % indices_per_byte) % indices_per_byte
-        table = self._tables.get(states.device)
-        packed = _native.fast().compress(states, table, self.bits) if table is not None and states.is_cuda and not torch.compiler.is_compiling() else None
+        table = self._tables.get(states.device)          # (of a HIP device, if there is one)
+        packed = _native.fast().compress(states, table, self.bits) if table is not None and not torch.compiler.is_compiling() else None
         if packed is None:
             with torch.no_grad():
                 packed = _native.call("compress", states, self.table(states.device), self.bits)
@@ -191,7 +191,7 @@ class MSECompressor:
         """Back to a float32 (B, H, S, D) tensor."""
         idx_bytes = compressed["idx_bytes"]
         table = self._tables.get(idx_bytes.device)
-        if table is not None and idx_bytes.is_cuda and not torch.compiler.is_compiling():
+        if table is not None and not torch.compiler.is_compiling():
             out = _native.fast().decompress(idx_bytes, compressed["vec_norms"], table, self.bits, compressed["shape"])
             if out is not None:
                 if type(out) is int:
@@ -275,16 +275,16 @@ class TurboQuantV3:
             )
         split_at = S - rw
         kc, vc = self.key_compressor, self.val_compressor
-        packed = None
-        if values.shape == keys.shape and keys.is_cuda and kc.head_dim == vc.head_dim == D:
-            packed = _native.compress_layer(keys, values, split_at, kc.table(keys.device), vc.table(keys.device), kc.bits, vc.bits)
+        packed, device = None, keys.device
+        if device.type == "cuda" and kc.head_dim == vc.head_dim == D:
+            packed = _native.compress_layer(keys, values, split_at, kc.table(device), vc.table(device), kc.bits, vc.bits)
         if packed is not None:
-            return tuple({
-                "compressed": {"idx_bytes": idx, "vec_norms": nrm, "shape": (B, H, split_at, D), "idx_pad": -D % (8 // comp.bits)},
-                "fp16": rest,
-                "shape": (B, H, S, D),
-                "split_at": split_at,
-            } for comp, (idx, nrm, rest) in ((kc, packed[0]), (vc, packed[1])))
+            (k_idx, k_nrm, k_rest), (v_idx, v_nrm, v_rest) = packed
+            shape, packed_shape = (B, H, S, D), (B, H, split_at, D)
+            return ({"compressed": {"idx_bytes": k_idx, "vec_norms": k_nrm, "shape": packed_shape, "idx_pad": -D % (8 // kc.bits)},
+                     "fp16": k_rest, "shape": shape, "split_at": split_at},
+                    {"compressed": {"idx_bytes": v_idx, "vec_norms": v_nrm, "shape": packed_shape, "idx_pad": -D % (8 // vc.bits)},
+                     "fp16": v_rest, "shape": shape, "split_at": split_at})
         return self._compress_by_tensor(keys, values, split_at)
 
     @torch.no_grad()
@@ -328,15 +328,14 @@ class TurboQuantV3:
         """Keys and values in one library call, or None where the dictionaries ask for something else than it does."""
         shape, split_at = compressed_k["shape"], compressed_k["split_at"]
         ck, cv, k_win, v_win = compressed_k["compressed"], compressed_v["compressed"], compressed_k["fp16"], compressed_v["fp16"]
-        B, H, S, D = shape
-        if (cv is None or compressed_v["shape"] != shape or compressed_v["split_at"] != split_at or k_win.shape != (B, H, S - split_at, D)
-                or ck["shape"] != (B, H, split_at, D) or cv["shape"] != ck["shape"] or not k_win.is_cuda):
+        device = k_win.device
+        if (cv is None or compressed_v["shape"] != shape or compressed_v["split_at"] != split_at or cv["shape"] != ck["shape"] or device.type != "cuda"):
             return None
         kc, vc = self.key_compressor, self.val_compressor
-        if kc.head_dim != D or vc.head_dim != D:
+        if kc.head_dim != shape[3] or vc.head_dim != shape[3]:
             return None
-        return _native.restore_layer((ck["idx_bytes"], ck["vec_norms"]), (cv["idx_bytes"], cv["vec_norms"]), split_at, kc.table(k_win.device),
-                                     vc.table(k_win.device), kc.bits, vc.bits, k_win, v_win)
+        return _native.restore_layer((ck["idx_bytes"], ck["vec_norms"]), (cv["idx_bytes"], cv["vec_norms"]), split_at, kc.table(device),
+                                     vc.table(device), kc.bits, vc.bits, k_win, v_win, shapes=(shape, ck["shape"]))
 
     def memory_bytes(self, B: int, H: int, S: int) -> dict:
         """Bytes stored including the uncompressed window (compressors_v3.py:235-265)."""

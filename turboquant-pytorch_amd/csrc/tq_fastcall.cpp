@@ -9,14 +9,16 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
 #include "../../include/tqamd.h"
 
 namespace {
 
-PyObject *g_raw_stream = nullptr;      // torch's: device index -> handle of the current stream
 PyObject *g_workspace = nullptr, *g_drop_workspace = nullptr;      // _native's: ticket counters of (device, stream)
 PyObject *g_scratch = nullptr, *g_arrived = nullptr;               // _native's: (device index, stream) -> tensor
 PyObject *g_tag = nullptr, *g_device = nullptr;                    // attribute names
@@ -86,12 +88,7 @@ struct Stream {
     explicit Stream(const at::Tensor &t) : dev(t.device().index()) {
         int current = -1;
         if (hipGetDevice(&current) != hipSuccess || current != dev) return;
-        PyObject *index = PyLong_FromLong(dev), *h = index ? PyObject_CallOneArg(g_raw_stream, index) : nullptr;
-        Py_XDECREF(index);
-        if (!h) throw Raised{};
-        handle = PyLong_AsUnsignedLongLong(h);
-        Py_DECREF(h);
-        if (PyErr_Occurred()) throw Raised{};
+        handle = (unsigned long long)reinterpret_cast<uintptr_t>(c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream());
         ok = true;
     }
     void *raw() const { return reinterpret_cast<void *>(handle); }
@@ -133,7 +130,12 @@ struct Workspace {
     ~Workspace() { Py_XDECREF(held); }
 };
 
+// From the allocator, without the dispatcher (which takes about as long again) unless somebody listens there: modes of torch, its function
+// transforms, algorithms that have to be deterministic (torch fills new memory then).
 inline at::Tensor empty(at::IntArrayRef shape, at::ScalarType type, const at::Tensor &like) {
+    constexpr c10::DispatchKeySet always({c10::DispatchKey::BackendSelect, c10::DispatchKey::ADInplaceOrView});
+    if ((c10::impl::tls_local_dispatch_key_set().included_ - always).empty() && !at::globalContext().deterministicAlgorithms())
+        return at::Tensor(at::detail::empty_cuda(shape, type, like.device(), std::nullopt));
     return at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
 }
 
@@ -229,7 +231,7 @@ PyObject *decompress(PyObject *const *a) {
     return THPVariable_Wrap(out);
 }
 
-// compress_layer(keys, values, tokens, table_k, table_v, bits_k, bits_v) -> (k_idx, k_norms, v_idx, v_norms, keys[:, :, tokens:], values[:, :, tokens:])
+// compress_layer(keys, values, tokens, table_k, table_v, bits_k, bits_v) -> ((k_idx, k_norms, keys[:, :, tokens:]), (v_idx, v_norms, values[:, :, tokens:]))
 PyObject *compress_layer(PyObject *const *a) {
     TENSOR(k, a[0]); TENSOR(v, a[1]);
     const int dt = dtype_code(k);
@@ -253,7 +255,18 @@ PyObject *compress_layer(PyObject *const *a) {
     const int rc = launch(lib.compress_layer, (const void *)address(k), (const void *)address(v), dt, n_rows, n_tokens, row_stride, ss, (const void *)address(tk),
                           (const void *)address(tv), (int)D, (int)bk, (int)bv, address(ki), (uint16_t *)address(kn), address(vi), (uint16_t *)address(vn), ws.address, s.raw());
     if (rc) { ws.drop(); return PyLong_FromLong(rc); }
-    return wrapped({ki, kn, vi, vn, k.slice(2, tokens), v.slice(2, tokens)});
+    PyObject *first = wrapped({ki, kn, k.slice(2, tokens)}), *second = nullptr, *both = nullptr;
+    try {
+        second = wrapped({vi, vn, v.slice(2, tokens)});
+        if (!(both = PyTuple_Pack(2, first, second))) throw Raised{};
+    } catch (...) {
+        Py_DECREF(first);
+        Py_XDECREF(second);
+        throw;
+    }
+    Py_DECREF(first);
+    Py_DECREF(second);
+    return both;
 }
 
 // the windows [B,H,n_win,D] behind `tokens` packed tokens a row: shared by the two callers below
@@ -276,6 +289,24 @@ PyObject *restore(PyObject *any, const at::Tensor &ki, const at::Tensor &kn, con
                           H > 1 ? sh : 0ll, (void *)address(k), (void *)address(v), dt, ws.address, s.raw());
     if (rc) { ws.drop(); return PyLong_FromLong(rc); }
     return wrapped({k, v});
+}
+
+inline bool tuple_is(PyObject *o, std::initializer_list<long long> want) {
+    if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != (Py_ssize_t)want.size()) return false;
+    Py_ssize_t i = 0;
+    for (long long w : want) if (integer(PyTuple_GET_ITEM(o, i++)) != w) return false;
+    return true;
+}
+
+// restore_dicts(k_idx, k_norms, v_idx, v_norms, tokens, table_k, table_v, bits_k, bits_v, k_win, v_win, shape, packed_shape): restore_layer where the
+// shapes of the two dictionaries are those of the tensors, None otherwise
+PyObject *restore_layer(PyObject *const *a);
+PyObject *restore_dicts(PyObject *const *a) {
+    TENSOR(kw, a[9]);
+    NEED(kw.dim() == 4);
+    const long long tokens = integer(a[4]), B = kw.size(0), H = kw.size(1), D = kw.size(3);
+    NEED(tuple_is(a[11], {B, H, tokens + kw.size(2), D}) && tuple_is(a[12], {B, H, tokens, D}));
+    return restore_layer(a);
 }
 
 // restore_layer(k_idx, k_norms, v_idx, v_norms, tokens, table_k, table_v, bits_k, bits_v, k_win, v_win) -> (keys, values); dense packed buffers
@@ -421,10 +452,10 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// init(addresses of the entry points in the order of Entries, raw_stream, workspace, drop_workspace, scratch, arrived, tag)
+// init(addresses of the entry points in the order of Entries, workspace, drop_workspace, scratch, arrived, tag)
 PyObject *init(PyObject *, PyObject *args) {
     PyObject *addresses, *tag;
-    if (!PyArg_ParseTuple(args, "O!OOOO!O!U", &PyTuple_Type, &addresses, &g_raw_stream, &g_workspace, &g_drop_workspace, &PyDict_Type, &g_scratch, &PyDict_Type, &g_arrived, &tag))
+    if (!PyArg_ParseTuple(args, "O!OOO!O!U", &PyTuple_Type, &addresses, &g_workspace, &g_drop_workspace, &PyDict_Type, &g_scratch, &PyDict_Type, &g_arrived, &tag))
         return nullptr;
     void *p[sizeof(Entries) / sizeof(void *)];
     if (PyTuple_GET_SIZE(addresses) != (Py_ssize_t)(sizeof(p) / sizeof(p[0]))) {
@@ -437,7 +468,7 @@ PyObject *init(PyObject *, PyObject *args) {
     }
     static_assert(sizeof(lib) == sizeof(p), "one address each");
     memcpy(&lib, p, sizeof(p));
-    for (PyObject *o : {g_raw_stream, g_workspace, g_drop_workspace, g_scratch, g_arrived}) Py_INCREF(o);      // kept for the life of the process
+    for (PyObject *o : {g_workspace, g_drop_workspace, g_scratch, g_arrived}) Py_INCREF(o);      // kept for the life of the process
     Py_INCREF(tag);
     g_tag = tag;
     g_device = PyUnicode_InternFromString("device");
@@ -447,7 +478,7 @@ PyObject *init(PyObject *, PyObject *args) {
 #define TQ_ENTRY(f, n) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<f, n>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"init", &init, METH_VARARGS, nullptr},
-    TQ_ENTRY(compress, 3), TQ_ENTRY(decompress, 5), TQ_ENTRY(compress_layer, 7), TQ_ENTRY(restore_layer, 11), TQ_ENTRY(restore_store, 13),
+    TQ_ENTRY(compress, 3), TQ_ENTRY(decompress, 5), TQ_ENTRY(compress_layer, 7), TQ_ENTRY(restore_layer, 11), TQ_ENTRY(restore_dicts, 13), TQ_ENTRY(restore_store, 13),
     TQ_ENTRY(decode_append, 7), TQ_ENTRY(decode_attend, 7), TQ_ENTRY(qjl_compress, 4), TQ_ENTRY(qjl_scores, 8),
     {nullptr, nullptr, 0, nullptr},
 };
