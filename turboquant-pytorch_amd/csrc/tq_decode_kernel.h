@@ -62,48 +62,53 @@ constexpr int decode_run(int d, int ipbk, int ipbv) { return d == 256 || (d > 64
 
 // Rotated queries of a row, q_rot[g][j] = scale * sum_i Pi[j][i] q[g][i]: a wave's 32 coordinates on the matrix cores, from the operands
 // of the key codec's table (Pi as three bf16 terms that add up to its float32 value, or for fp16 queries as two fp16 terms, 22 bits).
-// Loads and products apart, so that other loads can be under way between them.
+// Loads and products apart, so that other loads can be under way between them.  A row has 16 heads at most: two tiles of 16 x 16, which
+// take half the time of one of 32 x 32 (the table's operands are for that one: lane (row i, half hk) of step s has inputs 16 s + 8 hk ...;
+// here a lane picks the pieces that it needs).
 template <int D, bool BF>
 struct Rotation {
-    static constexpr int STEPS = D / 16, CH = STEPS < 8 ? STEPS : 8, TERMS = BF ? 3 : 2;     // CH: steps whose operands are in flight together
-    tq_u4 q[CH], p[TERMS][CH];
+    static constexpr int STEPS = D / 32, CH = STEPS < 4 ? STEPS : 4, TERMS = BF ? 3 : 2;     // CH: steps whose operands are in flight together
+    static_assert(STEPS % CH == 0, "whole chunks");
+    tq_u4 q[CH], p[2][TERMS][CH];
     const uint8_t *qsrc, *asrc;
     __device__ __forceinline__ void fetch(int s0) {
 #pragma unroll
         for (int s = 0; s < CH; ++s) {
-            q[s] = tq_gload16(qsrc + (s0 + s) * 32);
+            q[s] = tq_gload16(qsrc + (s0 + s) * 64);
 #pragma unroll
-            for (int t = 0; t < TERMS; ++t) p[t][s] = tq_gload16(asrc + (size_t)t * TQ_OPERAND_BYTES_FOR(D) + (size_t)(s0 + s) * 1024u);
+            for (int t = 0; t < TERMS; ++t)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) p[b][t][s] = tq_gload16(asrc + (size_t)t * TQ_OPERAND_BYTES_FOR(D) + (size_t)(s0 + s) * 2048u + 256u * b);
         }
     }
     // queries: the row's, [group][D]
     __device__ __forceinline__ void load(const uint8_t *queries, uint32_t group, const uint8_t *table_k, uint32_t tile, uint32_t lane) {
-        const uint32_t n = lane & 31u, hk = lane >> 5;
-        qsrc = queries + ((size_t)(n < group ? n : 0u) * D + 8u * hk) * 2u;
-        asrc = table_k + (BF ? TQ_OFF_A_BF16(D) : TQ_OFF_A_F16) + ((size_t)tile * STEPS * 64u + lane) * 16u;
+        const uint32_t n16 = lane & 15u, q4 = lane >> 4;
+        qsrc = queries + ((size_t)(n16 < group ? n16 : 0u) * D + 8u * q4) * 2u;
+        asrc = table_k + (BF ? TQ_OFF_A_BF16(D) : TQ_OFF_A_F16) + ((size_t)tile * (D / 16 * 64u) + q4 * 32u + n16) * 16u;
         fetch(0);
     }
     // qrot: [MAX_GROUP] rows of `stride` floats
     __device__ __forceinline__ void finish(float *qrot, uint32_t stride, float scale, uint32_t tile, uint32_t lane) {
-        static_assert(STEPS % CH == 0, "whole chunks");
-        const uint32_t n = lane & 31u, hk = lane >> 5;
-        tq_f16v acc = tq_zero16();
+        const uint32_t n16 = lane & 15u, q4 = lane >> 4;
+        tq_f4v acc[2] = {tq_f4v{0.f, 0.f, 0.f, 0.f}, tq_f4v{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll 1
         for (int s0 = 0;;) {
 #pragma unroll
             for (int s = 0; s < CH; ++s)
 #pragma unroll
-                for (int t = 0; t < TERMS; ++t) acc = BF ? mfma_bf16(p[t][s], q[s], acc) : mfma_f16(p[t][s], q[s], acc);
+                for (int t = 0; t < TERMS; ++t)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) acc[b] = BF ? mfma16_bf16(p[b][t][s], q[s], acc[b]) : mfma16_f16(p[b][t][s], q[s], acc[b]);
             s0 += CH;
             if (s0 >= STEPS) break;
             fetch(s0);
         }
         const float f = BF ? scale : scale * (1.0f / (float)(1 << TQ_F16_PI_SHIFT));
-        if (n < (uint32_t)MAX_GROUP) {
 #pragma unroll
-            for (int r = 0; r < 16; r += 4)
-                *reinterpret_cast<float4 *>(qrot + n * stride + 32u * tile + 16u * hk + r) = make_float4(acc[r] * f, acc[r + 1] * f, acc[r + 2] * f, acc[r + 3] * f);
-        }
+        for (int b = 0; b < 2; ++b)       // row i of the table's 32 holds coordinate 16 (i / 4 % 2) + 4 (i / 8) + i % 4
+            *reinterpret_cast<float4 *>(qrot + n16 * stride + 32u * tile + 16u * (q4 & 1u) + 8u * b + 4u * (q4 >> 1)) =
+                make_float4(acc[b][0] * f, acc[b][1] * f, acc[b][2] * f, acc[b][3] * f);
     }
 };
 
