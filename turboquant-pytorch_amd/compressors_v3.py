@@ -335,7 +335,7 @@ class TurboQuantV3:
         if kc.head_dim != shape[3] or vc.head_dim != shape[3]:
             return None
         return _native.restore_layer((ck["idx_bytes"], ck["vec_norms"]), (cv["idx_bytes"], cv["vec_norms"]), split_at, kc.table(device),
-                                     vc.table(device), kc.bits, vc.bits, k_win, v_win, shapes=(shape, ck["shape"]))
+                                     vc.table(device), kc.bits, vc.bits, k_win, v_win, None, 0, (shape, ck["shape"]))
 
     def memory_bytes(self, B: int, H: int, S: int) -> dict:
         """Bytes stored including the uncompressed window (compressors_v3.py:235-265)."""
