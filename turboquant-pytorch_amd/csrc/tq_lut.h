@@ -39,33 +39,39 @@ constexpr int LUT_THREADS = 512;     // threads of the block that stages the tab
 // keys' entry in the first half of a row and the values' in the second.  The address of a lane's slot of an entry is then the byte,
 // moved up by eight bits, with the lane's offset below it: one v_perm_b32, where 128-byte rows took two or three instructions (and
 // v_dot4_u32_u8, one as well, is followed by idle cycles before its result can be used as an address).
-// Consecutive threads write consecutive 16-byte pieces, so the writes are free of conflicts; the eight threads of a table
-// row read the same entry.
+// Eight consecutive threads write the 128 bytes of a table's half row, so the writes are free of conflicts; they read the same four entries
+// with one or two loads (a load for each entry, eight of them a thread for keys and values, stood in front of the other loads of a
+// block's start: 32 layers of 8 x 32768 tokens, K4/V2 628 -> 617 us, 16 of 32 x 6000 at 64 260 -> 258, 16 of 4 x 25627 266 -> 263).
 template <int B, typename T>
 __device__ __forceinline__ T lut_entry(const uint8_t *lut, uint32_t raw, uint32_t slot) {      // entry <byte B of raw>
     return *reinterpret_cast<const T *>(lut + __builtin_amdgcn_perm(raw, slot, 0x0c0c0000u | ((4u + B) << 8)));
 }
 template <int IPB>
 struct Lut {
-    static constexpr int ES = 2 * IPB;
-    static constexpr int TRIPS = 256 * 8 / LUT_THREADS;
-    tq_u4 v[TRIPS];
+    static constexpr int ES = 2 * IPB, ROWS = 256 * 8 / LUT_THREADS;        // a thread has ROWS entries in a row, which it loads together
+    static constexpr int WORDS = ROWS * ES / 4;
+    static_assert(ROWS == 4, "entries of a thread");
+    uint32_t v[WORDS];
     __device__ __forceinline__ void load(const uint8_t *src, uint32_t tid) {
+        const uint8_t *g = src + (tid >> 3) * (ROWS * ES);
+        if constexpr (WORDS == 2) { const tq_u2 x = tq_gload8(g); v[0] = x[0]; v[1] = x[1]; }
+        else {
 #pragma unroll
-        for (int k = 0; k < TRIPS; ++k) {
-            const TQ_GLOBAL uint8_t *g = (const TQ_GLOBAL uint8_t *)src + ((k * LUT_THREADS + tid) >> 3) * ES;
-            if constexpr (ES == 2) v[k][0] = *reinterpret_cast<const TQ_GLOBAL uint16_t *>(g);
-            else if constexpr (ES == 4) v[k][0] = *reinterpret_cast<const TQ_GLOBAL uint32_t *>(g);
-            else if constexpr (ES == 8) { const tq_u2 x = *reinterpret_cast<const TQ_GLOBAL tq_u2 *>(g); v[k][0] = x[0]; v[k][1] = x[1]; }
-            else v[k] = *reinterpret_cast<const TQ_GLOBAL tq_u4 *>(g);
+            for (int k = 0; k < WORDS; k += 4) {
+                const tq_u4 x = tq_gload16(g + 4 * k);
+                v[k] = x[0]; v[k + 1] = x[1]; v[k + 2] = x[2]; v[k + 3] = x[3];
+            }
         }
     }
     __device__ __forceinline__ void store(uint8_t *lds, uint32_t tid) {
 #pragma unroll
-        for (int k = 0; k < TRIPS; ++k) {
-            const tq_u4 x = ES <= 4 ? tq_u4{v[k][0], v[k][0], v[k][0], v[k][0]} : ES == 8 ? tq_u4{v[k][0], v[k][1], v[k][0], v[k][1]} : v[k];
-            const uint32_t piece = k * LUT_THREADS + tid;
-            *reinterpret_cast<tq_u4 *>(lds + (piece >> 3) * 256u + (piece & 7u) * 16u) = x;
+        for (int k = 0; k < ROWS; ++k) {
+            tq_u4 x;
+            if constexpr (ES == 2) { const uint32_t e = (v[k / 2] >> (16 * (k % 2))) & 0xffffu; x = tq_u4{e, e, e, e}; }
+            else if constexpr (ES == 4) x = tq_u4{v[k], v[k], v[k], v[k]};
+            else if constexpr (ES == 8) x = tq_u4{v[2 * k], v[2 * k + 1], v[2 * k], v[2 * k + 1]};
+            else x = tq_u4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+            *reinterpret_cast<tq_u4 *>(lds + ((tid >> 3) * ROWS + k) * 256u + (tid & 7u) * 16u) = x;
         }
     }
 };
