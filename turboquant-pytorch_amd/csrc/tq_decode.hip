@@ -195,8 +195,10 @@ int decode_splits(long long rows, long long tokens) {
     // One block is resident per compute unit.  A launch takes as many rounds of blocks as rows * splits fill the chip, each as
     // long as a block's tokens plus about what 2000 tokens take for tables, query rotation and result, and 400 more where the splits
     // of a row have to be merged; every record to merge counts like 12 tokens.  Blocks of less than 192 tokens gain nothing.
-    // (Best of a sweep / what this rule takes, us a launch, K4/V2: 8 x 32768 tokens 18.3 / 18.4 with 32 splits, 20.0 with 16 and 25.3 with 48;
-    // 2 x 8738 12.4 / 12.6; 8 x 1024 12.0 / 12.4, 14.9 in one split; 160 x 6000 34.6 / 34.6 in one split, 40.4 with 3; 128 x 4182 23.2 with 2.)
+    // (Best of a sweep / what this rule takes, us a layer with its append, K4/V2: 8 x 32768 tokens 19.1 / 19.1 with 32 splits, 21.1 with 16 and 26.2
+    // with 48; 2 x 8738 14.0 / 14.0; 32 x 6000 at 64, K6/V4, 15.8 / 15.8 with 8, 18.0 with 4; 128 x 4182, K3/V2, 24.6 with 2, 29.3 with 1, 33.1
+    // with 4; off the best 8 x 6289, K6/V4, 16.0 with 32 / 17.0 with 22 and 2 x 8574 at 96, K6/V4, 13.6 with 39 / 14.3 with 26.  A launch alone, when it was
+    // some 2 us longer: 8 x 1024 12.0 / 12.4, 14.9 in one split; 160 x 6000 34.6 / 34.6 in one split, 40.4 with 3.)
     long long most = (tokens + 191) / 192;
     if (most > MAX_SPLITS) most = MAX_SPLITS;
     long long best = 1, best_cost = 0;

@@ -57,7 +57,8 @@ __device__ __forceinline__ float fold(float a, float b) {
     return __uint_as_float(two[0]) + __uint_as_float(two[1]);
 }
 
-// Tokens a wave takes per trip: 32 where registers are short.
+// Tokens a wave takes per trip: 32 where registers are short, and with a byte per code from 96 on (64 fit by now, but take longer: 128 x 8192
+// tokens, K6/V4, 4 heads 393 -> 404 us for eight layers, K8/V8 474 -> 489; 96 wide, K8/V8, 7 heads 255 -> 277).
 constexpr int decode_run(int d, int ipbk, int ipbv) { return d == 256 || (d > 64 && (ipbk == 1 || ipbv == 1)) ? 32 : 64; }
 
 // Rotated queries of a row, q_rot[g][j] = scale * sum_i Pi[j][i] q[g][i]: a wave's 32 coordinates on the matrix cores, from the operands
@@ -329,6 +330,12 @@ struct WindowTile {
 // A tile of the window used to stand before the block's barrier: everybody in it waited 2.3 us (256 wide 4.4) for the wave that had it, and the row for the
 // block.  It is finished behind the barrier now; records are merged without loops around their loads.  us a layer, 4 heads, K4/V2: 8 rows x 32768
 // tokens 21.0 -> 20.3; 4 x 6000 16.4 -> 15.0; 64 wide, 32 x 6000 15.8 -> 14.8; 256 wide, 8 x 16384 35.3 -> 33.0.
+// Where the 17 us of a launch of 8 rows x 32768 tokens lie now (clock stamps, medians of the last block): 3.6 until the first tables and operands are
+// there and the barrier is passed, 0.5 the queries' operands, 4.7 two runs a wave (what reading 26 MB takes), 1.0 the 8 tokens over, 1.2 the waves' sums, 0.9 stores and
+// count, 2.3 the records of 32 blocks, 0.9 back through Pi_v.  What moved it last, a layer with its append: counters apart and Pi_v early 21.7 -> 20.9,
+// history past the caches 19.8, products of 16 x 16 and tables in fewer loads 19.3.  (One loop body for whole and partial runs: a trip of it takes
+// 2.05 us for 1.9 and the partial one still 1.0, a chain of latencies.  All waves rotating, or a barrier between the operands and the history: nothing
+// at 128, 1 % longer at 96.)
 // Before that, whole step of 32 layers 948 -> 778 us (734 since the append asks for all of its loads at once, see tq_decode.hip); 64 wide, 32 rows x 6000 tokens, K6/V4, 16 layers 394 -> 336; 512 rows x 16384 tokens, 8 layers 1565 -> 1404.
 // The matrix products have 16 columns and a row of the cache seldom 16 query heads.  C blocks of 16 tokens share them (C = 4 for up to 4
 // heads, 2 for up to 8): every block's scores are computed for the heads repeated C times, a lane keeps those of its own column's
@@ -908,8 +915,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     float *ysum = reinterpret_cast<float *>(&lds_area[0][0]);     // [head][D]: sums in the rotated space
     float *wsum = ysum + MAX_GROUP * D;                           // [head][D]: the window's, plain
     // Where few records meet there is one trip to memory: references and sums of exp of a head's records (a lane each), the sums (four columns
-    // a lane, every fourth record; the quarters of a wave are added in registers) and the rows of Pi_v, which are needed last, are under way
-    // together.  No loop holds a load there: behind one the compiler waits for everything in flight, the rows of Pi_v among it (32 rows x 6000
+    // a lane, every fourth record; the quarters of a wave are added in registers) and, if they are not on their way already, the rows of Pi_v,
+    // which are needed last, are under way together.  No loop holds a load there: behind one the compiler waits for everything in flight, the rows of Pi_v among it (32 rows x 6000
     // tokens, 64 wide, from the last arrival to merged sums: 1.9 us with loops, now 1.4).  What is left grows with the records: one compute unit reads
     // what other dies wrote at some 27 KB/us (8 rows x 32768, 66 KB: 2.4 us; 256 wide, 8 x 9906, 120 KB and 256 KB of Pi_v: 5.2).  Little code: it runs once and is fetched for the first time
     // (33 loads a lane, written out: 2.0 us from the first to the last of them, now 0.4).
