@@ -184,3 +184,54 @@ def test_v2_scores_of_a_negated_view(pkg):
     got, want = comp.asymmetric_attention_scores(torch._neg_view(q), packed), comp.asymmetric_attention_scores(-q, packed)
     scale = q.double().norm(dim=-1)[..., None] * x.double().norm(dim=-1)[:, :, None, :]
     assert float(((got.double() - want.double()).abs() / scale).max()) < 3e-5      # (two kernels: as in test_v2_scores_of_few_queries_equal_those_of_many)
+
+
+def test_outputs_are_seen_by_those_who_listen(pkg):
+    """Outputs come from the allocator directly, and through torch's dispatcher where a mode or deterministic algorithms want to see them; inference
+    mode makes inference tensors either way."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    comp = pkg.MSECompressor(128, 4, seed=42, device=DEV)
+    x = outlier_kv((1, 2, 70, 128), seed=3, dtype=torch.bfloat16).to(DEV)
+    want = comp.compress(x)
+    full = comp.decompress(want)
+    with Seen() as seen:
+        _same(comp.compress(x), want)
+        _same(comp.decompress(want), full)
+    assert sum("empty" in n for n in seen.names) >= 3
+    torch.use_deterministic_algorithms(True)
+    try:
+        _same(comp.compress(x), want)
+        _same(comp.decompress(want), full)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    with torch.inference_mode():
+        got = comp.compress(x)
+        out = comp.decompress(got)
+    assert out.is_inference() and got["idx_bytes"].is_inference() and torch.equal(out, full)
+
+
+def test_decompress_kv_with_shapes_that_are_not_the_tensors(pkg):
+    """Dictionaries whose shapes are lists, or numbers of another type, restore as tuples of integers do; shapes of other tensors are not taken."""
+    comp = pkg.TurboQuantV3(128, key_bits=4, value_bits=2, residual_window=16, layer_idx=8, device=DEV)
+    k = outlier_kv((1, 2, 70, 128), seed=4, dtype=torch.float16).to(DEV)
+    pair = comp.compress_kv(k, k)
+    want = comp.decompress_kv(*pair)
+    for form in (list, lambda t: tuple(float(i) for i in t), torch.Size):
+        if form is list or form is torch.Size:
+            other = [dict(c, shape=form(c["shape"]), compressed=dict(c["compressed"], shape=form(c["compressed"]["shape"]))) for c in pair]
+            _same(comp.decompress_kv(*other), want)
+        else:
+            assert pkg._native.fast().restore_dicts(*[pair[i]["compressed"][n] for i in (0, 1) for n in ("idx_bytes", "vec_norms")], 54, comp.key_compressor.table(k.device),
+                                                    comp.val_compressor.table(k.device), 4, 2, pair[0]["fp16"], pair[1]["fp16"], form(pair[0]["shape"]),
+                                                    pair[0]["compressed"]["shape"]) is None
+    assert comp._restore(*[dict(c, shape=(1, 2, 71, 128)) for c in pair]) is None

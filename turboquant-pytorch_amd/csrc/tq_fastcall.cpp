@@ -294,7 +294,10 @@ PyObject *restore(PyObject *any, const at::Tensor &ki, const at::Tensor &kn, con
 inline bool tuple_is(PyObject *o, std::initializer_list<long long> want) {
     if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != (Py_ssize_t)want.size()) return false;
     Py_ssize_t i = 0;
-    for (long long w : want) if (integer(PyTuple_GET_ITEM(o, i++)) != w) return false;
+    for (long long w : want) {
+        PyObject *const v = PyTuple_GET_ITEM(o, i++);
+        if (!PyLong_Check(v) || integer(v) != w) return false;
+    }
     return true;
 }
 
