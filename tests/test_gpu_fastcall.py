@@ -235,3 +235,15 @@ def test_decompress_kv_with_shapes_that_are_not_the_tensors(pkg):
                                                     comp.val_compressor.table(k.device), 4, 2, pair[0]["fp16"], pair[1]["fp16"], form(pair[0]["shape"]),
                                                     pair[0]["compressed"]["shape"]) is None
     assert comp._restore(*[dict(c, shape=(1, 2, 71, 128)) for c in pair]) is None
+
+
+def test_outputs_are_recorded_for_the_profiler(pkg):
+    """torch's profiler (and any other observer of operators) sees the outputs being made, on the calling thread and by name."""
+    comp = pkg.MSECompressor(128, 4, seed=42, device=DEV)
+    layer = pkg.TurboQuantV3(128, key_bits=4, value_bits=2, residual_window=16, layer_idx=8, device=DEV)
+    x = outlier_kv((1, 2, 70, 128), seed=3, dtype=torch.bfloat16).to(DEV)
+    want = (comp.compress(x), layer.compress_kv(x, x))
+    for call, outputs in ((lambda: comp.compress(x), 2), (lambda: comp.decompress(want[0]), 1), (lambda: layer.compress_kv(x, x), 4), (lambda: layer.decompress_kv(*want[1]), 2)):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+            call()
+        assert sum(e.name.startswith("aten::empty") for e in prof.events()) == outputs, [e.name for e in prof.events()]

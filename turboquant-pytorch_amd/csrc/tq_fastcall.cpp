@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
@@ -131,10 +132,10 @@ struct Workspace {
 };
 
 // From the allocator, without the dispatcher (which takes about as long again) unless somebody listens there: modes of torch, its function
-// transforms, algorithms that have to be deterministic (torch fills new memory then).
+// transforms, its profiler and other observers of operators, algorithms that have to be deterministic (torch fills new memory then).
 inline at::Tensor empty(at::IntArrayRef shape, at::ScalarType type, const at::Tensor &like) {
     constexpr c10::DispatchKeySet always({c10::DispatchKey::BackendSelect, c10::DispatchKey::ADInplaceOrView});
-    if ((c10::impl::tls_local_dispatch_key_set().included_ - always).empty() && !at::globalContext().deterministicAlgorithms())
+    if ((c10::impl::tls_local_dispatch_key_set().included_ - always).empty() && !at::globalContext().deterministicAlgorithms() && !at::hasCallbacks())
         return at::Tensor(at::detail::empty_cuda(shape, type, like.device(), std::nullopt));
     return at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
 }
