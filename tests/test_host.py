@@ -802,6 +802,36 @@ def test_extension_built_against_something_else_is_not_used(pkg, monkeypatch):
     assert native.fast() is native.fast()
 
 
+@pytest.mark.parametrize("interface", [None, 1, 3])
+def test_extension_of_another_interface_is_not_used(pkg, monkeypatch, interface):
+    """A module left over from other sources, built for the same version of the library, is refused with how to build it, before anything of it is called."""
+    import types
+    from importlib import machinery
+    native = pkg._native
+
+    class Stale(types.ModuleType):
+        abi_version = native.lib().tq_abi_version()
+
+        def init(self, *args):
+            raise TypeError("function takes exactly 7 arguments")
+
+    class Loader:
+        def __init__(self, name, path):
+            pass
+
+        def create_module(self, spec):
+            return Stale(spec.name)
+
+        def exec_module(self, module):
+            if interface is not None:
+                module.interface = interface
+
+    monkeypatch.setattr(native, "_fast", None)
+    monkeypatch.setattr(machinery, "ExtensionFileLoader", Loader)
+    with pytest.raises(native.TqError, match="build"):
+        native.fast()
+
+
 def test_decode_attend_counts_the_float_that_aligns_its_scratch(pkg):
     """Records are written and exchanged between blocks 8 bytes at a time: scratch at an odd multiple of 4 loses its first float, which
     tq_decode_scratch_floats includes.  (Nothing is launched: the scratch is always one float short.)"""

@@ -23,6 +23,7 @@ CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libtqamd.so")
 FAST_NAME = "tqamd_fastcall"        # extension module: the eager calls from tensors to the library in one step each
 FAST_SOURCE = "tq_fastcall.cpp"
+FAST_INTERFACE = 2                  # INTERFACE there: what init and the functions take and answer
 # (the ones that take longest to compile first)
 SOURCES = ("tq_decode_d256.hip", "tq_decode_d96.hip", "tq_decode_d64.hip", "tq_decode_d128_narrow.hip", "tq_decode_d128_wide.hip", "tq_compress.hip", "tq_decompress.hip",
            "tq_wide_d224.hip", "tq_wide_d192.hip", "tq_wide_d160.hip", "tq_wide_d96.hip", "tq_anydim.hip", "tq_attend.hip", "tq_qjl.hip",
@@ -303,6 +304,8 @@ def fast():
             raise TqError(f"{path} cannot be loaded ({e}): {how}") from e
         if module.abi_version != L.tq_abi_version():
             raise TqError(f"{path} was built for version {module.abi_version} of the library, this is {L.tq_abi_version()}: {how}")
+        if getattr(module, "interface", None) != FAST_INTERFACE:       # (modules of before had none)
+            raise TqError(f"{path} was built from another state of {FAST_SOURCE}: {how}")
         entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend_spread", "tq_qjl_compress", "tq_qjl_query_scores")
         module.init(tuple(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in entries), _workspace, _drop_workspace, _step_scratch, _arrived, _TABLE_TAG)
         _fast = module

@@ -20,6 +20,8 @@
 
 namespace {
 
+constexpr int INTERFACE = 2;      // of this module to _native.py (FAST_INTERFACE there): raised with any change of what init or a function takes or answers
+
 PyObject *g_workspace = nullptr, *g_drop_workspace = nullptr;      // _native's: ticket counters of (device, stream)
 PyObject *g_scratch = nullptr, *g_arrived = nullptr;               // _native's: (device index, stream) -> tensor
 PyObject *g_tag = nullptr, *g_device = nullptr;                    // attribute names
@@ -492,7 +494,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "tqamd_fastcall", nullptr, -1, meth
 
 PyMODINIT_FUNC PyInit_tqamd_fastcall(void) {
     PyObject *m = PyModule_Create(&module);
-    if (m && PyModule_AddIntConstant(m, "abi_version", TQ_ABI_VERSION) < 0) {
+    if (m && (PyModule_AddIntConstant(m, "abi_version", TQ_ABI_VERSION) < 0 || PyModule_AddIntConstant(m, "interface", INTERFACE) < 0)) {
         Py_DECREF(m);
         return nullptr;
     }
