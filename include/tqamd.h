@@ -420,6 +420,10 @@ int tq_attend_step(const void *queries, int q_dtype, long long rows, int group, 
  *   is shared by launches that can overlap in time.
  * tq_decode_attend_spread: the same with n_arrived >= rows counters (TQ_ERR_CAPACITY if fewer): from 32 * rows on every row
  *   has a line of memory to itself, which few rows with many blocks each finish sooner with.
+ * tq_decode_attend_cached: the same for a layer of a cache of which a step reads cache_bytes bytes (packed codes, norms and window of all
+ *   layers together; 0: not known, as for the two calls above).  They decide with which loads the history is read, by whether the
+ *   cache can stay in the last-level cache from one step to the next; results are the same bytes either way.
+ * tq_decode_streams: 1 if such a history is read with the non-temporal hint, 0 if not.
  * tq_decode_supported: 1 if these calls take the combination, 0 otherwise.
  */
 typedef struct tq_decode_layer {
@@ -441,6 +445,10 @@ int tq_decode_attend(const tq_decode_layer *layer, const void *queries, int grou
 int tq_decode_attend_spread(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
                             long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, long long n_arrived, void *out,
                             void *stream);
+int tq_decode_attend_cached(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
+                            long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, long long n_arrived,
+                            long long cache_bytes, void *out, void *stream);
+int tq_decode_streams(const tq_decode_layer *layer, long long tokens, long long n_win, long long cache_bytes);
 int tq_decode_append(const tq_decode_layer *layer, const void *k_new, const void *v_new, long long k_new_stride, long long v_new_stride,
                      long long evict, long long put, long long packed_slot, void *stream);
 

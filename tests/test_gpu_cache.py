@@ -873,6 +873,47 @@ def test_decode_attention_of_a_layer_on_either_side_of_streaming(pkg, dim, bits)
             assert err < (1.5e-3 if dim == 128 else 3.5e-4), (tokens, group, err)
 
 
+@pytest.mark.parametrize("dim,bits", [(64, (6, 4)), (64, (2, 8)), (64, (4, 4)), (96, (2, 2)), (96, (4, 2)), (96, (8, 8)), (128, (4, 2)), (128, (1, 1)), (128, (2, 4)), (128, (8, 8)),
+                                      (256, (4, 2)), (256, (2, 8)), (256, (8, 4))])
+def test_decode_attention_gives_the_same_bytes_streamed(pkg, monkeypatch, dim, bits):
+    """A history read with the non-temporal hint and without it: the same products and sums in the same order.  One row and several, histories
+    that end inside a run, groups of every number of blocks; eager steps, captured ones and the C ABI's calls for a cache whose size is not known."""
+    native = pkg._native
+    g = torch.Generator().manual_seed(dim + bits[0])
+    fits, large = 1, 1 << 40
+    asked = []
+    real = native.fast()
+
+    class Spy:
+        def __getattr__(self, name):
+            if name != "decode_attend":
+                return getattr(real, name)
+            return lambda *args: asked.append(args[-1]) or real.decode_attend(*args)
+
+    for rows, tokens in ((1, 33), (2, 4099), (5, 1025)):
+        cache = pkg.V3Cache(bits[0], bits[1], residual_window=20, n_layers=40)
+        k, v = (torch.randn(1, rows, tokens + 20, dim, generator=g).half().to(DEV) for _ in range(2))
+        cache.append(k, v, 8)
+        st = cache._stores[8]
+        for group in (1, 5, 16):
+            q = torch.randn(1, rows * group, 1, dim, generator=g).half().to(DEV)
+            want = cache.attend(q, 8)
+            for size in (fits, large):
+                st.cache_slot_bytes, st.cache_window_bytes = 0, size
+                with monkeypatch.context() as m:
+                    m.setattr(native, "fast", Spy)
+                    assert torch.equal(cache.attend(q, 8), want), (rows, tokens, group, size)
+                assert asked[-1] == size and native.lib().tq_decode_streams(ctypes.addressof(st.record()), tokens, 20, size) == (size == large)
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph):
+                    out = cache.attend(q, 8)
+                for _ in range(2):
+                    out.zero_()
+                    graph.replay()
+                    torch.cuda.synchronize()
+                    assert torch.equal(out, want), (rows, tokens, group, size)
+
+
 @pytest.mark.parametrize("n_arrived", [5, 9, 10, 63, 64, 159, 160, 1000])
 def test_decode_attention_with_counters_at_any_spread(pkg, n_arrived):
     """5 rows whose arrival counters lie 1 to 32 apart, by how many there are: the same bytes, all counters zero again, none touched past the last."""

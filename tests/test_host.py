@@ -802,8 +802,8 @@ def test_extension_built_against_something_else_is_not_used(pkg, monkeypatch):
     assert native.fast() is native.fast()
 
 
-@pytest.mark.parametrize("interface", [None, 1, 3])
-def test_extension_of_another_interface_is_not_used(pkg, monkeypatch, interface):
+@pytest.mark.parametrize("apart", [None, -1, 1])
+def test_extension_of_another_interface_is_not_used(pkg, monkeypatch, apart):
     """A module left over from other sources, built for the same version of the library, is refused with how to build it, before anything of it is called."""
     import types
     from importlib import machinery
@@ -823,8 +823,8 @@ def test_extension_of_another_interface_is_not_used(pkg, monkeypatch, interface)
             return Stale(spec.name)
 
         def exec_module(self, module):
-            if interface is not None:
-                module.interface = interface
+            if apart is not None:
+                module.interface = native.FAST_INTERFACE + apart
 
     monkeypatch.setattr(native, "_fast", None)
     monkeypatch.setattr(machinery, "ExtensionFileLoader", Loader)
@@ -850,3 +850,59 @@ def test_decode_attend_spread_wants_a_counter_for_every_row(pkg):
     size = native.lib().tq_decode_scratch_floats(8, 4, 128, 1000, 128)
     attend = lambda n_arrived: native.lib().tq_decode_attend_spread(ctypes.addressof(layer), 4096, 4, 1.0, 0, 128, 1000, 4096, size, 4096, n_arrived, 4096, None)  # noqa: E731
     assert attend(7) == native.ERR_CAPACITY and attend(0) == native.ERR_CAPACITY
+
+
+# rows, tokens, dim, bits, layers, window -> streamed if the cache's size is known, if it is not
+@pytest.mark.parametrize("rows,tokens,dim,bits,layers,window,cache,alone", [
+    (8, 6289, 128, (6, 4), 16, 128, False, False),      # 9.4 MiB a layer, 158 MiB with the windows: stays in the last-level cache
+    (8, 6289, 128, (6, 4), 32, 128, True, False),       # 32 of them do not
+    (2, 8738, 128, (4, 2), 32, 128, False, False),
+    (8, 32768, 128, (4, 2), 32, 128, True, True),
+    (8, 32768, 128, (4, 2), 8, 128, False, True),       # eight layers of 25 MiB fit; who says nothing is taken to have sixteen
+    (32, 6000, 64, (6, 4), 16, 128, True, True),
+    (128, 655, 128, (4, 2), 16, 128, True, True),       # half of it windows
+    (128, 655, 128, (4, 2), 16, 0, False, False),
+    (512, 16384, 128, (4, 2), 1, 128, True, True),
+    (1, 0, 128, (4, 2), 16, 128, False, False),
+])
+def test_decode_attention_streams_what_the_last_level_cache_cannot_keep(pkg, rows, tokens, dim, bits, layers, window, cache, alone):
+    native = pkg._native
+    layer = native.TqDecodeLayer(*([4096] * 9), 1024 * dim, max(tokens, 1), rows, dim, native.TQ_BF16, *bits)
+    streams = lambda cache_bytes: native.lib().tq_decode_streams(ctypes.addressof(layer), tokens, window, cache_bytes)  # noqa: E731
+    width = sum(pkg.kv_cache._LayerStore._width(dim, b) for b in bits) + 4
+    per_layer = rows * (tokens * width + window * 4 * dim)
+    assert streams(layers * per_layer) == cache and streams(0) == alone
+    limit = 224 << 20
+    assert (streams(limit - 1), streams(limit)) == (0, 1) and streams(-1) == streams(0)
+
+
+def test_decode_streams_checks_its_arguments(pkg):
+    native = pkg._native
+    layer = native.TqDecodeLayer(*([4096] * 9), 128 * 128, 2000, 8, 128, native.TQ_BF16, 4, 2)
+    at = ctypes.addressof(layer)
+    assert native.lib().tq_decode_streams(None, 10, 0, 0) == native.lib().tq_decode_streams(0, 10, 0, 0) == -1
+    for tokens, window in ((-1, 0), (1 << 31, 0), (10, -1), (10, 513)):
+        assert native.lib().tq_decode_streams(at, tokens, window, 0) < 0
+    layer.bits_k = 9
+    assert native.lib().tq_decode_streams(at, 10, 0, 0) < 0
+
+
+def test_layers_know_the_size_of_their_cache(pkg, recorded, tmp_path):
+    """Every layer counts all layers of its cache, protected ones of other widths and ones added later among them; so do copies and loaded caches."""
+    cache = pkg.V3Cache(4, 2, residual_window=4, protected_layers=1, n_layers=8, capacity=64)
+    slot, window = [], 2 * 2 * 3 * 4 * 128 * 2
+    for layer, wide in ((0, True), (1, False), (2, False), (7, True)):
+        x = torch.randn(2, 3, 4, 128).to(torch.bfloat16)
+        cache.append(x, x, layer)
+        slot.append(2 * 3 * (128 + 128 + 4 if wide else 64 + 32 + 4))
+        for st in cache._stores.values():
+            st.n_compressed = 10
+            assert st.cache_bytes() == 10 * sum(slot) + len(slot) * window
+            st.n_compressed = 0
+    for other in (copy.deepcopy(cache), pickle.loads(pickle.dumps(cache))):
+        assert {st.cache_bytes() for st in other._stores.values()} == {4 * window}
+    cache.save(str(tmp_path / "cache"))
+    loaded = pkg.V3Cache.load(str(tmp_path / "cache"), device="cpu")
+    assert [(st.cache_slot_bytes, st.cache_window_bytes) for st in loaded._stores.values()] == [(sum(slot), 4 * window)] * 4
+    lone = pkg.kv_cache._LayerStore(cache._get_compressor(3, 128, "cpu"), 2, 3, 128, torch.bfloat16, torch.device("cpu"), 64, 4)
+    assert lone.cache_bytes() == 0      # a layer of no cache does not know

@@ -23,7 +23,7 @@ CSRC = os.path.join(_HERE, "csrc")
 LIB_PATH = os.path.join(CSRC, "libtqamd.so")
 FAST_NAME = "tqamd_fastcall"        # extension module: the eager calls from tensors to the library in one step each
 FAST_SOURCE = "tq_fastcall.cpp"
-FAST_INTERFACE = 2                  # INTERFACE there: what init and the functions take and answer
+FAST_INTERFACE = 3                  # INTERFACE there: what init and the functions take and answer
 # (the ones that take longest to compile first)
 SOURCES = ("tq_decode_d256.hip", "tq_decode_d96.hip", "tq_decode_d64.hip", "tq_decode_d128_narrow.hip", "tq_decode_d128_wide.hip", "tq_compress.hip", "tq_decompress.hip",
            "tq_wide_d224.hip", "tq_wide_d192.hip", "tq_wide_d160.hip", "tq_wide_d96.hip", "tq_anydim.hip", "tq_attend.hip", "tq_qjl.hip",
@@ -213,7 +213,7 @@ EXPORTS = (
     "tq_qjl_compress", "tq_qjl_compress_batched", "tq_qjl_scores", "tq_qjl_query_scores",
     "tq_scores", "tq_weighted_values", "tq_weighted_values_splits", "tq_attend_partials", "tq_attend_splits",
     "tq_attend_prepare", "tq_attend_merge", "tq_append_token", "tq_attend_step",
-    "tq_decode_supported", "tq_decode_scratch_floats", "tq_decode_attend", "tq_decode_attend_spread", "tq_decode_append",
+    "tq_decode_supported", "tq_decode_scratch_floats", "tq_decode_attend", "tq_decode_attend_spread", "tq_decode_attend_cached", "tq_decode_streams", "tq_decode_append",
     "tq_compress_layer", "tq_restore_layer",
 )
 
@@ -272,6 +272,8 @@ def lib() -> ctypes.CDLL:
     L.tq_decode_scratch_floats.argtypes = [ll, ci, ci, ll, ll]
     L.tq_decode_attend.argtypes = [vp, vp, ci, ctypes.c_float, ll, ll, ll, vp, ll, vp, vp, vp]
     L.tq_decode_attend_spread.argtypes = [vp, vp, ci, ctypes.c_float, ll, ll, ll, vp, ll, vp, ll, vp, vp]
+    L.tq_decode_attend_cached.argtypes = [vp, vp, ci, ctypes.c_float, ll, ll, ll, vp, ll, vp, ll, ll, vp, vp]
+    L.tq_decode_streams.argtypes = [vp, ll, ll, ll]
     L.tq_decode_append.argtypes = [vp, vp, vp, ll, ll, ll, ll, ll, vp]
     L.tq_compress_layer.argtypes = [vp, vp, ci, ll, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, vp, vp, vp, vp]
     L.tq_restore_layer.argtypes = [vp, vp, vp, vp, ll, ll, ll, ll, vp, vp, ci, ci, ci, vp, vp, ll, ll, ll, vp, vp, ci, vp, vp]
@@ -306,7 +308,7 @@ def fast():
             raise TqError(f"{path} was built for version {module.abi_version} of the library, this is {L.tq_abi_version()}: {how}")
         if getattr(module, "interface", None) != FAST_INTERFACE:       # (modules of before had none)
             raise TqError(f"{path} was built from another state of {FAST_SOURCE}: {how}")
-        entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend_spread", "tq_qjl_compress", "tq_qjl_query_scores")
+        entries = ("tq_compress", "tq_decompress", "tq_compress_layer", "tq_restore_layer", "tq_decode_append", "tq_decode_attend_cached", "tq_qjl_compress", "tq_qjl_query_scores")
         module.init(tuple(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in entries), _workspace, _drop_workspace, _step_scratch, _arrived, _TABLE_TAG)
         _fast = module
     return _fast
@@ -565,9 +567,9 @@ def arrival_counters(device: torch.device, stream: int, rows: int) -> torch.Tens
     return buf
 
 
-def decode_attend(layer: TqDecodeLayer, queries: torch.Tensor, group: int, scale: float, win_first: int, n_win: int, tokens: int) -> torch.Tensor:
-    """tq_decode_attend into a new tensor of the queries' shape.  Scratch and counters are kept per stream, except while a
-    graph is being captured: then they come from the graph's own memory and the counters are cleared inside the graph."""
+def decode_attend(layer: TqDecodeLayer, queries: torch.Tensor, group: int, scale: float, win_first: int, n_win: int, tokens: int, cache_bytes: int = 0) -> torch.Tensor:
+    """tq_decode_attend (with the cache's size, where it is known: tq_decode_attend_cached) into a new tensor of the queries' shape.  Scratch and counters
+    are kept per stream, except while a graph is being captured: then they come from the graph's own memory and the counters are cleared inside the graph."""
     L = lib()
     dev = queries.device
     with _on(dev):
@@ -580,11 +582,12 @@ def decode_attend(layer: TqDecodeLayer, queries: torch.Tensor, group: int, scale
         else:
             counters = arrival_counters(dev, stream, layer.rows)
         args = lambda buf: (ctypes.addressof(layer), queries.data_ptr(), group, scale, win_first, n_win, tokens, buf.data_ptr(), buf.numel(),  # noqa: E731
-                            counters.data_ptr(), out.data_ptr(), stream)
-        rc = L.tq_decode_attend(*args(scratch))
+                            counters.data_ptr(), *((layer.rows, cache_bytes) if cache_bytes else ()), out.data_ptr(), stream)
+        entry = L.tq_decode_attend_cached if cache_bytes else L.tq_decode_attend
+        rc = entry(*args(scratch))
         if rc == ERR_CAPACITY:
             scratch = step_scratch(dev, stream, int(L.tq_decode_scratch_floats(layer.rows, group, layer.head_dim, tokens, n_win)))
-            rc = L.tq_decode_attend(*args(scratch))
+            rc = entry(*args(scratch))
     if rc:
         _arrived.pop((dev.index if dev.index is not None else torch.cuda.current_device(), stream), None)
     check(rc, "tq_decode_attend")
@@ -935,7 +938,7 @@ def _(k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, q_rot):
     return q_rot.new_empty((q_rot.shape[0], q_rot.shape[1], max(splits, 1), q_rot.shape[2] + 2), dtype=torch.float32)
 
 
-def _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_v, k_win, v_win, scale):
+def _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_v, k_win, v_win, scale, cache_bytes):
     """attend_packed through tq_decode_attend."""
     B, Hq, _, D = q.shape
     H, S, n_w = k_idx.shape[1], k_idx.shape[2], k_win.shape[2]
@@ -958,7 +961,7 @@ def _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_
                           k_idx.data_ptr() if S else None, k_norms.data_ptr() if S else None, v_idx.data_ptr() if S else None,
                           v_norms.data_ptr() if S else None, table_k.data_ptr(), table_v.data_ptr(), pi_v.data_ptr(), win_stride,
                           (prs_k or S) if S else 0, rows, D, dtype_code(q.dtype), bits_k, bits_v)
-    return decode_attend(layer, q, Hq // H, scale, 0, n_w, S)
+    return decode_attend(layer, q, Hq // H, scale, 0, n_w, S, cache_bytes)
 
 
 def _check_attend_packed(queries, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_k_t, pi_v, k_win, v_win):
@@ -987,10 +990,10 @@ def _check_attend_packed(queries, k_idx, k_norms, v_idx, v_norms, table_k, table
 def _attend_packed_impl(queries: torch.Tensor, k_idx: torch.Tensor, k_norms: torch.Tensor, v_idx: torch.Tensor,
                         v_norms: torch.Tensor, table_k: torch.Tensor, table_v: torch.Tensor, bits_k: int, bits_v: int,
                         pi_k_t: torch.Tensor, pi_v: torch.Tensor, k_win: torch.Tensor, v_win: torch.Tensor,
-                        scale: float) -> torch.Tensor:
+                        scale: float, cache_bytes: int = 0) -> torch.Tensor:
     """Decode-step attention of queries [B,Hq,1,D] over a packed history ([B,H,S,..] store slices, S may be 0)
     plus uncompressed window tokens [B,H,n_w,D] (n_w may be 0, not both): one launch where tq_decode_attend takes the
-    combination, otherwise three."""
+    combination, otherwise three.  cache_bytes: what a step reads of all layers of the cache together (0: not known)."""
     _require_gpu(queries, "queries")
     _check_attend_packed(queries, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_k_t, pi_v, k_win, v_win)
     B, Hq, _, D = queries.shape
@@ -1004,7 +1007,7 @@ def _attend_packed_impl(queries: torch.Tensor, k_idx: torch.Tensor, k_norms: tor
     pi_k_t, pi_v = pi_k_t.contiguous(), pi_v.contiguous()       # copies only if the caller kept a strided view
     L = lib()
     if group <= 16 and n_w <= 512 and rows <= 65535 and (k_win.dtype == v_win.dtype == q.dtype) and decode_supported(D, q.dtype, bits_k, bits_v):
-        return _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_v, k_win, v_win, scale)
+        return _attend_packed_one_launch(q, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_v, k_win, v_win, scale, cache_bytes)
     stream = _stream_handle(dev)
     q_rot = torch.empty((B, Hq, D), dtype=torch.float32, device=dev)
     part_w = torch.empty((rows, group, D + 2), dtype=torch.float32, device=dev) if n_w else None
@@ -1047,7 +1050,7 @@ attend_packed_op = torch.library.custom_op("tqamd::attend_packed", _attend_packe
 
 
 @attend_packed_op.register_fake
-def _(queries, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_k_t, pi_v, k_win, v_win, scale):
+def _(queries, k_idx, k_norms, v_idx, v_norms, table_k, table_v, bits_k, bits_v, pi_k_t, pi_v, k_win, v_win, scale, cache_bytes=0):
     return torch.empty_like(queries)
 
 

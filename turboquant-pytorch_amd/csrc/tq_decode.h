@@ -15,7 +15,7 @@ struct TqDecodeArgs {
     uint8_t *out;                    // [rows, group, D]
     long long win_stride;
     float scale;
-    uint32_t tokens, packed_row_stride, group, chunk, n_win, bf16, arrived_stride;
+    uint32_t tokens, packed_row_stride, group, chunk, n_win, bf16, arrived_stride, stream;
 };
 
 namespace {

@@ -187,6 +187,15 @@ void launch_append(dim3 grid, hipStream_t s, const AppendArgs &a) {
     else hipLaunchKernelGGL((tq_decode_append_kernel<D, false>), grid, block, 0, s, a);
 }
 
+// Packed histories are read with the non-temporal hint (see launch_decode) where the cache cannot stay in the last-level cache, 256 MiB, from one step
+// to the next: from 224 MiB on that a step reads, packed store and windows of all layers.  us of plain loads / with the hint, a step with
+// its appends, 128 wide and 8 rows unless stated: 16 layers of K4/V2 at 158 MiB 252 / 258, 200 273 / 278, 232 281 / 279, 360 300 / 295; 32 layers at
+// 144 473 / 492, 208 486 / 491, 240 514 / 511, 528 593 / 556; 16 of 6289 tokens, K6/V4, at 158 267 / 275; 32 x 3932 tokens at 64, K6/V4,
+// 16 layers at 208 233 / 236, 32 x 5242 at 272 248 / 242; 256 wide, 16 layers at 192 504 / 509, 32 layers at 256 1035 / 987; 128 rows x 655 tokens, half
+// of it windows, 16 layers at 256 291 / 281.  Of 291 sizes drawn 4 lose more than 1 % by this line, of 224 MiB of packed store alone 28, of 8 MiB
+// a layer 53.  A caller that names no cache is taken to have sixteen layers like this one.
+constexpr long long CACHE_STREAMED = 224ll << 20, LAYER_STREAMED = CACHE_STREAMED / 16;
+
 // splits of the token range per row
 int decode_splits(long long rows, long long tokens) {
     if (rows <= 0 || tokens <= 0) return 1;
@@ -209,6 +218,12 @@ int decode_splits(long long rows, long long tokens) {
         if (rounds > 16 && s > 1) break;
     }
     return (int)best;
+}
+
+// Whether the packed history is read with the non-temporal hint (what it does: see launch_decode).
+bool streams(const tq_decode_layer *l, long long tokens, long long n_win, long long cache_bytes) {
+    const long long slot = l->head_dim / (8 / l->bits_k) + l->head_dim / (8 / l->bits_v) + 4, layer = l->rows * (tokens * slot + n_win * l->head_dim * 4);
+    return cache_bytes > 0 ? cache_bytes >= CACHE_STREAMED : layer >= LAYER_STREAMED;
 }
 
 long long scratch_floats(long long rows, int group, int head_dim, int splits, long long n_win) {
@@ -242,9 +257,16 @@ extern "C" long long tq_decode_scratch_floats(long long rows, int group, int hea
     return scratch_floats(rows, group, head_dim, decode_splits(rows, tokens), n_win) + 1;      // (see tq_decode_attend)
 }
 
-extern "C" int tq_decode_attend_spread(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
-                                       long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, long long n_arrived, void *out,
-                                       void *stream) {
+extern "C" int tq_decode_streams(const tq_decode_layer *layer, long long tokens, long long n_win, long long cache_bytes) {
+    const int rc = check_layer(layer);
+    if (rc) return rc;
+    if (tokens < 0 || tokens > 0x7fffffff || n_win < 0 || n_win > MAX_WINDOW) return TQ_ERR_SIZE;
+    return streams(layer, tokens, n_win, cache_bytes) ? 1 : 0;
+}
+
+extern "C" int tq_decode_attend_cached(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
+                                       long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, long long n_arrived,
+                                       long long cache_bytes, void *out, void *stream) {
     const int rc = check_layer(layer);
     if (rc) return rc;
     const int D = layer->head_dim;
@@ -285,6 +307,7 @@ extern "C" int tq_decode_attend_spread(const tq_decode_layer *layer, const void 
     a.chunk = (uint32_t)(((tokens + splits - 1) / splits + 15) / 16 * 16);
     a.n_win = (uint32_t)n_win;
     a.bf16 = layer->dtype == TQ_BF16 ? 1u : 0u;
+    a.stream = streams(layer, tokens, n_win, cache_bytes) ? 1u : 0u;
     if (!tokens) {       // no history: the loads that every wave starts with find the tables instead, and nothing is done with them
         a.k_idx = a.table_k; a.v_idx = a.table_v;
         a.k_norms = reinterpret_cast<const uint16_t *>(a.table_k); a.v_norms = reinterpret_cast<const uint16_t *>(a.table_v);
@@ -301,9 +324,15 @@ extern "C" int tq_decode_attend_spread(const tq_decode_layer *layer, const void 
     }
 }
 
+extern "C" int tq_decode_attend_spread(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
+                                       long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, long long n_arrived, void *out,
+                                       void *stream) {
+    return tq_decode_attend_cached(layer, queries, group, scale, win_first, n_win, tokens, scratch, scratch_size, arrived, n_arrived, 0, out, stream);
+}
+
 extern "C" int tq_decode_attend(const tq_decode_layer *layer, const void *queries, int group, float scale, long long win_first, long long n_win,
                                 long long tokens, float *scratch, long long scratch_size, uint32_t *arrived, void *out, void *stream) {
-    return tq_decode_attend_spread(layer, queries, group, scale, win_first, n_win, tokens, scratch, scratch_size, arrived, layer ? layer->rows : 0, out, stream);
+    return tq_decode_attend_cached(layer, queries, group, scale, win_first, n_win, tokens, scratch, scratch_size, arrived, layer ? layer->rows : 0, 0, out, stream);
 }
 
 extern "C" int tq_decode_append(const tq_decode_layer *layer, const void *k_new, const void *v_new, long long k_new_stride, long long v_new_stride,

@@ -1126,15 +1126,13 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     if (g0 < G) rotate_back(std::integral_constant<int, 4>{}, g0);
 }
 
-// STREAM: what decides is whether the history can still lie in the last-level cache (256 MB) when the next step comes for it.  A layer of 8 MiB is
-// taken for one that does not: 32 of them fill it, and so do the weights that a model reads between two steps.  Read with the
-// non-temporal hint, what is used once no longer drives out what every block of the next launch reads (tables, operands, code), and few rows start and
-// merge sooner.  us a pass without / with it, 128 wide unless stated: 32 layers of 8 x 32768 tokens 669 / 635, 16 of 32 x 6000 at 64 276 / 264, 24
-// of 128 x 4182 642 / 620, 8 of 512 x 16384 1378 / 1355.  Caches that fit lose by it: 32 of 2 x 8738 476 / 484, 16 of 8 x 6289 270 / 280.
+// STREAM (a.stream, see CACHE_STREAMED): the history read with the non-temporal hint.  What is used once then no longer drives out what every block of the next
+// launch reads (tables, operands, code), and few rows start and merge sooner.  us a pass without / with it, 128 wide unless stated: 32 layers of
+// 8 x 32768 tokens 669 / 635, 16 of 32 x 6000 at 64 276 / 264, 24 of 128 x 4182 642 / 620, 8 of 512 x 16384 1378 / 1355.  Norms, and 2-bit keys at 96 (six
+// bytes a lane, in loads of two), are read without it.
 template <int D, int IPBK, int IPBV, int C>
 int launch_decode(dim3 grid, hipStream_t s, const TqDecodeArgs &a) {
-    const uint64_t bytes = (uint64_t)grid.y * a.tokens * (D / IPBK + D / IPBV + 4);
-    if (bytes >= 8u << 20) hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, C, true>), grid, dim3(DTHREADS), 0, s, a);
+    if (a.stream) hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, C, true>), grid, dim3(DTHREADS), 0, s, a);
     else hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, C, false>), grid, dim3(DTHREADS), 0, s, a);
     return (int)hipGetLastError();
 }

@@ -20,7 +20,7 @@
 
 namespace {
 
-constexpr int INTERFACE = 2;      // of this module to _native.py (FAST_INTERFACE there): raised with any change of what init or a function takes or answers
+constexpr int INTERFACE = 3;      // of this module to _native.py (FAST_INTERFACE there): raised with any change of what init or a function takes or answers
 
 PyObject *g_workspace = nullptr, *g_drop_workspace = nullptr;      // _native's: ticket counters of (device, stream)
 PyObject *g_scratch = nullptr, *g_arrived = nullptr;               // _native's: (device index, stream) -> tensor
@@ -33,7 +33,7 @@ struct Entries {
     decltype(&tq_compress_layer) compress_layer;
     decltype(&tq_restore_layer) restore_layer;
     decltype(&tq_decode_append) decode_append;
-    decltype(&tq_decode_attend_spread) decode_attend;
+    decltype(&tq_decode_attend_cached) decode_attend;
     decltype(&tq_qjl_compress) qjl_compress;
     decltype(&tq_qjl_query_scores) qjl_query_scores;
 } lib{};
@@ -368,7 +368,7 @@ PyObject *decode_append(PyObject *const *a) {
     return PyLong_FromLong(rc);
 }
 
-// decode_attend(record, queries, k_win, scale, win_first, n_win, tokens) -> output; scratch and counters of the stream as _native keeps them
+// decode_attend(record, queries, k_win, scale, win_first, n_win, tokens, cache_bytes) -> output; scratch and counters of the stream as _native keeps them
 PyObject *decode_attend(PyObject *const *a) {
     TENSOR(q, a[1]); TENSOR(win, a[2]);
     NEED(win.dim() == 4 && q.dim() == 4 && q.scalar_type() == win.scalar_type() && q.device() == win.device());
@@ -392,7 +392,7 @@ PyObject *decode_attend(PyObject *const *a) {
     NEED(counters.numel() >= rows);
     at::Tensor out = empty(q.sizes(), q.scalar_type(), q);
     const int rc = launch(lib.decode_attend, reinterpret_cast<const tq_decode_layer *>(integer(a[0])), (const void *)address(q), (int)(Hq / H), (float)scale, integer(a[4]), n_win,
-                          integer(a[6]), (float *)address(buf), (long long)buf.numel(), (uint32_t *)address(counters), (long long)counters.numel(), (void *)address(out), s.raw());
+                          integer(a[6]), (float *)address(buf), (long long)buf.numel(), (uint32_t *)address(counters), (long long)counters.numel(), integer(a[7]), (void *)address(out), s.raw());
     NEED(rc == 0);           // (a buffer that is too small, or an argument the library refuses: nothing was launched)
     return THPVariable_Wrap(out);
 }
@@ -485,7 +485,7 @@ PyObject *init(PyObject *, PyObject *args) {
 PyMethodDef methods[] = {
     {"init", &init, METH_VARARGS, nullptr},
     TQ_ENTRY(compress, 3), TQ_ENTRY(decompress, 5), TQ_ENTRY(compress_layer, 7), TQ_ENTRY(restore_layer, 11), TQ_ENTRY(restore_dicts, 13), TQ_ENTRY(restore_store, 13),
-    TQ_ENTRY(decode_append, 7), TQ_ENTRY(decode_attend, 7), TQ_ENTRY(qjl_compress, 4), TQ_ENTRY(qjl_scores, 8),
+    TQ_ENTRY(decode_append, 7), TQ_ENTRY(decode_attend, 8), TQ_ENTRY(qjl_compress, 4), TQ_ENTRY(qjl_scores, 8),
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "tqamd_fastcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

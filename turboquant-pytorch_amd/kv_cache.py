@@ -51,6 +51,9 @@ class _StepConsts(NamedTuple):
 class _LayerStore:
     """Packed history and uncompressed window of one layer."""
 
+    # over all layers of the cache on this device: packed bytes of one token, and bytes of the windows; 0: not known
+    cache_slot_bytes = cache_window_bytes = 0
+
     def __init__(self, comp: TurboQuantV3, B: int, H: int, D: int, dtype: torch.dtype, device: torch.device,
                  capacity: int, window: int):
         self.comp = comp
@@ -89,6 +92,14 @@ class _LayerStore:
     def _width(D: int, bits: int) -> int:
         ipb = 8 // bits
         return -(-D // ipb)
+
+    def slot_bytes(self) -> int:
+        """Packed bytes (codes and norms) of one token over all rows."""
+        return self.B * self.H * (self._width(self.D, self.comp.key_bits) + self._width(self.D, self.comp.value_bits) + 4)
+
+    def cache_bytes(self) -> int:
+        """What a decode step reads of all layers of the cache, taken to be as long as this one (0: not known)."""
+        return self.n_compressed * self.cache_slot_bytes + self.cache_window_bytes
 
     def reserve(self, tokens: int) -> None:
         """Make room for `tokens` compressed tokens per (batch, head) row (amortised doubling)."""
@@ -263,10 +274,20 @@ class V3Cache:
         if st is None:
             st = _LayerStore(comp, B, H, D, key_states.dtype, device, self.capacity, self.residual_window)
             self._stores[layer_idx] = st
+            self._count_slots()
         elif (st.B, st.H, st.D) != (B, H, D):
             raise ValueError(f"layer {layer_idx}: states {tuple(key_states.shape)} do not match the cached "
                              f"batch/head/dim {(st.B, st.H, st.D)}")
         return st
+
+    def _count_slots(self) -> None:
+        """Tells every layer how much all layers on its device hold, by which `attend` chooses the loads of the history (called once per new layer)."""
+        total: Dict[torch.device, Tuple[int, int]] = {}
+        for st in self._stores.values():
+            slots, windows = total.get(st.k_win.device, (0, 0))
+            total[st.k_win.device] = (slots + st.slot_bytes(), windows + 2 * st.B * st.H * st.window_tokens * st.D * st.k_win.element_size())
+        for st in self._stores.values():
+            st.cache_slot_bytes, st.cache_window_bytes = total[st.k_win.device]
 
     def _push(self, st: _LayerStore, key_states: torch.Tensor, value_states: torch.Tensor) -> None:
         """Bookkeeping of generation_test_v2.py:96-126: the uncompressed tokens are (window ++ new); all but
@@ -391,7 +412,8 @@ class V3Cache:
                 packed = (torch.empty((B, st.H, 0, 1), dtype=torch.uint8, device=dev),
                           torch.empty((B, st.H, 0), dtype=torch.float16, device=dev)) * 2
             return _native.call("attend_packed", query_states, *packed, kc.table(), vc.table(),
-                                                 kc.bits, vc.bits, kc.pi_transposed(), vc.Pi, kw, vw, float(scale))
+                                                 kc.bits, vc.bits, kc.pi_transposed(), vc.Pi, kw, vw, float(scale),
+                                                 0 if torch.compiler.is_compiling() else st.cache_bytes())
         # rows padded to a multiple of 8 floats (the kernels read weights with 16-byte loads); the padding
         # scores are -inf, so the softmax runs over the whole contiguous buffer
         q4 = query_states.reshape(B, st.H, G, D).to(torch.float32)
@@ -418,7 +440,8 @@ class V3Cache:
         """The fused path of `attend` in one library call (rotate + window, packed history, merge), with the
         scratch kept per stream.  None when the queries are not laid out for it."""
         if st.one_launch and query_states.is_cuda:
-            out = _native.fast().decode_attend(ctypes.addressof(st.record()), query_states, st.k_win, scale, st.w0, st.n_recent, st.n_compressed)
+            out = _native.fast().decode_attend(ctypes.addressof(st.record()), query_states, st.k_win, scale, st.w0, st.n_recent, st.n_compressed,
+                                               st.cache_bytes())
             if out is not None:
                 return out
         B, Hq, _, D = query_states.shape

@@ -209,4 +209,5 @@ def load_cache(path: str, device="cuda", cls=None):
             st.extend_window(kw, vw)
         st.total_seq = info["total_seq"]
         cache._stores[idx] = st
+    cache._count_slots()
     return cache
