@@ -424,9 +424,11 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
     uint16_t kn_raw, vn_raw;
     // n_tok >= 1: what lies past the last token is read as that token.  One form for whole and partial runs: with a branch between two
     // the registers are merged behind it, and that waits for the loads just issued.
-    auto load16 = [](const uint8_t *p) __attribute__((always_inline)) { return STREAM ? tq_gload16_stream(p) : tq_gload16(p); };
-    auto load8 = [](const uint8_t *p) __attribute__((always_inline)) { return STREAM ? tq_gload8_stream(p) : tq_gload8(p); };
-    auto load4 = [](const uint8_t *p) __attribute__((always_inline)) { return STREAM ? tq_gload4_stream(p) : tq_gload4(p); };
+    constexpr bool KEYS = STREAM && !(IPBK == 1 && (D == 256 || (D == 128 && C == 1)));      // keys streamed as well (see launch_decode)
+    auto load16 = [](const uint8_t *p, auto hint) __attribute__((always_inline)) { return decltype(hint)::value ? tq_gload16_stream(p) : tq_gload16(p); };
+    auto load8 = [](const uint8_t *p, auto hint) __attribute__((always_inline)) { return decltype(hint)::value ? tq_gload8_stream(p) : tq_gload8(p); };
+    constexpr std::integral_constant<bool, KEYS> key_hint{};
+    constexpr std::integral_constant<bool, STREAM> value_hint{};
     auto issue_keys = [&](uint32_t t0, uint32_t n_tok) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < SUB; ++u)
@@ -437,20 +439,20 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
                 if constexpr (KB % 16 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 16; ++p) {
-                        const tq_u4 v = load16(src + 16 * p);
+                        const tq_u4 v = load16(src + 16 * p, key_hint);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) kraw[u][b][4 * p + i] = v[i];
                     }
                 } else if constexpr (KB % 8 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 8; ++p) {
-                        const tq_u2 v = load8(src + 8 * p);
+                        const tq_u2 v = load8(src + 8 * p, key_hint);
                         kraw[u][b][2 * p] = v[0]; kraw[u][b][2 * p + 1] = v[1];
                     }
                 } else if constexpr (KB % 4 == 0) {
 #pragma unroll
                     for (int p = 0; p < KB / 4; ++p)
-                        kraw[u][b][p] = load4(src + 4 * p);
+                        kraw[u][b][p] = KEYS ? tq_gload4_stream(src + 4 * p) : tq_gload4(src + 4 * p);
                 } else {
                     static_assert(KB % 2 == 0, "key bytes of a lane");
                     uint32_t h[KB / 2];
@@ -466,8 +468,8 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
 #pragma unroll
         for (int p = 0; p < NVP; ++p) {
             const uint32_t piece = min(p * 64u + lane, min((uint32_t)VPIECES, n_tok * (GBV / VPB)) - 1u);
-            if constexpr (VPB == 16) vpiece[p] = load16(vsrc + piece * 16u);
-            else { const tq_u2 v = load8(vsrc + piece * 8u); vpiece[p][0] = v[0]; vpiece[p][1] = v[1]; }
+            if constexpr (VPB == 16) vpiece[p] = load16(vsrc + piece * 16u, value_hint);
+            else { const tq_u2 v = load8(vsrc + piece * 8u, value_hint); vpiece[p][0] = v[0]; vpiece[p][1] = v[1]; }
         }
         const uint32_t own = min(lane, n_tok - 1u);       // (lanes past the end: see trip)
         kn_raw = tq_gload2(a.k_norms + slot0 + t0 + own);
@@ -1130,6 +1132,11 @@ __global__ __launch_bounds__(DTHREADS, DW / 4) void tq_decode_kernel(TqDecodeArg
 // launch reads (tables, operands, code), and few rows start and merge sooner.  us a pass without / with it, 128 wide unless stated: 32 layers of
 // 8 x 32768 tokens 669 / 635, 16 of 32 x 6000 at 64 276 / 264, 24 of 128 x 4182 642 / 620, 8 of 512 x 16384 1378 / 1355.  Norms, and 2-bit keys at 96 (six
 // bytes a lane, in loads of two), are read without it.
+// Keys of a byte a code at 256 (KEYS) are read without it too, and so they are at 128 for more than eight heads: a lane takes a line of theirs in several loads with
+// other lines between, and what the hint lets go in the meantime is fetched again.  Time with the hint on keys and values / on values alone, over plain loads:
+// 256 wide, K8/V4, 24 layers of 2 x 13512 tokens 1.044 / 0.957, 8 of 8 x 13512 1.021 / 0.941, 6 of 256 x 1140 1.066 / 0.992; 128 wide, K8/V4, 16 heads, 6 of
+// 256 x 2256 1.036 / 0.967.  With two codes a byte at 256, and with a byte a code at 64 and 96, the keys gain by it as well: 256 wide, K4/V2, 6 of
+// 32 x 18055 0.938 / 0.997, 8 of 128 x 1671 0.902 / 0.989; 64 wide, K8/V4, 16 heads, 6 of 256 x 4423 0.985 / 1.043.
 template <int D, int IPBK, int IPBV, int C>
 int launch_decode(dim3 grid, hipStream_t s, const TqDecodeArgs &a) {
     if (a.stream) hipLaunchKernelGGL((tq_decode_kernel<D, IPBK, IPBV, C, true>), grid, dim3(DTHREADS), 0, s, a);
