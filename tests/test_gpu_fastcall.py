@@ -1,4 +1,6 @@
 """The eager calls in one step (tqamd_fastcall) against the general path behind them, over the forms that either may be given."""
+import ctypes
+
 import pytest
 import torch
 
@@ -244,6 +246,44 @@ def test_outputs_are_recorded_for_the_profiler(pkg):
     x = outlier_kv((1, 2, 70, 128), seed=3, dtype=torch.bfloat16).to(DEV)
     want = (comp.compress(x), layer.compress_kv(x, x))
     for call, outputs in ((lambda: comp.compress(x), 2), (lambda: comp.decompress(want[0]), 1), (lambda: layer.compress_kv(x, x), 4), (lambda: layer.decompress_kv(*want[1]), 2)):
-        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], acc_events=True) as prof:
             call()
         assert sum(e.name.startswith("aten::empty") for e in prof.events()) == outputs, [e.name for e in prof.events()]
+
+
+def test_outputs_are_filled_for_deterministic_algorithms(pkg):
+    """torch fills new memory while algorithms have to be deterministic: a kernel more for every output, seen as nodes of a captured graph."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    comp = pkg.MSECompressor(128, 4, seed=42, device=DEV)
+    x = outlier_kv((1, 2, 70, 128), seed=3, dtype=torch.bfloat16).to(DEV)
+    want = comp.decompress(comp.compress(x))
+    nodes, before = [], torch.are_deterministic_algorithms_enabled()
+    try:
+        for on in (False, True):
+            torch.use_deterministic_algorithms(on)
+            graph = torch.cuda.CUDAGraph(keep_graph=True)
+            with torch.cuda.graph(graph):
+                out = comp.decompress(comp.compress(x))
+            n = ctypes.c_size_t()
+            assert hip.hipGraphGetNodes(graph.raw_cuda_graph(), None, ctypes.byref(n)) == 0
+            nodes.append(n.value)
+            torch.use_deterministic_algorithms(before)
+            for _ in range(3):
+                out.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out, want)
+    finally:
+        torch.use_deterministic_algorithms(before)
+    assert nodes == [2, 2 + 3], nodes
+
+
+def test_decompress_kv_with_shapes_of_floats(pkg):
+    """Shapes whose numbers are floats of the same value: what shapes of integers restore, or what the general path says to them."""
+    comp = pkg.TurboQuantV3(128, key_bits=4, value_bits=2, residual_window=16, layer_idx=8, device=DEV)
+    k = outlier_kv((1, 2, 70, 128), seed=4, dtype=torch.float16).to(DEV)
+    pair = comp.compress_kv(k, k)
+    floats = lambda t: tuple(float(i) for i in t)  # noqa: E731
+    other = [dict(c, shape=floats(c["shape"]), compressed=dict(c["compressed"], shape=floats(c["compressed"]["shape"]))) for c in pair]
+    _same(comp.decompress_kv(*other), comp.decompress_kv(*pair))
