@@ -330,7 +330,8 @@ struct WindowTile {
 // A tile of the window used to stand before the block's barrier: everybody in it waited 2.3 us (256 wide 4.4) for the wave that had it, and the row for the
 // block.  It is finished behind the barrier now; records are merged without loops around their loads.  us a layer, 4 heads, K4/V2: 8 rows x 32768
 // tokens 21.0 -> 20.3; 4 x 6000 16.4 -> 15.0; 64 wide, 32 x 6000 15.8 -> 14.8; 256 wide, 8 x 16384 35.3 -> 33.0.
-// Where the 17 us of a launch of 8 rows x 32768 tokens lie now (clock stamps, medians of the last block): 3.6 until the first tables and operands are
+// Where the 16 us of a launch of 8 rows x 32768 tokens lie now (clock stamps, medians of the last block; together 15.1, the rest is before the first stamp and behind the
+// last): 3.6 until the first tables and operands are
 // there and the barrier is passed, 0.5 the queries' operands, 4.7 two runs a wave (what reading 26 MB takes), 1.0 the 8 tokens over, 1.2 the waves' sums, 0.9 stores and
 // count, 2.3 the records of 32 blocks, 0.9 back through Pi_v.  What moved it last, a layer with its append: counters apart and Pi_v early 21.7 -> 20.9,
 // history past the caches 19.8, products of 16 x 16 and tables in fewer loads 19.3.  (One loop body for whole and partial runs: a trip of it takes
